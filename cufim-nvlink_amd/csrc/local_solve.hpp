@@ -154,7 +154,9 @@ FIM_HD inline T cand_exact(const T g[6], const T ph[4], T inf) {
 // reference update (compat mode, FP64 with the reference's float
 // intermediates), src/eikonal/cuda_fim.h:1256-1411.  Unusable nodes carry
 // DBL_MAX, the reference's "infinity".  Evaluated without FMA contraction so
-// results are bit-identical to the CPU restatement.
+// results are bit-identical to the CPU restatement, and without branches (an
+// invalid configuration is deselected at the end), so that the parts of a
+// candidate, long chains of dependent FP64 operations, run side by side.
 // ---------------------------------------------------------------------------
 FIM_HD inline double tri_ref(double e12, double e13, double e23, double phi1, double phi2) {
 #pragma clang fp contract(off)
@@ -164,21 +166,19 @@ FIM_HD inline double tri_ref(double e12, double e13, double e23, double phi1, do
   const double phi12 = phi2 - phi1;
   float dv = (float)(phi12 * phi12 - c);
   const float sv = (float)((double)dv * (b * b - a * c));
-  if (dv != 0.0 && sv >= 0.0) {
-    dv = (float)(c * (double)dv);
-    const float sq = sqrtf(sv);
-    const double base = b * phi12 * phi12 - b * c;
-    const float l1 = (float)(-(base - (double)sq * phi12) / (double)dv);
-    const float l2 = (float)(-(base + (double)sq * phi12) / (double)dv);
-    float r1 = (float)(phi2 - (double)l1 * phi12 +
-                       sqrt(a + 2.0 * (double)l1 * b + (double)(l1 * l1) * c));
-    if (!((l1 >= 0.0) && (l1 <= 1.0))) r1 = INFINITY;
-    float r2 = (float)(phi2 - (double)l2 * phi12 +
-                       sqrt(a + 2.0 * (double)l2 * b + (double)(l2 * l2) * c));
-    if (!((l2 >= 0.0) && (l2 <= 1.0))) r2 = INFINITY;
-    return (double)fminf(r1, r2);
-  }
-  return DBL_MAX;
+  const bool ok = dv != 0.0f && sv >= 0.0f;
+  dv = (float)(c * (double)dv);
+  const float sq = sqrtf(sv);
+  const double base = b * phi12 * phi12 - b * c;
+  const float l1 = (float)(-(base - (double)sq * phi12) / (double)dv);
+  const float l2 = (float)(-(base + (double)sq * phi12) / (double)dv);
+  const float t1 = (float)(phi2 - (double)l1 * phi12 +
+                           sqrt(a + 2.0 * (double)l1 * b + (double)(l1 * l1) * c));
+  const float t2 = (float)(phi2 - (double)l2 * phi12 +
+                           sqrt(a + 2.0 * (double)l2 * b + (double)(l2 * l2) * c));
+  const float r1 = ((l1 >= 0.0f) & (l1 <= 1.0f)) ? t1 : INFINITY;
+  const float r2 = ((l2 >= 0.0f) & (l2 <= 1.0f)) ? t2 : INFINITY;
+  return ok ? (double)fminf(r1, r2) : DBL_MAX;
 }
 
 // The reference tet candidate evaluates a closed form whose coefficients are
@@ -202,7 +202,6 @@ FIM_HD inline double tet_ref(double e13, double e23, double e34, double e12, dou
       (e * e * c * c - 2. * e * b * c * d + a * c * d * d + (b * b * c - a * c * c) * f) * p23 * p23 +
       2. * (e * c * d * d - b * d * d * d) * e +
       (e * e * c * c + (b * b - 2. * a * c) * d * d - 2. * (e * c * c - b * c * d) * e) * f;
-  if (sqt < 0.) return DBL_MAX;
   const double q1 = e * c * d * d - b * d * d * d + (e * c - b * d) * f * p13 * p13 -
                     2. * (e * c * d - b * d * d) * p13 * p23 +
                     (e * c * c - b * c * d) * p23 * p23 - (e * c * c - b * c * d) * f;
@@ -214,32 +213,41 @@ FIM_HD inline double tet_ref(double e13, double e23, double e34, double e12, dou
   const double m2 = (q1 - sqt * (d * p13 - c * p23)) / q2;
   const double k1 = -((f * m1 + e) * p13 - (d * m1 + b) * p23) / (d * p13 - c * p23);
   const double k2 = -((f * m2 + e) * p13 - (d * m2 + b) * p23) / (d * p13 - c * p23);
-  double w = 1 - k1 - m1, r1 = DBL_MAX, r2 = DBL_MAX;
-  if ((k1 > 0. && k1 < 1.) && (m1 > 0. && m1 < 1.) && w > 0.)
-    r1 = k1 * phi1 + m1 * phi2 + w * phi3 +
-         sqrt(a + 2. * k1 * b + k1 * k1 * c + 2. * k1 * m1 * d + 2. * m1 * e + m1 * m1 * f);
-  w = 1 - k2 - m2;
-  if ((k2 > 0. && k2 < 1.) && (m2 > 0. && m2 < 1.) && w > 0.)
-    r2 = k2 * phi1 + m2 * phi2 + w * phi3 +
-         sqrt(a + 2. * k2 * b + k2 * k2 * c + 2. * k2 * m2 * d + 2. * m2 * e + m2 * m2 * f);
-  return fmin(r1, r2);
+  const double w1 = 1 - k1 - m1, w2 = 1 - k2 - m2;
+  const double t1 = k1 * phi1 + m1 * phi2 + w1 * phi3 +
+                    sqrt(a + 2. * k1 * b + k1 * k1 * c + 2. * k1 * m1 * d + 2. * m1 * e + m1 * m1 * f);
+  const double t2 = k2 * phi1 + m2 * phi2 + w2 * phi3 +
+                    sqrt(a + 2. * k2 * b + k2 * k2 * c + 2. * k2 * m2 * d + 2. * m2 * e + m2 * m2 * f);
+  const bool in1 = (k1 > 0.) & (k1 < 1.) & (m1 > 0.) & (m1 < 1.) & (w1 > 0.);
+  const bool in2 = (k2 > 0.) & (k2 < 1.) & (m2 > 0.) & (m2 < 1.) & (w2 > 0.);
+  const double r = fmin(in1 ? t1 : DBL_MAX, in2 ? t2 : DBL_MAX);
+  return sqt < 0. ? DBL_MAX : r;
 }
 
-// reference candidate for node position t (runtime), after the upwind filter
-FIM_HD inline double cand_ref(const double g[6], const double ph[4], int t) {
+// reference candidate of the target from the other three nodes, relabelled, in
+// two parts of about equal cost: (a) the tet face and triangle 1-3, (b) the
+// other triangles and the edges; the candidate is the smaller
+FIM_HD inline double cand_ref_a(double e12, double e13, double e23, double e14, double e24, double e34, double p1,
+                                double p2, double p3) {
+  return fmin(tet_ref(e13, e23, e34, e12, e14, e24, p1, p2, p3), tri_ref(e13, e14, e34, p1, p3));
+}
+FIM_HD inline double cand_ref_b(double e12, double e23, double e14, double e24, double e34, double p1, double p2,
+                                double p3) {
 #pragma clang fp contract(off)
-  const int q1 = (t + 1) & 3, q2 = (t + 2) & 3, q3 = (t + 3) & 3;
-  const double e13 = g[edge_idx(q1, q3)], e23 = g[edge_idx(q2, q3)], e34 = g[edge_idx(q3, t)];
-  const double e12 = g[edge_idx(q1, q2)], e14 = g[edge_idx(q1, t)], e24 = g[edge_idx(q2, t)];
-  const double p1 = ph[q1], p2 = ph[q2], p3 = ph[q3];
-  double v = tet_ref(e13, e23, e34, e12, e14, e24, p1, p2, p3);
-  v = fmin(v, tri_ref(e12, e14, e24, p1, p2));
-  v = fmin(v, tri_ref(e23, e24, e34, p2, p3));
-  v = fmin(v, tri_ref(e13, e14, e34, p1, p3));
+  double v = fmin(tri_ref(e12, e14, e24, p1, p2), tri_ref(e23, e24, e34, p2, p3));
   v = fmin(v, p1 + sqrt(e14));
   v = fmin(v, p2 + sqrt(e24));
   v = fmin(v, p3 + sqrt(e34));
   return v;
+}
+
+// reference candidate for node position t (runtime), after the upwind filter
+FIM_HD inline double cand_ref(const double g[6], const double ph[4], int t) {
+  const int q1 = (t + 1) & 3, q2 = (t + 2) & 3, q3 = (t + 3) & 3;
+  const double e12 = g[edge_idx(q1, q2)], e13 = g[edge_idx(q1, q3)], e23 = g[edge_idx(q2, q3)];
+  const double e14 = g[edge_idx(q1, t)], e24 = g[edge_idx(q2, t)], e34 = g[edge_idx(q3, t)];
+  return fmin(cand_ref_a(e12, e13, e23, e14, e24, e34, ph[q1], ph[q2], ph[q3]),
+              cand_ref_b(e12, e23, e14, e24, e34, ph[q1], ph[q2], ph[q3]));
 }
 
 }  // namespace fim

@@ -35,6 +35,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <string>
@@ -1362,6 +1363,18 @@ __global__ void k_support_check(const float *phi_g, const uint32_t *best, uint32
 // ---------------------------------------------------------------------------
 // compat mode (reference time windows, FP64)
 // ---------------------------------------------------------------------------
+constexpr uint32_t kNoVertex = 0xffffffffu;
+
+// A submesh of k_compat_small: its constant data is one block of 16-byte
+// words (blob + boff): slot chunk offsets of the copies (nn + 1 u16), node ids
+// of the elements (8 B each), slots (u16, element << 2 | position, each copy's
+// padded to chunks of four with kNoSlot) and, if it is to be in LDS, the FP64
+// geometry (48 B per element).
+struct CompatSub {
+  uint32_t coff, nn, eoff, ne, ioff, boff, nw, nch;  // nw words, nch chunks of slots
+};
+constexpr uint16_t kNoSlot = 0xffffu;
+
 struct CompatArgs {
   const SubInfo *sub;
   const uint2 *e2n;
@@ -1374,12 +1387,21 @@ struct CompatArgs {
   double *phi;
   int8_t *st;
   unsigned long long *stats;  // sweeps, slot evaluations
-  uint32_t *pending;          // copies left narrow/next after the window
   double *nexte;              // per submesh: earliest window time its copies change
+  const uint32_t *list;       // submeshes of this window (k_compat_sync), *nlist of them
+  const uint32_t *nlist;
+  const uint32_t *cshared;    // per copy: its vertex if it has other copies, else kNoVertex
+  uint32_t *vrec, *vcnt;      // per submesh (at ioff): shared vertices whose copy changed, their number
+  unsigned long long *done;   // finished workgroups << 32 | pending copies
+  uint32_t *out;              // pinned host word: copies left narrow/next after the window
   uint32_t nsub;
   int32_t exact;
   double fw, cur, phi_start, dt, apd;
   uint32_t o_tphi, o_st, o_tst, o_snap, o_misc;
+  // k_compat_small
+  const CompatSub *csub;
+  const uint4 *blob;
+  uint32_t o_tmin, o_lp, o_lq, o_blob;
 };
 
 __device__ inline uint32_t block_sum(uint32_t v, uint32_t *slot) {
@@ -1411,6 +1433,34 @@ __device__ inline double block_min0(double v, unsigned long long *slot) {
   if ((threadIdx.x & 63) == 0) atomicMin(slot, dkey(v));
   __syncthreads();
   return threadIdx.x == 0 ? dkey_inv(*slot) : 0.0;
+}
+
+// A workgroup is through with its submeshes (one thread calls this): the last
+// of the min(max(n, 1), gridDim) workgroups that take part knows the window's
+// pending count from the one counter all of them add to, hands it to the host
+// and clears the counter, so a window needs no fill and no copy for it.
+__device__ inline void compat_finish(const CompatArgs &a, uint32_t nlist, uint32_t pend) {
+  const uint32_t part = min(max(nlist, 1u), gridDim.x);
+  if (blockIdx.x >= part) return;
+  const unsigned long long add = (1ull << 32) | pend;
+  const unsigned long long now = atomicAdd(a.done, add) + add;
+  if ((uint32_t)(now >> 32) == part) {
+    __hip_atomic_store(a.out, (uint32_t)now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(a.done, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// Records the shared vertices whose copies (c, of the lanes with `changed`)
+// the pass has changed in the submesh's range of vrec; cnt is one LDS word.
+// Lane 0 of a wave is active whenever another lane is.
+__device__ inline void compat_record(const CompatArgs &a, uint32_t ioff, bool changed, uint32_t c, uint32_t *cnt) {
+  const uint32_t v = changed ? a.cshared[c] : kNoVertex;
+  const uint64_t m = __ballot(v != kNoVertex);
+  if (m == 0) return;
+  uint32_t at = 0;
+  if ((threadIdx.x & 63) == 0) at = atomicAdd(cnt, (uint32_t)__popcll(m));
+  at = __builtin_amdgcn_readfirstlane(at);
+  if (v != kNoVertex) a.vrec[ioff + at + (uint32_t)__popcll(m & lanes_below())] = v;
 }
 
 // one (vertex, element) slot: src/eikonal/cuda_fim.h:1362-1411.  The slot's
@@ -1469,10 +1519,10 @@ __global__ __launch_bounds__(BS) void k_compat_compute(CompatArgs a) {
   const uint32_t tid = threadIdx.x;
   unsigned long long sweeps = 0, slots = 0;
   unsigned long long *evslot = reinterpret_cast<unsigned long long *>(misc + 2);
-  for (uint32_t s = blockIdx.x; s < a.nsub; s += gridDim.x) {
-    // a submesh with nothing narrow or next, whose frozen and tail copies all
-    // stay put at this window time, would come out of the pass unchanged
-    if (a.nexte[s] > a.cur) continue;
+  const uint32_t nlist = *a.nlist;
+  uint32_t pend_wg = 0;  // thread 0
+  for (uint32_t i = blockIdx.x; i < nlist; i += gridDim.x) {
+    const uint32_t s = a.list[i];
     const SubInfo si = a.sub[s];
     const uint32_t nn = si.nn;
     // update_states (cuda_fim.cu:1790-1845), applied to every submesh
@@ -1580,9 +1630,12 @@ __global__ __launch_bounds__(BS) void k_compat_compute(CompatArgs a) {
     const bool lean = idle && nn <= BS;
     uint32_t pend = 0;
     double ev = INFINITY;
+    if (tid == 0) misc[1] = 0u;
+    __syncthreads();
     for (uint32_t l = tid; l < nn; l += BS) {
       const double p = phi_l[l];
       const int8_t st = st_l[l];
+      compat_record(a, si.ioff, !lean || p != p0, si.coff + l, &misc[1]);
       if (!lean || p != p0 || st != st0) {
         a.phi[si.coff + l] = p;
         a.st[si.coff + l] = st;
@@ -1598,33 +1651,349 @@ __global__ __launch_bounds__(BS) void k_compat_compute(CompatArgs a) {
     }
     if (!lean) {
       pend = block_sum(pend, misc);
-      if (tid == 0 && pend) atomicAdd(a.pending, pend);
+      pend_wg += pend;
     }
     ev = block_min0(ev, evslot);
-    if (tid == 0) a.nexte[s] = ev;
+    if (tid == 0) {
+      a.nexte[s] = ev;
+      a.vcnt[s] = misc[1];
+    }
   }
+  if (tid == 0) compat_finish(a, nlist, pend_wg);
   if (tid == 0 && sweeps) atomicAdd(&a.stats[0], sweeps);
   for (int off = 32; off > 0; off >>= 1) slots += __shfl_xor(slots, off);
   if ((tid & 63) == 0 && slots) atomicAdd(&a.stats[1], slots);
 }
 
-// sync_step2 over vertices with several copies
-__global__ void k_compat_sync(const uint32_t *grp_v, uint32_t ngrp, const uint32_t *g2c_dsp,
-                              const uint32_t *g2c, const uint32_t *c2s, double *phi, int8_t *st,
-                              double *nexte) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < ngrp; i += gridDim.x * blockDim.x) {
-    const uint32_t v = grp_v[i];
-    double mn = DBL_MAX;
-    for (uint32_t k = g2c_dsp[v]; k < g2c_dsp[v + 1]; ++k) {
-      const double c = phi[g2c[k]];
-      if (c < mn) mn = c;
+// geometry index of e12 e13 e23 e14 e24 e34 after relabelling for target t
+// (3 bits each, e12 lowest)
+__device__ inline uint32_t compat_relabel(int t) {
+  constexpr auto pack = [](int t) {
+    const int q1 = (t + 1) & 3, q2 = (t + 2) & 3, q3 = (t + 3) & 3;
+    return (uint32_t)(edge_idx(q1, q2) | edge_idx(q1, q3) << 3 | edge_idx(q2, q3) << 6 | edge_idx(q1, t) << 9 |
+                      edge_idx(q2, t) << 12 | edge_idx(q3, t) << 15);
+  };
+  constexpr uint32_t r0 = pack(0), r1 = pack(1), r2 = pack(2), r3 = pack(3);
+  return t & 2 ? (t & 1 ? r3 : r2) : (t & 1 ? r1 : r0);
+}
+
+// The window's pass for submeshes of at most BS copies: one thread per copy
+// keeps the copy's time and states in registers, the submesh's (vertex,
+// element) slots, node ids and (GEO) FP64 geometry are in LDS for all sweeps
+// of the window.  The pass is a chain of short sweeps, so what a sweep costs
+// is its latency: barriers, memory round trips and rounds of the ~3,000-cycle
+// FP64 candidate.  Here
+//   - a phase's slots are appended to an LDS list by the threads that decide
+//     on them, four at a time, so a candidate round has live lanes and no slot
+//     is looked at in vain (the scan of every slot cost most of a sweep);
+//   - `up` holds the time a copy offers to others (DBL_MAX if it may not act),
+//     so a slot reads three words and no states;
+//   - the downwind neighbours of just-frozen copies are found through the
+//     elements (copies are neighbours when they share one);
+//   - a sweep in which nothing froze has two barriers, any other six;
+//   - the submesh's data comes straight into LDS, in flight together with the
+//     copies' times, so a submesh waits for memory three times in all.
+// Full slab, 10,152 submeshes of at most 128 copies, 150 windows of 2 ms: a
+// map takes 11.7 ms against 25.0 with the general kernel (k_compat_compute)
+// and the sync over all shared vertices; the pass 46 us per window against
+// 109.  Workgroups of 256 beat 128 (12.8 ms) and 512 (13.2 ms); registers for
+// five waves per SIMD spill (13.0 ms); submeshes taken from a counter instead
+// of in turn gain nothing (11.9 ms).
+template <int BS, bool GEO>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_compat_small(CompatArgs a) {
+#pragma clang fp contract(off)
+  extern __shared__ __align__(16) unsigned char lds[];
+  double *phi_l = reinterpret_cast<double *>(lds);
+  double *up = reinterpret_cast<double *>(lds + a.o_tphi);
+  unsigned long long *tmin = reinterpret_cast<unsigned long long *>(lds + a.o_tmin);
+  int8_t *st_l = reinterpret_cast<int8_t *>(lds + a.o_st);
+  uint2 *lp = reinterpret_cast<uint2 *>(lds + a.o_lp);  // slot chunks of narrow copies
+  uint2 *lq = reinterpret_cast<uint2 *>(lds + a.o_lq);  // slot chunks of marked neighbours
+  uint4 *blob = reinterpret_cast<uint4 *>(lds + a.o_blob);
+  // misc: [0,1] chunks in lp (by sweep parity), [2] chunks in lq, [4,5]
+  // block_min0's slot, [6] shared vertices recorded, [8..] just-frozen bits,
+  // [8 + BS / 32 ..] marked-neighbour bits
+  uint32_t *misc = reinterpret_cast<uint32_t *>(lds + a.o_misc);
+  uint32_t *fz = misc + 8, *mk = fz + BS / 32;
+  unsigned long long *evslot = reinterpret_cast<unsigned long long *>(misc + 4);
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t l = tid;
+  const double lo = a.phi_start - a.fw;
+  const uint32_t nlist = *a.nlist;
+  uint32_t s = a.list[blockIdx.x];  // gridDim <= nsub entries; read with nlist
+  unsigned long long sweeps = 0, slots = 0;
+  uint32_t pend_wg = 0;  // thread 0
+  auto offer = [&](int8_t st, double p) { return (st >= FIM_NARROW && p > lo) ? p : DBL_MAX; };
+  for (uint32_t i = blockIdx.x; i < nlist; i += gridDim.x) {
+    if (i != blockIdx.x) s = a.list[i];
+    const CompatSub si = a.csub[s];
+    const uint32_t nn = si.nn, ne = si.ne;
+    const bool own = l < nn;
+    const uint16_t *dsp = reinterpret_cast<const uint16_t *>(blob);
+    const uint2 *el = reinterpret_cast<const uint2 *>(blob + (2 * (nn + 1) + 15) / 16);
+    const uint2 *sw = reinterpret_cast<const uint2 *>(reinterpret_cast<const uint4 *>(el) + (8 * ne + 15) / 16);
+    const double *gl = reinterpret_cast<const double *>(reinterpret_cast<const uint4 *>(sw) + (8 * si.nch + 15) / 16);
+    // chunks of the slots of copy v appended to a list
+    auto append = [&](uint2 *list, uint32_t *cnt, uint32_t v) {
+      const uint32_t b = dsp[v], n = dsp[v + 1] - b, at = atomicAdd(cnt, n);
+      for (uint32_t k = 0; k < n; k += 3) {
+        const uint2 w0 = sw[b + k], w1 = sw[b + min(k + 1, n - 1)], w2 = sw[b + min(k + 2, n - 1)];
+        list[at + k] = w0;
+        list[at + min(k + 1, n - 1)] = w1;
+        list[at + min(k + 2, n - 1)] = w2;
+      }
+    };
+    // the submesh's block into LDS: a wave's 64 lanes take 64 consecutive words
+    for (uint32_t k0 = tid & ~63u; k0 < si.nw; k0 += BS)
+      if (k0 + lane < si.nw)
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const __attribute__((address_space(1))) uint32_t *>(
+                reinterpret_cast<uintptr_t>(a.blob + si.boff + k0 + lane)),
+            (__attribute__((address_space(3))) uint32_t *)(blob + k0), 16, 0, 0);
+    // update_states (cuda_fim.cu:1790-1845)
+    double p = DBL_MAX, p0 = 0.0;
+    int8_t st = FIM_FAR, st0 = FIM_FAR;
+    if (own) {
+      p = a.phi[si.coff + l];
+      st = a.st[si.coff + l];
+      p0 = p;
+      st0 = st;
+      if (st == FIM_NEXT) {
+        st = FIM_NARROW;
+      } else if (st == FIM_FROZEN) {
+        if (!(p + a.apd > a.cur)) st = FIM_TAIL;
+      } else if (st == FIM_TAIL) {
+        if (!(p + a.apd / 0.91 > a.cur)) {
+          p = DBL_MAX;
+          st = FIM_FAR;
+        }
+      }
     }
-    for (uint32_t k = g2c_dsp[v]; k < g2c_dsp[v + 1]; ++k) {
-      const uint32_t c = g2c[k];
-      if (mn < phi[c]) {
-        phi[c] = mn;
-        st[c] = FIM_NARROW;
-        nexte[c2s[c]] = -INFINITY;
+    if (tid < 8) misc[tid] = 0u;
+    if (tid < 2 * (BS / 32)) fz[tid] = 0u;
+    if (own) {
+      phi_l[l] = p;
+      up[l] = offer(st, p);
+      st_l[l] = st;
+      tmin[l] = kDmaxBits;
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the block is in LDS
+    __syncthreads();
+    if (own && st == FIM_NARROW) append(lp, &misc[0], l);
+    {
+      // candidates of the listed slots: times are >= 0, so the minimum of the
+      // FP64 bit patterns as integers is the minimum of the values.  A slot's
+      // reference candidate is worked out by two lanes of different waves
+      // (the tet face and a triangle; two triangles and the edges): half the
+      // chain, at half the slots per round.
+      auto evaluate = [&](const uint2 *chunks, uint32_t nch) {
+        const uint16_t *list = reinterpret_cast<const uint16_t *>(chunks);
+        const uint32_t n = 4 * nch;
+        const bool split = !a.exact && BS > 64;
+        const bool second = split && tid >= BS / 2;
+        for (uint32_t j = second ? tid - BS / 2 : tid; j < n; j += split ? BS / 2 : BS) {
+          const uint32_t w = list[j], le = w >> 2;
+          if (w == kNoSlot) continue;
+          const int t = (int)(w & 3u);
+          const uint2 q = el[le];
+          const unsigned long long nd = (unsigned long long)q.y << 32 | q.x;
+          auto node = [&](int k) { return (uint32_t)(nd >> (16 * (k & 3))) & 0xffffu; };
+          const double p1 = up[node(t + 1)], p2 = up[node(t + 2)], p3 = up[node(t + 3)];
+          const double *g = GEO ? gl + 6 * le : a.geo + 6 * ((size_t)si.eoff + le);
+          const uint32_t ix = compat_relabel(t);
+          const double e12 = g[ix & 7u], e13 = g[(ix >> 3) & 7u], e23 = g[(ix >> 6) & 7u], e14 = g[(ix >> 9) & 7u],
+                       e24 = g[(ix >> 12) & 7u], e34 = g[ix >> 15];
+          double v;
+          if (a.exact)
+            v = cand_core<double>(e12, e13, e23, e14, e24, e34, p1, p2, p3, DBL_MAX);
+          else if (!split)
+            v = fmin(cand_ref_a(e12, e13, e23, e14, e24, e34, p1, p2, p3),
+                     cand_ref_b(e12, e23, e14, e24, e34, p1, p2, p3));
+          else if (second)
+            v = cand_ref_b(e12, e23, e14, e24, e34, p1, p2, p3);
+          else
+            v = cand_ref_a(e12, e13, e23, e14, e24, e34, p1, p2, p3);
+          atomicMin(&tmin[node(t)], (unsigned long long)__double_as_longlong(v));
+        }
+        slots += n;
+      };
+      for (uint32_t par = 0;; par ^= 1u) {
+        __syncthreads();
+        const uint32_t n = misc[par];
+        if (n == 0) break;  // uniform
+        ++sweeps;
+        // a: candidates of narrow copies
+        evaluate(lp, n);
+        __syncthreads();
+        // b: reduce, window test, convergence test; a copy that stays narrow
+        // is listed for the next sweep
+        bool froze = false;
+        int8_t prev = FIM_FAR;  // state before being marked (c)
+        if (own && st == FIM_NARROW) {
+          const double c = __longlong_as_double((long long)tmin[l]), old = p;
+          const double nw = c < old ? c : old;
+          tmin[l] = kDmaxBits;
+          p = nw;
+          phi_l[l] = nw;
+          if (nw - a.phi_start > a.dt) {
+            st = FIM_NEXT;
+            st_l[l] = st;
+          } else if (fabs(old - nw) < (1e-6 * (1 + (old + nw) * .5))) {
+            froze = true;
+          } else {
+            append(lp, &misc[par ^ 1u], l);
+          }
+          up[l] = offer(st, p);
+        }
+        const uint64_t fm = __ballot(froze);
+        if (lane == 0) {
+          fz[tid >> 5] = (uint32_t)fm;
+          if (BS > 32) fz[(tid >> 5) + 1] = (uint32_t)(fm >> 32);
+        }
+        __syncthreads();
+        if (tid == 0) misc[par] = 0u;  // every thread has read it
+        uint32_t any = 0;
+#pragma unroll
+        for (int k = 0; k < BS / 32; ++k) any |= fz[k];
+        if (any == 0u) continue;  // uniform
+        // c: copies that are not narrow and lie downwind of a just-frozen
+        // neighbour are marked
+        for (uint32_t e = tid; e < ne; e += BS) {
+          const uint2 q = el[e];
+          const uint32_t nd[4] = {q.x & 0xffffu, q.x >> 16, q.y & 0xffffu, q.y >> 16};
+          double first = DBL_MAX;  // earliest just-frozen node
+          bool f = false;
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (flag_at(fz, nd[k])) {
+              f = true;
+              first = fmin(first, phi_l[nd[k]]);
+            }
+          if (!f) continue;
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (st_l[nd[k]] != FIM_NARROW && first < phi_l[nd[k]]) atomicOr(&mk[nd[k] >> 5], 1u << (nd[k] & 31u));
+        }
+        __syncthreads();
+        // d: candidates of marked copies (a marked copy offers nothing)
+        const bool marked = own && flag_at(mk, l);
+        if (marked) {
+          prev = st;
+          up[l] = DBL_MAX;
+          append(lq, &misc[2], l);
+        }
+        __syncthreads();
+        const uint32_t nq = misc[2];
+        if (nq) {  // uniform
+          evaluate(lq, nq);
+          __syncthreads();
+        }
+        // e, f: accept improvements; freeze
+        if (froze) {
+          st = FIM_FROZEN;
+          st_l[l] = st;
+          up[l] = offer(st, p);
+        }
+        if (marked) {
+          const double c = __longlong_as_double((long long)tmin[l]), old = p;
+          tmin[l] = kDmaxBits;
+          const double nw = c < old ? c : old;
+          p = nw;
+          phi_l[l] = nw;
+          st = prev;
+          if (nw < old) {
+            // accepted; a copy that was frozen freezes again (phase f)
+            st = prev == FIM_FROZEN ? (int8_t)FIM_FROZEN : (int8_t)FIM_NARROW;
+            if (st == FIM_NARROW) append(lp, &misc[par ^ 1u], l);
+          }
+          st_l[l] = st;
+          up[l] = offer(st, p);
+          atomicAnd(&mk[l >> 5], ~(1u << (l & 31u)));
+        }
+        if (tid == 0) misc[2] = 0u;
+      }
+    }
+    // write back what changed; ev: the earliest window time at which
+    // update_states would change a copy (frozen: p + apd, tail: p + apd /
+    // 0.91, as update_states computes them; narrow or next: now)
+    bool pend = false;
+    double ev = INFINITY;
+    compat_record(a, si.ioff, own && p != p0, si.coff + l, &misc[6]);
+    if (own) {
+      if (p != p0) a.phi[si.coff + l] = p;
+      if (st != st0) a.st[si.coff + l] = st;
+      pend = st == FIM_NARROW || st == FIM_NEXT;
+      if (pend)
+        ev = -INFINITY;
+      else if (st == FIM_FROZEN)
+        ev = p + a.apd;
+      else if (st == FIM_TAIL)
+        ev = p + a.apd / 0.91;
+    }
+    pend_wg += (uint32_t)__syncthreads_count(pend);
+    ev = block_min0(ev, evslot);
+    if (tid == 0) {
+      a.nexte[s] = ev;
+      a.vcnt[s] = misc[6];
+    }
+  }
+  if (tid == 0) {
+    compat_finish(a, nlist, pend_wg);
+    if (sweeps) atomicAdd(&a.stats[0], sweeps);
+    if (slots) atomicAdd(&a.stats[1], slots);
+  }
+}
+
+// Start of a window.  sync_step2 (min over the copies of each shared vertex)
+// and the list of submeshes the window's pass has to run on: those whose
+// copies' own clocks are due (nexte; -inf when something is narrow or next)
+// and those a shared vertex was lowered in.  A submesh left out would come out
+// of the pass unchanged: nothing narrow or next, and its frozen and tail
+// copies all stay put at this window time.
+// The copies of a vertex are equal after a sync and a seed sets all of them,
+// so only the vertices that the last window's pass recorded can differ: one
+// wave per submesh of that window's list goes through its records.  A vertex
+// recorded by several submeshes is merged by each of them: all find the same
+// minimum and write nothing else.
+struct CompatSyncArgs {
+  const SubInfo *sub;
+  const uint32_t *last, *nlast;  // the last window's list
+  const uint32_t *vrec, *vcnt;
+  const uint32_t *g2c_dsp, *g2c, *c2s;
+  double *phi;
+  int8_t *st;
+  const double *nexte;
+  uint32_t nsub;
+  double cur;
+  uint32_t *list, *cnt, *next_cnt;  // this window's list; the next one's count, cleared
+  uint32_t *mark, stamp;            // mark[s] == stamp: s is on this window's list
+};
+
+__global__ __launch_bounds__(256) void k_compat_sync(CompatSyncArgs a) {
+  auto queue = [&](uint32_t s) {
+    if (a.mark[s] != a.stamp && atomicExch(&a.mark[s], a.stamp) != a.stamp) a.list[atomicAdd(a.cnt, 1u)] = s;
+  };
+  const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+  if (t0 == 0) *a.next_cnt = 0u;
+  for (uint32_t s = t0; s < a.nsub; s += nt)
+    if (!(a.nexte[s] > a.cur)) queue(s);
+  const uint32_t nlast = *a.nlast;
+  for (uint32_t i = t0 >> 6; i < nlast; i += nt >> 6) {
+    const uint32_t s = a.last[i], n = a.vcnt[s], off = a.sub[s].ioff;
+    for (uint32_t r = threadIdx.x & 63; r < n; r += 64) {
+      const uint32_t v = a.vrec[off + r], b = a.g2c_dsp[v], e = a.g2c_dsp[v + 1];
+      double mn = DBL_MAX;
+      for (uint32_t k = b; k < e; ++k) {
+        const double c = a.phi[a.g2c[k]];
+        if (c < mn) mn = c;
+      }
+      for (uint32_t k = b; k < e; ++k) {
+        const uint32_t c = a.g2c[k];
+        if (mn < a.phi[c]) {
+          a.phi[c] = mn;
+          a.st[c] = FIM_NARROW;
+          queue(a.c2s[c]);
+        }
       }
     }
   }
@@ -1665,6 +2034,16 @@ T *dalloc(size_t n, std::vector<void *> &owned) {
   return static_cast<T *>(p);
 }
 
+// f(begin, end) over [0, n) on up to eight host threads
+template <class F>
+void parallel_ranges(size_t n, F &&f) {
+  const size_t nt = std::max<size_t>(1, std::min<size_t>({8, (size_t)std::thread::hardware_concurrency(), n / 512}));
+  std::vector<std::thread> ts;
+  for (size_t t = 1; t < nt; ++t) ts.emplace_back([&, t] { f(n * t / nt, n * (t + 1) / nt); });
+  f(0, n / nt);
+  for (auto &t : ts) t.join();
+}
+
 template <class T>
 T *dupload(const std::vector<T> &v, std::vector<void *> &owned) {
   T *p = dalloc<T>(v.size(), owned);
@@ -1702,8 +2081,7 @@ struct fim_ctx {
   float4 *d_hgt = nullptr;
   double *d_geo64 = nullptr;
   uint8_t *d_ereg = nullptr;
-  uint32_t *d_c2g = nullptr, *d_c2s = nullptr, *d_g2c_dsp = nullptr, *d_g2c = nullptr, *d_grp = nullptr;
-  uint32_t ngrp = 0;
+  uint32_t *d_c2g = nullptr, *d_c2s = nullptr, *d_g2c_dsp = nullptr, *d_g2c = nullptr;
   uint16_t *d_if_l = nullptr;
   uint4 *d_if_fo = nullptr;
   uint2 *d_if_os = nullptr;
@@ -1735,10 +2113,19 @@ struct fim_ctx {
   double *d_phi64 = nullptr;
   int8_t *d_st = nullptr;
   double *d_nexte = nullptr;  // per submesh: earliest window time a copy changes
-  uint32_t *d_pending = nullptr;
+  // submesh lists of this and the last window (by parity), their counts
+  // (three in rotation), the stamps of the last window that listed a submesh,
+  // the pass's end counter and its records of changed shared vertices
+  uint32_t *d_list = nullptr, *d_lcnt = nullptr, *d_mark = nullptr;
+  CompatSub *d_csub = nullptr;
+  uint4 *d_blob = nullptr;
+  uint32_t *d_cshared = nullptr, *d_vrec = nullptr, *d_vcnt = nullptr;
+  unsigned long long *d_done = nullptr;
+  uint32_t stamp = 0;
+  bool compat_small = false, compat_geo = false;  // k_compat_small, with geometry in LDS
   // shared
   unsigned long long *d_stats = nullptr;
-  uint32_t *h_pin = nullptr;
+  uint32_t *h_pin = nullptr, *d_pin = nullptr;  // pinned host words and their device address
   // seed staging: pinned host and device buffers of (instance, copy) pairs
   uint2 *h_seed = nullptr, *d_seed = nullptr;
   size_t seed_cap = 0;
@@ -1817,27 +2204,27 @@ const void *conv_kernel_ptr(bool staged, int block, int wpe, bool pairs) {
 void set_lds_attr(fim_ctx *c) {
   const void *f = conv_kernel_ptr(c->o.staged != 0, c->block, c->band_wpe, c->band_pairs);
   HIPCHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_conv));
-  const void *g = nullptr;
+}
+
+const void *compat_kernel_ptr(const fim_ctx *c) {
+  const bool geo = c->compat_geo;
+  if (c->compat_small) switch (c->block) {
+      case 64: return geo ? (const void *)k_compat_small<64, true> : (const void *)k_compat_small<64, false>;
+      case 128: return geo ? (const void *)k_compat_small<128, true> : (const void *)k_compat_small<128, false>;
+      case 512: return geo ? (const void *)k_compat_small<512, true> : (const void *)k_compat_small<512, false>;
+      default: return geo ? (const void *)k_compat_small<256, true> : (const void *)k_compat_small<256, false>;
+    }
   switch (c->block) {
-    case 64: g = (const void *)k_compat_compute<64>; break;
-    case 128: g = (const void *)k_compat_compute<128>; break;
-    case 512: g = (const void *)k_compat_compute<512>; break;
-    default: g = (const void *)k_compat_compute<256>; break;
+    case 64: return (const void *)k_compat_compute<64>;
+    case 128: return (const void *)k_compat_compute<128>;
+    case 512: return (const void *)k_compat_compute<512>;
+    default: return (const void *)k_compat_compute<256>;
   }
-  HIPCHECK(hipFuncSetAttribute(g, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_compat));
 }
 
 void launch_compat_compute(fim_ctx *c, const CompatArgs &a) {
-  // 8192 workgroups: more submeshes in flight than 4096 (-4 % per window on
-  // the slab's 10,162), no further gain from one workgroup per submesh
-  const int grid = (int)std::min<uint32_t>(c->nsub, 8192u);
-  switch (c->block) {
-    case 64: k_compat_compute<64><<<grid, 64, c->lds_compat, c->stream>>>(a); break;
-    case 128: k_compat_compute<128><<<grid, 128, c->lds_compat, c->stream>>>(a); break;
-    case 512: k_compat_compute<512><<<grid, 512, c->lds_compat, c->stream>>>(a); break;
-    default: k_compat_compute<256><<<grid, 256, c->lds_compat, c->stream>>>(a); break;
-  }
-  HIPCHECK(hipGetLastError());
+  void *args[] = {const_cast<CompatArgs *>(&a)};
+  HIPCHECK(hipLaunchKernel(compat_kernel_ptr(c), dim3(c->grid), dim3(c->block), args, c->lds_compat, c->stream));
 }
 
 int blocks_for(size_t n, int bs) { return (int)std::max<size_t>(1, std::min<size_t>((n + bs - 1) / bs, 65536)); }
@@ -2071,6 +2458,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
       c->d_g2c = dupload(p.g2c, ow);
       c->d_stats = dalloc<unsigned long long>(8, ow);
       HIPCHECK(hipHostMalloc((void **)&c->h_pin, 64, hipHostMallocDefault));
+      HIPCHECK(hipHostGetDevicePointer((void **)&c->d_pin, c->h_pin, 0));
       c->d_tmpu = dalloc<uint32_t>(4, ow);
       HIPCHECK(hipMemset(c->d_stats, 0, 8 * sizeof(unsigned long long)));
       if (o->mode == FIM_MODE_CONVERGE) {
@@ -2260,28 +2648,107 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->lds_compat = o_misc + 16;
         if (c->lds_compat > 160 * 1024)
           throw Error(FIM_ELIMIT, "largest submesh too large for compat mode LDS");
-        c->d_geo64 = dupload(p.geo64, ow);
-        c->d_grp = dupload(p.grp_v, ow);
-        c->ngrp = (uint32_t)p.grp_v.size();
-        c->d_n2e_dsp = dupload(p.n2e_dsp, ow);
-        c->d_n2e_le = dupload(p.n2e_le, ow);
-        c->d_n2e_pos = dupload(p.n2e_pos, ow);
-        c->d_n2n_dsp = dupload(p.n2n_dsp, ow);
-        c->d_n2n_lv = dupload(p.n2n_lv, ow);
+        const uint32_t s_tmin = 2 * al16(8 * nn), s_st = s_tmin + al16(8 * nn);
+        const uint32_t s_misc = s_st + al16(nn), s_blob = s_misc + al16(32 + 2 * 4 * ((uint32_t)c->block / 32));
+        uint32_t chunks = 0, words = 0, gwords = 0;  // largest submesh
+        std::vector<CompatSub> cs(p.nsub);
+        for (int64_t q = 0; q < p.nsub; ++q) {
+          const SubInfo &si = p.sub[q];
+          uint32_t nch = 0;
+          for (uint32_t l = 0; l < si.nn; ++l) nch += (p.n2e_dsp[si.coff + l + 1] - p.n2e_dsp[si.coff + l] + 3) / 4;
+          const uint32_t w = (2 * (si.nn + 1) + 15) / 16 + (8 * si.ne + 15) / 16 + (8 * nch + 15) / 16;
+          cs[q] = CompatSub{si.coff, si.nn, si.eoff, si.ne, si.ioff, 0u, w, nch};
+          chunks = std::max(chunks, nch);
+          words = std::max(words, w);
+          gwords = std::max(gwords, w + 3 * si.ne);
+        }
+        // k_compat_small needs a thread per copy and its data in LDS; 40 KB
+        // leave a CU the four workgroups that its registers admit.  Without
+        // the geometry in LDS (submeshes of 256 copies, say) it comes from L2.
+        const uint32_t lists = 2 * al16(8 * chunks);
+        constexpr uint32_t kSmallLds = 40 * 1024;
+        c->compat_small = nn <= (uint32_t)c->block && (uint32_t)c->ne_max < (kNoSlot >> 2) && chunks < (1u << 16) &&
+                          s_blob + 16 * words + lists <= kSmallLds;
+        c->compat_geo = c->compat_small && s_blob + 16 * gwords + lists <= kSmallLds;
+        const uint32_t s_lp = s_blob + 16 * (c->compat_geo ? gwords : words), s_lq = s_lp + al16(8 * chunks);
+        if (c->compat_small) {
+          c->lds_compat = s_blob + 16 * (c->compat_geo ? gwords : words) + lists;
+          size_t total = 0;
+          for (CompatSub &q : cs) {
+            if (c->compat_geo) q.nw += 3 * q.ne;
+            q.boff = (uint32_t)total;
+            total += q.nw;
+          }
+          if (total >= (1ull << 32)) throw Error(FIM_ELIMIT, "submesh blocks above 2^32 words");
+          std::unique_ptr<void, void (*)(void *)> mem(std::malloc(16 * std::max<size_t>(total, 1)), std::free);
+          if (!mem) throw std::bad_alloc();
+          uint4 *blob = static_cast<uint4 *>(mem.get());
+          parallel_ranges((size_t)p.nsub, [&](size_t b, size_t e) {
+            for (size_t i = b; i < e; ++i) {
+              const CompatSub &q = cs[i];
+              const size_t nd = (2 * (q.nn + 1) + 15) / 16, nel = (8 * q.ne + 15) / 16, nsl = (8 * q.nch + 15) / 16;
+              uint16_t *d = reinterpret_cast<uint16_t *>(blob + q.boff), *en = d + 8 * nd, *sl = en + 8 * nel;
+              blob[q.boff + nd - 1] = blob[q.boff + nd + nel - 1] = blob[q.boff + nd + nel + nsl - 1] =
+                  make_uint4(0u, 0u, 0u, 0u);  // the sections' ends
+              std::memcpy(en, &p.e2n_l[4 * (size_t)q.eoff], 8 * (size_t)q.ne);
+              uint32_t ch = 0;
+              for (uint32_t l = 0; l < q.nn; ++l) {
+                const uint32_t kb = p.n2e_dsp[q.coff + l], n = p.n2e_dsp[q.coff + l + 1] - kb;
+                d[l] = (uint16_t)ch;
+                for (uint32_t k = 0; k < (n + 3) / 4 * 4; ++k)
+                  sl[4 * ch + k] = k < n ? (uint16_t)(p.n2e_le[kb + k] << 2 | p.n2e_pos[kb + k]) : kNoSlot;
+                ch += (n + 3) / 4;
+              }
+              d[q.nn] = (uint16_t)ch;
+              if (c->compat_geo) std::memcpy(sl + 8 * nsl, &p.geo64[6 * (size_t)q.eoff], 48 * (size_t)q.ne);
+            }
+          });
+          c->d_csub = dupload(cs, ow);
+          c->d_blob = dalloc<uint4>(total, ow);
+          HIPCHECK(hipMemcpy(c->d_blob, blob, 16 * total, hipMemcpyHostToDevice));
+        }
+        if (!c->compat_geo) c->d_geo64 = dupload(p.geo64, ow);
+        if (!c->compat_small) {
+          c->d_n2e_dsp = dupload(p.n2e_dsp, ow);
+          c->d_n2e_le = dupload(p.n2e_le, ow);
+          c->d_n2e_pos = dupload(p.n2e_pos, ow);
+          c->d_n2n_dsp = dupload(p.n2n_dsp, ow);
+          c->d_n2n_lv = dupload(p.n2n_lv, ow);
+        }
         c->d_phi64 = dalloc<double>(c->ncopy, ow);
         c->d_st = dalloc<int8_t>(c->ncopy, ow);
-        c->d_pending = dalloc<uint32_t>(1, ow);
         c->d_nexte = dalloc<double>(c->nsub, ow);
+        c->d_list = dalloc<uint32_t>(2 * (size_t)c->nsub, ow);
+        c->d_mark = dalloc<uint32_t>(c->nsub, ow);
+        c->d_lcnt = dalloc<uint32_t>(3, ow);
+        {
+          std::vector<uint32_t> cs(p.ncopy, kNoVertex);
+          for (uint32_t v : p.grp_v)
+            for (uint32_t k = p.g2c_dsp[v]; k < p.g2c_dsp[v + 1]; ++k) cs[p.g2c[k]] = v;
+          c->d_cshared = dupload(cs, ow);
+        }
+        c->d_vrec = dalloc<uint32_t>(p.if_l.size(), ow);
+        c->d_vcnt = dalloc<uint32_t>(c->nsub, ow);
+        c->d_done = dalloc<unsigned long long>(1, ow);
+        HIPCHECK(hipMemset(c->d_mark, 0, sizeof(uint32_t) * c->nsub));
+        HIPCHECK(hipMemset(c->d_done, 0, sizeof(unsigned long long)));
+        HIPCHECK(hipFuncSetAttribute(compat_kernel_ptr(c), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)c->lds_compat));
+        int ncu = 256, per_cu = 0;
+        HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->dev));
+        HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, compat_kernel_ptr(c), c->block, c->lds_compat));
+        c->grid = (int)std::min<uint32_t>(c->nsub, (uint32_t)(ncu * std::max(per_cu, 1)));
         c->d_tmpd = dalloc<double>(c->nn, ow);
         c->d_tmpi = dalloc<int32_t>(c->nn, ow);
         c->lds_conv = 0;
         c->xa = CompatArgs{c->d_sub, c->d_e2n, c->d_geo64, c->d_n2e_dsp, c->d_n2e_le, c->d_n2e_pos,
                            c->d_n2n_dsp, c->d_n2n_lv, c->d_phi64, c->d_st, c->d_stats,
-                           c->d_pending, c->d_nexte, c->nsub, o->local == FIM_LOCAL_EXACT ? 1 : 0,
-                           0, 0, 0, 0, o->apd > 0 ? o->apd : 3e5,
-                           o_tphi, o_st, o_tst, o_snap, o_misc};
+                           c->d_nexte, nullptr, nullptr, c->d_cshared, c->d_vrec, c->d_vcnt,
+                           c->d_done, c->d_pin, c->nsub,
+                           o->local == FIM_LOCAL_EXACT ? 1 : 0, 0, 0, 0, 0, o->apd > 0 ? o->apd : 3e5,
+                           o_tphi, c->compat_small ? s_st : o_st, o_tst, o_snap,
+                           c->compat_small ? s_misc : o_misc, c->d_csub, c->d_blob, s_tmin, s_lp, s_lq, s_blob};
       }
-      set_lds_attr(c);
       HIPCHECK(hipStreamSynchronize(c->stream));
       *out = c;
     } catch (...) {
@@ -2314,7 +2781,8 @@ int fim_reset(fim_ctx *c) {
     } else {
       k_fill<double><<<blocks_for(c->ncopy, 256), 256, 0, c->stream>>>(c->d_phi64, c->ncopy, DBL_MAX);
       k_fill<int8_t><<<blocks_for(c->ncopy, 256), 256, 0, c->stream>>>(c->d_st, c->ncopy, (int8_t)FIM_FAR);
-      k_fill<double><<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>(c->d_nexte, c->nsub, -INFINITY);
+      k_fill<double><<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>(c->d_nexte, c->nsub, INFINITY);
+      k_fill<uint32_t><<<1, 64, 0, c->stream>>>(c->d_lcnt, 3, 0u);
     }
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(c->stream));
@@ -2439,18 +2907,23 @@ int fim_step(fim_ctx *c, double phi_start, double cur_time, double dt, double fr
     if (c->o.mode != FIM_MODE_COMPAT) throw Error(FIM_ESTATE, "fim_step needs compat mode");
     HIPCHECK(hipSetDevice(c->dev));
     HIPCHECK(hipEventRecord(c->ev0, c->stream));
-    if (c->ngrp)
-      k_compat_sync<<<blocks_for(c->ngrp, 256), 256, 0, c->stream>>>(
-          c->d_grp, c->ngrp, c->d_g2c_dsp, c->d_g2c, c->d_c2s, c->d_phi64, c->d_st, c->d_nexte);
-    k_fill<uint32_t><<<1, 64, 0, c->stream>>>(c->d_pending, 1, 0u);
+    const uint32_t stamp = ++c->stamp;
+    uint32_t *list = c->d_list + (stamp & 1u) * (size_t)c->nsub, *last = c->d_list + ((stamp & 1u) ^ 1u) * (size_t)c->nsub;
+    const CompatSyncArgs sy{c->d_sub, last, c->d_lcnt + (stamp + 2) % 3, c->d_vrec, c->d_vcnt, c->d_g2c_dsp, c->d_g2c,
+                            c->d_c2s, c->d_phi64, c->d_st, c->d_nexte, c->nsub, cur_time, list,
+                            c->d_lcnt + stamp % 3, c->d_lcnt + (stamp + 1) % 3, c->d_mark, stamp};
+    // a wave for every submesh the last window can have listed, up to 8 waves per SIMD
+    k_compat_sync<<<std::min<int>(blocks_for((size_t)c->nsub * 64, 256), 2048), 256, 0, c->stream>>>(sy);
+    HIPCHECK(hipGetLastError());
     CompatArgs a = c->xa;
+    a.list = list;
+    a.nlist = c->d_lcnt + stamp % 3;
     a.fw = front_width;
     a.cur = cur_time;
     a.phi_start = phi_start;
     a.dt = dt;
     launch_compat_compute(c, a);
     HIPCHECK(hipEventRecord(c->ev1, c->stream));
-    HIPCHECK(hipMemcpyAsync(c->h_pin, c->d_pending, 4, hipMemcpyDeviceToHost, c->stream));
     HIPCHECK(hipStreamSynchronize(c->stream));
     float ms = 0;
     HIPCHECK(hipEventElapsedTime(&ms, c->ev0, c->ev1));

@@ -85,6 +85,66 @@ def test_compat_box_rcb_partition():
     assert np.array_equal(phi, ophi)
 
 
+@pytest.mark.parametrize("block,max_nn", [(64, 64), (128, 96), (256, 128), (256, 256), (512, 300),
+                                          (64, 128), (256, 700)])
+def test_compat_submesh_kernels_bit_identical(block, max_nn):
+    """the thread-per-copy pass (copies <= block; geometry in LDS or not; one
+    wave, so a slot's candidate is not split over two) and the general pass
+    (copies > block), through re-entry (tail, far) and with shared vertices
+    lowered from outside: bit-identical to the oracle"""
+    cfg = dict(cases.SLAB, nx=17, ny=13, nz=5, lx=17e3, ly=13e3, lz=5e3)
+    m, om = cases.box(cfg, seed=5)
+    p = F.Pack(m, F.PART_RCB, max_nn=max_nn, seed=3)
+    e2s, _ = p.partition()
+    om = O.Mesh(om.xyz, om.e2n, fib=om.fib, vel=om.vel, atags=e2s.astype(np.int32))
+    dt, apd, steps = 2e3, 20e3, 45
+    stims = [(1, 0.0, [0, 700]), (1, 61e3, [5])]
+    s = F.Solver(p, mode=F.MODE_COMPAT, local=F.LOCAL_REF, apd=apd, block=block)
+    fw = m.front_width()
+    for _ in range(2):  # the second time through fim_reset in the middle of the state
+        s.reset()
+        cur = 0.0
+        for _ in range(steps):
+            ps = cur
+            cur += dt
+            for active, tstart, vtx in stims:
+                if active and ps <= tstart < cur:
+                    s.seed(vtx, tstart)
+            left = s.step(ps, cur, dt, fw)
+    phi, st = s.download()
+    s.close()
+    ophi, ost, _ = O.compat_solve(om, stims, dt, steps, apd=apd, front_width=fw, timed=True)
+    assert np.array_equal(st, ost)
+    assert np.array_equal(phi, ophi)
+    assert left >= np.sum((st == F.NARROW) | (st == F.NEXT))  # copies against vertices
+
+
+@pytest.mark.parametrize("block,max_nn", [(64, 64), (256, 256), (64, 128)])
+def test_compat_submesh_kernels_exact_candidates(block, max_nn):
+    """the same passes with the exact local update, against the oracle's
+    windows with that update (the windows are not a fixed-point solve; its
+    FP64 arithmetic differs from the device's by contraction only; bound 1e-4
+    of the latest time)"""
+    cfg = dict(cases.SLAB, nx=17, ny=13, nz=5, lx=17e3, ly=13e3, lz=5e3)
+    m, om = cases.box(cfg, seed=5)
+    p = F.Pack(m, F.PART_RCB, max_nn=max_nn, seed=3)
+    e2s, _ = p.partition()
+    om = O.Mesh(om.xyz, om.e2n, fib=om.fib, vel=om.vel, atags=e2s.astype(np.int32))
+    s = F.Solver(p, mode=F.MODE_COMPAT, local=F.LOCAL_EXACT, block=block)
+    fw = 1e9  # every earlier time may act: no upwind cut
+    s.reset()
+    s.seed([0], 0.0)
+    cur = 0.0
+    for _ in range(60):
+        s.step(cur, cur + 2e3, 2e3, fw)
+        cur += 2e3
+    phi, _ = s.download()
+    s.close()
+    ref, _, _ = O.compat_solve(om, [(1, 0.0, [0])], 2e3, 60, front_width=fw, variant=O.LOCAL_EXACT)
+    assert ref.max() < 1e50
+    assert np.max(np.abs(phi - ref)) <= 1e-4 * ref.max()
+
+
 def _converge(m, pack, sources, **kw):
     s = F.Solver(pack, **kw)
     s.seed(sources, 0.0)
