@@ -94,6 +94,10 @@ struct Pack {
   std::vector<float> hgt32;        // 4 per element: metric height of each node
                                    // above its opposite face, rounded down
   std::vector<double> geo64;       // 6 per element
+  std::vector<uint8_t> bnd8;       // 12 per element: for each node as target, lower bounds
+                                   // n . (x_target - x_i) of the other three nodes for a unit
+                                   // direction n, (byte - 128) * scale
+  std::vector<float> bnd_scale;    // 1 per element
   std::vector<uint8_t> ereg;       // 1 per element
   std::vector<uint32_t> c2g;       // per copy
   std::vector<uint32_t> c2s;       // per copy
@@ -117,7 +121,7 @@ Pack build_pack(const Mesh &m, const Partition &p, int32_t source);
 
 // element-list entries the converge-mode band kernel keeps per pass (more
 // marked elements take further passes)
-constexpr int32_t kElistCap = 2048;
+constexpr int32_t kElistCap = 2032;
 
 // dynamic LDS bytes the converge-mode kernel needs for the largest submesh
 int64_t converge_lds_bytes(int32_t nn_max, int32_t ne_max);

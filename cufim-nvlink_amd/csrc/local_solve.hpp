@@ -9,6 +9,7 @@
 
 #include <cfloat>
 #include <cmath>
+#include <cstdint>
 
 #ifndef FIM_HD
 #ifdef __HIPCC__
@@ -148,6 +149,41 @@ FIM_HD inline T cand_exact(const T g[6], const T ph[4], T inf) {
   return cand_core<T>(g[edge_idx(q1, q2)], g[edge_idx(q1, q3)], g[edge_idx(q2, q3)],
                       g[edge_idx(q1, TP)], g[edge_idx(q2, TP)], g[edge_idx(q3, TP)], ph[q1], ph[q2],
                       ph[q3], inf);
+}
+
+// Lower bounds of the exact candidates of an element's four targets (host; the
+// kernel skips targets that they show to be hopeless).  With u_i = x_T - x_i
+// (metric inner product) and any unit vector n, a candidate sum l_i p_i + |x_T -
+// sum l_i x_i| (l_i >= 0, sum 1) is at least min_i (p_i + n . u_i).  n points
+// here from the centroid of the opposite face to the target.  b[3 T + j] is
+// the product for node T + 1 + j (mod 4) as a byte, (byte - 128) * scale, rounded
+// down after a margin of 1e-4 |u_i| that lies far above the rounding of the
+// products and of the FP32 candidates.  A face whose centroid (almost) meets
+// the target gives no direction: -|u_i|.
+inline void cand_bounds(const double geo[6], uint8_t b[12], float *scale) {
+  double hi = 0.0, v[12], top = 0.0;
+  for (int k = 0; k < 6; ++k) hi = std::fmax(hi, geo[k]);
+  for (int t = 0; t < 4; ++t) {
+    const int q[3] = {(t + 1) & 3, (t + 2) & 3, (t + 3) & 3};
+    double s[3], ss = 0.0;  // u_a . (u_1 + u_2 + u_3), |u_1 + u_2 + u_3|^2
+    for (int a = 0; a < 3; ++a) {
+      s[a] = 0.0;
+      for (int c = 0; c < 3; ++c)
+        s[a] += a == c ? geo[edge_idx(q[a], t)]
+                       : 0.5 * (geo[edge_idx(q[a], t)] + geo[edge_idx(q[c], t)] - geo[edge_idx(q[a], q[c])]);
+      ss += s[a];
+    }
+    for (int a = 0; a < 3; ++a) {
+      const double len = std::sqrt(std::fmax(geo[edge_idx(q[a], t)], 0.0));
+      v[3 * t + a] = (ss > 1e-6 * hi ? s[a] / std::sqrt(ss) : -len) - 1e-4 * len;
+      top = std::fmax(top, std::fabs(v[3 * t + a]));
+    }
+  }
+  *scale = (float)(top / 127.0 * (1.0 + 1e-6));
+  for (int a = 0; a < 12; ++a) {
+    const double x = *scale > 0.0f ? std::floor(v[a] / *scale) + 128.0 : 0.0;
+    b[a] = (uint8_t)std::fmin(255.0, std::fmax(0.0, x));
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -4,8 +4,10 @@
 #include <cmath>
 #include <map>
 #include <numeric>
+#include <thread>
 
 #include "host.hpp"
+#include "local_solve.hpp"
 
 namespace fim {
 
@@ -189,7 +191,7 @@ int64_t converge_lds_bytes(int32_t nn_max, int32_t ne_max) {
   // same carve as the default converge-mode kernel: vertex times and
   // candidate minima (2 x f32 per vertex, rounded to 64), four vertex
   // bitmasks, two element bitmasks, element list (u16), source list (u16),
-  // 8 counters and 4 region factors, interface-copy bits and entry counts
+  // 8 counters, 4 region factors, 4 launch counters, interface-copy bits and entry counts
   auto al = [](int64_t x) { return (x + 15) & ~int64_t(15); };
   const int64_t nn64 = (nn_max + 63) & ~int64_t(63);
   const int64_t ne32 = (ne_max + 31) / 32;
@@ -197,7 +199,21 @@ int64_t converge_lds_bytes(int32_t nn_max, int32_t ne_max) {
   // four waves of a workgroup of 256: at least 4 x 320 u16)
   return 2 * al(4 * nn64) + 4 * al(4 * (nn64 / 32)) + 2 * al(4 * ne32) +
          al(2LL * std::min<int64_t>(ne_max, kElistCap)) +
-         al(std::max<int64_t>(2 * nn64, ne_max < (1 << 14) ? 2560 : 0)) + 48 + 2 * al(4 * (nn64 / 32));
+         al(std::max<int64_t>(2 * nn64, ne_max < (1 << 14) ? 2560 : 0)) + 80 + 2 * al(4 * (nn64 / 32));
+}
+
+static void element_bounds(Pack &k) {
+  k.bnd8.resize(12 * (size_t)k.ne_global);
+  k.bnd_scale.resize((size_t)k.ne_global);
+  auto run = [&](int64_t b, int64_t e) {
+    for (int64_t i = b; i < e; ++i) cand_bounds(&k.geo64[6 * i], &k.bnd8[12 * i], &k.bnd_scale[i]);
+  };
+  const int64_t nt = std::max<int64_t>(1, std::min<int64_t>({8, (int64_t)std::thread::hardware_concurrency(),
+                                                             k.ne_global / 4096}));
+  std::vector<std::thread> ts;
+  for (int64_t t = 1; t < nt; ++t) ts.emplace_back(run, k.ne_global * t / nt, k.ne_global * (t + 1) / nt);
+  run(0, k.ne_global / nt);
+  for (auto &t : ts) t.join();
 }
 
 Pack build_pack(const Mesh &m, const Partition &p, int32_t source) {
@@ -284,6 +300,7 @@ Pack build_pack(const Mesh &m, const Partition &p, int32_t source) {
     }
     for (int64_t l = 0; l < nn_s; ++l) g2l[p.l2g[p.s_vdsp[s] + l]] = -1;
   }
+  element_bounds(k);
   // global vertex -> copies, ascending submesh
   k.g2c_dsp.assign(m.nn + 1, 0);
   for (int64_t c = 0; c < k.ncopy; ++c) k.g2c_dsp[k.c2g[c] + 1]++;

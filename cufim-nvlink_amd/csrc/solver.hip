@@ -12,14 +12,15 @@
 //    elements evaluate exact candidates from 48-byte element records read
 //    from L2, and candidates merge with LDS atomicMin on the float bit
 //    pattern (times are >= 0, so the IEEE order equals the unsigned order).
-//    A work item writes its lowered interface copies as (entry, time)
-//    records into its own slot range and a descriptor (item, record count)
-//    into its work-unit slot (no global atomics); a second kernel
-//    (k_conv_sync), one wave per item slot, pushes them to the other copies
-//    of the vertex with global atomicMin, marks those dirty and queues their
-//    submesh on the next list; a third (k_conv_plan) cuts the next list into
-//    work units.  The kernels read only their own list, so results are
-//    independent of scheduling (atomic min and "set" flags commute).  Each
+//    At its end a work item pushes its lowered interface copies to the other
+//    copies of the vertex: global atomicMin into the copy's inbox entry of the
+//    next iteration, whose work item merges it when it stages the submesh,
+//    and the submesh is queued on the next list.  Inbox, queue flags and wake
+//    times exist twice, for even and odd iterations: a kernel reads one set
+//    and writes the other, so results are independent of scheduling (atomic
+//    min, max and "set" flags commute).  With more instances than a work
+//    unit holds, a second kernel (k_conv_plan) cuts the next list into work
+//    units; otherwise an iteration is one launch.  Each
 //    instance's time window counts from its own start iteration, so a
 //    converged instance can be recycled and seeded again mid-run.
 //    Iterations are captured in a hipGraph; the host reads one counter per
@@ -86,116 +87,38 @@ struct WorkList {
   uint32_t *bcnt;   // nsub: queued instances per submesh
   uint32_t *bins;   // nsub x ninst instance ids
   uint32_t *plan;   // work units
-  uint32_t *cnt;    // [0] units, [1] queued pairs, [2..9] per-XCD unit counters
-  uint2 *desc;      // push descriptors, slot u * unit + q for item q of unit u:
-                    // (instance * nsub + submesh, push records; 0 = none)
+  uint32_t *cnt;    // [0] units, [1] queued pairs, [2..9] per-XCD unit counters,
+                    // [10] number of the iteration that works through the list
 };
 
 constexpr uint32_t kXcd = 8;
+constexpr uint32_t kIterWord = 10;
 
-__device__ inline void enqueue(const WorkList &l, uint32_t *act, uint32_t inst, uint32_t s,
-                               uint32_t nsub, uint32_t ninst) {
-  if (atomicExch(&act[(size_t)inst * nsub + s], 1u) == 0u) {
+// Queue flags of the items of iteration k: act = 4 (k + 1) + why, so a flag
+// needs no clearing; kPushed outranks kQueued.
+constexpr uint32_t kQueued = 1, kPushed = 2;
+__device__ inline uint32_t act_tag(uint32_t iter) { return 4u * (iter + 1u); }
+
+// Where items are queued: a list and its iteration's queue flags.
+struct Queue {
+  WorkList l;
+  uint32_t *act;    // n_inst x nsub
+  uint32_t tag;     // act_tag of the list's iteration
+  uint32_t nsub, ninst;
+  uint32_t direct;  // a bucket is one work unit: planned by its first item
+
+  // for kernels between iterations: the list's own iteration number tells the
+  // flags' parity and tag
+  __device__ void enter() {
+    const uint32_t iter = l.cnt[kIterWord];
+    act += (iter & 1u) * (size_t)ninst * nsub;
+    tag = act_tag(iter);
+  }
+  __device__ void add(uint32_t inst, uint32_t s, uint32_t why) const {
+    if (atomicMax(&act[(size_t)inst * nsub + s], tag + why) >= tag) return;
     const uint32_t j = atomicAdd(&l.bcnt[s], 1u);
     l.bins[(size_t)s * ninst + j] = inst;
-  }
-}
-
-// A work item queues itself for the next iteration.  Its act flag was
-// cleared when the item started and only the item's own workgroup can set
-// it before the iteration's sync kernel runs, so no exchange is needed.
-__device__ inline void requeue(const WorkList &l, uint32_t *act, uint32_t inst, uint32_t s,
-                               uint32_t nsub, uint32_t ninst) {
-  act[(size_t)inst * nsub + s] = 1u;
-  const uint32_t j = atomicAdd(&l.bcnt[s], 1u);
-  l.bins[(size_t)s * ninst + j] = inst;
-}
-
-// Every item of a list leaves its push descriptor in its unit slot
-// (instance * nsub + submesh, push records of its activation, 0 if none), so
-// the interface push finds an item's records with one load.
-__device__ inline void push_descriptor(const WorkList &l, uint32_t slot, size_t entry, uint32_t n) {
-  l.desc[slot] = make_uint2((uint32_t)entry, n);
-}
-
-struct UnitRange {
-  uint32_t b, e, nb;  // units [b, e); nb workgroups of the grid run on this XCD
-};
-
-__device__ inline UnitRange xcd_range(uint32_t U, uint32_t y, uint32_t G) {
-  UnitRange r;
-  r.b = (uint32_t)(((uint64_t)U * y) / kXcd);
-  r.e = (uint32_t)(((uint64_t)U * (y + 1)) / kXcd);
-  r.nb = G > y ? (G - y + kXcd - 1) / kXcd : 0u;
-  return r;
-}
-
-// Iterates the (instance, submesh) pairs of a list for one workgroup; every
-// thread of the workgroup calls next() together.  `slot` is one LDS word.
-struct UnitCursor {
-  const uint32_t *bcnt, *bins, *plan;
-  uint32_t *grab;
-  uint32_t *slot;
-  uint32_t U, G, x, y, d, ninst, unit, maxch;
-  UnitRange R;
-  uint32_t s, base, n_in, i;
-  uint32_t uidx = 0;  // unit of the current item
-  uint2 *desc;
-  bool first;
-
-  __device__ UnitCursor(const WorkList &l, uint32_t *lds_slot, uint32_t ninst_, uint32_t unit_,
-                        uint32_t maxch_)
-      : bcnt(l.bcnt), bins(l.bins), plan(l.plan), grab(l.cnt + 2), slot(lds_slot), U(l.cnt[0]),
-        G(gridDim.x), x(blockIdx.x % kXcd), y(blockIdx.x % kXcd), d(0), ninst(ninst_),
-        unit(unit_), maxch(maxch_), s(0), base(0), n_in(0), i(0), desc(l.desc), first(true) {
-    R = xcd_range(U, x, G);
-  }
-
-  __device__ bool next(uint32_t &inst, uint32_t &sub) {
-    if (++i < n_in) {
-      inst = bins[base + i];
-      sub = s;
-      return true;
-    }
-    for (;;) {
-      uint32_t u;
-      if (first) {
-        u = R.b + blockIdx.x / kXcd;
-        first = false;
-      } else {
-        // dynamic units follow the R.nb static ones; a plain read of the
-        // counter skips exhausted eighths without an atomic
-        if (threadIdx.x == 0) {
-          const uint32_t dyn = R.b + R.nb;
-          uint32_t v = 0xffffffffu;
-          if (dyn < R.e &&
-              dyn + __hip_atomic_load(&grab[y], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < R.e)
-            v = dyn + atomicAdd(&grab[y], 1u);
-          *slot = v;
-        }
-        __syncthreads();
-        u = *slot;
-        __syncthreads();
-      }
-      if (u < R.e) {
-        const uint32_t pu = plan[u];
-        s = pu / maxch;
-        const uint32_t j = pu - s * maxch;
-        n_in = min(unit, bcnt[s] - j * unit);
-        base = s * ninst + j * unit;
-        i = 0;
-        uidx = u;
-        // slots of a partial unit that no item fills
-        if (threadIdx.x == 0)
-          for (uint32_t q = n_in; q < unit; ++q) desc[u * unit + q] = make_uint2(0u, 0u);
-        inst = bins[base];
-        sub = s;
-        return true;
-      }
-      if (++d == kXcd) return false;
-      y = (x + d) % kXcd;
-      R = xcd_range(U, y, G);
-    }
+    if (direct && j == 0) l.plan[atomicAdd(&l.cnt[0], 1u)] = s;
   }
 };
 
@@ -266,26 +189,28 @@ struct ConvArgs {
   const float *rscale;   // n_inst x 4 geometry multipliers (1/s^2)
   float *phi;            // n_inst x ncopy
   uint8_t *dirty;        // n_inst x ncopy
-  uint32_t *act;         // n_inst x nsub
-  float *wake;           // n_inst x nsub: lower bound of the dirty vertex times
+  uint32_t *act;         // 2 x n_inst x nsub: queue flags, by iteration parity
+  float *wown;           // n_inst x nsub: earliest time the item left dirty
+  float *wpush;          // 2 x n_inst x nsub: earliest time pushed to the item
   const uint16_t *if_l;  // per interface entry: local copy id
   const uint2 *ifm;      // per submesh, wps words: interface-copy bits of 32
                          // local copies and the interface entries before them
-  uint2 *prec;           // push records (entry, time bits): instance i,
-                         // submesh s use [i * n_if + ioff(s), + ni(s))
+  uint32_t *inbox;       // 2 x n_inst x n_if: earliest time pushed to an interface copy
+  const uint4 *if_fo;    // per entry: first other copy, its submesh, its entry,
+  const uint4 *if_os;    // index + 1 in if_os of the next other copy (0 = none)
   WorkList cur;          // work list of this iteration
   WorkList nxt;          // work list of the next iteration (requeues)
   unsigned long long *stats;  // activations, sweeps, element evaluations,
                               // iterations, algorithmic bytes
-  const uint32_t *iter;  // global iteration counter (advanced by the sync kernel)
+  uint32_t *old_cnt;     // counters of the list of the last iteration
   const uint32_t *start; // n_inst: iteration an instance was (re)seeded at; its
                          // window is window * (iter - start + 1)
   const uint32_t *n2e_dsp;  // per copy: incident local elements (staged kernel)
   const uint16_t *n2e_le;
-  const uint4 *erec;        // band kernel: 48 B per element (ElemRecord layout)
+  const uint4 *erec;        // band kernel: 48 B per element (below)
   const uint32_t *adj_ptr;  // band kernel: per copy, chunk offset << 6 | chunk count
   const uint4 *adj;         // 8 incident local element ids (u16) per chunk, 0xffff padded
-  uint32_t nsub, ncopy, ninst;
+  uint32_t nsub, ncopy, ninst, direct;
   float eps;
   const float *winst;    // n_inst: time window added per global iteration of
                          // each instance (us), 0 = off (plain FIM order)
@@ -297,36 +222,244 @@ struct ConvArgs {
   uint32_t o_phin, o_flg, o_tch, o_dfr, o_e2n, o_geo, o_list, o_vlist, o_misc, o_wrt, o_ifc;
 };
 
-// Writes the interface copies lowered by this activation (bits in tch) as
-// push records into the item's slot range and, when there are any, the
-// item's push descriptor into its list; the entries are found through the
-// interface list (if_l).  Every thread of the workgroup calls it; cnt is one
-// LDS word.
-template <int BS>
-__device__ inline void push_lowered_scan(const ConvArgs &a, const SubInfo &si, uint32_t inst,
-                                         size_t entry, uint32_t dslot, const uint32_t *tch,
-                                         const float *phi_l, uint32_t *cnt) {
-  const uint32_t tid = threadIdx.x, lane = tid & 63;
-  if (tid == 0) *cnt = 0u;
-  __syncthreads();
-  uint2 *rec = a.prec + (size_t)inst * a.n_if + si.ioff;
-  for (uint32_t j0 = 0; j0 < si.ni; j0 += BS) {
-    const uint32_t j = j0 + tid;
-    uint32_t l = 0;
-    bool p = false;
-    if (j < si.ni) {
-      l = a.if_l[si.ioff + j];
-      p = flag_at(tch, l);
+// The kernel's arguments where they lie (scalar loads from the constant
+// segment).  The empty asm makes every call a pointer of its own, so that what
+// a phase reads through it is loaded in that phase: held from the kernel's
+// start, 50 pointers and counts do not fit the scalar registers and were
+// spilled to lanes of vector registers (800 v_readlane in a kernel that is
+// bound by vector issue).
+using KArgs = const __attribute__((address_space(4))) ConvArgs *;
+__device__ inline KArgs kargs() {
+  KArgs k = (KArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  return k;
+}
+
+struct UnitRange {
+  uint32_t b, e, nb;  // units [b, e); nb workgroups of the grid run on this XCD
+};
+
+__device__ inline UnitRange xcd_range(uint32_t U, uint32_t y, uint32_t G) {
+  UnitRange r;
+  r.b = (uint32_t)(((uint64_t)U * y) / kXcd);
+  r.e = (uint32_t)(((uint64_t)U * (y + 1)) / kXcd);
+  r.nb = G > y ? (G - y + kXcd - 1) / kXcd : 0u;
+  return r;
+}
+
+// Iterates the (instance, submesh) pairs of a list for one workgroup; every
+// thread of the workgroup calls next() together.  `slot` is one LDS word.
+struct UnitCursor {
+  uint32_t s = 0, base = 0, n_in = 0, i = 0;
+  bool first = true;
+
+  // a further unit from the eighths' counters (own eighth first), U if none is
+  // left.  The first wave looks at all eight at once: one round trip for the
+  // workgroup that finds nothing (one after the other took 6 us, at the end of
+  // every launch); when no eighth has more units than workgroups, none.
+  __device__ static uint32_t fetch(const uint32_t *cnt, uint32_t U, uint32_t *slot) {
+    const uint32_t G = gridDim.x;
+    if ((U + kXcd - 1) / kXcd <= G / kXcd) return U;
+    if (threadIdx.x < 64) {
+      uint32_t *grab = const_cast<uint32_t *>(cnt) + 2;
+      const uint32_t y = (blockIdx.x + threadIdx.x) % kXcd;
+      const UnitRange R = xcd_range(U, y, G);
+      const uint32_t dyn = R.b + R.nb;
+      uint32_t got = U;
+      for (;;) {
+        // a plain read of the counter skips exhausted eighths without an atomic
+        const bool open = threadIdx.x < kXcd && dyn < R.e &&
+                          dyn + __hip_atomic_load(&grab[y], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < R.e;
+        const uint64_t m = __ballot(open);
+        if (m == 0) break;
+        const int w = __ffsll((unsigned long long)m) - 1;
+        if ((int)threadIdx.x == w) {
+          const uint32_t v = dyn + atomicAdd(&grab[y], 1u);
+          if (v < R.e) got = v;
+        }
+        got = __shfl(got, w);
+        if (got < U) break;
+      }
+      if (threadIdx.x == 0) *slot = got;
     }
-    const uint64_t m = __ballot(p);
-    if (m == 0) continue;  // uniform across the wave
-    uint32_t wb = 0;
-    if (lane == 0) wb = atomicAdd(cnt, (uint32_t)__popcll(m));
-    wb = __shfl(wb, 0);
-    if (p) rec[wb + __popcll(m & lanes_below())] = make_uint2(si.ioff + j, __float_as_uint(phi_l[l]));
+    __syncthreads();
+    const uint32_t v = *slot;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(v);
+  }
+
+  __device__ bool next(uint32_t &inst, uint32_t &sub, uint32_t *slot) {
+    const KArgs k = kargs();
+    if (++i < n_in) {
+      inst = k->cur.bins[base + i];
+      sub = s;
+      return true;
+    }
+    const uint32_t U = k->cur.cnt[0];
+    uint32_t u = U;
+    if (first) {
+      first = false;
+      const UnitRange R = xcd_range(U, blockIdx.x % kXcd, gridDim.x);
+      u = R.b + blockIdx.x / kXcd;
+      if (u >= R.e) u = fetch(k->cur.cnt, U, slot);
+    } else {
+      if (k->direct) {  // no plan kernel clears the bucket
+        __syncthreads();  // every thread has read its count
+        if (threadIdx.x == 0) k->cur.bcnt[s] = 0u;
+      }
+      u = fetch(k->cur.cnt, U, slot);
+    }
+    if (u >= U) return false;
+    const uint32_t pu = k->cur.plan[u], maxch = k->maxch, unit = k->unit;
+    s = maxch == 1 ? pu : pu / maxch;
+    const uint32_t j = pu - s * maxch;
+    n_in = min(unit, k->cur.bcnt[s] - j * unit);
+    base = s * k->ninst + j * unit;
+    i = 0;
+    inst = k->cur.bins[base];
+    sub = s;
+    return true;
+  }
+};
+
+// Start of a kernel of iteration k: the next iteration's number, and, where no
+// plan kernel sets them, the counters of the list that was worked through in
+// iteration k - 1 and is filled in k + 1.  Returns k.
+__device__ inline uint32_t start_iteration() {
+  const KArgs k = kargs();
+  const uint32_t iter = k->cur.cnt[kIterWord];
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) {
+      k->nxt.cnt[kIterWord] = iter + 1u;
+      if (k->cur.cnt[0] > 0) atomicAdd(&k->stats[3], 1ull);
+    }
+    if (k->direct && threadIdx.x < kIterWord) k->old_cnt[threadIdx.x] = 0u;
+  }
+  return iter;
+}
+
+__device__ inline Queue next_queue(KArgs k, uint32_t iter) {
+  return Queue{WorkList{k->nxt.bcnt, k->nxt.bins, k->nxt.plan, k->nxt.cnt},
+               k->act + ((iter + 1u) & 1u) * (size_t)k->ninst * k->nsub, act_tag(iter + 1u), k->nsub, k->ninst,
+               k->direct};
+}
+
+// Pushes the time v of interface entry e (instance inst) to the vertex's other
+// copies, for the next iteration.  A copy's time only falls, so a stale read
+// of it (its item may run now) lets at most a useless push through, and the
+// smallest push to a copy is always below what it reads; min, max and flags
+// commute, so the merged times do not depend on any order.
+__device__ inline void push_entry(KArgs k, const Queue &nq, uint32_t inst, uint32_t e, uint32_t v,
+                                  uint32_t iter) {
+  const uint32_t par = (iter + 1u) & 1u;
+  const uint32_t *phi = reinterpret_cast<const uint32_t *>(k->phi) + (size_t)inst * k->ncopy;
+  uint32_t *inbox = k->inbox + ((size_t)par * k->ninst + inst) * k->n_if;
+  uint32_t *wpush = reinterpret_cast<uint32_t *>(k->wpush) + ((size_t)par * k->ninst + inst) * k->nsub;
+  const uint32_t *act = nq.act + (size_t)inst * k->nsub;
+  uint4 o = k->if_fo[e];  // most entries have one other copy
+  for (;;) {
+    // three reads in flight together
+    const uint32_t cur = __hip_atomic_load(phi + o.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t wcur = __hip_atomic_load(wpush + o.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t queued = __hip_atomic_load(act + o.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v < cur) {
+      __hip_atomic_fetch_min(inbox + o.z, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (v < wcur) __hip_atomic_fetch_min(wpush + o.y, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (queued < nq.tag + kPushed) nq.add(inst, o.y, kPushed);
+    }
+    if (o.w == 0u) break;
+    o = k->if_os[o.w - 1u];
+  }
+}
+
+// One item as it is taken from the list.
+struct Item {
+  bool pushed;    // something was pushed to it
+  float own;      // earliest time it left dirty itself
+  float wake;     // nothing in it can act before this time
+};
+
+// its place in wpush and act of iteration iter's parity; its inbox entries
+__device__ inline size_t item_parity(KArgs k, uint32_t inst, uint32_t s, uint32_t iter) {
+  return ((iter & 1u) * (size_t)k->ninst + inst) * k->nsub + s;
+}
+__device__ inline size_t item_inbox(KArgs k, uint32_t ioff, uint32_t inst, uint32_t iter) {
+  return ((iter & 1u) * (size_t)k->ninst + inst) * k->n_if + ioff;
+}
+
+__device__ inline Item take_item(KArgs k, uint32_t inst, uint32_t s, uint32_t iter) {
+  Item t;
+  const size_t pe = item_parity(k, inst, s, iter);
+  t.own = k->wown[(size_t)inst * k->nsub + s];
+  const float wp = k->wpush[pe];
+  t.pushed = (k->act[pe] & 3u) == kPushed;
+  t.wake = fminf(t.own, wp);
+  return t;
+}
+
+// End of an item: the earliest time it left dirty itself; one thread.
+__device__ inline void end_item(KArgs k, const Queue &nq, uint32_t inst, uint32_t s, uint32_t iter, bool pushed,
+                                float wake) {
+  k->wown[(size_t)inst * k->nsub + s] = wake;
+  if (pushed) k->wpush[item_parity(k, inst, s, iter)] = F_INF;
+  if (wake < F_INF) nq.add(inst, s, kQueued);
+}
+
+// An item that cannot act in this iteration stays queued.  What was pushed to
+// it goes into the copies' times now (the inbox of this parity is written
+// again in the next iteration); pushes that lower nothing leave no trace.
+// low: one LDS word.  Every thread of the workgroup calls it.
+template <int BS>
+__device__ inline void defer_item(const SubInfo &si, const Item &t, uint32_t inst, uint32_t s, uint32_t iter,
+                                  uint32_t *low) {
+  const KArgs k = kargs();
+  const Queue nq = next_queue(k, iter);
+  if (!t.pushed) {
+    if (threadIdx.x == 0) nq.add(inst, s, kQueued);
+    return;
+  }
+  __syncthreads();  // the LDS word is free
+  if (threadIdx.x == 0) *low = __float_as_uint(t.own);
+  __syncthreads();
+  uint32_t *phi = reinterpret_cast<uint32_t *>(k->phi) + (size_t)inst * k->ncopy + si.coff;
+  uint32_t *inbox = k->inbox + item_inbox(k, si.ioff, inst, iter);
+  for (uint32_t j = threadIdx.x; j < si.ni; j += BS) {
+    const uint32_t v = inbox[j];
+    if (v == __float_as_uint(F_INF)) continue;
+    inbox[j] = __float_as_uint(F_INF);
+    const uint32_t l = k->if_l[si.ioff + j];
+    if (v < phi[l]) {
+      phi[l] = v;
+      k->dirty[(size_t)inst * k->ncopy + si.coff + l] = 1;
+      atomicMin(low, v);
+    }
   }
   __syncthreads();
-  if (tid == 0) push_descriptor(a.cur, dslot, entry, *cnt);
+  if (threadIdx.x == 0) end_item(k, nq, inst, s, iter, true, __uint_as_float(*low));
+}
+
+// the time of an interface copy of an item that was pushed to: the smaller of
+// its own v and its inbox entry's, which is emptied; true if lowered
+__device__ inline bool merge_inbox(uint32_t *entry, float *phi, float &v) {
+  const float x = __uint_as_float(*entry);
+  if (!(x < F_INF)) return false;
+  *entry = __float_as_uint(F_INF);
+  if (!(x < v)) return false;
+  v = x;
+  *phi = x;
+  return true;
+}
+
+// Pushes the interface copies lowered by this activation (bits in tch), found
+// through the interface list.
+template <int BS>
+__device__ inline void push_lowered_scan(const Queue &nq, const SubInfo &si, uint32_t inst, uint32_t iter,
+                                         const uint32_t *tch, const float *phi_l) {
+  const KArgs k = kargs();
+  for (uint32_t j = threadIdx.x; j < si.ni; j += BS) {
+    const uint32_t l = k->if_l[si.ioff + j];
+    if (flag_at(tch, l)) push_entry(k, nq, inst, si.ioff + j, __float_as_uint(phi_l[l]), iter);
+  }
 }
 
 // One workgroup per work item (instance, submesh).  STAGED copies the
@@ -352,30 +485,25 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
   uint32_t *misc = reinterpret_cast<uint32_t *>(lds + a.o_misc);
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
-  UnitCursor cursor(a.cur, &misc[4], a.ninst, a.unit, a.maxch);
-  if (blockIdx.x == 0 && tid == 0 && cursor.U > 0) atomicAdd(&a.stats[3], 1ull);
+  UnitCursor cursor;
+  const uint32_t iter_now = start_iteration();
   unsigned long long sweeps = 0, evals = 0, acts = 0, abytes = 0, vupd = 0;
-  // time window of this iteration: flagged vertices later than W wait
-  const uint32_t iter_now = *a.iter;
 
   uint32_t inst, s;
-  while (cursor.next(inst, s)) {
-    const size_t entry = (size_t)inst * a.nsub + s;
+  while (cursor.next(inst, s, &misc[4])) {
     const float wi = a.winst[inst];
+    // time window of this iteration: flagged vertices later than W wait
     const float W = wi > 0.0f ? wi * (float)(iter_now - a.start[inst] + 1u) : F_INF;
     const SubInfo si = a.sub[s];
+    const Item item = take_item(kargs(), inst, s, iter_now);
     const size_t cb = (size_t)inst * a.ncopy + si.coff;
     const uint32_t nn = si.nn, ne = si.ne;
     const uint32_t nv64 = (nn + 63u) & ~63u;
     const uint32_t new32 = (ne + 31u) >> 5;
-    if (tid == 0) a.act[entry] = 0u;
     // nothing in this submesh can act before the window reaches its wake
     // time: keep it queued without staging anything
-    if (a.wake[entry] > W) {
-      if (tid == 0) {
-        requeue(a.nxt, a.act, inst, s, a.nsub, a.ninst);
-        push_descriptor(a.cur, cursor.uidx * a.unit + cursor.i, entry, 0u);
-      }
+    if (item.wake > W) {
+      defer_item<BS>(si, item, inst, s, iter_now, &misc[5]);
       continue;
     }
     // stage vertex times and dirty flags
@@ -383,11 +511,18 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
       const uint32_t l = l0 + tid;
       bool d = false, late = false;
       if (l < nn) {
-        const float v = a.phi[cb + l];
-        phi_l[l] = v;
-        phi_n[l] = __float_as_uint(v);
+        float v = a.phi[cb + l];
         d = a.dirty[cb + l] != 0;
         if (d) a.dirty[cb + l] = 0;
+        if (item.pushed) {
+          const uint2 w = a.ifm[(size_t)s * a.wps + (l >> 5)];
+          if ((w.x >> (l & 31)) & 1u)
+            d |= merge_inbox(a.inbox + item_inbox(kargs(), si.ioff, inst, iter_now) + w.y +
+                                 __popc(w.x & ((1u << (l & 31)) - 1u)),
+                             a.phi + cb + l, v);
+        }
+        phi_l[l] = v;
+        phi_n[l] = __float_as_uint(v);
         late = d && v > W;
         d = d && !late;
       }
@@ -593,7 +728,7 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
       __syncthreads();
     }
     sweeps += it;
-    acts += 1;
+    acts += it > 0;
     // algorithmic bytes of the activation: copies read and written (phi 4+4,
     // flag 1+1), interface entries (index 4, read 4, write 4) and the
     // element data used (nodes 8 + geometry 24) -- all elements when staged,
@@ -608,7 +743,7 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
       __syncthreads();
       used = misc[3];
     }
-    abytes += 32ull * used + 10ull * nn + 12ull * si.ni;
+    if (it > 0) abytes += 32ull * used + 10ull * nn + 12ull * si.ni;
     // write back decreased copies and push the lowered interface copies.
     // Deferred vertices (and sources left by the sweep cap) stay dirty and
     // the submesh is queued for the next iteration.
@@ -621,13 +756,10 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
         atomicMin(&misc[1], __float_as_uint(phi_l[l]));
       }
     }
-    push_lowered_scan<BS>(a, si, inst, entry, cursor.uidx * a.unit + cursor.i, tch, phi_l, &misc[6]);
+    const Queue nq = next_queue(kargs(), iter_now);
+    push_lowered_scan<BS>(nq, si, inst, iter_now, tch, phi_l);
     __syncthreads();
-    if (tid == 0) {
-      const float wk = __uint_as_float(misc[1]);
-      a.wake[entry] = wk;
-      if (wk < F_INF) requeue(a.nxt, a.act, inst, s, a.nsub, a.ninst);
-    }
+    if (tid == 0) end_item(kargs(), nq, inst, s, iter_now, item.pushed, __uint_as_float(misc[1]));
     __syncthreads();
   }
   if (tid == 0 && acts) {
@@ -644,12 +776,46 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
 //   [0] nodes 0,1 (u16 each; bit 15 and bit 31 carry the region id's bits 0
 //       and 1), nodes 2,3 (u16 each), geometry e12 e13 (f32)
 //   [1] geometry e23 e14 e24 e34 (f32)
-//   [2] node heights h0..h3 (f32)
+//   [2] candidate bounds: for the targets T = 0..3, n . (x_T - x_i) of the
+//       nodes i = T+1, T+2, T+3 (Pack::bnd8), their scale (f32)
 // Local copy ids are below 2^15, so the two region bits are free.
+
+// The targets with a source among the other nodes whose candidates can still
+// lower them: a candidate is at least min_i (p_i + n . u_i).  With n along the
+// target's distance from the centroid of the opposite face this keeps 33 % of
+// the targets of a settled slab; the plane's height over that face (n
+// perpendicular to it, four floats, the bound before) 50 %, two directions
+// 23 %, three 20 %.  One direction in bytes is what fits the record's 48 B: the
+// records of the fronts that an XCD works on just about fill its L2, and a
+// record of 80 B for two directions lost in L2 misses (twice as many) what
+// fewer candidates saved.  Three directions from the squared lengths, without
+// a table, take 100 instructions and 30 more registers (28 % slower).
+__device__ inline uint32_t live_targets(const uint4 b, float hs, const float ph[4], const int f[4]) {
+  const uint32_t w[3] = {b.x, b.y, b.z};
+  const float sc = __uint_as_float(b.w) * hs;
+  const int nf = f[0] + f[1] + f[2] + f[3];
+  float p[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) p[k] = fmaf(-128.0f, sc, ph[k]);
+  uint32_t tm = 0;
+#pragma unroll
+  for (int T = 0; T < 4; ++T) {
+    float v[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int k = 3 * T + j;
+      v[j] = fmaf((float)((w[k >> 2] >> (8 * (k & 3))) & 0xffu), sc, p[(T + 1 + j) & 3]);
+    }
+    tm |= (nf - f[T] > 0 && ph[T] > fminf(v[0], fminf(v[1], v[2]))) ? 1u << T : 0u;
+  }
+  return tm;
+}
 constexpr uint32_t kAdjPad = 0xffffffffu;
 // (element, target) pair ring of one wave in the band kernel: up to 63 pairs
 // left from earlier rounds plus 4 targets of 64 elements
 constexpr uint32_t kPairRing = 320;
+// counters and flags of a workgroup, region factors, launch counters
+constexpr uint32_t kMiscBytes = 80;
 
 // marks the (up to two) local elements of one adjacency word in the LDS
 // bitmask; the atomics return nothing, the list is built from the bitmask
@@ -666,11 +832,11 @@ __device__ inline void mark_chunk(uint32_t *emark, const uint4 q) {
   mark_word(emark, q.w);
 }
 
-// marks the incident elements of copy c (global copy id): up to four 8-entry
-// chunks of the padded adjacency are loaded before any is used
-__device__ inline void mark_incident(const ConvArgs &a, uint32_t c, uint32_t *emark) {
-  const uint32_t ap = a.adj_ptr[c];
-  const uint4 *ch = a.adj + (ap >> 6);
+// marks the incident elements of local copy c: up to four 8-entry chunks of
+// the padded adjacency are loaded before any is used
+__device__ inline void mark_incident(const uint32_t *adj_ptr, const uint4 *adj, uint32_t c, uint32_t *emark) {
+  const uint32_t ap = adj_ptr[c];
+  const uint4 *ch = adj + (ap >> 6);
   const uint32_t nch = ap & 63u;
   const uint4 pad = make_uint4(kAdjPad, kAdjPad, kAdjPad, kAdjPad);
   const uint4 q0 = ch[0];
@@ -722,48 +888,50 @@ __device__ inline void wave_append(bool pred, uint32_t l, uint16_t *list, uint32
 // that the LDS carve allows anyway, so registers left over by a large
 // submesh's LDS footprint are used instead of spilled.
 template <int BS, int WPE, bool PAIRS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) void k_conv_band(ConvArgs a) {
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) void k_conv_band(ConvArgs) {
   extern __shared__ __align__(16) unsigned char lds[];
+  const KArgs k0 = kargs();
   float *phi_l = reinterpret_cast<float *>(lds);
-  uint32_t *phi_n = reinterpret_cast<uint32_t *>(lds + a.o_phin);
-  uint32_t *flg = reinterpret_cast<uint32_t *>(lds + a.o_flg);  // sources of the sweep
-  uint32_t *tch = reinterpret_cast<uint32_t *>(lds + a.o_tch);  // decreased this activation
-  uint32_t *dfr = reinterpret_cast<uint32_t *>(lds + a.o_dfr);  // flagged, beyond the window
-  uint32_t *wrt = reinterpret_cast<uint32_t *>(lds + a.o_wrt);  // lowered in this sweep
-  uint32_t *ifc = reinterpret_cast<uint32_t *>(lds + a.o_ifc);  // interface copies
-  uint32_t *ipre = ifc + a.wps;  // interface entries before each word
-  uint32_t *emark = reinterpret_cast<uint32_t *>(lds + a.o_e2n);
-  uint32_t *eseen = reinterpret_cast<uint32_t *>(lds + a.o_geo);
-  uint16_t *elist = reinterpret_cast<uint16_t *>(lds + a.o_list);
-  uint16_t *vlist = reinterpret_cast<uint16_t *>(lds + a.o_vlist);
+  uint32_t *phi_n = reinterpret_cast<uint32_t *>(lds + k0->o_phin);
+  uint32_t *flg = reinterpret_cast<uint32_t *>(lds + k0->o_flg);  // sources of the sweep
+  uint32_t *tch = reinterpret_cast<uint32_t *>(lds + k0->o_tch);  // decreased this activation
+  uint32_t *dfr = reinterpret_cast<uint32_t *>(lds + k0->o_dfr);  // flagged, beyond the window
+  uint32_t *wrt = reinterpret_cast<uint32_t *>(lds + k0->o_wrt);  // lowered in this sweep
+  uint32_t *ifc = reinterpret_cast<uint32_t *>(lds + k0->o_ifc);  // interface copies
+  uint32_t *ipre = ifc + k0->wps;  // interface entries before each word
+  uint32_t *emark = reinterpret_cast<uint32_t *>(lds + k0->o_e2n);
+  uint32_t *eseen = reinterpret_cast<uint32_t *>(lds + k0->o_geo);
+  uint16_t *elist = reinterpret_cast<uint16_t *>(lds + k0->o_list);
+  uint16_t *vlist = reinterpret_cast<uint16_t *>(lds + k0->o_vlist);
   // misc: [0] listed elements, [2] listed sources, [3] distinct elements,
-  // [4] work cursor, [5] earliest deferred time, [6] push records,
-  // [8..11] the instance's region factors
-  uint32_t *misc = reinterpret_cast<uint32_t *>(lds + a.o_misc);
+  // [4] work cursor, [5] earliest deferred time, [6], [7] lowered interface copies,
+  // [8..11] the instance's region factors, [12..19] launch counters
+  uint32_t *misc = reinterpret_cast<uint32_t *>(lds + k0->o_misc);
   const float *rsl = reinterpret_cast<const float *>(misc + 8);
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
-  UnitCursor cursor(a.cur, &misc[4], a.ninst, a.unit, a.maxch);
-  if (blockIdx.x == 0 && tid == 0 && cursor.U > 0) atomicAdd(&a.stats[3], 1ull);
-  unsigned long long sweeps = 0, evals = 0, acts = 0, abytes = 0, vupd = 0;
-  const uint32_t iter_now = *a.iter;
+  UnitCursor cursor;
+  const uint32_t iter_now = start_iteration();
+  // counters of the launch (thread 0): activations, sweeps, element
+  // evaluations, algorithmic bytes
+  unsigned long long *ctr = reinterpret_cast<unsigned long long *>(misc + 12);
+  if (tid == 0) ctr[0] = ctr[1] = ctr[2] = ctr[3] = 0ull;
+  unsigned long long vupd = 0;
 
+  uint32_t npush = 6;  // misc word of the push count, 6 and 7 in turn
   uint32_t inst, s;
-  while (cursor.next(inst, s)) {
-    const size_t entry = (size_t)inst * a.nsub + s;
-    const float wi = a.winst[inst];
-    const float W = wi > 0.0f ? wi * (float)(iter_now - a.start[inst] + 1u) : F_INF;
-    const SubInfo si = a.sub[s];
-    const size_t cb = (size_t)inst * a.ncopy + si.coff;
+  while (cursor.next(inst, s, &misc[4])) {
+    const KArgs ks = kargs();
+    const float wi = ks->winst[inst];
+    // time window of this iteration: flagged vertices later than W wait
+    const float W = wi > 0.0f ? wi * (float)(iter_now - ks->start[inst] + 1u) : F_INF;
+    const SubInfo si = ks->sub[s];
+    const Item item = take_item(ks, inst, s, iter_now);
     const uint32_t nn = si.nn, ne = si.ne;
     const uint32_t nv64 = (nn + 63u) & ~63u;
     const uint32_t new32 = (ne + 31u) >> 5;  // element bitmask words
-    if (tid == 0) a.act[entry] = 0u;
-    if (a.wake[entry] > W) {
-      if (tid == 0) {
-        requeue(a.nxt, a.act, inst, s, a.nsub, a.ninst);
-        push_descriptor(a.cur, cursor.uidx * a.unit + cursor.i, entry, 0u);
-      }
+    if (item.wake > W) {
+      defer_item<BS>(si, item, inst, s, iter_now, &misc[5]);
       continue;
     }
     for (uint32_t k = tid; k < new32; k += BS) {
@@ -775,27 +943,38 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
       misc[2] = 0u;
       misc[3] = 0u;
       misc[5] = __float_as_uint(F_INF);
-      misc[6] = 0u;
+      misc[npush] = 0u;
     }
-    if (tid < 4) misc[8 + tid] = __float_as_uint(a.rscale[4 * (size_t)inst + tid]);
+    if (tid < 4) misc[8 + tid] = __float_as_uint(ks->rscale[4 * (size_t)inst + tid]);
     __syncthreads();
     // stage vertex times; dirty flags split into sources and deferred
+    float *phi_g = ks->phi + (size_t)inst * ks->ncopy + si.coff;
+    uint8_t *dirty_g = ks->dirty + (size_t)inst * ks->ncopy + si.coff;
+    uint32_t *inbox_g = ks->inbox + item_inbox(ks, si.ioff, inst, iter_now);
+    const uint2 *ifm_g = ks->ifm + (size_t)s * ks->wps;
     for (uint32_t l0 = 0; l0 < nv64; l0 += BS) {
       const uint32_t l = l0 + tid;
       const uint32_t wb = l0 + wave * 64;
       if (wb < nv64) {
         bool d = false, late = false;
+        const uint2 fw = ifm_g[l >> 5];
         if (l < nn) {
-          const float v = a.phi[cb + l];
+          float v = phi_g[l];
+          d = dirty_g[l] != 0;
+          if (d) dirty_g[l] = 0;
+          if (item.pushed && ((fw.x >> (l & 31)) & 1u))
+            d |= merge_inbox(inbox_g + fw.y + __popc(fw.x & ((1u << (l & 31)) - 1u)), phi_g + l, v);
           phi_l[l] = v;
           phi_n[l] = __float_as_uint(v);
-          d = a.dirty[cb + l] != 0;
-          if (d) a.dirty[cb + l] = 0;
           late = d && v > W;
           d = d && !late;
         }
         const uint64_t m = __ballot(d), md = __ballot(late);
         const uint32_t k = wb >> 5;
+        if ((lane & 31) == 0) {
+          ifc[l >> 5] = fw.x;
+          ipre[l >> 5] = fw.y;
+        }
         if (lane == 0) {
           flg[k] = (uint32_t)m;
           flg[k + 1] = (uint32_t)(m >> 32);
@@ -808,29 +987,30 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
           wrt[k] = 0u;
           wrt[k + 1] = 0u;
         }
-        if (lane == 2 || lane == 3) {
-          const uint2 w = a.ifm[(size_t)s * a.wps + k + (lane - 2)];
-          ifc[k + lane - 2] = w.x;
-          ipre[k + lane - 2] = w.y;
-        }
         wave_append(d, l, vlist, &misc[2]);
       }
     }
     __syncthreads();
 
-    uint32_t it = 0;
+    uint32_t it = 0, evals = 0;
     bool capped = false;
+    const KArgs kw = kargs();
+    const uint32_t elcap = kw->elcap;
+    const int32_t max_local = kw->max_local;
+    const float eps = kw->eps;
+    const uint4 *erec = kw->erec + 3 * (size_t)si.eoff, *adj = kw->adj;
+    const uint32_t *adj_ptr = kw->adj_ptr + si.coff;
     for (;;) {
       const uint32_t nsrc = misc[2];
       if (nsrc == 0) break;
-      if ((a.max_local > 0 && it >= (uint32_t)a.max_local) || it >= (uint32_t)kHardLocalCap) {
+      if ((max_local > 0 && it >= (uint32_t)max_local) || it >= (uint32_t)kHardLocalCap) {
         capped = true;
         break;
       }
       ++it;
       // mark the elements incident to the sources, then list the marked
       // elements in id order (clearing the marks, one word per thread)
-      for (uint32_t i = tid; i < nsrc; i += BS) mark_incident(a, si.coff + vlist[i], emark);
+      for (uint32_t i = tid; i < nsrc; i += BS) mark_incident(adj_ptr, adj, vlist[i], emark);
       __syncthreads();
       // element-list passes of at most elcap elements: a word's elements
       // beyond the cap stay marked for the next pass (the sweep still
@@ -851,9 +1031,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
           uint32_t base = 0;
           if (lane == 0 && tot) base = atomicAdd(&misc[0], tot);  // lane 0 is active here
           uint32_t pos = __builtin_amdgcn_readfirstlane(base) + pre;
-          if (rest && pos < a.elcap) {
+          if (rest && pos < elcap) {
             uint32_t take = 0;
-            while (rest && pos < a.elcap) {
+            while (rest && pos < elcap) {
               const uint32_t b = __ffs(rest) - 1;
               rest &= rest - 1;
               take |= 1u << b;
@@ -865,7 +1045,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
         }
         __syncthreads();
         const uint32_t listed = misc[0];
-        const uint32_t nact = min(listed, a.elcap);
+        const uint32_t nact = min(listed, elcap);
         evals += nact;
         if (tid == 0) misc[2] = 0u;  // every thread has read the source count
         // candidates of the listed elements
@@ -884,11 +1064,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
               uint32_t tm = 0, e = 0;
               if (i < nact) {
                 e = elist[i];
-                const uint4 *rec = a.erec + 3 * ((size_t)si.eoff + e);
+                const uint4 *rec = erec + 3 * e;
                 const uint4 r0 = rec[0], r2 = rec[2];
                 const float hs = csqrt(rsl[((r0.x >> 15) & 1u) | ((r0.x >> 30) & 2u)]);
-                const float h[4] = {__uint_as_float(r2.x) * hs, __uint_as_float(r2.y) * hs,
-                                    __uint_as_float(r2.z) * hs, __uint_as_float(r2.w) * hs};
                 const uint32_t nd[4] = {r0.x & 0x7fffu, (r0.x >> 16) & 0x7fffu, r0.y & 0xffffu,
                                         r0.y >> 16};
                 float ph[4];
@@ -898,13 +1076,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
                   ph[k] = phi_l[nd[k]];
                   f[k] = flag_at(flg, nd[k]) ? 1 : 0;
                 }
-                const int nf = f[0] + f[1] + f[2] + f[3];
-                // targets with a source among the other nodes whose bound
-                // (earliest other node + metric height) is still below their time
-                tm |= (nf - f[0] > 0 && ph[0] > fminf(ph[1], fminf(ph[2], ph[3])) + h[0]) ? 1u : 0u;
-                tm |= (nf - f[1] > 0 && ph[1] > fminf(ph[0], fminf(ph[2], ph[3])) + h[1]) ? 2u : 0u;
-                tm |= (nf - f[2] > 0 && ph[2] > fminf(ph[0], fminf(ph[1], ph[3])) + h[2]) ? 4u : 0u;
-                tm |= (nf - f[3] > 0 && ph[3] > fminf(ph[0], fminf(ph[1], ph[2])) + h[3]) ? 8u : 0u;
+                tm = live_targets(r2, hs, ph, f);
               }
   #pragma unroll
               for (uint32_t T = 0; T < 4; ++T) {
@@ -926,7 +1098,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
                 if (pos >= kPairRing) pos -= kPairRing;
                 const uint32_t code = pq[pos];
                 const uint32_t e = code & 0x3fffu, T = code >> 14;
-                const uint4 *rec = a.erec + 3 * ((size_t)si.eoff + e);
+                const uint4 *rec = erec + 3 * e;
                 const uint4 r0 = rec[0], r1 = rec[1];
                 const float sc = rsl[((r0.x >> 15) & 1u) | ((r0.x >> 30) & 2u)];
                 const float g[6] = {__uint_as_float(r0.z) * sc, __uint_as_float(r0.w) * sc,
@@ -980,8 +1152,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
         } else {
           for (uint32_t i = tid; i < nact; i += BS) {
             const uint32_t e = elist[i];
-            const uint4 *rec = a.erec + 3 * ((size_t)si.eoff + e);
-            const uint4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+            const uint4 r0 = erec[3 * e], r1 = erec[3 * e + 1];
             const float sc = rsl[((r0.x >> 15) & 1u) | ((r0.x >> 30) & 2u)];
             const float g[6] = {__uint_as_float(r0.z) * sc, __uint_as_float(r0.w) * sc,
                                 __uint_as_float(r1.x) * sc, __uint_as_float(r1.y) * sc,
@@ -994,9 +1165,6 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
               sq[k] = csqrt(g[k]);
               rc[k] = __builtin_amdgcn_rcpf(g[k]);
             }
-            const float hs = csqrt(sc);
-            const float h[4] = {__uint_as_float(r2.x) * hs, __uint_as_float(r2.y) * hs,
-                                __uint_as_float(r2.z) * hs, __uint_as_float(r2.w) * hs};
             const uint32_t nd[4] = {r0.x & 0x7fffu, (r0.x >> 16) & 0x7fffu, r0.y & 0xffffu,
                                     r0.y >> 16};
             float ph[4];
@@ -1006,11 +1174,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
               ph[k] = phi_l[nd[k]];
               f[k] = flag_at(flg, nd[k]) ? 1 : 0;
             }
-            const int nf = f[0] + f[1] + f[2] + f[3];
-            // targets with a source among the other nodes whose bound (earliest
-            // other node + metric height) is still below their time
-    #define FIM_TARGET(T, A, B, C)                                                        \
-            if (nf - f[T] > 0 && ph[T] > fminf(ph[A], fminf(ph[B], ph[C])) + h[T]) {         \
+            const uint32_t tm = live_targets(erec[3 * e + 2], csqrt(sc), ph, f);
+    #define FIM_TARGET(T)                                                                 \
+            if (tm & (1u << T)) {                                                             \
               const float c = cand_exact_sh<T, float>(g, sq, rc, ph, F_INF);                 \
               ++vupd;                                                                         \
               if (c < ph[T]) {                                                                \
@@ -1019,16 +1185,16 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
                   atomicOr(&wrt[nd[T] >> 5], 1u << (nd[T] & 31));                             \
               }                                                                               \
             }
-            FIM_TARGET(0, 1, 2, 3)
-            FIM_TARGET(1, 0, 2, 3)
-            FIM_TARGET(2, 0, 1, 3)
-            FIM_TARGET(3, 0, 1, 2)
+            FIM_TARGET(0)
+            FIM_TARGET(1)
+            FIM_TARGET(2)
+            FIM_TARGET(3)
     #undef FIM_TARGET
           }
         }
         __syncthreads();
         if (tid == 0) misc[0] = 0u;  // every thread has read the element count
-        if (listed <= a.elcap) break;  // uniform: read after a barrier
+        if (listed <= elcap) break;  // uniform: read after a barrier
         __syncthreads();
       }
       // accept the written vertices: the sources of the next sweep
@@ -1052,7 +1218,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
             if (nv < ov) {
               phi_l[l] = nv;
               dc = true;
-              if ((ov - nv) >= a.eps * (1.0f + 0.5f * (ov + nv))) {
+              if ((ov - nv) >= eps * (1.0f + 0.5f * (ov + nv))) {
                 lt = nv > W;
                 sg = !lt;
               }
@@ -1078,8 +1244,6 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
       }
       __syncthreads();
     }
-    sweeps += it;
-    acts += 1;
     // algorithmic bytes: copies (phi 4+4, flag 1+1), interface entries
     // (4+4+4) and the distinct elements evaluated (32 B: 24 B of FP32
     // geometry + 8 B of node ids; the 16 B of node heights in the record
@@ -1088,11 +1252,12 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     for (uint32_t k = tid; k < new32; k += BS) cnt += __popc(eseen[k]);
     cnt = wave_sum_small<9>(cnt);  // at most 8 words of 32 per thread
     if (lane == 0 && cnt) atomicAdd(&misc[3], cnt);
-    // write back decreased copies, lowered interface copies as push records
-    // into the item's slot range (entry = interface copies before it);
-    // deferred vertices (and sources left by the sweep cap) stay dirty and
-    // the submesh is queued again
-    uint2 *rec = a.prec + (size_t)inst * a.n_if + si.ioff;
+    // write back decreased copies and list the lowered interface copies (in
+    // the source list's space); deferred vertices (and sources left by the
+    // sweep cap) stay dirty and the submesh is queued again
+    const KArgs ke = kargs();
+    float *phi_e = ke->phi + (size_t)inst * ke->ncopy + si.coff;
+    uint8_t *dirty_e = ke->dirty + (size_t)inst * ke->ncopy + si.coff;
     uint32_t dmin = 0xffffffffu;  // earliest time left dirty, per lane
     for (uint32_t l0 = 0; l0 < nv64; l0 += BS) {
       const uint32_t l = l0 + tid;  // uniform trip count: ballots below
@@ -1104,117 +1269,89 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
       bool p = false;
       if (l < nn) {
         if (flag_at(tch, l)) {
-          a.phi[cb + l] = phi_l[l];
+          phi_e[l] = phi_l[l];
           p = flag_at(ifc, l);
         }
         if (flag_at(dfr, l) || (capped && flag_at(flg, l))) {
-          a.dirty[cb + l] = 1;
+          dirty_e[l] = 1;
           dmin = min(dmin, __float_as_uint(phi_l[l]));
         }
       }
-      const uint64_t m = __ballot(p);
-      if (m) {
-        uint32_t wb = 0;
-        if (lane == 0) wb = atomicAdd(&misc[6], (uint32_t)__popcll(m));
-        wb = __builtin_amdgcn_readfirstlane(wb);  // every lane of the wave is active
-        if (p) {
-          const uint32_t w = l >> 5;
-          const uint32_t j = ipre[w] + __popc(ifc[w] & ((1u << (l & 31)) - 1u));
-          rec[wb + __popcll(m & lanes_below())] = make_uint2(si.ioff + j, __float_as_uint(phi_l[l]));
-        }
-      }
+      wave_append(p, l, vlist, &misc[npush]);
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) dmin = min(dmin, (uint32_t)__shfl_xor(dmin, off));
     if (lane == 0 && dmin != 0xffffffffu) atomicMin(&misc[5], dmin);
     __syncthreads();
+    const Queue nq = next_queue(ke, iter_now);
     if (tid == 0) {
-      push_descriptor(a.cur, cursor.uidx * a.unit + cursor.i, entry, misc[6]);
-      abytes += 32ull * misc[3] + 10ull * nn + 12ull * si.ni;
-      const float wk = __uint_as_float(misc[5]);
-      a.wake[entry] = wk;
-      if (wk < F_INF) requeue(a.nxt, a.act, inst, s, a.nsub, a.ninst);
+      if (it > 0) {  // pushes that lowered nothing make no activation
+        ctr[0] += 1ull;
+        ctr[1] += it;
+        ctr[2] += evals;
+        ctr[3] += 32ull * misc[3] + 10ull * nn + 12ull * si.ni;
+      }
+      end_item(ke, nq, inst, s, iter_now, item.pushed, __uint_as_float(misc[5]));
     }
-    __syncthreads();
+    // the last waves first: the first wave, which ends the item, is free to
+    // fetch the next one meanwhile
+    for (uint32_t i = BS - 1 - tid, n = misc[npush]; i < n; i += BS) {
+      const uint32_t l = vlist[i], w = l >> 5;
+      const uint32_t j = ipre[w] + __popc(ifc[w] & ((1u << (l & 31)) - 1u));
+      push_entry(ke, nq, inst, si.ioff + j, __float_as_uint(phi_l[l]), iter_now);
+    }
+    // no barrier: what the push reads (times, list, interface bits) is written
+    // again only after the next item's first barrier, its count is another word
+    npush ^= 1u;
   }
-  if (tid == 0 && acts) {
-    atomicAdd(&a.stats[0], acts);
-    atomicAdd(&a.stats[1], sweeps);
-    atomicAdd(&a.stats[2], evals);
-    atomicAdd(&a.stats[4], abytes);
+  unsigned long long *stats = kargs()->stats;
+  if (tid == 0 && ctr[0]) {
+    atomicAdd(&stats[0], ctr[0]);
+    atomicAdd(&stats[1], ctr[1]);
+    atomicAdd(&stats[2], ctr[2]);
+    atomicAdd(&stats[4], ctr[3]);
   }
   for (int off = 32; off > 0; off >>= 1) vupd += __shfl_xor(vupd, off);
-  if (lane == 0 && vupd) atomicAdd(&a.stats[5], vupd);
+  if (lane == 0 && vupd) atomicAdd(&stats[5], vupd);
 }
 
-
-struct SyncArgs {
-  const SubInfo *sub;
-  const uint4 *if_fo;  // per entry: first other copy, its submesh, then [z, w) in if_os
-  const uint2 *if_os;  // per other copy: (copy, its submesh)
-  const uint2 *prec;
-  float *phi;
+// Merges what is left in the inbox (the run stopped before the items it was
+// pushed to were worked through) into the copies' times, so that a context's
+// state is in its times, flags and list alone.
+struct DrainArgs {
+  const uint32_t *ifc;  // per interface entry: its copy
+  const uint32_t *c2s;
+  uint32_t *inbox;
+  float *phi, *wown;
   uint8_t *dirty;
-  uint32_t *act;
-  float *wake;
-  WorkList cur, nxt;
-  uint32_t *iter;
-  uint32_t nsub, ncopy, ninst, n_if, unit, maxch;
+  const uint32_t *iter;
+  uint32_t n_if, ncopy, nsub, ninst;
 };
 
-// interface push: one wave per item slot of the iteration's work units (its
-// push descriptor), a lane per push record;
-// min over copies, order independent.  The kernel waits on memory, so it
-// runs on its own full-occupancy grid.
-__global__ __launch_bounds__(256) void k_conv_sync(SyncArgs a) {
-  // the compute kernel of this iteration has finished reading the counter
-  if (blockIdx.x == 0 && threadIdx.x == 0) *a.iter += 1u;
-  const uint32_t lane = threadIdx.x & 63, wpb = blockDim.x >> 6;
-  const uint32_t NI = a.cur.cnt[0] * a.unit, nw = gridDim.x * wpb;
-  for (uint32_t w = blockIdx.x * wpb + (threadIdx.x >> 6); w < NI; w += nw) {
-    const uint2 d = a.cur.desc[w];
-    const uint32_t inst = d.x / a.nsub, s = d.x - inst * a.nsub, n = d.y;
-    if (n) {
-      const uint2 *rec = a.prec + (size_t)inst * a.n_if + a.sub[s].ioff;
-      const size_t ib = (size_t)inst * a.ncopy;
-      for (uint32_t r = lane; r < n; r += 64) {
-        const uint2 e = rec[r];
-        const uint32_t v = e.y;
-        // most entries have one other copy: the entry's record holds it
-        const uint4 fo = a.if_fo[e.x];
-        uint2 o = make_uint2(fo.x, fo.y);
-        for (uint32_t k = fo.z;;) {
-          const size_t pe = (size_t)inst * a.nsub + o.y;
-          uint32_t *p = reinterpret_cast<uint32_t *>(a.phi + ib + o.x);
-          uint32_t *wk = reinterpret_cast<uint32_t *>(a.wake + pe);
-          // Only pushes (no compute kernel runs now) lower phi and wake and
-          // only pushes set act, so a stale read errs on the safe side (an
-          // extra atomic); the smallest push to a copy always sees v below
-          // what it reads, so the flags it sets (dirty, wake, queued) are the
-          // same whatever the order, and the minima need no return value.
-          // The three reads are issued together.
-          const uint32_t cur = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          const uint32_t wcur = __hip_atomic_load(wk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          const uint32_t queued = __hip_atomic_load(&a.act[pe], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          if (v < cur) {
-            __hip_atomic_fetch_min(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            a.dirty[ib + o.x] = 1;
-            if (v < wcur) __hip_atomic_fetch_min(wk, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (queued == 0u) enqueue(a.nxt, a.act, inst, o.y, a.nsub, a.ninst);
-          }
-          if (k >= fo.w) break;
-          o = a.if_os[k++];
-        }
+__global__ __launch_bounds__(256) void k_conv_drain(DrainArgs a) {
+  uint32_t *inbox = a.inbox + (*a.iter & 1u) * (size_t)a.ninst * a.n_if;
+  for (uint32_t inst = blockIdx.y; inst < a.ninst; inst += gridDim.y)
+    for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < a.n_if; e += gridDim.x * blockDim.x) {
+      const size_t i = (size_t)inst * a.n_if + e;
+      const uint32_t v = inbox[i];
+      if (v == __float_as_uint(F_INF)) continue;
+      inbox[i] = __float_as_uint(F_INF);
+      const uint32_t c = a.ifc[e];
+      const size_t gc = (size_t)inst * a.ncopy + c;
+      if (__uint_as_float(v) < a.phi[gc]) {
+        a.phi[gc] = __uint_as_float(v);
+        a.dirty[gc] = 1;
+        atomicMin(reinterpret_cast<uint32_t *>(a.wown) + (size_t)inst * a.nsub + a.c2s[c], v);
       }
     }
-  }
 }
 
 // seeds: (instance, copy) pairs get min(phi, t0), are flagged, and their
 // submesh is queued on the current list
 __global__ void k_conv_seed(const uint2 *ic, uint32_t n, float t0, const uint32_t *c2s, float *phi,
-                            uint8_t *dirty, uint32_t *act, float *wake, WorkList l0, uint32_t nsub,
-                            uint32_t ncopy, uint32_t ninst) {
+                            uint8_t *dirty, float *wake, Queue q, uint32_t ncopy) {
+  const uint32_t nsub = q.nsub;
+  q.enter();
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const uint32_t inst = ic[i].x, c = ic[i].y;
     const size_t gc = (size_t)inst * ncopy + c;
@@ -1222,18 +1359,19 @@ __global__ void k_conv_seed(const uint2 *ic, uint32_t n, float t0, const uint32_
     dirty[gc] = 1;
     const uint32_t s = c2s[c];
     atomicMin(reinterpret_cast<uint32_t *>(wake + (size_t)inst * nsub + s), __float_as_uint(t0));
-    enqueue(l0, act, inst, s, nsub, ninst);
+    q.add(inst, s, kQueued);
   }
 }
 
 // per instance: 1 if any (instance, submesh) pair is queued
-__global__ __launch_bounds__(256) void k_inst_active(const uint32_t *act, uint32_t nsub, uint32_t *out) {
+__global__ __launch_bounds__(256) void k_inst_active(Queue q, uint32_t *out) {
   __shared__ uint32_t any;
   if (threadIdx.x == 0) any = 0u;
+  q.enter();
   __syncthreads();
-  const uint32_t *row = act + (size_t)blockIdx.x * nsub;
+  const uint32_t *row = q.act + (size_t)blockIdx.x * q.nsub;
   uint32_t v = 0u;
-  for (uint32_t s = threadIdx.x; s < nsub; s += blockDim.x) v |= row[s];
+  for (uint32_t s = threadIdx.x; s < q.nsub; s += blockDim.x) v |= row[s] >= q.tag ? 1u : 0u;
   if (v) atomicOr(&any, 1u);
   __syncthreads();
   if (threadIdx.x == 0) out[blockIdx.x] = any;
@@ -1269,11 +1407,11 @@ __global__ void k_conv_init(const float *phi0, const uint32_t *c2g, uint32_t ins
   }
 }
 
-__global__ void k_conv_queue_all(uint32_t inst, uint32_t nsub, uint32_t ninst, uint32_t *act,
-                                 float *wake, WorkList l0) {
-  for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < nsub; s += gridDim.x * blockDim.x) {
-    wake[(size_t)inst * nsub + s] = 0.0f;
-    enqueue(l0, act, inst, s, nsub, ninst);
+__global__ void k_conv_queue_all(uint32_t inst, float *wake, Queue q) {
+  q.enter();
+  for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < q.nsub; s += gridDim.x * blockDim.x) {
+    wake[(size_t)inst * q.nsub + s] = 0.0f;
+    q.add(inst, s, kQueued);
   }
 }
 
@@ -2034,10 +2172,11 @@ T *dalloc(size_t n, std::vector<void *> &owned) {
   return static_cast<T *>(p);
 }
 
-// f(begin, end) over [0, n) on up to eight host threads
+// f(begin, end) over [0, n) on up to eight host threads, at least `least` each
+// (starting a thread costs about 50 us)
 template <class F>
-void parallel_ranges(size_t n, F &&f) {
-  const size_t nt = std::max<size_t>(1, std::min<size_t>({8, (size_t)std::thread::hardware_concurrency(), n / 512}));
+void parallel_ranges(size_t n, size_t least, F &&f) {
+  const size_t nt = std::max<size_t>(1, std::min<size_t>({8, (size_t)std::thread::hardware_concurrency(), n / least}));
   std::vector<std::thread> ts;
   for (size_t t = 1; t < nt; ++t) ts.emplace_back([&, t] { f(n * t / nt, n * (t + 1) / nt); });
   f(0, n / nt);
@@ -2068,7 +2207,7 @@ struct fim_ctx {
   int dev = 0;
   hipStream_t stream = nullptr;
   fim_opts o{};
-  uint32_t nsub = 0, ncopy = 0, ninst = 1, nn = 0;
+  uint32_t nsub = 0, ncopy = 0, ninst = 1, nn = 0, n_if = 0;
   int64_t ne = 0;
   int32_t nn_max = 0, ne_max = 0;
   std::vector<void *> owned;
@@ -2083,8 +2222,7 @@ struct fim_ctx {
   uint8_t *d_ereg = nullptr;
   uint32_t *d_c2g = nullptr, *d_c2s = nullptr, *d_g2c_dsp = nullptr, *d_g2c = nullptr;
   uint16_t *d_if_l = nullptr;
-  uint4 *d_if_fo = nullptr;
-  uint2 *d_if_os = nullptr;
+  uint4 *d_if_fo = nullptr, *d_if_os = nullptr;
   uint32_t *d_n2e_dsp = nullptr, *d_n2n_dsp = nullptr;
   uint16_t *d_n2e_le = nullptr, *d_n2n_lv = nullptr;
   uint8_t *d_n2e_pos = nullptr;
@@ -2103,12 +2241,15 @@ struct fim_ctx {
   std::vector<float> h_rscale, h_winst;
   bool params_dirty = false;
   uint32_t *d_flag = nullptr;   // n_inst: scratch for instance queries / lists
-  uint2 *d_prec = nullptr;  // push records: n_inst x (interface entries)
+  uint32_t *d_inbox = nullptr;  // 2 x n_inst x interface entries
+  uint32_t *d_ifc = nullptr;    // per interface entry: its copy
+  bool inbox_left = false;      // the last run stopped with pushes in the inbox
+  bool direct_plan = false;     // a bucket is one work unit
   uint2 *d_ifm = nullptr;
   uint32_t wps = 1;
   WorkList wl[3] = {};
   uint32_t unit = 2, maxch = 1;
-  float *d_wake = nullptr;
+  float *d_wake = nullptr, *d_wpush = nullptr;
   // compat state
   double *d_phi64 = nullptr;
   int8_t *d_st = nullptr;
@@ -2139,10 +2280,9 @@ struct fim_ctx {
   hipEvent_t evc = nullptr;  // end of an iteration chunk's read-back
   std::vector<hipEvent_t> kev;  // profile: events around each captured compute launch
   ConvArgs ca{};
-  SyncArgs sa{};
   CompatArgs xa{};
   uint32_t lds_conv = 0, lds_compat = 0;
-  int grid = 0, sync_grid = 0, block = 256, graph_iters = 8;
+  int grid = 0, block = 256, graph_iters = 8;
   int band_wpe = 8;  // waves per SIMD the band kernel's registers are sized for
   bool band_pairs = false;  // band kernel evaluates (element, target) pairs
   bool direct = false;      // launch iterations directly instead of replaying the graph
@@ -2238,22 +2378,19 @@ void launch_plan(fim_ctx *c, int l, int z) {
 }
 
 // one global iteration k: work lists rotate over three buffers; iteration k
-// reads list k%3 and appends to (k+1)%3, whose units are planned after the
-// interface push; the buckets of list k%3 are cleared then
+// reads list k%3 and appends to (k+1)%3, whose units are planned then (by the
+// items themselves when a bucket is one unit) and the buckets of list k%3
+// cleared
 void enqueue_iteration(fim_ctx *c, int k, bool timed) {
   const int p = k % 3, q = (k + 1) % 3;
   if (timed) HIPCHECK(hipEventRecord(c->kev[2 * k], c->stream));
   ConvArgs a = c->ca;
   a.cur = c->wl[p];
   a.nxt = c->wl[q];
+  a.old_cnt = c->wl[(k + 2) % 3].cnt;
   launch_conv_compute(c, a);
   if (timed) HIPCHECK(hipEventRecord(c->kev[2 * k + 1], c->stream));
-  SyncArgs s = c->sa;
-  s.cur = c->wl[p];
-  s.nxt = c->wl[q];
-  k_conv_sync<<<c->sync_grid, 256, 0, c->stream>>>(s);
-  HIPCHECK(hipGetLastError());
-  launch_plan(c, q, p);
+  if (!c->direct_plan) launch_plan(c, q, p);
 }
 
 void build_graph(fim_ctx *c) {
@@ -2267,6 +2404,23 @@ void build_graph(fim_ctx *c) {
   }
   HIPCHECK(hipStreamEndCapture(c->stream, &c->graph));
   HIPCHECK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
+}
+
+// the list that the next run starts on, for kernels between runs
+Queue list0(const fim_ctx *c) {
+  return Queue{c->wl[0], c->d_act, 0u, c->nsub, c->ninst, c->direct_plan ? 1u : 0u};
+}
+
+// before a call reads or replaces times while pushes may be in the inbox
+void settle(fim_ctx *c) {
+  if (!c->inbox_left) return;
+  c->inbox_left = false;
+  if (c->n_if == 0) return;
+  const DrainArgs a{c->d_ifc, c->d_c2s, c->d_inbox, c->d_phi, c->d_wake, c->d_dirty, c->wl[0].cnt + kIterWord,
+                    c->n_if, c->ncopy, c->nsub, c->ninst};
+  k_conv_drain<<<dim3(std::min(blocks_for(c->n_if, 256), 256), std::min<uint32_t>(c->ninst, 1024u)), 256, 0,
+                 c->stream>>>(a);
+  HIPCHECK(hipGetLastError());
 }
 
 void check_inst(const fim_ctx *c, int32_t inst) {
@@ -2338,12 +2492,12 @@ float *ctx_field_buffer(fim_ctx *c) { return c->d_tmpf; }
 
 void ctx_init_field(fim_ctx *c, int32_t inst, bool all_active) {
   check_inst(c, inst);
+  settle(c);
   k_conv_init<<<blocks_for(c->ncopy, 256), 256, 0, c->stream>>>(c->d_tmpf, c->d_c2g, (uint32_t)inst,
                                                                  c->d_phi, c->d_dirty, c->ncopy,
                                                                  all_active ? 1 : 0);
   if (all_active)
-    k_conv_queue_all<<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>((uint32_t)inst, c->nsub, c->ninst,
-                                                                       c->d_act, c->d_wake, c->wl[0]);
+    k_conv_queue_all<<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>((uint32_t)inst, c->d_wake, list0(c));
   HIPCHECK(hipGetLastError());
 }
 
@@ -2380,6 +2534,7 @@ void flush_params(fim_ctx *c) {
 // the per-vertex candidate minimum
 double support_into(fim_ctx *c, int32_t inst, uint32_t *best) {
   flush_params(c);
+  settle(c);
   k_fill<uint32_t><<<blocks_for(c->nn, 256), 256, 0, c->stream>>>(best, c->nn, 0x7f800000u);
   k_conv_support<<<(int)std::min<uint32_t>(c->nsub, 4096u), 256, 0, c->stream>>>(
       c->d_sub, c->nsub, c->d_e2n, c->d_geo32, c->d_ereg, c->d_rscale, c->d_phi, c->d_c2g,
@@ -2479,7 +2634,8 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         const uint32_t vlist_bytes =
             o->staged ? 0u
                       : al16(std::max<uint32_t>(2 * nn64, c->band_pairs ? (uint32_t)(c->block / 64) * 2u * kPairRing : 0u));
-        const uint32_t tail_bytes = vlist_bytes + 48 + (o->staged ? 0u : 3u * al16(4 * (nn64 / 32)));
+        const uint32_t misc_bytes = o->staged ? 48u : kMiscBytes;  // staged: 8 words, 4 region factors
+        const uint32_t tail_bytes = vlist_bytes + misc_bytes + (o->staged ? 0u : 3u * al16(4 * (nn64 / 32)));
         // The band kernel lists at most elcap elements per pass: at least
         // kElistCap, more if the LDS left over by the workgroups the wave
         // slots admit (8 waves per SIMD) holds more
@@ -2493,7 +2649,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         }
         const uint32_t o_vlist = o_list + al16(2 * elcap);
         const uint32_t o_misc = o_vlist + vlist_bytes;
-        const uint32_t o_wrt = o_misc + 48;  // misc: 8 words, 4 region factors
+        const uint32_t o_wrt = o_misc + misc_bytes;
         // unstaged: interface-copy bits and entry counts (2 x nn64/32 words)
         const uint32_t o_ifc = o_wrt + (o->staged ? 0u : al16(4 * (nn64 / 32)));
         c->lds_conv = o_ifc + (o->staged ? 0u : 2u * al16(4 * (nn64 / 32)));
@@ -2512,17 +2668,20 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         if (!o->staged) {
           if (c->nn_max > 32768) throw Error(FIM_ELIMIT, "submeshes above 32768 copies");
           std::vector<uint4> rec(3 * (size_t)p.ne_global);
-          for (int64_t e = 0; e < p.ne_global; ++e) {
-            const uint16_t *n = &p.e2n_l[4 * e];
-            const uint32_t r = p.ereg.empty() ? 0u : (p.ereg[e] & 3u);
-            const float *g = &p.geo32[6 * e], *h = &p.hgt32[4 * e];
-            auto fb = [](float x) { uint32_t u; std::memcpy(&u, &x, 4); return u; };
-            rec[3 * e] = make_uint4((uint32_t)n[0] | ((uint32_t)n[1] << 16) | ((r & 1u) << 15) |
-                                        ((r & 2u) << 30),
-                                    (uint32_t)n[2] | ((uint32_t)n[3] << 16), fb(g[0]), fb(g[1]));
-            rec[3 * e + 1] = make_uint4(fb(g[2]), fb(g[3]), fb(g[4]), fb(g[5]));
-            rec[3 * e + 2] = make_uint4(fb(h[0]), fb(h[1]), fb(h[2]), fb(h[3]));
-          }
+          parallel_ranges((size_t)p.ne_global, 65536, [&](size_t b, size_t end) {
+            for (size_t e = b; e < end; ++e) {
+              const uint16_t *n = &p.e2n_l[4 * e];
+              const uint32_t r = p.ereg.empty() ? 0u : (p.ereg[e] & 3u);
+              const float *g = &p.geo32[6 * e];
+              auto fb = [](float x) { uint32_t u; std::memcpy(&u, &x, 4); return u; };
+              rec[3 * e] = make_uint4((uint32_t)n[0] | ((uint32_t)n[1] << 16) | ((r & 1u) << 15) | ((r & 2u) << 30),
+                                      (uint32_t)n[2] | ((uint32_t)n[3] << 16), fb(g[0]), fb(g[1]));
+              rec[3 * e + 1] = make_uint4(fb(g[2]), fb(g[3]), fb(g[4]), fb(g[5]));
+              uint32_t w[3];
+              std::memcpy(w, &p.bnd8[12 * e], 12);
+              rec[3 * e + 2] = make_uint4(w[0], w[1], w[2], fb(p.bnd_scale[e]));
+            }
+          });
           c->d_erec = dupload(rec, ow);
           std::vector<uint32_t> aptr(p.ncopy);
           std::vector<uint16_t> adj;
@@ -2543,25 +2702,35 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         }
         c->d_if_l = dupload(p.if_l, ow);
         {
-          std::vector<uint2> os(p.if_other.size());
-          for (size_t k = 0; k < os.size(); ++k) os[k] = make_uint2(p.if_other[k], p.c2s[p.if_other[k]]);
-          std::vector<uint4> fo(p.if_l.size());
+          // interface entry of a copy
+          std::vector<uint32_t> ifc(p.if_l.size()), ent(p.ncopy, 0u);
+          for (const SubInfo &si : p.sub)
+            for (uint32_t e = si.ioff; e < si.ioff + si.ni; ++e) {
+              ifc[e] = si.coff + p.if_l[e];
+              ent[ifc[e]] = e;
+            }
+          c->d_ifc = dupload(ifc, ow);
+          std::vector<uint4> os(p.if_other.size()), fo(p.if_l.size());
           for (size_t e = 0; e < fo.size(); ++e) {
             const uint32_t k0 = p.if_dsp[e], k1 = p.if_dsp[e + 1];
             if (k1 <= k0) throw Error(FIM_EINVAL, "interface entry without another copy");
-            fo[e] = make_uint4(os[k0].x, os[k0].y, k0 + 1, k1);
+            for (uint32_t k = k0; k < k1; ++k) {
+              const uint32_t o = p.if_other[k];
+              os[k] = make_uint4(o, p.c2s[o], ent[o], k + 1 < k1 ? k + 2 : 0u);
+            }
+            fo[e] = os[k0];
           }
           c->d_if_os = dupload(os, ow);
           c->d_if_fo = dupload(fo, ow);
         }
         const size_t ncs = (size_t)c->ninst * c->ncopy, nss = (size_t)c->ninst * c->nsub;
-        // push descriptors name an item by instance * nsub + submesh in 32 bits
         if (nss >= (1ull << 32)) throw Error(FIM_ELIMIT, "instances x submeshes exceed 2^32");
         c->d_phi = dalloc<float>(ncs, ow);
         c->d_dirty = dalloc<uint8_t>(ncs, ow);
         {
-          // push records: one slot per (instance, interface entry)
-          c->d_prec = dalloc<uint2>((size_t)c->ninst * p.if_l.size(), ow);
+          const size_t nib = 2 * (size_t)c->ninst * p.if_l.size();
+          c->d_inbox = dalloc<uint32_t>(nib, ow);
+          if (nib) k_fill<uint32_t><<<blocks_for(nib, 256), 256, 0, c->stream>>>(c->d_inbox, nib, 0x7f800000u);
           c->d_start = dalloc<uint32_t>(c->ninst, ow);
           c->h_winst.assign(c->ninst, (float)std::max(0.0, o->window));
           c->d_winst = dupload(c->h_winst, ow);
@@ -2586,20 +2755,23 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
           }
           c->d_ifm = dupload(ifm, ow);
         }
-        c->d_act = dalloc<uint32_t>(nss, ow);
+        c->d_act = dalloc<uint32_t>(2 * nss, ow);
         c->d_wake = dalloc<float>(nss, ow);
+        c->d_wpush = dalloc<float>(2 * nss, ow);
         c->unit = o->unit > 0 ? (uint32_t)o->unit : 2u;
         c->maxch = (c->ninst + c->unit - 1) / c->unit;
         if ((uint64_t)c->nsub * c->maxch >= (1ull << 32)) throw Error(FIM_ELIMIT, "too many work units");
-        // 16 words per list (units, pairs, 8 XCD counters), then the
-        // iteration counter at word 48
-        c->d_cnt = dalloc<uint32_t>(64, ow);
+        // a bucket that fits one unit is planned by its first item; only
+        // batches of more instances need the plan kernel (4 us, and as much
+        // again between two launches, out of 60 for an iteration of a single
+        // solve on the 2M-tet slab)
+        c->direct_plan = c->maxch == 1;
+        c->d_cnt = dalloc<uint32_t>(48, ow);  // 16 words per list
         for (int k = 0; k < 3; ++k) {
           c->wl[k].bcnt = dalloc<uint32_t>(c->nsub, ow);
           c->wl[k].bins = dalloc<uint32_t>(nss, ow);
           c->wl[k].plan = dalloc<uint32_t>((size_t)c->nsub * c->maxch, ow);
           c->wl[k].cnt = c->d_cnt + 16 * k;
-          c->wl[k].desc = dalloc<uint2>((size_t)c->nsub * c->maxch * c->unit, ow);
         }
         c->d_rscale = dalloc<float>(4 * (size_t)c->ninst, ow);
         c->d_tmpf = dalloc<float>(c->nn, ow);
@@ -2624,20 +2796,17 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         per_cu = std::max(per_cu, 1);
         c->grid = o->grid > 0 ? o->grid : ncu * per_cu;
         c->grid = std::max(c->grid, (int)kXcd);  // every XCD eighth needs a workgroup
-        c->sync_grid = ncu * 8;  // eight workgroups of 256 fill a CU's wave slots
         c->lds_compat = 0;
         c->ca = ConvArgs{c->d_sub, c->d_e2n, c->d_geo32, c->d_hgt, c->d_ereg, c->d_rscale, c->d_phi,
-                         c->d_dirty, c->d_act, c->d_wake, c->d_if_l, c->d_ifm, c->d_prec,
-                         WorkList{}, WorkList{}, c->d_stats, c->d_cnt + 48, c->d_start,
+                         c->d_dirty, c->d_act, c->d_wake, c->d_wpush, c->d_if_l, c->d_ifm, c->d_inbox, c->d_if_fo,
+                         c->d_if_os, WorkList{}, WorkList{}, c->d_stats, nullptr, c->d_start,
                          c->d_n2e_dsp, c->d_n2e_le, c->d_erec, c->d_adj_ptr, c->d_adj,
-                         c->nsub, c->ncopy, c->ninst, (float)(o->eps_rel > 0 ? o->eps_rel : 1e-6),
+                         c->nsub, c->ncopy, c->ninst, c->direct_plan ? 1u : 0u,
+                         (float)(o->eps_rel > 0 ? o->eps_rel : 1e-6),
                          c->d_winst, o->local_iters, c->unit, c->maxch, (uint32_t)p.if_l.size(),
                          c->wps, elcap, o_phin, o_flg, o_tch, o_dfr, o_e2n, o_geo, o_list, o_vlist, o_misc,
                          o_wrt, o_ifc};
-        c->sa = SyncArgs{c->d_sub, c->d_if_fo, c->d_if_os, c->d_prec,
-                         c->d_phi, c->d_dirty, c->d_act, c->d_wake, WorkList{}, WorkList{},
-                         c->d_cnt + 48, c->nsub, c->ncopy, c->ninst, (uint32_t)p.if_l.size(),
-                         c->unit, c->maxch};
+        c->n_if = (uint32_t)p.if_l.size();
       } else {
         const uint32_t nn = (uint32_t)c->nn_max;
         const uint32_t o_tphi = al16(8 * nn);
@@ -2683,7 +2852,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
           std::unique_ptr<void, void (*)(void *)> mem(std::malloc(16 * std::max<size_t>(total, 1)), std::free);
           if (!mem) throw std::bad_alloc();
           uint4 *blob = static_cast<uint4 *>(mem.get());
-          parallel_ranges((size_t)p.nsub, [&](size_t b, size_t e) {
+          parallel_ranges((size_t)p.nsub, 256, [&](size_t b, size_t e) {
             for (size_t i = b; i < e; ++i) {
               const CompatSub &q = cs[i];
               const size_t nd = (2 * (q.nn + 1) + 15) / 16, nel = (8 * q.ne + 15) / 16, nsl = (8 * q.nch + 15) / 16;
@@ -2770,11 +2939,13 @@ int fim_reset(fim_ctx *c) {
     HIPCHECK(hipSetDevice(c->dev));
     if (c->o.mode == FIM_MODE_CONVERGE) {
       const size_t ncs = (size_t)c->ninst * c->ncopy, nss = (size_t)c->ninst * c->nsub;
+      settle(c);  // empties the inbox
       k_fill<float><<<blocks_for(ncs, 256), 256, 0, c->stream>>>(c->d_phi, ncs, F_INF);
       k_fill<uint8_t><<<blocks_for(ncs, 256), 256, 0, c->stream>>>(c->d_dirty, ncs, (uint8_t)0);
-      k_fill<uint32_t><<<blocks_for(nss, 256), 256, 0, c->stream>>>(c->d_act, nss, 0u);
+      k_fill<uint32_t><<<blocks_for(2 * nss, 256), 256, 0, c->stream>>>(c->d_act, 2 * nss, 0u);
       k_fill<float><<<blocks_for(nss, 256), 256, 0, c->stream>>>(c->d_wake, nss, F_INF);
-      k_fill<uint32_t><<<1, 64, 0, c->stream>>>(c->d_cnt, 64, 0u);
+      k_fill<float><<<blocks_for(2 * nss, 256), 256, 0, c->stream>>>(c->d_wpush, 2 * nss, F_INF);
+      k_fill<uint32_t><<<1, 64, 0, c->stream>>>(c->d_cnt, 48, 0u);
       k_fill<uint32_t><<<blocks_for(c->ninst, 256), 256, 0, c->stream>>>(c->d_start, c->ninst, 0u);
       for (int k = 0; k < 3; ++k)
         k_fill<uint32_t><<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>(c->wl[k].bcnt, c->nsub, 0u);
@@ -2814,8 +2985,7 @@ void seed_pairs(fim_ctx *c, const std::vector<uint2> &ic, double t0) {
   const int g = blocks_for(ic.size(), 256);
   if (c->o.mode == FIM_MODE_CONVERGE) {
     k_conv_seed<<<g, 256, 0, c->stream>>>(c->d_seed, (uint32_t)ic.size(), (float)t0, c->d_c2s, c->d_phi,
-                                          c->d_dirty, c->d_act, c->d_wake, c->wl[0], c->nsub,
-                                          c->ncopy, c->ninst);
+                                          c->d_dirty, c->d_wake, list0(c), c->ncopy);
   } else {
     k_compat_seed<<<g, 256, 0, c->stream>>>(c->d_seed, (uint32_t)ic.size(), t0, c->d_c2s, c->d_phi64,
                                             c->d_st, c->d_nexte);
@@ -2890,11 +3060,11 @@ int fim_init_field(fim_ctx *c, int32_t inst, const float *phi0) {
     for (uint32_t v = 0; v < c->nn; ++v)
       if (!(phi0[v] >= 0.0f)) throw Error(FIM_EINVAL, "initial field must be >= 0 (inf allowed)");
     HIPCHECK(hipSetDevice(c->dev));
+    settle(c);
     HIPCHECK(hipMemcpyAsync(c->d_tmpf, phi0, c->nn * sizeof(float), hipMemcpyHostToDevice, c->stream));
     k_conv_init<<<blocks_for(c->ncopy, 256), 256, 0, c->stream>>>(c->d_tmpf, c->d_c2g, (uint32_t)inst,
                                                                    c->d_phi, c->d_dirty, c->ncopy, 1);
-    k_conv_queue_all<<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>((uint32_t)inst, c->nsub, c->ninst,
-                                                                       c->d_act, c->d_wake, c->wl[0]);
+    k_conv_queue_all<<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>((uint32_t)inst, c->d_wake, list0(c));
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(c->stream));
   });
@@ -2960,9 +3130,10 @@ void run_begin(fim_ctx *c, int32_t max_iters, bool reset_stats, RunState &r) {
     c->stats.compute_ms = 0.0;
     c->stats.compute_launches = 0;
   }
+  c->inbox_left = true;  // until the run has ended with nothing queued
   HIPCHECK(hipEventRecord(c->ev0, c->stream));
   // units of the list the seeds (or an earlier run) filled
-  launch_plan(c, 0, -1);
+  if (!c->direct_plan) launch_plan(c, 0, -1);
   r = RunState{};
   r.max_iters = max_iters;
 }
@@ -3011,6 +3182,7 @@ void run_end(fim_ctx *c, RunState &r) {
   c->stats.global_iters = (int64_t)st[3];
   c->stats.alg_bytes = (int64_t)st[4];
   c->stats.vertex_updates = (int64_t)st[5];
+  c->inbox_left = r.left != 0;
   c->stats.compute_ms += r.kms;
   c->stats.compute_launches += r.klaunch;
 }
@@ -3113,7 +3285,7 @@ int fim_active(fim_ctx *c, int32_t *active) {
     if (!c || !active) throw Error(FIM_EINVAL, "null argument");
     if (c->o.mode != FIM_MODE_CONVERGE) throw Error(FIM_ESTATE, "fim_active needs converge mode");
     HIPCHECK(hipSetDevice(c->dev));
-    k_inst_active<<<c->ninst, 256, 0, c->stream>>>(c->d_act, c->nsub, c->d_flag);
+    k_inst_active<<<c->ninst, 256, 0, c->stream>>>(list0(c), c->d_flag);
     HIPCHECK(hipGetLastError());
     std::vector<uint32_t> h(c->ninst);
     HIPCHECK(hipMemcpyAsync(h.data(), c->d_flag, sizeof(uint32_t) * c->ninst, hipMemcpyDeviceToHost, c->stream));
@@ -3130,7 +3302,7 @@ int fim_recycle(fim_ctx *c, int32_t n, const int32_t *insts) {
     if (v.empty()) return;
     HIPCHECK(hipSetDevice(c->dev));
     // only instances with nothing queued may be recycled
-    k_inst_active<<<c->ninst, 256, 0, c->stream>>>(c->d_act, c->nsub, c->d_flag);
+    k_inst_active<<<c->ninst, 256, 0, c->stream>>>(list0(c), c->d_flag);
     HIPCHECK(hipGetLastError());
     std::vector<uint32_t> h(c->ninst);
     HIPCHECK(hipMemcpyAsync(h.data(), c->d_flag, sizeof(uint32_t) * c->ninst, hipMemcpyDeviceToHost, c->stream));
@@ -3143,7 +3315,7 @@ int fim_recycle(fim_ctx *c, int32_t n, const int32_t *insts) {
     HIPCHECK(hipMemcpyAsync(c->d_flag, v.data(), sizeof(uint32_t) * v.size(), hipMemcpyHostToDevice, c->stream));
     const size_t total = ((size_t)c->ncopy + c->nsub) * v.size();
     k_inst_reset<<<blocks_for(total, 256), 256, 0, c->stream>>>(c->d_flag, (uint32_t)v.size(), c->d_phi, c->d_dirty,
-                                                               c->d_wake, c->d_start, c->d_cnt + 48, c->ncopy,
+                                                               c->d_wake, c->d_start, c->wl[0].cnt + kIterWord, c->ncopy,
                                                                c->nsub);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(c->stream));
@@ -3190,6 +3362,7 @@ int fim_residual(fim_ctx *c, int32_t inst, double *res) {
     check_inst(c, inst);
     HIPCHECK(hipSetDevice(c->dev));
     flush_params(c);
+    settle(c);
     k_fill<uint32_t><<<1, 64, 0, c->stream>>>(c->d_tmpu, 1, 0u);
     k_conv_residual<<<(int)std::min<uint32_t>(c->nsub, 4096u), 256, 0, c->stream>>>(
         c->d_sub, c->nsub, c->d_e2n, c->d_geo32, c->d_ereg, c->d_rscale, c->d_phi,

@@ -347,6 +347,65 @@ def test_converge_work_units_and_grid_change_nothing(unit, grid):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("n_inst,unit", [(1, 0), (3, 4), (5, 2)])
+def test_interrupted_runs_change_nothing(n_inst, unit):
+    """a run stopped after a few iterations, with pushes on their way to the
+    copies of other submeshes, then looked at (residual, support), resumed,
+    reset or given a new field: bitwise the maps of uninterrupted solves (one
+    work unit per bucket, and several)"""
+    cfg = cases.scaled(cases.SLAB, 8)
+    m, _ = cases.box(cfg, seed=9)
+    p = F.Pack(m, F.PART_RCB, max_nn=200, seed=9)
+    srcs = [cases.pacing_sites(cfg, 1 + k % 3, seed=500 + k) for k in range(n_inst)]
+    s = F.Solver(p, n_instances=n_inst, window=500.0, unit=unit, graph_iters=3)
+
+    def seed():
+        s.reset()
+        s.seed_batch(srcs, 0.0)
+
+    def maps():
+        return [s.download(inst=i)[0] for i in range(n_inst)]
+
+    seed()
+    s.run()
+    base = maps()
+    seed()
+    left = 1
+    for k in range(1000):
+        left = s.advance(3, reset_stats=k == 0)
+        if k % 2:
+            assert s.residual(inst=k % n_inst) >= 0.0 and s.support(inst=0) >= 0.0
+        if left == 0:
+            break
+    assert left == 0
+    for a, b in zip(base, maps()):
+        assert np.array_equal(a, b)
+    assert all(s.residual(inst=i) <= 1e-5 for i in range(n_inst))
+    # reset in the middle of a run leaves nothing behind
+    seed()
+    assert s.advance(6, reset_stats=True) > 0
+    seed()
+    s.run()
+    for a, b in zip(base, maps()):
+        assert np.array_equal(a, b)
+    # a field given in the middle of a run is what is solved from (its window
+    # is further on then: the fixed point, not the last bits)
+    up = (base[0] + 3000.0).astype(np.float32)
+    up[srcs[0]] = 0.0
+    s.reset()
+    s.init_field(up, inst=0)
+    s.run()
+    warm = s.download(inst=0)[0]
+    seed()
+    assert s.advance(6, reset_stats=True) > 0
+    s.init_field(up, inst=0)
+    s.run()
+    assert np.max(np.abs(s.download(inst=0)[0] - warm)) <= 1e-4 * warm.max()
+    for a, b in zip(base[1:], maps()[1:]):
+        assert np.array_equal(a, b)
+    s.close()
+
+
 def test_run_multi_contexts_change_nothing():
     """12 instances at their own windows, solved by one context and by three
     contexts of 5 + 4 + 3 instances run together (fim_run_multi, one host

@@ -38,6 +38,7 @@ float ls_exact32(const float *g, const float *ph, int t) {
   }
 }
 double ls_ref(const double *g, const double *ph, int t) { return fim::cand_ref(g, ph, t); }
+void ls_bounds(const double *g, unsigned char *b, float *scale) { fim::cand_bounds(g, b, scale); }
 }
 """
 
@@ -176,3 +177,36 @@ def test_shared_root_candidate_equals_plain_candidate(tmp_path):
         pf_ = np.where(ph >= 1e299, np.float32(3.0e38), ph).astype(np.float32)
         bad += lib.ls_shared_equal(_ptr(gf, C.c_float), _ptr(pf_, C.c_float))
     assert bad == 0
+
+
+def test_candidate_bounds_lie_below_every_candidate(shim):
+    """cand_bounds on ordinary, strongly anisotropic, flat and needle-shaped
+    elements: for random times of the other nodes (some unreached, some equal,
+    some far apart) the bound is at most the exact candidate.  The bound has a
+    margin of 1e-4 of an edge, so nothing is allowed for rounding."""
+    shim.ls_bounds.restype = None
+    shim.ls_bounds.argtypes = [C.POINTER(C.c_double), C.POINTER(C.c_uint8), C.POINTER(C.c_float)]
+    rng = np.random.default_rng(11)
+    pd = C.POINTER(C.c_double)
+    tight = 0
+    for k in range(4000):
+        x = rng.normal(size=(4, 3)) * [1.0, rng.choice([1.0, 0.2, 1e-3]), rng.choice([1.0, 0.1, 1e-4])]
+        if k % 7 == 0:
+            x[3] = x[:3].mean(0) + 1e-5 * rng.normal(size=3)  # target in the face's centroid
+        x *= 10.0 ** rng.uniform(-2, 5)
+        g = np.array([np.sum((x[a] - x[b]) ** 2) for a, b in ((0, 1), (0, 2), (1, 2), (0, 3), (1, 3), (2, 3))])
+        b = np.zeros(12, np.uint8)
+        sc = C.c_float()
+        shim.ls_bounds(g.ctypes.data_as(pd), b.ctypes.data_as(C.POINTER(C.c_uint8)), C.byref(sc))
+        v = (b.astype(np.float64) - 128.0) * sc.value
+        size = np.sqrt(g.max())
+        for t in range(4):
+            ph = rng.uniform(0, size, 4) * rng.choice([0.0, 0.1, 1.0, 3.0])
+            if rng.random() < 0.2:
+                ph[rng.integers(4)] = 1e300
+            o = [(t + 1 + j) % 4 for j in range(3)]
+            bound = min(ph[o[j]] + v[3 * t + j] for j in range(3))
+            c = shim.ls_exact64(g.ctypes.data_as(pd), ph.ctypes.data_as(pd), t)
+            assert bound <= c, (k, t, bound, c, g, ph)
+            tight += bound > min(ph[o]) + 0.3 * (c - min(ph[o]))
+    assert tight > 4000  # they do bound: most lie well above the earliest node
