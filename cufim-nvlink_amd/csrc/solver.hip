@@ -63,8 +63,20 @@ __device__ inline uint64_t lanes_below() {
   return lane ? (~0ull >> (64 - lane)) : 0ull;
 }
 
+// x as a value of its own: what is computed from it is not kept in registers
+// from an earlier phase
+__device__ inline uint32_t fresh(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 __device__ inline bool flag_at(const uint32_t *bits, uint32_t l) {
   return (bits[l >> 5] >> (l & 31)) & 1u;
+}
+
+// set bits of the word of l below l
+__device__ inline uint32_t bits_below(const uint32_t *bits, uint32_t l) {
+  return __popc(bits[l >> 5] & ((1u << (l & 31)) - 1u));
 }
 
 // ---------------------------------------------------------------------------
@@ -208,8 +220,9 @@ struct ConvArgs {
   const uint32_t *n2e_dsp;  // per copy: incident local elements (staged kernel)
   const uint16_t *n2e_le;
   const uint4 *erec;        // band kernel: 48 B per element (below)
-  const uint32_t *adj_ptr;  // band kernel: per copy, chunk offset << 6 | chunk count
-  const uint4 *adj;         // 8 incident local element ids (u16) per chunk, 0xffff padded
+  const uint4 *adj;         // band kernel: per copy, four words of 8 incident local element ids
+  const uint32_t *adj_ptr;  // copies of more than 32 elements: offset << 6 | words in adj_more
+  const uint4 *adj_more;
   uint32_t nsub, ncopy, ninst, direct;
   float eps;
   const float *winst;    // n_inst: time window added per global iteration of
@@ -810,19 +823,17 @@ __device__ inline uint32_t live_targets(const uint4 b, float hs, const float ph[
   }
   return tm;
 }
-constexpr uint32_t kAdjPad = 0xffffffffu;
-// (element, target) pair ring of one wave in the band kernel: up to 63 pairs
-// left from earlier rounds plus 4 targets of 64 elements
-constexpr uint32_t kPairRing = 320;
+// (element, target) pair ring of one wave in the band kernel: pairs left from
+// earlier rounds of 64 ilp plus 4 targets of 64 elements
+constexpr uint32_t pair_ring(int ilp) { return 64u * (uint32_t)ilp + 256u; }
 // counters and flags of a workgroup, region factors, launch counters
 constexpr uint32_t kMiscBytes = 80;
 
-// marks the (up to two) local elements of one adjacency word in the LDS
-// bitmask; the atomics return nothing, the list is built from the bitmask
+// marks the two local elements of one adjacency word in the LDS bitmask; the
+// atomics return nothing, the list is built from the bitmask
 __device__ inline void mark_word(uint32_t *emark, uint32_t w) {
-  const uint32_t lo = w & 0xffffu, hi = w >> 16;
-  if (lo != 0xffffu) atomicOr(&emark[lo >> 5], 1u << (lo & 31));
-  if (hi != 0xffffu) atomicOr(&emark[hi >> 5], 1u << (hi & 31));
+  atomicOr(&emark[(w & 0xffffu) >> 5], 1u << (w & 31u));
+  atomicOr(&emark[w >> 21], 1u << ((w >> 16) & 31u));
 }
 
 __device__ inline void mark_chunk(uint32_t *emark, const uint4 q) {
@@ -832,22 +843,31 @@ __device__ inline void mark_chunk(uint32_t *emark, const uint4 q) {
   mark_word(emark, q.w);
 }
 
-// marks the incident elements of local copy c: up to four 8-entry chunks of
-// the padded adjacency are loaded before any is used
-__device__ inline void mark_incident(const uint32_t *adj_ptr, const uint4 *adj, uint32_t c, uint32_t *emark) {
-  const uint32_t ap = adj_ptr[c];
-  const uint4 *ch = adj + (ap >> 6);
-  const uint32_t nch = ap & 63u;
-  const uint4 pad = make_uint4(kAdjPad, kAdjPad, kAdjPad, kAdjPad);
-  const uint4 q0 = ch[0];
-  const uint4 q1 = nch > 1 ? ch[1] : pad;
-  const uint4 q2 = nch > 2 ? ch[2] : pad;
-  const uint4 q3 = nch > 3 ? ch[3] : pad;
+// marks the incident elements of local copy c.  Every copy has four 16-byte
+// words of eight ids in a row, found without a pointer (a dependent load from
+// L2 less per sweep) and filled up with its first element, which may be marked
+// any number of times; a wave skips words that only repeat.  A copy of more
+// than 32 elements has kAdjMore in place of the last id and lists the others
+// through adj_ptr.
+constexpr uint32_t kAdjMore = 0xffffu;
+__device__ inline void mark_incident(const uint4 *adj, const uint32_t *adj_ptr, const uint4 *adj_more, uint32_t c,
+                                     uint32_t *emark) {
+  const uint4 *ch = adj + 4 * (size_t)c;
+  const uint4 q0 = ch[0], q1 = ch[1], q2 = ch[2];
+  uint4 q3 = ch[3];
+  const uint32_t first = q0.x & 0xffffu;
   mark_chunk(emark, q0);
   mark_chunk(emark, q1);
-  mark_chunk(emark, q2);
-  mark_chunk(emark, q3);
-  for (uint32_t k = 4; k < nch; ++k) mark_chunk(emark, ch[k]);
+  if (__any((q2.x & 0xffffu) != first)) mark_chunk(emark, q2);
+  if (__any((q3.x & 0xffffu) != first)) {
+    const bool more = q3.w >> 16 == kAdjMore;
+    if (more) q3.w = (q3.w & 0xffffu) | first << 16;
+    mark_chunk(emark, q3);
+    if (more) {
+      const uint32_t ap = adj_ptr[c];
+      for (uint32_t k = 0; k < (ap & 63u); ++k) mark_chunk(emark, adj_more[(ap >> 6) + k]);
+    }
+  }
 }
 
 // sum over the wave of n < 2^BITS, one ballot per bit; every lane of the
@@ -871,22 +891,35 @@ __device__ inline void wave_append(bool pred, uint32_t l, uint16_t *list, uint32
 }
 
 // Unstaged converge kernel.  Per sweep it touches only the band that is
-// active, in three steps separated by barriers:
+// active, in three steps, a barrier after each:
 //   mark: the sources (a compact list) mark their incident elements through
 //     the vertex -> element adjacency in an LDS bitmask (atomics without
-//     return), then one thread per bitmask word lists the marked elements in
-//     id order and clears the word;
-//   evaluate: the listed elements compute candidates from L2-resident
-//     element records; LDS atomicMin winners set a "written" bit;
+//     return);
+//   evaluate: each wave lists the marked elements of its words of the bitmask
+//     and computes their candidates from L2-resident element records; LDS
+//     atomicMin winners set a "written" bit;
 //   accept: each written vertex takes its new time; a significant decrease
 //     (reference criterion, cuda_fim.cu:2154) makes it a source of the next
 //     sweep, or a deferred vertex if it lies beyond the window.
 // Element data never enters LDS.  PAIRS evaluates (element, target) pairs
 // in full rounds of 64 instead of an element's four targets per lane (local
-// element ids below 2^14).  WPE is the number of waves per SIMD the
-// register budget is sized for (512 / WPE VGPRs): the launch picks the one
-// that the LDS carve allows anyway, so registers left over by a large
-// submesh's LDS footprint are used instead of spilled.
+// element ids below 2^14).  WPE is the number of waves per SIMD the register
+// budget is sized for (512 / WPE VGPRs): the launch picks the one that the LDS
+// carve allows anyway, so registers left over by a large submesh's LDS footprint
+// are used instead of spilled; with WPE <= 4 a wave works on two rounds of
+// pairs side by side (ILP).
+//
+// What bounds it is latency: with 8 waves per SIMD the vector units issue 41-50 %
+// of the time and waves wait 65-70 % of theirs (L2 misses of records and
+// times, LDS round trips, barriers).  Cycles per item of the 2M slab (256 x 2
+// instances, 2816 copies; a single solve, 1024 copies): staging 24k / 6.9k,
+// mark 13k / 7k, list and evaluate 79k / 27k, accept 17k / 5k, write-back 6k /
+// 3k, push 3k / 2.5k, next item 6k / 2.6k; 155k / 63k in all before the lists
+// were split over the waves, blocks with nothing to do were skipped by whole
+// waves and the adjacency lost its pointer.  A single solve's iteration lasts
+// as long as its longest item (107k cycles), a batch's launch is 1,450 items
+// deep.  Loading the next 64 listed elements ahead of the current ones gained
+// nothing.
 template <int BS, int WPE, bool PAIRS>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) void k_conv_band(ConvArgs) {
   extern __shared__ __align__(16) unsigned char lds[];
@@ -903,12 +936,15 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
   uint32_t *eseen = reinterpret_cast<uint32_t *>(lds + k0->o_geo);
   uint16_t *elist = reinterpret_cast<uint16_t *>(lds + k0->o_list);
   uint16_t *vlist = reinterpret_cast<uint16_t *>(lds + k0->o_vlist);
-  // misc: [0] listed elements, [2] listed sources, [3] distinct elements,
+  // misc: [0] element evaluations, [2] listed sources, [3] distinct elements,
   // [4] work cursor, [5] earliest deferred time, [6], [7] lowered interface copies,
   // [8..11] the instance's region factors, [12..19] launch counters
   uint32_t *misc = reinterpret_cast<uint32_t *>(lds + k0->o_misc);
   const float *rsl = reinterpret_cast<const float *>(misc + 8);
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr uint32_t NW = BS / 64;
+  constexpr int ILP = WPE <= 4 ? 2 : 1;
+  uint32_t tid = threadIdx.x;
+  const uint32_t lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   UnitCursor cursor;
   const uint32_t iter_now = start_iteration();
@@ -916,12 +952,13 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
   // evaluations, algorithmic bytes
   unsigned long long *ctr = reinterpret_cast<unsigned long long *>(misc + 12);
   if (tid == 0) ctr[0] = ctr[1] = ctr[2] = ctr[3] = 0ull;
-  unsigned long long vupd = 0;
+  uint32_t vupd = 0;  // candidates of the lane in this launch
 
   uint32_t npush = 6;  // misc word of the push count, 6 and 7 in turn
   uint32_t inst, s;
   while (cursor.next(inst, s, &misc[4])) {
     const KArgs ks = kargs();
+    tid = fresh(tid);
     const float wi = ks->winst[inst];
     // time window of this iteration: flagged vertices later than W wait
     const float W = wi > 0.0f ? wi * (float)(iter_now - ks->start[inst] + 1u) : F_INF;
@@ -930,10 +967,12 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     const uint32_t nn = si.nn, ne = si.ne;
     const uint32_t nv64 = (nn + 63u) & ~63u;
     const uint32_t new32 = (ne + 31u) >> 5;  // element bitmask words
+    const uint32_t nww = wave < new32 ? (new32 - wave + NW - 1) / NW : 0u;  // words of this wave
     if (item.wake > W) {
       defer_item<BS>(si, item, inst, s, iter_now, &misc[5]);
       continue;
     }
+    const uint2 *ifm_g = ks->ifm + (size_t)s * ks->wps;
     for (uint32_t k = tid; k < new32; k += BS) {
       emark[k] = 0u;
       eseen[k] = 0u;
@@ -945,36 +984,58 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
       misc[5] = __float_as_uint(F_INF);
       misc[npush] = 0u;
     }
+    for (uint32_t q = tid; q < nv64 / 32; q += BS) {
+      const uint2 fw = ifm_g[q];
+      ifc[q] = fw.x;
+      ipre[q] = fw.y;
+    }
     if (tid < 4) misc[8 + tid] = __float_as_uint(ks->rscale[4 * (size_t)inst + tid]);
     __syncthreads();
     // stage vertex times; dirty flags split into sources and deferred
     float *phi_g = ks->phi + (size_t)inst * ks->ncopy + si.coff;
     uint8_t *dirty_g = ks->dirty + (size_t)inst * ks->ncopy + si.coff;
     uint32_t *inbox_g = ks->inbox + item_inbox(ks, si.ioff, inst, iter_now);
-    const uint2 *ifm_g = ks->ifm + (size_t)s * ks->wps;
+    // the loads of a wave's next block of 64 copies are issued before the
+    // current one is used
+    struct Staged {
+      float v, x;  // time, time pushed
+      uint32_t d;
+    };
+    auto fetch = [&](uint32_t l) {
+      Staged g{F_INF, F_INF, 0u};
+      if (l < nn) {
+        g.v = phi_g[l];
+        g.d = dirty_g[l];
+        if (item.pushed && flag_at(ifc, l)) g.x = __uint_as_float(inbox_g[ipre[l >> 5] + bits_below(ifc, l)]);
+      }
+      return g;
+    };
+    Staged next = fetch(tid);
     for (uint32_t l0 = 0; l0 < nv64; l0 += BS) {
       const uint32_t l = l0 + tid;
       const uint32_t wb = l0 + wave * 64;
       if (wb < nv64) {
-        bool d = false, late = false;
-        const uint2 fw = ifm_g[l >> 5];
+        const Staged g = next;
+        next = fetch(l + BS);
+        bool d = g.d != 0;
+        float v = g.v;
+        if (d) dirty_g[l] = 0;
+        if (g.x < F_INF) {  // merged into the time, and emptied
+          inbox_g[ipre[l >> 5] + bits_below(ifc, l)] = __float_as_uint(F_INF);
+          if (g.x < v) {
+            v = g.x;
+            phi_g[l] = v;
+            d = true;
+          }
+        }
         if (l < nn) {
-          float v = phi_g[l];
-          d = dirty_g[l] != 0;
-          if (d) dirty_g[l] = 0;
-          if (item.pushed && ((fw.x >> (l & 31)) & 1u))
-            d |= merge_inbox(inbox_g + fw.y + __popc(fw.x & ((1u << (l & 31)) - 1u)), phi_g + l, v);
           phi_l[l] = v;
           phi_n[l] = __float_as_uint(v);
-          late = d && v > W;
-          d = d && !late;
         }
+        const bool late = d && v > W;
+        d = d && !late;
         const uint64_t m = __ballot(d), md = __ballot(late);
         const uint32_t k = wb >> 5;
-        if ((lane & 31) == 0) {
-          ifc[l >> 5] = fw.x;
-          ipre[l >> 5] = fw.y;
-        }
         if (lane == 0) {
           flg[k] = (uint32_t)m;
           flg[k + 1] = (uint32_t)(m >> 32);
@@ -993,12 +1054,14 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     __syncthreads();
 
     uint32_t it = 0, evals = 0;
+    tid = fresh(tid);
     bool capped = false;
     const KArgs kw = kargs();
-    const uint32_t elcap = kw->elcap;
+    const uint32_t wcap = kw->elcap / NW;
+    uint16_t *wlist = elist + wave * wcap;
     const int32_t max_local = kw->max_local;
     const float eps = kw->eps;
-    const uint4 *erec = kw->erec + 3 * (size_t)si.eoff, *adj = kw->adj;
+    const uint4 *erec = kw->erec + 3 * (size_t)si.eoff, *adj = kw->adj + 4 * (size_t)si.coff, *adj_more = kw->adj_more;
     const uint32_t *adj_ptr = kw->adj_ptr + si.coff;
     for (;;) {
       const uint32_t nsrc = misc[2];
@@ -1008,46 +1071,62 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
         break;
       }
       ++it;
-      // mark the elements incident to the sources, then list the marked
-      // elements in id order (clearing the marks, one word per thread)
-      for (uint32_t i = tid; i < nsrc; i += BS) mark_incident(adj_ptr, adj, vlist[i], emark);
+      // mark the elements incident to the sources
+      for (uint32_t i = tid; i < nsrc; i += BS) mark_incident(adj, adj_ptr, adj_more, vlist[i], emark);
       __syncthreads();
-      // element-list passes of at most elcap elements: a word's elements
-      // beyond the cap stay marked for the next pass (the sweep still
-      // evaluates every marked element against the same times)
-      for (;;) {
-        for (uint32_t k = tid; k < new32; k += BS) {
-          // list offsets: a wave prefix sum of the word counts (<= 32, six
-          // bits) from one ballot per bit, one LDS reservation per wave
-          uint32_t rest = emark[k];
-          const uint32_t n = __popc(rest);
-          uint32_t pre = 0, tot = 0;
+      if (tid == 0) misc[2] = 0u;  // every thread has read the source count
+      // Each wave lists and evaluates the marked elements of its own words of
+      // the bitmask (every NW-th: neighbours go to different waves), without a
+      // barrier in between.  Lane i holds word i: offsets from a wave prefix sum
+      // of the word counts (<= 32, six bits) with one ballot per bit, then two
+      // words at a time, a lane per bit.  A pass lists at most wcap elements;
+      // what is left of the words stays marked for the next pass (the sweep
+      // still evaluates every marked element against the same times).
+      for (uint32_t i0 = 0; i0 < nww;) {
+        const uint32_t kw = wave + NW * (i0 + lane);
+        const uint32_t rest = i0 + lane < nww ? emark[kw] : 0u;
+        const uint32_t n = __popc(rest);
+        uint32_t pos = 0, tot = 0;
 #pragma unroll
-          for (int b = 0; b < 6; ++b) {
-            const uint64_t m = __ballot((n >> b) & 1u);
-            pre += (uint32_t)__popcll(m & lanes_below()) << b;
-            tot += (uint32_t)__popcll(m) << b;
-          }
-          uint32_t base = 0;
-          if (lane == 0 && tot) base = atomicAdd(&misc[0], tot);  // lane 0 is active here
-          uint32_t pos = __builtin_amdgcn_readfirstlane(base) + pre;
-          if (rest && pos < elcap) {
-            uint32_t take = 0;
-            while (rest && pos < elcap) {
-              const uint32_t b = __ffs(rest) - 1;
-              rest &= rest - 1;
-              take |= 1u << b;
-              elist[pos++] = (uint16_t)(k * 32 + b);
-            }
-            emark[k] = rest;
-            eseen[k] |= take;
-          }
+        for (int b = 0; b < 6; ++b) {
+          const uint64_t m = __ballot((n >> b) & 1u);
+          pos += (uint32_t)__popcll(m & lanes_below()) << b;
+          tot += (uint32_t)__popcll(m) << b;
         }
-        __syncthreads();
-        const uint32_t listed = misc[0];
-        const uint32_t nact = min(listed, elcap);
+        const uint32_t word0 = i0;
+        uint32_t take = rest;
+        if (tot > wcap) {  // uniform: the list is full after some word's first bits
+          uint32_t room = pos < wcap ? wcap - pos : 0u;
+          take = 0u;
+          for (uint32_t left = rest; left && room; --room) {
+            take |= left & (0u - left);
+            left &= left - 1u;
+          }
+        } else {
+          i0 += 64;
+        }
+        if (tot == 0) continue;  // uniform
+        if (rest) {
+          emark[kw] = rest & ~take;
+          eseen[kw] |= take;
+        }
+        for (uint64_t some = __ballot(take != 0u); some;) {
+          const int i1 = __ffsll((unsigned long long)some) - 1;
+          some &= some - 1;
+          const bool two = some != 0;
+          const int i2 = two ? __ffsll((unsigned long long)some) - 1 : i1;
+          some &= some - 1;  // 0 stays 0
+          const uint32_t t1 = __builtin_amdgcn_readlane(take, i1), t2 = __builtin_amdgcn_readlane(take, i2);
+          const uint32_t p1 = __builtin_amdgcn_readlane(pos, i1), p2 = __builtin_amdgcn_readlane(pos, i2);
+          const bool hi = lane >= 32;
+          const uint32_t bit = lane & 31u, tw = hi ? (two ? t2 : 0u) : t1;
+          if ((tw >> bit) & 1u)
+            wlist[(hi ? p2 : p1) + __popc(tw & ((1u << bit) - 1u))] =
+                (uint16_t)((wave + NW * (word0 + (hi ? i2 : i1))) * 32 + bit);
+        }
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t nact = min(tot, wcap);
         evals += nact;
-        if (tid == 0) misc[2] = 0u;  // every thread has read the source count
         // candidates of the listed elements
         if constexpr (PAIRS) {
           // (element, target) pairs: a pass over 64 listed elements per wave
@@ -1055,15 +1134,16 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
           // wave-private ring (LDS, in the source list's space, idle until the
           // accept step); full rounds of 64 pairs then evaluate one target
           // per lane, so no lane idles on a pruned target
-          uint16_t *pq = vlist + wave * kPairRing;
+          constexpr uint32_t kRing = pair_ring(ILP);
+          uint16_t *pq = vlist + wave * kRing;
           uint32_t qh = 0, qn = 0;  // ring head and fill, uniform across the wave
-          for (uint32_t c0 = wave * 64;; c0 += BS) {
+          for (uint32_t c0 = 0;; c0 += 64) {
             const bool more = c0 < nact;  // uniform across the wave
             if (more) {
               const uint32_t i = c0 + lane;
               uint32_t tm = 0, e = 0;
               if (i < nact) {
-                e = elist[i];
+                e = wlist[i];
                 const uint4 *rec = erec + 3 * e;
                 const uint4 r0 = rec[0], r2 = rec[2];
                 const float hs = csqrt(rsl[((r0.x >> 15) & 1u) | ((r0.x >> 30) & 2u)]);
@@ -1084,19 +1164,22 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
                 const uint64_t m = __ballot(p);
                 if (p) {
                   uint32_t pos = qh + qn + (uint32_t)__popcll(m & lanes_below());
-                  if (pos >= kPairRing) pos -= kPairRing;
+                  if (pos >= kRing) pos -= kRing;
                   pq[pos] = (uint16_t)(e | (T << 14));
                 }
                 qn += (uint32_t)__popcll(m);
               }
               __builtin_amdgcn_wave_barrier();
             }
-            while (qn >= 64u || (!more && qn > 0u)) {
-              const uint32_t take = qn < 64u ? qn : 64u;
-              if (lane < take) {
-                uint32_t pos = qh + lane;
-                if (pos >= kPairRing) pos -= kPairRing;
-                const uint32_t code = pq[pos];
+            while (qn >= 64u * ILP || (!more && qn > 0u)) {
+              const uint32_t take = min(qn, 64u * ILP);
+              float gp[ILP][6], pp[ILP][4];
+              uint32_t nt[ILP];
+              auto load = [&](int u) {
+                uint32_t pos = qh + 64u * u + lane;
+                if (pos >= kRing) pos -= kRing;
+                // a lane without a pair works on element 0 and drops the result
+                const uint32_t code = 64u * u + lane < take ? pq[pos] : 0u;
                 const uint32_t e = code & 0x3fffu, T = code >> 14;
                 const uint4 *rec = erec + 3 * e;
                 const uint4 r0 = rec[0], r1 = rec[1];
@@ -1104,54 +1187,70 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
                 const float g[6] = {__uint_as_float(r0.z) * sc, __uint_as_float(r0.w) * sc,
                                     __uint_as_float(r1.x) * sc, __uint_as_float(r1.y) * sc,
                                     __uint_as_float(r1.z) * sc, __uint_as_float(r1.w) * sc};
-                const uint32_t nd[4] = {r0.x & 0x7fffu, (r0.x >> 16) & 0x7fffu, r0.y & 0xffffu,
-                                        r0.y >> 16};
                 // relabel so that the target is node 3 (others T+1, T+2, T+3):
-                // the same candidate as for node position T
+                // the same candidate as for node position T.  The node ids
+                // rotate as one 64-bit word.
+                const uint64_t ids = (uint64_t)r0.y << 32 | (r0.x & 0x7fff7fffu);
+                const uint64_t rot = ids >> (16u * T) | ids << ((64u - 16u * T) & 63u);
                 const bool t1 = T & 1u, t2 = T & 2u;
                 auto sel = [&](float x0, float x1, float x2, float x3) {
                   return t2 ? (t1 ? x3 : x2) : (t1 ? x1 : x0);
                 };
-                auto seli = [&](uint32_t x0, uint32_t x1, uint32_t x2, uint32_t x3) {
-                  return t2 ? (t1 ? x3 : x2) : (t1 ? x1 : x0);
-                };
                 // edge (i,j) of the relabelled element for T = 0, 1, 2, 3
-                const float gp[6] = {sel(g[2], g[5], g[3], g[0]), sel(g[4], g[1], g[4], g[1]),
-                                     sel(g[5], g[3], g[0], g[2]), sel(g[0], g[2], g[5], g[3]),
-                                     sel(g[1], g[4], g[1], g[4]), sel(g[3], g[0], g[2], g[5])};
-                const uint32_t n1 = seli(nd[1], nd[2], nd[3], nd[0]);
-                const uint32_t n2 = seli(nd[2], nd[3], nd[0], nd[1]);
-                const uint32_t n3 = seli(nd[3], nd[0], nd[1], nd[2]);
-                const uint32_t nt = seli(nd[0], nd[1], nd[2], nd[3]);
-                const float pp[4] = {phi_l[n1], phi_l[n2], phi_l[n3], phi_l[nt]};
+                gp[u][0] = sel(g[2], g[5], g[3], g[0]);
+                gp[u][1] = t1 ? g[1] : g[4];
+                gp[u][2] = sel(g[5], g[3], g[0], g[2]);
+                gp[u][3] = sel(g[0], g[2], g[5], g[3]);
+                gp[u][4] = t1 ? g[4] : g[1];
+                gp[u][5] = sel(g[3], g[0], g[2], g[5]);
+                nt[u] = (uint32_t)rot & 0xffffu;
+                pp[u][0] = phi_l[(uint32_t)rot >> 16];
+                pp[u][1] = phi_l[(uint32_t)(rot >> 32) & 0xffffu];
+                pp[u][2] = phi_l[(uint32_t)(rot >> 48)];
+                pp[u][3] = phi_l[nt[u]];
+              };
+              auto value = [&](int u) {
                 float sq[6], rc[6];
   #pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                  rc[k] = __builtin_amdgcn_rcpf(gp[k]);
-                  sq[k + 3] = csqrt(gp[k + 3]);
+                  rc[k] = __builtin_amdgcn_rcpf(gp[u][k]);
+                  sq[k + 3] = csqrt(gp[u][k + 3]);
                   sq[k] = 0.0f;
                   rc[k + 3] = 0.0f;
                 }
-                const float c = cand_exact_sh<3, float>(gp, sq, rc, pp, F_INF);
+                return cand_exact_sh<3, float>(gp[u], sq, rc, pp[u], F_INF);
+              };
+              auto commit = [&](int u, float c) {
                 ++vupd;
-                if (c < pp[3]) {
-                  const uint32_t cbits = __float_as_uint(c);
+                if (c < pp[u][3]) {
                   // below the staged time: the minimum ends below it too, so the
                   // written bit needs no returned value
-                  atomicMin(&phi_n[nt], cbits);
-                  atomicOr(&wrt[nt >> 5], 1u << (nt & 31));
+                  atomicMin(&phi_n[nt[u]], __float_as_uint(c));
+                  atomicOr(&wrt[nt[u] >> 5], 1u << (nt[u] & 31));
                 }
+              };
+              if constexpr (ILP == 1) {
+                if (lane < take) {
+                  load(0);
+                  commit(0, value(0));
+                }
+              } else {
+                load(0);
+                load(1);
+                const float c0 = value(0), c1 = value(1);
+                if (lane < take) commit(0, c0);
+                if (64u + lane < take) commit(1, c1);
               }
               qh += take;
-              if (qh >= kPairRing) qh -= kPairRing;
+              if (qh >= kRing) qh -= kRing;
               qn -= take;
               __builtin_amdgcn_wave_barrier();
             }
             if (!more) break;
           }
         } else {
-          for (uint32_t i = tid; i < nact; i += BS) {
-            const uint32_t e = elist[i];
+          for (uint32_t i = lane; i < nact; i += 64) {
+            const uint32_t e = wlist[i];
             const uint4 r0 = erec[3 * e], r1 = erec[3 * e + 1];
             const float sc = rsl[((r0.x >> 15) & 1u) | ((r0.x >> 30) & 2u)];
             const float g[6] = {__uint_as_float(r0.z) * sc, __uint_as_float(r0.w) * sc,
@@ -1192,27 +1291,26 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     #undef FIM_TARGET
           }
         }
-        __syncthreads();
-        if (tid == 0) misc[0] = 0u;  // every thread has read the element count
-        if (listed <= elcap) break;  // uniform: read after a barrier
-        __syncthreads();
+        __builtin_amdgcn_wave_barrier();
       }
+      __syncthreads();
       // accept the written vertices: the sources of the next sweep
-      for (uint32_t l0 = 0; l0 < nv64; l0 += BS) {
-        const uint32_t l = l0 + tid;
-        const uint32_t wb = l0 + wave * 64;
-        if (wb < nv64) {
-          const uint32_t k = wb >> 5;
-          // a block of 64 copies with nothing written has no sources
-          if ((wrt[k] | wrt[k + 1]) == 0u) {  // uniform: same LDS words
-            if (lane == 0) {
-              flg[k] = 0u;
-              flg[k + 1] = 0u;
-            }
-            continue;
-          }
+      // lane i of a wave looks at its block i of 64 copies: blocks with nothing
+      // written have no sources, the others are gone through
+      for (uint32_t b0 = wave; b0 < nv64 / 64; b0 += BS) {
+        const uint32_t bl = b0 + lane * (BS / 64);
+        uint2 wr = make_uint2(0u, 0u);
+        if (bl < nv64 / 64) {
+          wr = reinterpret_cast<const uint2 *>(wrt)[bl];
+          if ((wr.x | wr.y) == 0u) reinterpret_cast<uint2 *>(flg)[bl] = make_uint2(0u, 0u);
+        }
+        for (uint64_t some = __ballot((wr.x | wr.y) != 0u); some; some &= some - 1) {
+          const int i = __ffsll((unsigned long long)some) - 1;
+          const uint32_t k = 2 * (b0 + (uint32_t)i * (BS / 64)), l = 32 * k + lane;
+          const uint64_t w = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(wr.y, i) << 32 |
+                             (uint32_t)__builtin_amdgcn_readlane(wr.x, i);
           bool sg = false, lt = false, dc = false;
-          if (l < nn && ((wrt[l >> 5] >> (l & 31)) & 1u)) {
+          if ((w >> lane) & 1u) {
             const float ov = phi_l[l];
             const float nv = __uint_as_float(phi_n[l]);
             if (nv < ov) {
@@ -1252,32 +1350,53 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     for (uint32_t k = tid; k < new32; k += BS) cnt += __popc(eseen[k]);
     cnt = wave_sum_small<9>(cnt);  // at most 8 words of 32 per thread
     if (lane == 0 && cnt) atomicAdd(&misc[3], cnt);
-    // write back decreased copies and list the lowered interface copies (in
-    // the source list's space); deferred vertices (and sources left by the
-    // sweep cap) stay dirty and the submesh is queued again
+    if (lane == 0 && evals) atomicAdd(&misc[0], evals);
+    // write back decreased copies and list the lowered interface copies
+    // (interface entry << 16 | copy, in the space of the candidate minima);
+    // deferred vertices (and sources left by the sweep cap) stay dirty and the
+    // submesh is queued again.  Lane i of a wave looks at its block i of 64
+    // copies; blocks with nothing lowered or left dirty are skipped.
     const KArgs ke = kargs();
+    tid = fresh(tid);
     float *phi_e = ke->phi + (size_t)inst * ke->ncopy + si.coff;
     uint8_t *dirty_e = ke->dirty + (size_t)inst * ke->ncopy + si.coff;
     uint32_t dmin = 0xffffffffu;  // earliest time left dirty, per lane
-    for (uint32_t l0 = 0; l0 < nv64; l0 += BS) {
-      const uint32_t l = l0 + tid;  // uniform trip count: ballots below
-      const uint32_t k = (l0 + wave * 64) >> 5;
-      // blocks of 64 copies with nothing lowered or left dirty are skipped
-      if (l0 + wave * 64 >= nv64 ||
-          (tch[k] | tch[k + 1] | dfr[k] | dfr[k + 1] | (capped ? (flg[k] | flg[k + 1]) : 0u)) == 0u)
-        continue;  // uniform across the wave
-      bool p = false;
-      if (l < nn) {
-        if (flag_at(tch, l)) {
-          phi_e[l] = phi_l[l];
-          p = flag_at(ifc, l);
-        }
-        if (flag_at(dfr, l) || (capped && flag_at(flg, l))) {
-          dirty_e[l] = 1;
-          dmin = min(dmin, __float_as_uint(phi_l[l]));
+    for (uint32_t b0 = wave; b0 < nv64 / 64; b0 += BS) {
+      const uint32_t bl = b0 + lane * (BS / 64);
+      uint2 tc = make_uint2(0u, 0u), df = tc;
+      if (bl < nv64 / 64) {
+        tc = reinterpret_cast<const uint2 *>(tch)[bl];
+        df = reinterpret_cast<const uint2 *>(dfr)[bl];
+        if (capped) {
+          const uint2 fl = reinterpret_cast<const uint2 *>(flg)[bl];
+          df.x |= fl.x;
+          df.y |= fl.y;
         }
       }
-      wave_append(p, l, vlist, &misc[npush]);
+      for (uint64_t some = __ballot((tc.x | tc.y | df.x | df.y) != 0u); some; some &= some - 1) {
+        const int i = __ffsll((unsigned long long)some) - 1;
+        const uint32_t l = 64 * (b0 + (uint32_t)i * (BS / 64)) + lane;
+        const uint64_t t = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(tc.y, i) << 32 |
+                           (uint32_t)__builtin_amdgcn_readlane(tc.x, i);
+        const uint64_t q = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(df.y, i) << 32 |
+                           (uint32_t)__builtin_amdgcn_readlane(df.x, i);
+        const float v = phi_l[l];
+        bool p = false;
+        if ((t >> lane) & 1u) {
+          phi_e[l] = v;
+          p = flag_at(ifc, l);
+        }
+        if ((q >> lane) & 1u) {
+          dirty_e[l] = 1;
+          dmin = min(dmin, __float_as_uint(v));
+        }
+        const uint64_t m = __ballot(p);
+        if (m == 0) continue;
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&misc[npush], (uint32_t)__popcll(m));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (p) phi_n[at + (uint32_t)__popcll(m & lanes_below())] = (ipre[l >> 5] + bits_below(ifc, l)) << 16 | l;
+      }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) dmin = min(dmin, (uint32_t)__shfl_xor(dmin, off));
@@ -1288,7 +1407,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
       if (it > 0) {  // pushes that lowered nothing make no activation
         ctr[0] += 1ull;
         ctr[1] += it;
-        ctr[2] += evals;
+        ctr[2] += misc[0];
         ctr[3] += 32ull * misc[3] + 10ull * nn + 12ull * si.ni;
       }
       end_item(ke, nq, inst, s, iter_now, item.pushed, __uint_as_float(misc[5]));
@@ -1296,12 +1415,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     // the last waves first: the first wave, which ends the item, is free to
     // fetch the next one meanwhile
     for (uint32_t i = BS - 1 - tid, n = misc[npush]; i < n; i += BS) {
-      const uint32_t l = vlist[i], w = l >> 5;
-      const uint32_t j = ipre[w] + __popc(ifc[w] & ((1u << (l & 31)) - 1u));
-      push_entry(ke, nq, inst, si.ioff + j, __float_as_uint(phi_l[l]), iter_now);
+      const uint32_t q = phi_n[i];
+      push_entry(ke, nq, inst, si.ioff + (q >> 16), __float_as_uint(phi_l[q & 0xffffu]), iter_now);
     }
-    // no barrier: what the push reads (times, list, interface bits) is written
-    // again only after the next item's first barrier, its count is another word
+    // no barrier: what the push reads (times, list) is written again only after
+    // the next item's first barrier, its count is another word
     npush ^= 1u;
   }
   unsigned long long *stats = kargs()->stats;
@@ -1311,8 +1429,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     atomicAdd(&stats[2], ctr[2]);
     atomicAdd(&stats[4], ctr[3]);
   }
-  for (int off = 32; off > 0; off >>= 1) vupd += __shfl_xor(vupd, off);
-  if (lane == 0 && vupd) atomicAdd(&stats[5], vupd);
+  unsigned long long vsum = vupd;
+  for (int off = 32; off > 0; off >>= 1) vsum += __shfl_xor(vsum, off);
+  if (lane == 0 && vsum) atomicAdd(&stats[5], vsum);
 }
 
 // Merges what is left in the inbox (the run stopped before the items it was
@@ -2226,7 +2345,7 @@ struct fim_ctx {
   uint32_t *d_n2e_dsp = nullptr, *d_n2n_dsp = nullptr;
   uint16_t *d_n2e_le = nullptr, *d_n2n_lv = nullptr;
   uint8_t *d_n2e_pos = nullptr;
-  uint4 *d_erec = nullptr, *d_adj = nullptr;
+  uint4 *d_erec = nullptr, *d_adj = nullptr, *d_adj_more = nullptr;
   uint32_t *d_adj_ptr = nullptr;
   // converge state
   float *d_phi = nullptr, *d_rscale = nullptr;
@@ -2291,54 +2410,34 @@ struct fim_ctx {
 
 namespace {
 
-const void *conv_kernel_ptr(bool staged, int block, int wpe, bool pairs);
-
-void launch_conv_compute(fim_ctx *c, const ConvArgs &a) {
-  if (c->o.staged) {
-    switch (c->block) {
-      case 64: k_conv_compute<64, true><<<c->grid, 64, c->lds_conv, c->stream>>>(a); break;
-      case 128: k_conv_compute<128, true><<<c->grid, 128, c->lds_conv, c->stream>>>(a); break;
-      case 512: k_conv_compute<512, true><<<c->grid, 512, c->lds_conv, c->stream>>>(a); break;
-      default: k_conv_compute<256, true><<<c->grid, 256, c->lds_conv, c->stream>>>(a); break;
-    }
-  } else {
-    switch (c->block) {
-      case 64: k_conv_band<64, 8, false><<<c->grid, 64, c->lds_conv, c->stream>>>(a); break;
-      case 128: k_conv_band<128, 8, false><<<c->grid, 128, c->lds_conv, c->stream>>>(a); break;
-      case 512:
-        if (c->band_pairs) k_conv_band<512, 8, true><<<c->grid, 512, c->lds_conv, c->stream>>>(a);
-        else k_conv_band<512, 8, false><<<c->grid, 512, c->lds_conv, c->stream>>>(a);
-        break;
-      default: {
-        const void *f = conv_kernel_ptr(false, 256, c->band_wpe, c->band_pairs);
-        void *args[] = {const_cast<ConvArgs *>(&a)};
-        HIPCHECK(hipLaunchKernel(f, dim3(c->grid), dim3(256), args, c->lds_conv, c->stream));
-        break;
-      }
-    }
-  }
-  HIPCHECK(hipGetLastError());
-}
-
 const void *conv_kernel_ptr(bool staged, int block, int wpe, bool pairs) {
   switch (block) {
     case 64: return staged ? (const void *)k_conv_compute<64, true> : (const void *)k_conv_band<64, 8, false>;
     case 128: return staged ? (const void *)k_conv_compute<128, true> : (const void *)k_conv_band<128, 8, false>;
-    case 512: return staged ? (const void *)k_conv_compute<512, true>
-                            : (pairs ? (const void *)k_conv_band<512, 8, true> : (const void *)k_conv_band<512, 8, false>);
+    case 512:
+      if (staged) return (const void *)k_conv_compute<512, true>;
+      if (!pairs) return (const void *)k_conv_band<512, 8, false>;
+      return wpe <= 4 ? (const void *)k_conv_band<512, 4, true> : (const void *)k_conv_band<512, 8, true>;
     default:
       if (staged) return (const void *)k_conv_compute<256, true>;
       if (pairs) {
+        if (wpe <= 4) return (const void *)k_conv_band<256, 4, true>;
         if (wpe == 5) return (const void *)k_conv_band<256, 5, true>;
         if (wpe == 6) return (const void *)k_conv_band<256, 6, true>;
         if (wpe == 7) return (const void *)k_conv_band<256, 7, true>;
         return (const void *)k_conv_band<256, 8, true>;
       }
-      if (wpe == 5) return (const void *)k_conv_band<256, 5, false>;
+      if (wpe <= 5) return (const void *)k_conv_band<256, 5, false>;
       if (wpe == 6) return (const void *)k_conv_band<256, 6, false>;
       if (wpe == 7) return (const void *)k_conv_band<256, 7, false>;
       return (const void *)k_conv_band<256, 8, false>;
   }
+}
+
+void launch_conv_compute(fim_ctx *c, const ConvArgs &a) {
+  void *args[] = {const_cast<ConvArgs *>(&a)};
+  HIPCHECK(hipLaunchKernel(conv_kernel_ptr(c->o.staged != 0, c->block, c->band_wpe, c->band_pairs), dim3(c->grid),
+                           dim3(c->block), args, c->lds_conv, c->stream));
 }
 
 void set_lds_attr(fim_ctx *c) {
@@ -2631,21 +2730,37 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         // workgroups of 256 and 512 evaluate (element, target) pairs when
         // local element ids fit 14 bits; the pair rings live in the source list
         c->band_pairs = !o->staged && (c->block == 256 || c->block == 512) && c->ne_max < (1 << 14);
+        c->unit = o->unit > 0 ? (uint32_t)o->unit : 2u;
+        c->maxch = (c->ninst + c->unit - 1) / c->unit;
+        if ((uint64_t)c->nsub * c->maxch >= (1ull << 32)) throw Error(FIM_ELIMIT, "too many work units");
+        // a bucket that fits one unit is planned by its first item; only
+        // batches of more instances need the plan kernel (4 us, and as much
+        // again between two launches, out of 60 for an iteration of a single
+        // solve on the 2M-tet slab)
+        c->direct_plan = c->maxch == 1;
+        int ncu = 256;
+        HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->dev));
+        // A list of at most one unit per submesh leaves the CUs with a few waves
+        // each when the mesh has few submeshes: the kernel gets registers for
+        // two pair rounds side by side then (ILP of k_conv_band)
+        const bool few = c->band_pairs && c->direct_plan && o->waves == 0 && c->nsub <= 4u * (uint32_t)ncu;
+        if (few) c->band_wpe = 4;
         const uint32_t vlist_bytes =
             o->staged ? 0u
-                      : al16(std::max<uint32_t>(2 * nn64, c->band_pairs ? (uint32_t)(c->block / 64) * 2u * kPairRing : 0u));
+                      : al16(std::max<uint32_t>(2 * nn64, c->band_pairs ? (uint32_t)(c->block / 64) * 2u * pair_ring(few ? 2 : 1) : 0u));
         const uint32_t misc_bytes = o->staged ? 48u : kMiscBytes;  // staged: 8 words, 4 region factors
         const uint32_t tail_bytes = vlist_bytes + misc_bytes + (o->staged ? 0u : 3u * al16(4 * (nn64 / 32)));
-        // The band kernel lists at most elcap elements per pass: at least
-        // kElistCap, more if the LDS left over by the workgroups the wave
-        // slots admit (8 waves per SIMD) holds more
+        // The band kernel lists at most elcap elements per pass, an equal share
+        // per wave: all elements of a wave's words where they fit, else at least
+        // kElistCap, more if the LDS left over by the workgroups the wave slots
+        // admit (8 waves per SIMD) holds more
         uint32_t elcap = (uint32_t)c->ne_max;
         if (!o->staged) {
-          const uint32_t wg_slots = std::max<uint32_t>(1u, 32u / ((uint32_t)c->block / 64u));
+          const uint32_t nw = (uint32_t)c->block / 64u, wg_slots = std::max<uint32_t>(1u, 32u / nw);
           const uint32_t budget = (160u * 1024u / wg_slots) & ~15u;
           const uint32_t base = o_list + tail_bytes;
           const uint32_t room = budget > base ? ((budget - base) / 2u) & ~7u : 0u;
-          elcap = std::min<uint32_t>((uint32_t)c->ne_max, std::max<uint32_t>((uint32_t)kElistCap, room));
+          elcap = std::min<uint32_t>(32u * nw * ((ne32 + nw - 1u) / nw), std::max<uint32_t>((uint32_t)kElistCap, room));
         }
         const uint32_t o_vlist = o_list + al16(2 * elcap);
         const uint32_t o_misc = o_vlist + vlist_bytes;
@@ -2683,22 +2798,26 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
             }
           });
           c->d_erec = dupload(rec, ow);
-          std::vector<uint32_t> aptr(p.ncopy);
-          std::vector<uint16_t> adj;
+          // four words of eight element ids per copy (mark_incident)
+          std::vector<uint4> adj(4 * (size_t)p.ncopy), more;
+          std::vector<uint32_t> aptr(p.ncopy, 0u);
           for (int64_t cc = 0; cc < p.ncopy; ++cc) {
-            const uint32_t kb = p.n2e_dsp[cc], ke = p.n2e_dsp[cc + 1];
-            const uint32_t nch = (ke - kb + 7) / 8;
-            if (nch == 0 || nch > 63) throw Error(FIM_ELIMIT, "vertex with no or over 504 incident elements");
-            const size_t off = adj.size() / 8;
+            const uint32_t kb = p.n2e_dsp[cc], n = p.n2e_dsp[cc + 1] - kb;
+            if (n == 0 || n > 504) throw Error(FIM_ELIMIT, "vertex with no or over 504 incident elements");
+            uint16_t *q = reinterpret_cast<uint16_t *>(&adj[4 * (size_t)cc]);
+            for (uint32_t k = 0; k < 32; ++k) q[k] = p.n2e_le[kb + (k < n ? k : 0u)];
+            if (n <= 32) continue;
+            q[31] = (uint16_t)kAdjMore;
+            const size_t off = more.size(), words = (n - 31 + 7) / 8;
             if (off >= (1u << 26)) throw Error(FIM_ELIMIT, "adjacency above 2^26 chunks");
-            aptr[cc] = (uint32_t)(off << 6) | nch;
-            for (uint32_t k = kb; k < ke; ++k) adj.push_back(p.n2e_le[k]);
-            while (adj.size() % 8) adj.push_back(0xffffu);
+            aptr[cc] = (uint32_t)(off << 6 | words);
+            more.resize(off + words);
+            uint16_t *o = reinterpret_cast<uint16_t *>(&more[off]);
+            for (uint32_t k = 0; k < 8 * words; ++k) o[k] = p.n2e_le[kb + (31 + k < n ? 31 + k : 0u)];
           }
+          c->d_adj = dupload(adj, ow);
           c->d_adj_ptr = dupload(aptr, ow);
-          std::vector<uint4> adj4(adj.size() / 8);
-          std::memcpy(adj4.data(), adj.data(), adj.size() * 2);
-          c->d_adj = dupload(adj4, ow);
+          c->d_adj_more = dupload(more, ow);
         }
         c->d_if_l = dupload(p.if_l, ow);
         {
@@ -2758,14 +2877,6 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->d_act = dalloc<uint32_t>(2 * nss, ow);
         c->d_wake = dalloc<float>(nss, ow);
         c->d_wpush = dalloc<float>(2 * nss, ow);
-        c->unit = o->unit > 0 ? (uint32_t)o->unit : 2u;
-        c->maxch = (c->ninst + c->unit - 1) / c->unit;
-        if ((uint64_t)c->nsub * c->maxch >= (1ull << 32)) throw Error(FIM_ELIMIT, "too many work units");
-        // a bucket that fits one unit is planned by its first item; only
-        // batches of more instances need the plan kernel (4 us, and as much
-        // again between two launches, out of 60 for an iteration of a single
-        // solve on the 2M-tet slab)
-        c->direct_plan = c->maxch == 1;
         c->d_cnt = dalloc<uint32_t>(48, ow);  // 16 words per list
         for (int k = 0; k < 3; ++k) {
           c->wl[k].bcnt = dalloc<uint32_t>(c->nsub, ow);
@@ -2777,13 +2888,11 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->d_tmpf = dalloc<float>(c->nn, ow);
         k_fill<float><<<blocks_for(4 * (size_t)c->ninst, 256), 256, 0, c->stream>>>(c->d_rscale, 4 * (size_t)c->ninst, 1.0f);
         c->h_rscale.assign(4 * (size_t)c->ninst, 1.0f);
-        int ncu = 256;
-        HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->dev));
         // one resident wave of workgroups: registers, LDS and wave slots.
         // Workgroups of 256 put one wave on each SIMD, so the LDS carve
         // alone caps the waves per SIMD at 160 KB / carve; the band kernel
         // variant sized for that many waves gets the registers left over.
-        {
+        if (!few) {
           const uint32_t lds_cap = 160u * 1024u / std::max<uint32_t>(c->lds_conv, 1u);
           c->band_wpe = lds_cap <= 5u ? 5 : (lds_cap >= 8u ? 8 : (int)lds_cap);
           if (o->waves > 0) c->band_wpe = std::min(c->band_wpe, std::max(o->waves, 5));
@@ -2800,7 +2909,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->ca = ConvArgs{c->d_sub, c->d_e2n, c->d_geo32, c->d_hgt, c->d_ereg, c->d_rscale, c->d_phi,
                          c->d_dirty, c->d_act, c->d_wake, c->d_wpush, c->d_if_l, c->d_ifm, c->d_inbox, c->d_if_fo,
                          c->d_if_os, WorkList{}, WorkList{}, c->d_stats, nullptr, c->d_start,
-                         c->d_n2e_dsp, c->d_n2e_le, c->d_erec, c->d_adj_ptr, c->d_adj,
+                         c->d_n2e_dsp, c->d_n2e_le, c->d_erec, c->d_adj, c->d_adj_ptr, c->d_adj_more,
                          c->nsub, c->ncopy, c->ninst, c->direct_plan ? 1u : 0u,
                          (float)(o->eps_rel > 0 ? o->eps_rel : 1e-6),
                          c->d_winst, o->local_iters, c->unit, c->maxch, (uint32_t)p.if_l.size(),

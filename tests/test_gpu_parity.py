@@ -347,6 +347,47 @@ def test_converge_work_units_and_grid_change_nothing(unit, grid):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("block,max_nn", [(256, 300), (512, 300), (512, 1500)])
+def test_few_submesh_variant_agrees(block, max_nn):
+    """a list of at most one unit per submesh runs the variant that works on
+    two rounds of pairs at a time; waves=8 asks for the other: bitwise the same
+    maps"""
+    cfg = cases.scaled(cases.SLAB, 5)
+    m, _ = cases.box(cfg, seed=4)
+    p = F.Pack(m, F.PART_RCB, max_nn=max_nn, seed=4)
+    src = cases.pacing_sites(cfg, 3, seed=41)
+    maps = [_converge(m, p, src, block=block, waves=w, window=1500.0)[0] for w in (0, 8)]
+    assert np.array_equal(maps[0], maps[1])
+
+
+@pytest.mark.parametrize("n", [14, 20, 60, 240])
+def test_vertices_of_many_elements(n):
+    """a fan of tets around one vertex, and each of them split once: 24, 36,
+    116 and 476 elements at the centre (below and above the 32 ids that a copy
+    keeps in a row), against the FP64 oracle"""
+    from scipy.spatial import ConvexHull
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(n, 3))
+    x *= 5000.0 / np.linalg.norm(x, axis=1, keepdims=True)
+    tri = ConvexHull(x).simplices
+    out = 2.0 * x
+    xyz = np.concatenate([[[0.0, 0.0, 0.0]], x, out])
+    e2n = [[0, 1 + a, 1 + b, 1 + c] for a, b, c in tri]
+    for t in tri:  # the prism outside each face, split along ascending ids
+        a, b, c = sorted(int(v) for v in t)
+        A, B, C = 1 + n + a, 1 + n + b, 1 + n + c
+        e2n += [[1 + a, 1 + b, 1 + c, C], [1 + a, 1 + b, B, C], [1 + a, A, B, C]]
+    e2n = np.array(e2n)
+    m = F.Mesh.from_arrays(xyz, e2n)
+    xyz, e2n, _ = m.arrays()
+    fib, vel = m.material()
+    om = O.Mesh(xyz, e2n, fib=fib, vel=vel)
+    for src in ([n + 1], [0]):
+        phi, _, _, _, _ = _converge(m, F.Pack(m, F.PART_RCB, max_nn=4096, seed=1), src)
+        ref, _ = O.fim_solve(om, src, variant=O.LOCAL_EXACT)
+        _check_fp32(phi, ref)
+
+
 @pytest.mark.parametrize("n_inst,unit", [(1, 0), (3, 4), (5, 2)])
 def test_interrupted_runs_change_nothing(n_inst, unit):
     """a run stopped after a few iterations, with pushes on their way to the
