@@ -10,7 +10,7 @@
 // 64 inputs, the padding weights stay zero):
 //   W0[256 x 64] b0[256]  (W_l[256 x 256] b_l[256]) x 5  w_out[256] b_out
 // A training step is three kernels:
-//   k_mlp_chain<true>: per tile of 64 rows, the six forward layers with the
+//   k_mlp_chain: per tile of 64 rows, the six forward layers with the
 //     activations kept in LDS, the output layer and squared error, and the
 //     five backward-data layers dZ_{l-1} = (dZ_l W_l) * SiLU'(Z_{l-1});
 //     Z_0..Z_4 and dZ_0..dZ_5 leave the tile for the weight gradients;
@@ -18,7 +18,7 @@
 //     partial sums over spans of rows (H = SiLU(Z) recomputed from Z);
 //   k_reduce_parts + k_adam: the sum of the partials, the Adam update and
 //     the BF16 weight copies.
-// Prediction is k_mlp_chain<false> (forward and output layer only).
+// Prediction is k_mlp_infer (forward and output layer only).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -140,10 +140,12 @@ constexpr size_t CHAIN_LDS = (size_t)TR * HP * 2 + (HID + TR + 2) * 4;
 // 64 fg + 32 j) = T(rows, 0..K) B, with T the tile in LDS (row-major, pitch
 // HP) and B given by fragments (fragment (mb, ks) of B^T at bfr).  The next
 // step's weight fragments are loaded before the current step's products.
-template <int K>
+// The first K of KW inputs take part; SWAP gives the transposed product
+// (accumulator rows are features, columns rows of the tile).
+template <int K, int KW, bool SWAP>
 __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restrict__ bfr, uint32_t rg, uint32_t fg,
                                     uint32_t lane, f32x16 (&acc)[2][2]) {
-  constexpr int NS = K / 16;
+  constexpr int NS = K / 16, NW = KW / 16;
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -151,16 +153,18 @@ __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restri
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-  const u16x8 *bp0 = reinterpret_cast<const u16x8 *>(bfr) + (size_t)(2 * fg) * NS * 64 + lane;
-  const u16x8 *bp1 = bp0 + NS * 64;
+  const u16x8 *bp0 = reinterpret_cast<const u16x8 *>(bfr) + (size_t)(2 * fg) * NW * 64 + lane;
+  const u16x8 *bp1 = bp0 + NW * 64;
   const uint16_t *ta0 = Ts + (64 * rg + l32) * HP + 8 * lh;
   const uint16_t *ta1 = ta0 + 32 * HP;
   // weight fragments two steps ahead, tile fragments one step ahead
   u16x8 b[2][2], t[2][2];
   b[0][0] = bp0[0];
   b[0][1] = bp1[0];
-  b[1][0] = bp0[64];
-  b[1][1] = bp1[64];
+  if (NS > 1) {
+    b[1][0] = bp0[64];
+    b[1][1] = bp1[64];
+  }
   t[0][0] = *reinterpret_cast<const u16x8 *>(ta0);
   t[0][1] = *reinterpret_cast<const u16x8 *>(ta1);
 #pragma unroll
@@ -170,10 +174,11 @@ __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restri
       t[c ^ 1][0] = *reinterpret_cast<const u16x8 *>(ta0 + 16 * (s + 1));
       t[c ^ 1][1] = *reinterpret_cast<const u16x8 *>(ta1 + 16 * (s + 1));
     }
-    acc[0][0] = mfma(t[c][0], b[c][0], acc[0][0]);
-    acc[0][1] = mfma(t[c][0], b[c][1], acc[0][1]);
-    acc[1][0] = mfma(t[c][1], b[c][0], acc[1][0]);
-    acc[1][1] = mfma(t[c][1], b[c][1], acc[1][1]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[i][j] = SWAP ? mfma(b[c][j], t[c][i], acc[i][j]) : mfma(t[c][i], b[c][j], acc[i][j]);
     if (s + 2 < NS) {
       b[c][0] = bp0[(s + 2) * 64];
       b[c][1] = bp1[(s + 2) * 64];
@@ -188,13 +193,12 @@ struct ChainArgs {
   const uint16_t *X0;        // inputs, k-step layout, K0 columns
   const uint16_t *wb, *wbt;  // fragment-ordered BF16 weights
   const float *w;            // FP32 masters (biases, output layer)
-  const float *tgt;          // training: targets / t_scale
-  uint16_t *Z[NL - 1];       // training: Z_0..Z_4, k-step layout
-  uint16_t *dZ[NL];          // training: dZ_0..dZ_5, k-step layout
-  float *g, *loss;           // training: output-layer gradient (accumulated), loss sum
-  float *out;                // inference: predictions
+  const float *tgt;          // targets / t_scale
+  uint16_t *Z[NL - 1];       // Z_0..Z_4, k-step layout
+  uint16_t *dZ[NL];          // dZ_0..dZ_5, k-step layout
+  float *g, *loss;           // output-layer gradient (accumulated), loss sum
   uint32_t nreal;            // rows with data; the rest of the last tile is padding
-  float inv_b, t_scale, delta;
+  float inv_b;
 };
 
 // The whole network for one tile of TR = 64 RG rows, activations in LDS
@@ -202,14 +206,12 @@ struct ChainArgs {
 // 4; RG = 1, so one group of four waves), columns 64 fg .. +63 (fg = wave % 4)
 // of every product, as 2 x 2 accumulators of 32 x 32.
 //   forward: Z_l = H_{l-1} W_l^T + b_l, H_l = SiLU(Z_l) (BF16 in LDS; Z_l to
-//     HBM in the k-step layout when training);
-//   output: y = H_5 . w_out + b_out (inference: t = y t_scale + delta);
-//   training: e = y - t, dZ_5 = (2 e / B) w_out SiLU'(Z_5), the output-layer
+//     HBM in the k-step layout);
+//   output: y = H_5 . w_out + b_out, e = y - t, dZ_5 = (2 e / B) w_out SiLU'(Z_5), the output-layer
 //     gradient, then dZ_{l-1} = (dZ_l W_l) * SiLU'(Z_{l-1}) for l = 5..1 with
 //     dZ_l in LDS; every dZ_l goes to HBM in the k-step layout.
 // Rounding to BF16 where the separate-kernel formulation stores values:
 // Z, H and dZ; SiLU'(Z) of the stored Z.
-template <bool TRAIN>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_mlp_chain(ChainArgs a) {
   extern __shared__ __align__(16) unsigned char chain_lds[];
   uint16_t *Ts = reinterpret_cast<uint16_t *>(chain_lds);
@@ -240,9 +242,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 #pragma unroll 1
   for (int l = 0; l < NL; ++l) {
     if (l == 0)
-      tile_product<K0>(Ts, a.wb + offb_w(0), rg, fg, lane, acc);
+      tile_product<K0, K0, false>(Ts, a.wb + offb_w(0), rg, fg, lane, acc);
     else
-      tile_product<HID>(Ts, a.wb + offb_w(l), rg, fg, lane, acc);
+      tile_product<HID, HID, false>(Ts, a.wb + offb_w(l), rg, fg, lane, acc);
     __syncthreads();  // every wave has read the layer's input
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -253,7 +255,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] += bias;
     }
-    uint16_t *zl = TRAIN && l < NL - 1 ? a.Z[l] + r0 * HID : nullptr;
+    uint16_t *zl = l < NL - 1 ? a.Z[l] + r0 * HID : nullptr;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -289,10 +291,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     p += __shfl_xor(p, 2);
     const float y = p + a.w[OFF_BO];
     const size_t grow = r0 + row;
-    if (!TRAIN) {
-      if ((tid & 3u) == 0 && grow < a.nreal) a.out[grow] = y * a.t_scale + a.delta;
-      return;
-    }
     const float e = grow < a.nreal ? y - a.tgt[grow] : 0.0f;
     const float dy = 2.0f * e * a.inv_b;
     if ((tid & 3u) == 0) dys[row] = dy;
@@ -341,7 +339,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   // backward through the hidden layers
 #pragma unroll 1
   for (int l = NL - 1; l >= 1; --l) {
-    tile_product<HID>(Ts, a.wbt + offbt(l), rg, fg, lane, acc);
+    tile_product<HID, HID, false>(Ts, a.wbt + offbt(l), rg, fg, lane, acc);
     __syncthreads();  // every wave has read dZ_l
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -369,6 +367,110 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     }
     __syncthreads();
   }
+}
+
+// ---------------------------------------------------------------------------
+// Inference: the same forward pass, t = y t_scale + delta, with the products
+// transposed (Z_l^T = W_l H_{l-1}^T, the same sums in the same order): a lane's
+// accumulators then hold four neighbouring features of one row, which leave as
+// one 8-byte LDS write of two packed conversions, where the training kernel
+// (whose HBM layout wants four rows of one feature) writes four single values.
+// Per 64-row tile and layer a wave has 2,048 cycles of matrix work, about as
+// much VALU work in its epilogue (64 values: two transcendentals and five more
+// instructions each) and 2,048 cycles of weight fragments through the L1, so the
+// shorter epilogue is what the form gives: 362,894 rows in 267 us (0.90
+// PFLOP/s; a large library product reaches 1.2),
+// from 285 us and 10 us more to write the input rows.
+// The input rows are made here, not read back from memory: row r is given
+// (x), or solve r / m at vertex sample[r % m] (r itself without a sample).
+// The first product needs one k-step for the 16 inputs, not the padded four.
+// ---------------------------------------------------------------------------
+struct InferArgs {
+  const float *x;             // given rows (n x 16), or null
+  const float *coords, *mp;   // normalised coordinates; per solve MAPP parameters
+  const uint32_t *sample;     // m vertices, or null
+  uint32_t m;
+  const uint16_t *wb;
+  const float *w;
+  float *out;
+  uint32_t nreal;
+  float t_scale, delta;
+};
+
+constexpr int MAPP = 16;  // per map: 13 floats = three normalised site positions, four factors - 1
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_mlp_infer(InferArgs a) {
+  extern __shared__ __align__(16) unsigned char chain_lds[];
+  uint16_t *Ts = reinterpret_cast<uint16_t *>(chain_lds);
+  float *wos = reinterpret_cast<float *>(chain_lds + TR * HP * 2);  // w_out
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, fg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t l32 = lane & 31u, lh = lane >> 5;
+  const uint32_t r0 = blockIdx.x * TR;
+  wos[tid] = a.w[OFF_WO + tid];
+  {
+    // four threads a row, four inputs each; rows past the end repeat the last
+    const uint32_t row = tid >> 2, c0 = (tid & 3u) * 4, r = min(r0 + row, a.nreal - 1u);
+    float f[4];
+    if (a.x) {
+      const float4 v = *reinterpret_cast<const float4 *>(a.x + (size_t)r * NIN + c0);
+      f[0] = v.x;
+      f[1] = v.y;
+      f[2] = v.z;
+      f[3] = v.w;
+    } else {
+      const uint32_t j = a.sample ? r / a.m : 0u, v = a.sample ? a.sample[r - j * a.m] : r;
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t c = c0 + k;
+        f[k] = c < 3 ? a.coords[3 * (size_t)v + c] : a.mp[MAPP * (size_t)j + (c - 3)];
+      }
+    }
+    u16x4 h;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) h[k] = f2bf(f[k]);
+    *reinterpret_cast<u16x4 *>(Ts + row * HP + c0) = h;
+  }
+  __syncthreads();
+  f32x16 acc[2][2];
+#pragma unroll 1
+  for (int l = 0; l < NL; ++l) {
+    const uint16_t *wl = a.wb + offb_w(l);
+    if (l == 0)
+      tile_product<NIN, K0, true>(Ts, wl, 0, fg, lane, acc);
+    else
+      tile_product<HID, HID, true>(Ts, wl, 0, fg, lane, acc);
+    const float *bl = a.w + off_b(l) + 64 * fg + 4 * lh;
+    __syncthreads();  // every wave has read the layer's input
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 b = *reinterpret_cast<const float4 *>(bl + 32 * j + 8 * q);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          u16x4 h;
+          h[0] = f2bf(silu(acc[i][j][4 * q] + b.x));
+          h[1] = f2bf(silu(acc[i][j][4 * q + 1] + b.y));
+          h[2] = f2bf(silu(acc[i][j][4 * q + 2] + b.z));
+          h[3] = f2bf(silu(acc[i][j][4 * q + 3] + b.w));
+          *reinterpret_cast<u16x4 *>(Ts + (32 * i + l32) * HP + 64 * fg + 32 * j + 8 * q + 4 * lh) = h;
+        }
+      }
+    __syncthreads();
+  }
+  // output layer: four threads per row, 64 columns each
+  const uint32_t row = tid >> 2, c0 = (tid & 3u) * 64;
+  float p = 0.0f;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const u16x8 h = *reinterpret_cast<const u16x8 *>(Ts + row * HP + c0 + 8 * u);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) p += bf2f(h[k]) * wos[c0 + 8 * u + k];
+  }
+  p += __shfl_xor(p, 1);
+  p += __shfl_xor(p, 2);
+  const float y = p + a.w[OFF_BO];
+  if ((tid & 3u) == 0 && r0 + row < a.nreal) a.out[r0 + row] = y * a.t_scale + a.delta;
 }
 
 // ---------------------------------------------------------------------------
@@ -529,9 +631,6 @@ __device__ inline uint64_t mix64(uint64_t x) {
   return x ^ (x >> 31);
 }
 
-// per map: 13 floats = three normalised site positions, four factors - 1
-constexpr int MAPP = 16;
-
 // the 16 inputs of one row into X0 (k-step layout; the padding columns
 // NIN..K0-1 are zero from the start and never written)
 __device__ inline void write_features(uint16_t *X0, size_t row, const float *vxyz, const float *mp) {
@@ -558,24 +657,6 @@ __global__ void k_sample(const float *coords, const float *mparams, const float 
     const uint32_t j = (uint32_t)((h >> 32) % nmaps), v = (uint32_t)((h & 0xffffffffu) % nn);
     write_features(X0, m, coords + 3 * (size_t)v, mparams + MAPP * (size_t)j);
     tgt[m] = T[(size_t)j * nn + v] * inv_ts;
-  }
-}
-
-// rows of one map: every vertex (padding rows repeat vertex 0)
-__global__ void k_map_rows(const float *coords, const float *mp, uint32_t nn, uint32_t rows,
-                           uint16_t *X0) {
-  for (uint32_t m = blockIdx.x * blockDim.x + threadIdx.x; m < rows; m += gridDim.x * blockDim.x)
-    write_features(X0, m, coords + 3 * (size_t)(m < nn ? m : 0), mp);
-}
-
-// rows of several solves over one vertex sample: row r is solve r / m at
-// sample vertex r % m (padding rows repeat the last real row)
-__global__ void k_sample_rows(const float *coords, const float *mp, const uint32_t *sample, uint32_t m,
-                              uint32_t nreal, uint32_t rows, uint16_t *X0) {
-  for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
-    const uint32_t q = r < nreal ? r : nreal - 1;
-    const uint32_t j = q / m, v = sample[q - j * m];
-    write_features(X0, r, coords + 3 * (size_t)v, mp + MAPP * (size_t)j);
   }
 }
 
@@ -736,19 +817,12 @@ uint32_t tile_rows(uint32_t rows) { return (rows + TR - 1) / TR * TR; }
 
 float t_scale(const fim_nn *n) { return (float)(n->o.t_scale > 0 ? n->o.t_scale : 1e5); }
 
-// predictions for rows 0..nreal-1 of X0 (filled up to tile_rows(nreal)):
-// out[r] = y_r t_scale + delta
-void infer(fim_nn *n, uint32_t nreal, float delta, float *out) {
-  ChainArgs a{};
-  a.X0 = n->X0;
-  a.wb = n->wb;
-  a.wbt = n->wbt;
-  a.w = n->w;
-  a.out = out;
-  a.nreal = nreal;
-  a.t_scale = t_scale(n);
-  a.delta = delta;
-  k_mlp_chain<false><<<tile_rows(nreal) / TR, NT, CHAIN_LDS, n->stream>>>(a);
+// predictions out[r] = y_r t_scale + delta for the rows 0..nreal-1 that x, or
+// (coords, mp, sample, m), describe (InferArgs)
+void infer(fim_nn *n, const float *x, const float *mp, const uint32_t *sample, uint32_t m, uint32_t nreal, float delta,
+           float *out) {
+  const InferArgs a{x, n->coords, mp, sample, m, n->wb, n->w, out, nreal, t_scale(n), delta};
+  k_mlp_infer<<<(nreal + TR - 1) / TR, 256, CHAIN_LDS, n->stream>>>(a);
   HIPCHECK(hipGetLastError());
 }
 
@@ -771,7 +845,7 @@ void train_pass(fim_nn *n, uint32_t B) {
   a.loss = n->loss;
   a.nreal = B;
   a.inv_b = 1.0f / (float)B;
-  k_mlp_chain<true><<<rows / TR, NT, CHAIN_LDS, n->stream>>>(a);
+  k_mlp_chain<<<rows / TR, NT, CHAIN_LDS, n->stream>>>(a);
   // weight gradients: S spans of whole 32-row steps, one partial sum each
   const uint32_t S = std::min<uint32_t>(n->nsplit, rows / 32);
   WGradArgs wa;
@@ -852,13 +926,9 @@ int guarded(F &&f) {
 
 // prediction for all vertices of one solve into dst (device, nn floats)
 void predict_map_device(fim_nn *n, const std::vector<float> &mp, float delta, float *dst) {
-  const uint32_t rows = tile_rows(n->nn);
-  ensure_rows(n, rows);
-  HIPCHECK(hipMemcpyAsync(n->mparams + (size_t)n->max_maps * MAPP, mp.data(), MAPP * sizeof(float),
-                          hipMemcpyHostToDevice, n->stream));
-  k_map_rows<<<grid_for(rows), 256, 0, n->stream>>>(n->coords, n->mparams + (size_t)n->max_maps * MAPP,
-                                                    n->nn, rows, n->X0);
-  infer(n, n->nn, delta, dst);
+  float *md = n->mparams + (size_t)n->max_maps * MAPP;
+  HIPCHECK(hipMemcpyAsync(md, mp.data(), MAPP * sizeof(float), hipMemcpyHostToDevice, n->stream));
+  infer(n, nullptr, md, nullptr, 0u, n->nn, delta, dst);
 }
 
 }  // namespace
@@ -939,9 +1009,9 @@ int fim_nn_create(const fim_mesh *mesh, const fim_nn_opts *o, fim_nn **out) {
       n->tgt = nn_alloc<float>(n, n->cap);
       n->out = nn_alloc<float>(n, n->cap);
       n->parts = nn_alloc<float>(n, (size_t)n->nsplit * OFF_WO);
-      HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_chain<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_chain, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)CHAIN_LDS));
-      HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_chain<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_infer, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)CHAIN_LDS));
       HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_wgrad, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    WG_LDS * 2));
@@ -1119,15 +1189,13 @@ int fim_nn_predict(fim_nn *n, const float *x, int64_t count, float *t) {
     if (!n || (!x && count > 0) || (!t && count > 0) || count < 0) throw Error(FIM_EINVAL, "null argument");
     if (count == 0) return;
     if (count > (int64_t)n->cap) throw Error(FIM_ELIMIT, "batch larger than the surrogate's row capacity");
-    const uint32_t rows = tile_rows((uint32_t)count);
-    ensure_rows(n, rows);
+    ensure_rows(n, tile_rows((uint32_t)count));
     HIPCHECK(hipSetDevice(n->dev));
     float *xd = nullptr;
     HIPCHECK(hipMalloc(&xd, (size_t)count * NIN * sizeof(float)));
     try {
       HIPCHECK(hipMemcpyAsync(xd, x, (size_t)count * NIN * sizeof(float), hipMemcpyHostToDevice, n->stream));
-      k_input_rows<<<grid_for(rows), 256, 0, n->stream>>>(xd, (uint32_t)count, rows, n->X0);
-      infer(n, (uint32_t)count, 0.0f, n->out);
+      infer(n, xd, nullptr, nullptr, 0u, (uint32_t)count, 0.0f, n->out);
       HIPCHECK(hipMemcpyAsync(t, n->out, (size_t)count * sizeof(float), hipMemcpyDeviceToHost, n->stream));
       HIPCHECK(hipStreamSynchronize(n->stream));
     } catch (...) {
@@ -1171,10 +1239,7 @@ int fim_nn_predict_max(fim_nn *n, int32_t count, const int64_t *sites, const flo
       for (uint32_t j0 = 0; j0 < (uint32_t)count; j0 += per) {
         const uint32_t nj = std::min<uint32_t>(per, (uint32_t)count - j0);
         const uint32_t nreal = nj * (uint32_t)m;
-        const uint32_t rows = tile_rows(nreal);  // <= cap: cap is a whole number of tiles
-        k_sample_rows<<<grid_for(rows), 256, 0, n->stream>>>(n->coords, md + (size_t)j0 * MAPP, sd, (uint32_t)m,
-                                                             nreal, rows, n->X0);
-        infer(n, nreal, 0.0f, n->out);
+        infer(n, nullptr, md + (size_t)j0 * MAPP, sd, (uint32_t)m, nreal, 0.0f, n->out);
         k_solve_max<<<std::min<uint32_t>((nj + 3) / 4, 4096), 256, 0, n->stream>>>(n->out, (uint32_t)m, nj,
                                                                                   od + j0);
         HIPCHECK(hipGetLastError());

@@ -55,6 +55,28 @@ def test_forward_matches_oracle(small_slab):
     nn.close()
 
 
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 1000])
+def test_inference_tiles(small_slab, rows):
+    """Rows at and around the 64-row tile: the oracle's values, and each row
+    the same whatever tile and place it has and whichever form names it (a
+    given row, a vertex of a map, a sample vertex)."""
+    _, m = small_slab
+    nn = F.Surrogate(m, seed=1)
+    p = M.init_params(5)
+    nn.set_params(p)
+    sites, f = [3, m.nn // 2], np.array([0.7, 1.2, 1.0, 0.9], np.float32)
+    vtx = (np.arange(1000, dtype=np.int64) * 7) % m.nn
+    ref = M.forward(p, nn.features(vtx, sites, f))[0] * TS
+    vtx = vtx[:rows]
+    x = nn.features(vtx, sites, f)
+    y = nn.predict(x)
+    assert np.max(np.abs(y - ref[:rows])) <= 1e-2 * (np.ptp(ref) + 1e-3 * TS)
+    assert np.array_equal(nn.predict(x[::-1].copy())[::-1], y)
+    assert np.array_equal(nn.predict_map(sites, f)[vtx], y)
+    assert nn.predict_max([(sites, f)] * 3, vtx).tolist() == [y.max()] * 3
+    nn.close()
+
+
 @pytest.mark.parametrize("b", [256, 2112])
 def test_gradient_matches_oracle(small_slab, b):
     """b = 256: four row tiles, eight weight-gradient spans of one 32-row
