@@ -6,18 +6,18 @@
 // Hidden-layer products run on MFMA (v_mfma_f32_32x32x16_bf16): BF16 weights
 // and activations, FP32 accumulation; FP32 master weights and Adam moments.
 //
-// Device layout of the FP32 master parameters (the first layer is padded to
-// 64 inputs, the padding weights stay zero):
-//   W0[256 x 64] b0[256]  (W_l[256 x 256] b_l[256]) x 5  w_out[256] b_out
-// A training step is three kernels:
-//   k_mlp_chain: per tile of 64 rows, the six forward layers with the
+// Device layout of the FP32 master parameters (the caller's order):
+//   W0[256 x 16] b0[256]  (W_l[256 x 256] b_l[256]) x 5  w_out[256] b_out
+// A training step is three launches (seven, with a kernel to write the rows, two
+// clears and a reduction before Adam, took 302 against 283 us at 65,536 rows):
+//   k_mlp_chain: the rows of a tile of 64, the six forward layers with the
 //     activations kept in LDS, the output layer and squared error, and the
 //     five backward-data layers dZ_{l-1} = (dZ_l W_l) * SiLU'(Z_{l-1});
 //     Z_0..Z_4 and dZ_0..dZ_5 leave the tile for the weight gradients;
 //   k_mlp_wgrad: dW_l = dZ_l^T H_{l-1} and db_l = column sums of dZ_l as
 //     partial sums over spans of rows (H = SiLU(Z) recomputed from Z);
-//   k_reduce_parts + k_adam: the sum of the partials, the Adam update and
-//     the BF16 weight copies.
+//   k_adam: the sum of the partials in a fixed order (so a step gives the same
+//     bits each time), the Adam update and the BF16 weight copies.
 // Prediction is k_mlp_infer (forward and output layer only).
 #include <hip/hip_runtime.h>
 
@@ -41,10 +41,9 @@ namespace nn {
 namespace {
 
 constexpr int NIN = FIM_NN_INPUTS;  // logical inputs
-constexpr int K0 = 64;              // padded inputs
 constexpr int HID = FIM_NN_HIDDEN;
 constexpr int NL = FIM_NN_LAYERS;
-constexpr size_t W0_N = (size_t)HID * K0;
+constexpr size_t W0_N = (size_t)HID * NIN;
 constexpr size_t WL_N = (size_t)HID * HID;
 
 // FP32 master offsets
@@ -52,7 +51,8 @@ constexpr size_t off_w(int l) { return l == 0 ? 0 : W0_N + HID + (size_t)(l - 1)
 constexpr size_t off_b(int l) { return off_w(l) + (l == 0 ? W0_N : WL_N); }
 constexpr size_t OFF_WO = off_w(NL);  // = off_b(5) + HID
 constexpr size_t OFF_BO = OFF_WO + HID;
-constexpr size_t NPAD = OFF_BO + 1;
+constexpr size_t NPAR = OFF_BO + 1;
+constexpr size_t PST = (NPAR + 1 + 63) / 64 * 64;  // a partial gradient: the parameters, then the loss sum; whole lines
 // BF16 weight copies in MFMA fragment order (below): wb holds W_l as the
 // operand of the forward products (l = 0..5), wbt W_l^T as the operand of the
 // backward-data products (l = 1..5)
@@ -61,6 +61,7 @@ constexpr size_t NWB = W0_N + (size_t)(NL - 1) * WL_N;
 constexpr size_t offbt(int l) { return (size_t)(l - 1) * WL_N; }
 constexpr size_t NWBT = (size_t)(NL - 1) * WL_N;
 static_assert(off_w(NL) == off_b(NL - 1) + HID, "layout");
+static_assert(off_b(0) % 4 == 0 && (WL_N + HID) % 4 == 0, "biases are read four at a time");
 static_assert((size_t)HID * NIN + HID + (NL - 1) * (WL_N + HID) + HID + 1 == FIM_NN_PARAMS,
               "logical parameter count");
 
@@ -132,20 +133,22 @@ constexpr int RG = 1;         // row groups of 64 per tile of the fused chain ke
 constexpr int TR = 64 * RG;   // rows per tile
 constexpr int NT = 256 * RG;  // threads per workgroup: four waves per row group
 constexpr int HP = HID + 8;   // LDS row pitch of the tile (BF16 values)
-// LDS of the chain kernel: the tile, w_out, dy per row, loss and
-// bias-gradient sums
-constexpr size_t CHAIN_LDS = (size_t)TR * HP * 2 + (HID + TR + 2) * 4;
+// LDS of the chain kernel: the tile, w_out, target and then dy per row, each
+// wave's loss and bias-gradient sums
+constexpr size_t CHAIN_LDS = (size_t)TR * HP * 2 + (HID + TR + 2 * NT / 64) * 4;
+static_assert(TR == 64, "batches are multiples of 64 rows and have to fill whole tiles");
+constexpr int NOUT = HID + 4;  // per tile: w_out and b_out gradients, loss sum, two unused
 
 // One layer's product for the tile: acc[i][j] (rows 64 rg + 32 i, columns
 // 64 fg + 32 j) = T(rows, 0..K) B, with T the tile in LDS (row-major, pitch
 // HP) and B given by fragments (fragment (mb, ks) of B^T at bfr).  The next
 // step's weight fragments are loaded before the current step's products.
-// The first K of KW inputs take part; SWAP gives the transposed product
-// (accumulator rows are features, columns rows of the tile).
-template <int K, int KW, bool SWAP>
+// SWAP gives the transposed product (accumulator rows are features, columns
+// rows of the tile).
+template <int K, bool SWAP>
 __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restrict__ bfr, uint32_t rg, uint32_t fg,
                                     uint32_t lane, f32x16 (&acc)[2][2]) {
-  constexpr int NS = K / 16, NW = KW / 16;
+  constexpr int NS = K / 16;
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -153,8 +156,8 @@ __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restri
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-  const u16x8 *bp0 = reinterpret_cast<const u16x8 *>(bfr) + (size_t)(2 * fg) * NW * 64 + lane;
-  const u16x8 *bp1 = bp0 + NW * 64;
+  const u16x8 *bp0 = reinterpret_cast<const u16x8 *>(bfr) + (size_t)(2 * fg) * NS * 64 + lane;
+  const u16x8 *bp1 = bp0 + NS * 64;
   const uint16_t *ta0 = Ts + (64 * rg + l32) * HP + 8 * lh;
   const uint16_t *ta1 = ta0 + 32 * HP;
   // weight fragments two steps ahead, tile fragments one step ahead
@@ -189,15 +192,28 @@ __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restri
   }
 }
 
+constexpr int MAPP = 16;  // per map: 13 floats = three normalised site positions, four factors - 1
+
+__device__ inline uint64_t mix64(uint64_t x) {
+  x += 0x9E3779B97F4A7C15ull;
+  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+  x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+  return x ^ (x >> 31);
+}
+
 struct ChainArgs {
-  const uint16_t *X0;        // inputs, k-step layout, K0 columns
+  const float *x, *tgt;       // given rows (n x 16) and targets / t_scale, or null:
+  const float *coords, *mp;   // row r is a (map, vertex) pair drawn by (seed, r)
+  const float *T;             // maps x nn times
+  uint32_t nn, nmaps;
+  uint64_t seed;
+  float inv_ts;
+  uint16_t *X0;              // inputs, k-step layout, NIN columns (for the weight gradients)
   const uint16_t *wb, *wbt;  // fragment-ordered BF16 weights
   const float *w;            // FP32 masters (biases, output layer)
-  const float *tgt;          // targets / t_scale
   uint16_t *Z[NL - 1];       // Z_0..Z_4, k-step layout
   uint16_t *dZ[NL];          // dZ_0..dZ_5, k-step layout
-  float *g, *loss;           // output-layer gradient (accumulated), loss sum
-  uint32_t nreal;            // rows with data; the rest of the last tile is padding
+  float *tp;                 // per tile: output-layer gradient (HID + 1), loss sum
   float inv_b;
 };
 
@@ -207,11 +223,13 @@ struct ChainArgs {
 // of every product, as 2 x 2 accumulators of 32 x 32.
 //   forward: Z_l = H_{l-1} W_l^T + b_l, H_l = SiLU(Z_l) (BF16 in LDS; Z_l to
 //     HBM in the k-step layout);
-//   output: y = H_5 . w_out + b_out, e = y - t, dZ_5 = (2 e / B) w_out SiLU'(Z_5), the output-layer
-//     gradient, then dZ_{l-1} = (dZ_l W_l) * SiLU'(Z_{l-1}) for l = 5..1 with
+//   output: y = H_5 . w_out + b_out, e = y - t, dZ_5 = (2 e / B) w_out
+//     SiLU'(Z_5), the tile's output-layer gradient and loss, then dZ_{l-1} = (dZ_l W_l) * SiLU'(Z_{l-1}) for l = 5..1 with
 //     dZ_l in LDS; every dZ_l goes to HBM in the k-step layout.
 // Rounding to BF16 where the separate-kernel formulation stores values:
 // Z, H and dZ; SiLU'(Z) of the stored Z.
+// At 65,536 rows 384 MB out and 206 MB in, in 172 us (3.4 TB/s): memory and the
+// two barriers a layer bound it (86.7 GFLOP, 0.5 PFLOP/s).
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_mlp_chain(ChainArgs a) {
   extern __shared__ __align__(16) unsigned char chain_lds[];
   uint16_t *Ts = reinterpret_cast<uint16_t *>(chain_lds);
@@ -228,23 +246,52 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   auto ks_acc = [&](int i, int j, int q) -> uint32_t {
     return ks_lane + i * 32 * HID + (q >> 1) * 16 * HID + j * 32 * 16 + (q & 1) * 8;
   };
-  if (tid < 2) misc[tid] = 0.0f;
   for (uint32_t c = tid; c < HID; c += NT) wos[c] = a.w[OFF_WO + c];
-  // inputs: 16-byte pieces of the k-step layout (8 rows of one column)
-  for (uint32_t p = tid; p < TR * K0 / 8; p += NT) {
-    const uint32_t kb = p / (2 * K0), c = (p >> 1) % K0, hf = p & 1u;
-    const u16x8 v = *reinterpret_cast<const u16x8 *>(a.X0 + ((((r0 >> 4) + kb) * K0 + c) << 4) + 8 * hf);
+  // the rows, four threads each with four inputs; every row has data (batches
+  // are multiples of the tile)
+  {
+    const uint32_t row = tid >> 2, c0 = (tid & 3u) * 4;
+    float f[4], t;
+    if (a.x) {
+      const float4 v = *reinterpret_cast<const float4 *>(a.x + (r0 + row) * NIN + c0);
+      f[0] = v.x;
+      f[1] = v.y;
+      f[2] = v.z;
+      f[3] = v.w;
+      t = a.tgt[r0 + row];
+    } else {
+      const uint64_t h = mix64(a.seed ^ mix64((uint64_t)(r0 + row) + 1));
+      const uint32_t j = (uint32_t)(h >> 32) % a.nmaps, v = (uint32_t)h % a.nn;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) Ts[(kb * 16 + 8 * hf + j) * HP + c] = v[j];
+      for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t c = c0 + k;
+        f[k] = c < 3 ? a.coords[3 * (size_t)v + c] : a.mp[MAPP * (size_t)j + (c - 3)];
+      }
+      t = a.T[(size_t)j * a.nn + v] * a.inv_ts;
+    }
+    u16x4 h;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) h[k] = f2bf(f[k]);
+    *reinterpret_cast<u16x4 *>(Ts + row * HP + c0) = h;
+    if ((tid & 3u) == 0) dys[row] = t;
   }
   __syncthreads();
+  // and for the weight gradients: 16-byte pieces of the k-step layout (8 rows
+  // of one column)
+  if (tid < TR * NIN / 8) {
+    const uint32_t kb = tid / (2 * NIN), c = (tid >> 1) % NIN, hf = tid & 1u;
+    u16x8 v;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = Ts[(kb * 16 + 8 * hf + j) * HP + c];
+    *reinterpret_cast<u16x8 *>(a.X0 + ((((r0 >> 4) + kb) * NIN + c) << 4) + 8 * hf) = v;
+  }
   f32x16 acc[2][2];
 #pragma unroll 1
   for (int l = 0; l < NL; ++l) {
     if (l == 0)
-      tile_product<K0, K0, false>(Ts, a.wb + offb_w(0), rg, fg, lane, acc);
+      tile_product<NIN, false>(Ts, a.wb + offb_w(0), rg, fg, lane, acc);
     else
-      tile_product<HID, HID, false>(Ts, a.wb + offb_w(l), rg, fg, lane, acc);
+      tile_product<HID, false>(Ts, a.wb + offb_w(l), rg, fg, lane, acc);
     __syncthreads();  // every wave has read the layer's input
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -290,8 +337,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     p += __shfl_xor(p, 1);
     p += __shfl_xor(p, 2);
     const float y = p + a.w[OFF_BO];
-    const size_t grow = r0 + row;
-    const float e = grow < a.nreal ? y - a.tgt[grow] : 0.0f;
+    const float e = y - dys[row];
     const float dy = 2.0f * e * a.inv_b;
     if ((tid & 3u) == 0) dys[row] = dy;
     float ls = (tid & 3u) == 0 ? e * e : 0.0f, gb = (tid & 3u) == 0 ? dy : 0.0f;
@@ -300,8 +346,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
       gb += __shfl_xor(gb, off);
     }
     if (lane == 0) {
-      atomicAdd(&misc[0], ls);
-      atomicAdd(&misc[1], gb);
+      misc[wave] = ls;
+      misc[NT / 64 + wave] = gb;
     }
   }
   __syncthreads();
@@ -309,11 +355,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   if (tid < HID) {
     float gw = 0.0f;
     for (uint32_t row = 0; row < TR; ++row) gw += dys[row] * bf2f(Ts[row * HP + tid]);
-    atomicAdd(&a.g[OFF_WO + tid], gw);
+    a.tp[(size_t)blockIdx.x * NOUT + tid] = gw;
   }
-  if (tid == 0) {
-    atomicAdd(a.loss, misc[0]);
-    atomicAdd(&a.g[OFF_BO], misc[1]);
+  if (tid < 2) {  // b_out, loss
+    const float *q = misc + (tid == 0 ? NT / 64 : 0);
+    float v = 0.0f;
+    for (int k = 0; k < NT / 64; ++k) v += q[k];
+    a.tp[(size_t)blockIdx.x * NOUT + HID + tid] = v;
   }
   __syncthreads();  // H_5 is read; dZ_5 takes its place
   // dZ_5 = dy w_out SiLU'(Z_5)
@@ -339,7 +387,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   // backward through the hidden layers
 #pragma unroll 1
   for (int l = NL - 1; l >= 1; --l) {
-    tile_product<HID, HID, false>(Ts, a.wbt + offbt(l), rg, fg, lane, acc);
+    tile_product<HID, false>(Ts, a.wbt + offbt(l), rg, fg, lane, acc);
     __syncthreads();  // every wave has read dZ_l
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -383,7 +431,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 // from 285 us and 10 us more to write the input rows.
 // The input rows are made here, not read back from memory: row r is given
 // (x), or solve r / m at vertex sample[r % m] (r itself without a sample).
-// The first product needs one k-step for the 16 inputs, not the padded four.
 // ---------------------------------------------------------------------------
 struct InferArgs {
   const float *x;             // given rows (n x 16), or null
@@ -396,8 +443,6 @@ struct InferArgs {
   uint32_t nreal;
   float t_scale, delta;
 };
-
-constexpr int MAPP = 16;  // per map: 13 floats = three normalised site positions, four factors - 1
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_mlp_infer(InferArgs a) {
   extern __shared__ __align__(16) unsigned char chain_lds[];
@@ -436,9 +481,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   for (int l = 0; l < NL; ++l) {
     const uint16_t *wl = a.wb + offb_w(l);
     if (l == 0)
-      tile_product<NIN, K0, true>(Ts, wl, 0, fg, lane, acc);
+      tile_product<NIN, true>(Ts, wl, 0, fg, lane, acc);
     else
-      tile_product<HID, HID, true>(Ts, wl, 0, fg, lane, acc);
+      tile_product<HID, true>(Ts, wl, 0, fg, lane, acc);
     const float *bl = a.w + off_b(l) + 64 * fg + 4 * lh;
     __syncthreads();  // every wave has read the layer's input
 #pragma unroll
@@ -481,12 +526,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 // staged 32 rows at a time into LDS in their k-step layout (SiLU applied
 // once per element); every fragment is then one 16-byte LDS read.  Eight
 // waves tile the 256 x K output: 4 x 2 waves of 64 x 128 (K = 256) or 8 x 1
-// waves of 32 x 64 (K = 64).
+// waves of 32 x 16 (K = 16: the inputs; the other half of the 32-wide product
+// repeats them and is dropped).  Layer 0's workgroups also add up their span's
+// share of the output-layer gradient and the loss.  At 65,536 rows it reads
+// 384 MB in 101 us (3.8 TB/s, of 4.7 TB/s that a large copy reaches).
 // ---------------------------------------------------------------------------
 struct WGradArgs {
   const uint16_t *dZ[NL];   // k-step layout, HID columns
-  const uint16_t *Hin[NL];  // l = 0: X0 (K0 columns); l >= 1: Z_{l-1} (HID columns)
-  float *P;                 // partial sums, OFF_WO floats per span
+  const uint16_t *Hin[NL];  // l = 0: X0 (NIN columns); l >= 1: Z_{l-1} (HID columns)
+  const float *tp;          // per tile: output-layer gradient, loss sum
+  float *P;                 // partial sums, PST floats per span
   uint32_t steps;           // 32-row steps of the batch; span s takes steps
                             // [s steps / S, (s + 1) steps / S), S = gridDim.x
 };
@@ -500,7 +549,8 @@ constexpr int WG_LDS = 2 * 2 * 2 * HID * KSP;  // BF16 values
 template <int K>
 __device__ inline void wgrad_body(const WGradArgs &a, uint32_t l, uint16_t *lds) {
   constexpr int WN = K == HID ? 4 : 8, WK = 8 / WN;
-  constexpr int BN = HID / WN / 32, BK = K / WK / 32;
+  constexpr int BN = HID / WN / 32, BK = K == HID ? K / WK / 32 : 1;
+  constexpr int HU = K == HID ? 2 : 1;  // pieces of H per thread and step
   constexpr uint32_t BUF = 2 * 2 * HID * KSP;  // one buffer: dZ (2 x HID x KSP) then H (2 x K x KSP)
   constexpr uint32_t HPC = 2 * K * 16 / 8;    // 16-byte pieces of H per step
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -514,7 +564,7 @@ __device__ inline void wgrad_body(const WGradArgs &a, uint32_t l, uint16_t *lds)
   // step i is multiplied and step i + 1 is staged.  Every load is issued (the
   // step index clamped), so the number of loads in flight is the same on
   // every path and each wait leaves the two younger steps in flight.
-  u16x8 rz[3][2], rh[3][2];
+  u16x8 rz[3][2], rh[3][HU];
   float csum = 0.0f;  // column sum of dZ for column tid / 2
   auto gload = [&](int slot, uint32_t i) {
     const uint32_t st = s0 + (i < n ? i : n - 1);
@@ -523,7 +573,7 @@ __device__ inline void wgrad_body(const WGradArgs &a, uint32_t l, uint16_t *lds)
     rz[slot][0] = sz[tid];
     rz[slot][1] = sz[tid + 512];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) rh[slot][u] = sh[(tid + 512u * u) % HPC];
+    for (int u = 0; u < HU; ++u) rh[slot][u] = sh[(tid + 512u * u) % HPC];
   };
   // stages relative step i (zeros beyond the span) into LDS buffer buf
   auto lstore = [&](int slot, uint32_t buf, uint32_t i) {
@@ -545,15 +595,15 @@ __device__ inline void wgrad_body(const WGradArgs &a, uint32_t l, uint16_t *lds)
 #pragma unroll
     for (int j = 0; j < 8; ++j) csum += bf2f(z0[j]) + bf2f(z1[j]);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const uint32_t p = tid + 512u * u;
-      if (p < HPC) {
-        u16x8 v = masked(rh[slot][u]);
-        if (K == HID)
+    for (int u = 0; u < HU; ++u) {
+      // the 64 pieces of the inputs by every wave alike (the same values to
+      // the same place): a branch around them cost 4 of the 100 us
+      const uint32_t p = (tid + 512u * u) % HPC;
+      u16x8 v = masked(rh[slot][u]);
+      if (K == HID)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = f2bf(silu(bf2f(v[j])));
-        *reinterpret_cast<u16x8 *>(bh + (p >> 1) * KSP + 8 * (p & 1u)) = v;
-      }
+        for (int j = 0; j < 8; ++j) v[j] = f2bf(silu(bf2f(v[j])));
+      *reinterpret_cast<u16x8 *>(bh + (p >> 1) * KSP + 8 * (p & 1u)) = v;
     }
   };
   f32x16 acc[BN][BK];
@@ -573,7 +623,7 @@ __device__ inline void wgrad_body(const WGradArgs &a, uint32_t l, uint16_t *lds)
         fa[i] = *reinterpret_cast<const u16x8 *>(bz + (u * HID + wn * BN * 32 + 32 * i + l32) * KSP + 8 * lh);
 #pragma unroll
       for (int j = 0; j < BK; ++j)
-        fb[j] = *reinterpret_cast<const u16x8 *>(bh + (u * K + wk * BK * 32 + 32 * j + l32) * KSP + 8 * lh);
+        fb[j] = *reinterpret_cast<const u16x8 *>(bh + (u * K + (K == HID ? wk * BK * 32 + 32 * j + l32 : l32 % K)) * KSP + 8 * lh);
 #pragma unroll
       for (int i = 0; i < BN; ++i)
 #pragma unroll
@@ -596,7 +646,7 @@ __device__ inline void wgrad_body(const WGradArgs &a, uint32_t l, uint16_t *lds)
       __syncthreads();
     }
   }
-  float *P = a.P + (size_t)blockIdx.x * OFF_WO;
+  float *P = a.P + (size_t)blockIdx.x * PST;
 #pragma unroll
   for (int i = 0; i < BN; ++i)
 #pragma unroll
@@ -605,10 +655,41 @@ __device__ inline void wgrad_body(const WGradArgs &a, uint32_t l, uint16_t *lds)
       for (int r = 0; r < 16; ++r) {
         const uint32_t n = wn * BN * 32 + 32 * i + 8 * (r >> 2) + 4 * lh + (r & 3);
         const uint32_t k = wk * BK * 32 + 32 * j + l32;
-        P[off_w(l) + (size_t)n * K + k] = acc[i][j][r];
+        if (K == HID || k < K) P[off_w(l) + (size_t)n * K + k] = acc[i][j][r];
       }
   csum += __shfl_xor(csum, 1);
   if ((tid & 1u) == 0) P[off_b(l) + (tid >> 1)] = csum;
+  if (K != HID) {
+    // the span's share of the tiles' output-layer sums: wave w takes tiles
+    // t0 + w, t0 + w + 8, .., and the eight are added in order (all in flight
+    // at once: one thread per sum over the 26 tiles of a span took 6 us more
+    // of the 100 us kernel at 65,536 rows)
+    const uint32_t nt = a.steps / 2;
+    const uint32_t t0 = (uint32_t)((uint64_t)blockIdx.x * nt / gridDim.x);
+    const uint32_t t1 = (uint32_t)((uint64_t)(blockIdx.x + 1) * nt / gridDim.x);
+    float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    float e = 0.0f;
+#pragma unroll 4
+    for (uint32_t t = t0 + wave; t < t1; t += 8) {
+      const float *q = a.tp + (size_t)t * NOUT;
+      const float4 u = reinterpret_cast<const float4 *>(q)[lane];
+      e += q[HID + (lane & 1u)];
+      v.x += u.x;
+      v.y += u.y;
+      v.z += u.z;
+      v.w += u.w;
+    }
+    float *sums = reinterpret_cast<float *>(lds);  // every wave is past the last product
+    reinterpret_cast<float4 *>(sums + wave * NOUT)[lane] = v;
+    if (lane < 2) sums[wave * NOUT + HID + lane] = e;
+    __syncthreads();
+    if (tid < HID + 2) {
+      float r = 0.0f;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) r += sums[w * NOUT + tid];
+      P[OFF_WO + tid] = r;
+    }
+  }
 }
 
 __global__ __launch_bounds__(512) void k_mlp_wgrad(WGradArgs a) {
@@ -616,7 +697,7 @@ __global__ __launch_bounds__(512) void k_mlp_wgrad(WGradArgs a) {
   uint16_t *lds = reinterpret_cast<uint16_t *>(wg_lds);
   const uint32_t l = blockIdx.y;
   if (l == 0)
-    wgrad_body<K0>(a, 0, lds);
+    wgrad_body<NIN>(a, 0, lds);
   else
     wgrad_body<HID>(a, l, lds);
 }
@@ -624,42 +705,6 @@ __global__ __launch_bounds__(512) void k_mlp_wgrad(WGradArgs a) {
 // ---------------------------------------------------------------------------
 // small kernels
 // ---------------------------------------------------------------------------
-__device__ inline uint64_t mix64(uint64_t x) {
-  x += 0x9E3779B97F4A7C15ull;
-  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
-  x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
-  return x ^ (x >> 31);
-}
-
-// the 16 inputs of one row into X0 (k-step layout; the padding columns
-// NIN..K0-1 are zero from the start and never written)
-__device__ inline void write_features(uint16_t *X0, size_t row, const float *vxyz, const float *mp) {
-  for (int k = 0; k < 3; ++k) X0[ks_off(row, k, K0)] = f2bf(vxyz[k]);
-  for (int k = 0; k < 13; ++k) X0[ks_off(row, 3 + k, K0)] = f2bf(mp[k]);
-}
-
-__device__ inline void zero_features(uint16_t *X0, size_t row) {
-  for (int k = 0; k < NIN; ++k) X0[ks_off(row, k, K0)] = 0;
-}
-
-// training rows: random (map, vertex) samples; rows B..rows-1 (padding of
-// the last tile) are zero with target 0
-__global__ void k_sample(const float *coords, const float *mparams, const float *T, uint32_t nn,
-                         uint32_t nmaps, uint64_t seed, uint32_t B, uint32_t rows, float inv_ts, uint16_t *X0,
-                         float *tgt) {
-  for (uint32_t m = blockIdx.x * blockDim.x + threadIdx.x; m < rows; m += gridDim.x * blockDim.x) {
-    if (m >= B) {
-      zero_features(X0, m);
-      tgt[m] = 0.0f;
-      continue;
-    }
-    const uint64_t h = mix64(seed ^ mix64((uint64_t)m + 1));
-    const uint32_t j = (uint32_t)((h >> 32) % nmaps), v = (uint32_t)((h & 0xffffffffu) % nn);
-    write_features(X0, m, coords + 3 * (size_t)v, mparams + MAPP * (size_t)j);
-    tgt[m] = T[(size_t)j * nn + v] * inv_ts;
-  }
-}
-
 // per solve: the largest of its m predictions (one wave per solve)
 __global__ __launch_bounds__(256) void k_solve_max(const float *t, uint32_t m, uint32_t nsolve, float *out) {
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -671,65 +716,72 @@ __global__ __launch_bounds__(256) void k_solve_max(const float *t, uint32_t m, u
   }
 }
 
-// given inputs (n x 16 floats) -> BF16 rows of X0 (rows n..rows-1 zero)
-__global__ void k_input_rows(const float *x, uint32_t n, uint32_t rows, uint16_t *X0) {
-  for (uint32_t m = blockIdx.x * blockDim.x + threadIdx.x; m < rows; m += gridDim.x * blockDim.x)
-    for (int k = 0; k < NIN; ++k) X0[ks_off(m, k, K0)] = m < n ? f2bf(x[(size_t)m * NIN + k]) : (uint16_t)0;
+// One element of the sum of the S partial gradients (eight loads in flight:
+// partial k goes to accumulator k % 8, and the eight are added in a fixed
+// order, so the sum is reproducible)
+__device__ inline float sum_parts(const float *P, uint32_t S, size_t i) {
+  float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  uint32_t k = 0;
+  for (; k + 8 <= S; k += 8) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a[j] += P[(size_t)(k + j) * PST + i];
+  }
+  for (; k < S; ++k) a[k & 7u] += P[(size_t)k * PST + i];
+  return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
 }
 
-// sum of the batch-split partials
-// (eight loads in flight per thread: partial k goes to accumulator k % 8,
-// and the eight are added in a fixed order, so the sum is reproducible)
-__global__ void k_reduce_parts(const float *P, uint32_t S, size_t n, float *g) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    uint32_t k = 0;
-    for (; k + 8 <= S; k += 8) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) a[j] += P[(size_t)(k + j) * n + i];
+// BF16 copies of parameter i, if it is a hidden-layer weight
+__device__ inline void put_bf16(uint32_t i, float w, uint16_t *wb, uint16_t *wbt) {
+  constexpr uint32_t L1 = (uint32_t)off_w(1), LS = (uint32_t)(WL_N + HID);
+  if (i < W0_N) {
+    wb[frag_off(i / NIN, i % NIN, NIN)] = f2bf(w);
+  } else if (i >= L1 && i < OFF_WO) {
+    const uint32_t l = (i - L1) / LS, q = (i - L1) % LS;  // hidden layer l + 1
+    if (q < WL_N) {
+      const uint32_t n = q / HID, k = q % HID;
+      wb[W0_N + l * WL_N + frag_off(n, k, HID)] = f2bf(w);
+      wbt[l * WL_N + frag_off(k, n, HID)] = f2bf(w);
     }
-    for (; k < S; ++k) a[k & 7u] += P[(size_t)k * n + i];
-    g[i] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
   }
 }
 
-// Adam on the FP32 masters; BF16 copies of the hidden-layer weights
+// gradient and loss sum (element NPAR)
+__global__ __launch_bounds__(256) void k_reduce_parts(const float *P, uint32_t S, float *g) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i <= NPAR) g[i] = sum_parts(P, S, i);
+}
+
+// Adam on the FP32 masters with the sum of S partial gradients; BF16 copies of
+// the hidden-layer weights; the loss sum, where the partials carry one.  One
+// element a thread: bound by the partials' bytes (40 x 1.33 MB).
 struct AdamArgs {
-  float *w, *m, *v;
-  const float *g;
+  float *w, *m, *v, *loss;
+  const float *P;
   uint16_t *wb, *wbt;
+  uint32_t S;
   float lr, b1, b2, eps, c1, c2;  // c1 = 1 - b1^t, c2 = 1 - b2^t
 };
 
-__global__ void k_adam(AdamArgs a) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < NPAD; i += (size_t)gridDim.x * blockDim.x) {
-    const float g = a.g[i];
-    const float m = a.b1 * a.m[i] + (1.0f - a.b1) * g;
-    const float v = a.b2 * a.v[i] + (1.0f - a.b2) * g * g;
-    a.m[i] = m;
-    a.v[i] = v;
-    const float w = a.w[i] - a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
-    a.w[i] = w;
-    // weights of layer l live at off_w(l) .. off_b(l) in the masters
-    for (int l = 0; l < NL; ++l)
-      if (i >= off_w(l) && i < off_b(l)) {
-        const size_t q = i - off_w(l);
-        const uint32_t K = l == 0 ? K0 : HID, n = (uint32_t)(q / K), k = (uint32_t)(q % K);
-        a.wb[offb_w(l) + frag_off(n, k, K)] = f2bf(w);
-        if (l > 0) a.wbt[offbt(l) + frag_off(k, n, HID)] = f2bf(w);
-      }
+__global__ __launch_bounds__(256) void k_adam(AdamArgs a) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i > NPAR || (i == NPAR && !a.loss)) return;
+  const float g = sum_parts(a.P, a.S, i);
+  if (i == NPAR) {
+    *a.loss = g;
+    return;
   }
+  const float m = a.b1 * a.m[i] + (1.0f - a.b1) * g;
+  const float v = a.b2 * a.v[i] + (1.0f - a.b2) * g * g;
+  a.m[i] = m;
+  a.v[i] = v;
+  const float w = a.w[i] - a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
+  a.w[i] = w;
+  put_bf16(i, w, a.wb, a.wbt);
 }
 
-__global__ void k_to_bf16(const float *w, uint16_t *wb, uint16_t *wbt) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < NPAD; i += (size_t)gridDim.x * blockDim.x)
-    for (int l = 0; l < NL; ++l)
-      if (i >= off_w(l) && i < off_b(l)) {
-        const size_t q = i - off_w(l);
-        const uint32_t K = l == 0 ? K0 : HID, n = (uint32_t)(q / K), k = (uint32_t)(q % K);
-        wb[offb_w(l) + frag_off(n, k, K)] = f2bf(w[i]);
-        if (l > 0) wbt[offbt(l) + frag_off(k, n, HID)] = f2bf(w[i]);
-      }
+__global__ __launch_bounds__(256) void k_to_bf16(const float *w, uint16_t *wb, uint16_t *wbt) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < NPAR) put_bf16(i, w[i], wb, wbt);
 }
 
 __global__ void k_zero_sites(const uint32_t *v, uint32_t n, float *f) {
@@ -766,7 +818,7 @@ struct fim_nn {
   // activations (rows = cap, a multiple of the chain kernel's tile), k-step layout
   uint32_t cap = 0;
   uint16_t *X0 = nullptr, *Z[NL - 1] = {}, *dZ[NL] = {};
-  float *tgt = nullptr, *out = nullptr, *parts = nullptr, *loss = nullptr;
+  float *tgt = nullptr, *out = nullptr, *parts = nullptr, *tp = nullptr;
   uint32_t nsplit = 1;  // row spans of the weight gradients (partial sums)
   // dataset
   float *coords = nullptr, *T = nullptr, *mparams = nullptr;
@@ -826,47 +878,54 @@ void infer(fim_nn *n, const float *x, const float *mp, const uint32_t *sample, u
   HIPCHECK(hipGetLastError());
 }
 
-// forward and backward pass over rows 0..B-1 of X0 (targets in n->tgt; rows
-// up to tile_rows(B) filled, as padding): gradient in n->g, loss sum in
-// n->loss
-void train_pass(fim_nn *n, uint32_t B) {
-  const uint32_t rows = tile_rows(B);
-  HIPCHECK(hipMemsetAsync(n->g + OFF_WO, 0, (NPAD - OFF_WO) * sizeof(float), n->stream));
-  HIPCHECK(hipMemsetAsync(n->loss, 0, sizeof(float), n->stream));
+// Forward and backward pass over B rows (a multiple of the tile): those of
+// (x, n->tgt) or, without x, pairs of the dataset drawn by `seed`.  Leaves
+// the partial gradients in n->parts; returns how many.
+uint32_t train_pass(fim_nn *n, const float *x, uint64_t seed, uint32_t B) {
   ChainArgs a{};
+  a.x = x;
+  a.tgt = n->tgt;
+  a.coords = n->coords;
+  a.mp = n->mparams;
+  a.T = n->T;
+  a.nn = n->nn;
+  a.nmaps = (uint32_t)n->nmaps;
+  a.seed = seed;
+  a.inv_ts = 1.0f / t_scale(n);
   a.X0 = n->X0;
   a.wb = n->wb;
   a.wbt = n->wbt;
   a.w = n->w;
-  a.tgt = n->tgt;
   for (int l = 0; l < NL - 1; ++l) a.Z[l] = n->Z[l];
   for (int l = 0; l < NL; ++l) a.dZ[l] = n->dZ[l];
-  a.g = n->g;
-  a.loss = n->loss;
-  a.nreal = B;
+  a.tp = n->tp;
   a.inv_b = 1.0f / (float)B;
-  k_mlp_chain<<<rows / TR, NT, CHAIN_LDS, n->stream>>>(a);
+  k_mlp_chain<<<B / TR, NT, CHAIN_LDS, n->stream>>>(a);
   // weight gradients: S spans of whole 32-row steps, one partial sum each
-  const uint32_t S = std::min<uint32_t>(n->nsplit, rows / 32);
+  const uint32_t S = std::min<uint32_t>(n->nsplit, B / 32);
   WGradArgs wa;
   for (int l = 0; l < NL; ++l) {
     wa.dZ[l] = n->dZ[l];
     wa.Hin[l] = l == 0 ? n->X0 : n->Z[l - 1];
   }
+  wa.tp = n->tp;
   wa.P = n->parts;
-  wa.steps = rows / 32;
+  wa.steps = B / 32;
   k_mlp_wgrad<<<dim3(S, NL), 512, WG_LDS * 2, n->stream>>>(wa);
-  k_reduce_parts<<<grid_for(OFF_WO), 256, 0, n->stream>>>(n->parts, S, OFF_WO, n->g);
   HIPCHECK(hipGetLastError());
+  return S;
 }
 
-void adam(fim_nn *n) {
+// one Adam step with the sum of S partial gradients
+void adam(fim_nn *n, const float *P, uint32_t S, float *loss) {
   n->t += 1;
   AdamArgs a;
   a.w = n->w;
   a.m = n->m;
   a.v = n->v;
-  a.g = n->g;
+  a.loss = loss;
+  a.P = P;
+  a.S = S;
   a.wb = n->wb;
   a.wbt = n->wbt;
   a.lr = (float)(n->o.lr > 0 ? n->o.lr : 1e-3);
@@ -875,36 +934,8 @@ void adam(fim_nn *n) {
   a.eps = (float)(n->o.adam_eps > 0 ? n->o.adam_eps : 1e-8);
   a.c1 = (float)(1.0 - std::pow((double)a.b1, (double)n->t));
   a.c2 = (float)(1.0 - std::pow((double)a.b2, (double)n->t));
-  k_adam<<<grid_for(NPAD), 256, 0, n->stream>>>(a);
+  k_adam<<<NPAR / 256 + 1, 256, 0, n->stream>>>(a);
   HIPCHECK(hipGetLastError());
-}
-
-// logical <-> device parameter order
-void to_device_order(const float *logical, std::vector<float> &dev) {
-  dev.assign(NPAD, 0.0f);
-  size_t q = 0;
-  for (int r = 0; r < HID; ++r)
-    for (int k = 0; k < NIN; ++k) dev[off_w(0) + (size_t)r * K0 + k] = logical[q++];
-  for (int r = 0; r < HID; ++r) dev[off_b(0) + r] = logical[q++];
-  for (int l = 1; l < NL; ++l) {
-    for (size_t i = 0; i < WL_N; ++i) dev[off_w(l) + i] = logical[q++];
-    for (int r = 0; r < HID; ++r) dev[off_b(l) + r] = logical[q++];
-  }
-  for (int r = 0; r < HID; ++r) dev[OFF_WO + r] = logical[q++];
-  dev[OFF_BO] = logical[q++];
-}
-
-void to_logical_order(const std::vector<float> &dev, float *logical) {
-  size_t q = 0;
-  for (int r = 0; r < HID; ++r)
-    for (int k = 0; k < NIN; ++k) logical[q++] = dev[off_w(0) + (size_t)r * K0 + k];
-  for (int r = 0; r < HID; ++r) logical[q++] = dev[off_b(0) + r];
-  for (int l = 1; l < NL; ++l) {
-    for (size_t i = 0; i < WL_N; ++i) logical[q++] = dev[off_w(l) + i];
-    for (int r = 0; r < HID; ++r) logical[q++] = dev[off_b(l) + r];
-  }
-  for (int r = 0; r < HID; ++r) logical[q++] = dev[OFF_WO + r];
-  logical[q++] = dev[OFF_BO];
 }
 
 template <class F>
@@ -973,7 +1004,7 @@ int fim_nn_create(const fim_mesh *mesh, const fim_nn_opts *o, fim_nn **out) {
       // once (32 / 48 / 64 spans measured 4-8 % slower per training step)
       n->nsplit = 40;
       // parameters: He-uniform hidden layers, small output layer, zero biases
-      std::vector<float> w(NPAD, 0.0f);
+      std::vector<float> w(NPAR, 0.0f);
       uint64_t st = o->seed ^ 0x5DEECE66Dull;
       auto uni = [&]() {
         st += 0x9E3779B97F4A7C15ull;
@@ -987,35 +1018,34 @@ int fim_nn_create(const fim_mesh *mesh, const fim_nn_opts *o, fim_nn **out) {
         const int fan = l == 0 ? NIN : HID;
         const double a = std::sqrt(6.0 / fan);
         for (int r = 0; r < HID; ++r)
-          for (int k = 0; k < fan; ++k) w[off_w(l) + (size_t)r * (l == 0 ? K0 : HID) + k] = (float)(a * uni());
+          for (int k = 0; k < fan; ++k) w[off_w(l) + (size_t)r * fan + k] = (float)(a * uni());
       }
       for (int r = 0; r < HID; ++r) w[OFF_WO + r] = (float)(0.1 * std::sqrt(6.0 / HID) * uni());
-      n->w = nn_alloc<float>(n, NPAD);
-      n->g = nn_alloc<float>(n, NPAD);
-      n->m = nn_alloc<float>(n, NPAD);
-      n->v = nn_alloc<float>(n, NPAD);
+      n->w = nn_alloc<float>(n, NPAR);
+      n->g = nn_alloc<float>(n, PST);
+      n->m = nn_alloc<float>(n, NPAR);
+      n->v = nn_alloc<float>(n, NPAR);
       n->wb = nn_alloc<uint16_t>(n, NWB);
       n->wbt = nn_alloc<uint16_t>(n, NWBT);
-      HIPCHECK(hipMemcpy(n->w, w.data(), NPAD * sizeof(float), hipMemcpyHostToDevice));
-      HIPCHECK(hipMemset(n->m, 0, NPAD * sizeof(float)));
-      HIPCHECK(hipMemset(n->v, 0, NPAD * sizeof(float)));
-      HIPCHECK(hipMemset(n->g, 0, NPAD * sizeof(float)));
-      k_to_bf16<<<grid_for(NPAD), 256, 0, n->stream>>>(n->w, n->wb, n->wbt);
+      HIPCHECK(hipMemcpy(n->w, w.data(), NPAR * sizeof(float), hipMemcpyHostToDevice));
+      HIPCHECK(hipMemset(n->m, 0, NPAR * sizeof(float)));
+      HIPCHECK(hipMemset(n->v, 0, NPAR * sizeof(float)));
+      HIPCHECK(hipMemset(n->g, 0, PST * sizeof(float)));
+      k_to_bf16<<<(NPAR + 255) / 256, 256, 0, n->stream>>>(n->w, n->wb, n->wbt);
       HIPCHECK(hipGetLastError());
-      n->X0 = nn_alloc<uint16_t>(n, (size_t)n->cap * K0);
-      HIPCHECK(hipMemset(n->X0, 0, (size_t)n->cap * K0 * sizeof(uint16_t)));  // padding columns stay 0
+      n->X0 = nn_alloc<uint16_t>(n, (size_t)n->cap * NIN);
       for (int l = 0; l < NL - 1; ++l) n->Z[l] = nn_alloc<uint16_t>(n, (size_t)n->cap * HID);
       for (int l = 0; l < NL; ++l) n->dZ[l] = nn_alloc<uint16_t>(n, (size_t)n->cap * HID);
       n->tgt = nn_alloc<float>(n, n->cap);
       n->out = nn_alloc<float>(n, n->cap);
-      n->parts = nn_alloc<float>(n, (size_t)n->nsplit * OFF_WO);
+      n->parts = nn_alloc<float>(n, (size_t)n->nsplit * PST);
+      n->tp = nn_alloc<float>(n, (size_t)(n->cap / TR) * NOUT);
       HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_chain, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)CHAIN_LDS));
       HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_infer, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)CHAIN_LDS));
       HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_wgrad, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    WG_LDS * 2));
-      n->loss = nn_alloc<float>(n, 1);
       n->coords = nn_alloc<float>(n, 3 * (size_t)n->nn);
       HIPCHECK(hipMemcpy(n->coords, n->coords_h.data(), 3 * (size_t)n->nn * sizeof(float), hipMemcpyHostToDevice));
       n->T = nn_alloc<float>(n, (size_t)n->max_maps * n->nn);
@@ -1036,10 +1066,8 @@ int fim_nn_get_params(fim_nn *n, float *params) {
   return guarded([&] {
     if (!n || !params) throw Error(FIM_EINVAL, "null argument");
     HIPCHECK(hipSetDevice(n->dev));
-    std::vector<float> dev(NPAD);
-    HIPCHECK(hipMemcpyAsync(dev.data(), n->w, NPAD * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+    HIPCHECK(hipMemcpyAsync(params, n->w, NPAR * sizeof(float), hipMemcpyDeviceToHost, n->stream));
     HIPCHECK(hipStreamSynchronize(n->stream));
-    to_logical_order(dev, params);
   });
 }
 
@@ -1047,10 +1075,8 @@ int fim_nn_set_params(fim_nn *n, const float *params) {
   return guarded([&] {
     if (!n || !params) throw Error(FIM_EINVAL, "null argument");
     HIPCHECK(hipSetDevice(n->dev));
-    std::vector<float> dev;
-    to_device_order(params, dev);
-    HIPCHECK(hipMemcpyAsync(n->w, dev.data(), NPAD * sizeof(float), hipMemcpyHostToDevice, n->stream));
-    k_to_bf16<<<grid_for(NPAD), 256, 0, n->stream>>>(n->w, n->wb, n->wbt);
+    HIPCHECK(hipMemcpyAsync(n->w, params, NPAR * sizeof(float), hipMemcpyHostToDevice, n->stream));
+    k_to_bf16<<<(NPAR + 255) / 256, 256, 0, n->stream>>>(n->w, n->wb, n->wbt);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(n->stream));
   });
@@ -1060,10 +1086,8 @@ int fim_nn_adam_step(fim_nn *n, const float *grad) {
   return guarded([&] {
     if (!n || !grad) throw Error(FIM_EINVAL, "null argument");
     HIPCHECK(hipSetDevice(n->dev));
-    std::vector<float> dev;
-    to_device_order(grad, dev);  // padding entries stay 0
-    HIPCHECK(hipMemcpyAsync(n->g, dev.data(), NPAD * sizeof(float), hipMemcpyHostToDevice, n->stream));
-    adam(n);
+    HIPCHECK(hipMemcpyAsync(n->g, grad, NPAR * sizeof(float), hipMemcpyHostToDevice, n->stream));
+    adam(n, n->g, 1, nullptr);
     HIPCHECK(hipStreamSynchronize(n->stream));
   });
 }
@@ -1072,14 +1096,11 @@ int fim_nn_get_moments(fim_nn *n, float *m, float *v, int64_t *steps) {
   return guarded([&] {
     if (!n) throw Error(FIM_EINVAL, "null argument");
     HIPCHECK(hipSetDevice(n->dev));
-    std::vector<float> dev(NPAD);
     for (int k = 0; k < 2; ++k) {
       float *dst = k == 0 ? m : v;
       if (!dst) continue;
-      HIPCHECK(hipMemcpyAsync(dev.data(), k == 0 ? n->m : n->v, NPAD * sizeof(float), hipMemcpyDeviceToHost,
-                              n->stream));
+      HIPCHECK(hipMemcpyAsync(dst, k == 0 ? n->m : n->v, NPAR * sizeof(float), hipMemcpyDeviceToHost, n->stream));
       HIPCHECK(hipStreamSynchronize(n->stream));
-      to_logical_order(dev, dst);
     }
     if (steps) *steps = n->t;
   });
@@ -1135,7 +1156,7 @@ int fim_nn_gradient(fim_nn *n, const float *x, const float *t, int32_t b, double
   return guarded([&] {
     if (!n || !x || !t || !loss || !grad) throw Error(FIM_EINVAL, "null argument");
     if (b <= 0 || b % 64) throw Error(FIM_EINVAL, "batch must be a positive multiple of 64");
-    ensure_rows(n, tile_rows((uint32_t)b));
+    ensure_rows(n, (uint32_t)b);
     HIPCHECK(hipSetDevice(n->dev));
     std::vector<float> ts(b);
     for (int32_t i = 0; i < b; ++i) ts[i] = t[i] / t_scale(n);
@@ -1144,15 +1165,13 @@ int fim_nn_gradient(fim_nn *n, const float *x, const float *t, int32_t b, double
     try {
       HIPCHECK(hipMemcpyAsync(xd, x, (size_t)b * NIN * sizeof(float), hipMemcpyHostToDevice, n->stream));
       HIPCHECK(hipMemcpyAsync(n->tgt, ts.data(), (size_t)b * sizeof(float), hipMemcpyHostToDevice, n->stream));
-      k_input_rows<<<grid_for(tile_rows((uint32_t)b)), 256, 0, n->stream>>>(xd, (uint32_t)b,
-                                                                            tile_rows((uint32_t)b), n->X0);
-      train_pass(n, (uint32_t)b);
-      std::vector<float> dev(NPAD);
+      const uint32_t S = train_pass(n, xd, 0, (uint32_t)b);
+      k_reduce_parts<<<NPAR / 256 + 1, 256, 0, n->stream>>>(n->parts, S, n->g);
+      HIPCHECK(hipGetLastError());
       float l = 0.0f;
-      HIPCHECK(hipMemcpyAsync(dev.data(), n->g, NPAD * sizeof(float), hipMemcpyDeviceToHost, n->stream));
-      HIPCHECK(hipMemcpyAsync(&l, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream));
+      HIPCHECK(hipMemcpyAsync(grad, n->g, NPAR * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+      HIPCHECK(hipMemcpyAsync(&l, n->g + NPAR, sizeof(float), hipMemcpyDeviceToHost, n->stream));
       HIPCHECK(hipStreamSynchronize(n->stream));
-      to_logical_order(dev, grad);
       *loss = (double)l / b;
     } catch (...) {
       (void)hipFree(xd);
@@ -1167,18 +1186,14 @@ int fim_nn_train(fim_nn *n, int32_t steps, int32_t batch, uint64_t seed, double 
     if (!n) throw Error(FIM_EINVAL, "null argument");
     if (steps < 0 || batch <= 0 || batch % 64) throw Error(FIM_EINVAL, "bad training arguments");
     if (n->nmaps == 0) throw Error(FIM_ESTATE, "surrogate dataset is empty");
-    const uint32_t rows = tile_rows((uint32_t)batch);
-    ensure_rows(n, rows);
+    ensure_rows(n, (uint32_t)batch);
     HIPCHECK(hipSetDevice(n->dev));
     float l = 0.0f;
     for (int32_t s = 0; s < steps; ++s) {
-      k_sample<<<grid_for(rows), 256, 0, n->stream>>>(n->coords, n->mparams, n->T, n->nn, (uint32_t)n->nmaps,
-                                                      seed * 0x100000001B3ull + (uint64_t)s, (uint32_t)batch,
-                                                      rows, 1.0f / t_scale(n), n->X0, n->tgt);
-      train_pass(n, (uint32_t)batch);
-      adam(n);
+      const uint32_t S = train_pass(n, nullptr, seed * 0x100000001B3ull + (uint64_t)s, (uint32_t)batch);
+      adam(n, n->parts, S, n->g + NPAR);
     }
-    HIPCHECK(hipMemcpyAsync(&l, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream));
+    HIPCHECK(hipMemcpyAsync(&l, n->g + NPAR, sizeof(float), hipMemcpyDeviceToHost, n->stream));
     HIPCHECK(hipStreamSynchronize(n->stream));
     if (loss) *loss = (double)l / batch;
   });

@@ -101,6 +101,30 @@ def test_gradient_matches_oracle(small_slab, b):
     nn.close()
 
 
+@pytest.mark.parametrize("b", [64, 128, 2624])
+def test_partial_gradients_cover_every_row_once(small_slab, b):
+    """One tile over two spans, two over four, 41 tiles over 40 spans: the
+    gradient of the batch against the mean over its 64-row parts (the same
+    rows in the same tiles, so only FP32 summation order and the scale 1/b
+    before BF16 rounding differ: 2^-8 per value of a sum of signed terms, held
+    to 1e-2 of the block's norm), and the same bits twice."""
+    _, m = small_slab
+    nn = F.Surrogate(m, seed=1)
+    nn.set_params(M.init_params(7))
+    rng = np.random.default_rng(2)
+    x = rng.uniform(-1, 1, (b, M.NIN)).astype(np.float32)
+    t = rng.uniform(0.0, 2.0 * TS, b).astype(np.float32)
+    loss, g = nn.gradient(x, t)
+    parts = [nn.gradient(x[i:i + 64], t[i:i + 64]) for i in range(0, b, 64)]
+    assert abs(loss - np.mean([p[0] for p in parts])) <= 1e-5 * loss
+    ref = np.mean([p[1].astype(np.float64) for p in parts], axis=0)
+    for name, sl in _blocks():
+        assert np.linalg.norm(g[sl] - ref[sl]) <= 1e-2 * np.linalg.norm(ref[sl]), name
+    again = nn.gradient(x, t)
+    assert again[0] == loss and np.array_equal(again[1], g)
+    nn.close()
+
+
 def test_adam_steps_match_oracle(small_slab):
     """k_adam against the oracle's Adam: three steps with known gradients
     through the C ABI; FP32 masters and both moments agree with the FP64
