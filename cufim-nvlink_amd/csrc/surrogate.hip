@@ -9,7 +9,8 @@
 // Device layout of the FP32 master parameters (the caller's order):
 //   W0[256 x 16] b0[256]  (W_l[256 x 256] b_l[256]) x 5  w_out[256] b_out
 // A training step is three launches (seven, with a kernel to write the rows, two
-// clears and a reduction before Adam, took 302 against 283 us at 65,536 rows):
+// clears and a reduction before Adam, took 302 against 283 us at 65,536 rows, before the chain kernel held more
+// weights in flight):
 //   k_mlp_chain: the rows of a tile of 64, the six forward layers with the
 //     activations kept in LDS, the output layer and squared error, and the
 //     five backward-data layers dZ_{l-1} = (dZ_l W_l) * SiLU'(Z_{l-1});
@@ -129,9 +130,8 @@ __device__ inline f32x16 mfma(const u16x8 a, const u16x8 b, const f32x16 c) {
                                                  0, 0, 0);
 }
 
-constexpr int RG = 1;         // row groups of 64 per tile of the fused chain kernel
-constexpr int TR = 64 * RG;   // rows per tile
-constexpr int NT = 256 * RG;  // threads per workgroup: four waves per row group
+constexpr int TR = 64;        // rows per tile
+constexpr int NT = 256;       // threads per workgroup: four waves of 64 columns
 constexpr int HP = HID + 8;   // LDS row pitch of the tile (BF16 values)
 // LDS of the chain kernel: the tile, w_out, target and then dy per row, each
 // wave's loss and bias-gradient sums
@@ -139,14 +139,14 @@ constexpr size_t CHAIN_LDS = (size_t)TR * HP * 2 + (HID + TR + 2 * NT / 64) * 4;
 static_assert(TR == 64, "batches are multiples of 64 rows and have to fill whole tiles");
 constexpr int NOUT = HID + 4;  // per tile: w_out and b_out gradients, loss sum, two unused
 
-// One layer's product for the tile: acc[i][j] (rows 64 rg + 32 i, columns
+// One layer's product for the tile: acc[i][j] (rows 32 i, columns
 // 64 fg + 32 j) = T(rows, 0..K) B, with T the tile in LDS (row-major, pitch
 // HP) and B given by fragments (fragment (mb, ks) of B^T at bfr).  The next
 // step's weight fragments are loaded before the current step's products.
 // SWAP gives the transposed product (accumulator rows are features, columns
 // rows of the tile).
 template <int K, bool SWAP>
-__device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restrict__ bfr, uint32_t rg, uint32_t fg,
+__device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restrict__ bfr, uint32_t fg,
                                     uint32_t lane, f32x16 (&acc)[2][2]) {
   constexpr int NS = K / 16;
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
@@ -158,7 +158,7 @@ __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restri
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
   const u16x8 *bp0 = reinterpret_cast<const u16x8 *>(bfr) + (size_t)(2 * fg) * NS * 64 + lane;
   const u16x8 *bp1 = bp0 + NS * 64;
-  const uint16_t *ta0 = Ts + (64 * rg + l32) * HP + 8 * lh;
+  const uint16_t *ta0 = Ts + l32 * HP + 8 * lh;
   const uint16_t *ta1 = ta0 + 32 * HP;
   // weight fragments two steps ahead, tile fragments one step ahead
   u16x8 b[2][2], t[2][2];
@@ -192,6 +192,60 @@ __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restri
   }
 }
 
+// The same for a hidden layer with DEEP k-steps of weight fragments in flight
+// across layers and barriers: b holds the first DEEP steps of this layer's
+// weights on entry and of `next`'s on return.  170 registers, so two waves a
+// SIMD; with the Z of the backward loaded before the product as well, the
+// training kernel takes 167 against 175 us for 65,536 rows and 47 against
+// 61 us for 4,160 (four waves a SIMD, two steps); eight steps 169 and 47.
+// Inference, whose epilogue is shorter, is faster with four waves (267
+// against 310 us for 362,894 rows).
+constexpr int DEEP = 4;
+using Ring = u16x8[DEEP][2];
+__device__ inline const u16x8 *frags(const uint16_t *bfr, uint32_t fg, uint32_t lane) {
+  return reinterpret_cast<const u16x8 *>(bfr) + (size_t)(2 * fg) * (HID / 16) * 64 + lane;
+}
+__device__ inline void deep_fill(Ring &b, const u16x8 *bp) {
+#pragma unroll
+  for (int s = 0; s < DEEP; ++s) {
+    b[s][0] = bp[64 * s];
+    b[s][1] = bp[64 * (HID / 16 + s)];
+  }
+}
+__device__ inline void deep_product(const uint16_t *Ts, const u16x8 *bp, const u16x8 *next, uint32_t lane, Ring &b,
+                                    f32x16 (&acc)[2][2]) {
+  constexpr int NS = HID / 16;
+  const uint32_t l32 = lane & 31u, lh = lane >> 5;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+  const uint16_t *ta0 = Ts + l32 * HP + 8 * lh;
+  const uint16_t *ta1 = ta0 + 32 * HP;
+  u16x8 t[2][2];
+  t[0][0] = *reinterpret_cast<const u16x8 *>(ta0);
+  t[0][1] = *reinterpret_cast<const u16x8 *>(ta1);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const int c = s & 1, d = s % DEEP;
+    if (s + 1 < NS) {
+      t[c ^ 1][0] = *reinterpret_cast<const u16x8 *>(ta0 + 16 * (s + 1));
+      t[c ^ 1][1] = *reinterpret_cast<const u16x8 *>(ta1 + 16 * (s + 1));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[i][j] = mfma(t[c][i], b[d][j], acc[i][j]);
+    const u16x8 *q = s + DEEP < NS ? bp + 64 * (s + DEEP) : next + 64 * (s + DEEP - NS);
+    b[d][0] = q[0];
+    b[d][1] = q[64 * NS];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 constexpr int MAPP = 16;  // per map: 13 floats = three normalised site positions, four factors - 1
 
 __device__ inline uint64_t mix64(uint64_t x) {
@@ -217,10 +271,8 @@ struct ChainArgs {
   float inv_b;
 };
 
-// The whole network for one tile of TR = 64 RG rows, activations in LDS
-// between layers.  Four waves per row group: rows 64 rg .. +63 (rg = wave /
-// 4; RG = 1, so one group of four waves), columns 64 fg .. +63 (fg = wave % 4)
-// of every product, as 2 x 2 accumulators of 32 x 32.
+// The whole network for one tile of 64 rows, activations in LDS between
+// layers.  Four waves: wave fg has columns 64 fg .. +63 of every product, as 2 x 2 accumulators of 32 x 32.
 //   forward: Z_l = H_{l-1} W_l^T + b_l, H_l = SiLU(Z_l) (BF16 in LDS; Z_l to
 //     HBM in the k-step layout);
 //   output: y = H_5 . w_out + b_out, e = y - t, dZ_5 = (2 e / B) w_out
@@ -228,25 +280,27 @@ struct ChainArgs {
 //     dZ_l in LDS; every dZ_l goes to HBM in the k-step layout.
 // Rounding to BF16 where the separate-kernel formulation stores values:
 // Z, H and dZ; SiLU'(Z) of the stored Z.
-// At 65,536 rows 384 MB out and 206 MB in, in 172 us (3.4 TB/s): memory and the
+// At 65,536 rows 384 MB out and 206 MB in, in 167 us (3.5 TB/s): memory and the
 // two barriers a layer bound it (86.7 GFLOP, 0.5 PFLOP/s).
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_mlp_chain(ChainArgs a) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mlp_chain(ChainArgs a) {
   extern __shared__ __align__(16) unsigned char chain_lds[];
   uint16_t *Ts = reinterpret_cast<uint16_t *>(chain_lds);
   float *wos = reinterpret_cast<float *>(chain_lds + TR * HP * 2);  // w_out
   float *dys = wos + HID;
   float *misc = dys + TR;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t rg = wave >> 2, fg = wave & 3u, l32 = lane & 31u, lh = lane >> 5;
+  const uint32_t fg = wave, l32 = lane & 31u, lh = lane >> 5;
   const size_t r0 = (size_t)blockIdx.x * TR;
   // k-step offset, within the tile's rows, of the four accumulator values
-  // (rows 64 rg + 32 i + 8 q + 4 lh + 0..3, column 64 fg + 32 j + l32) of
+  // (rows 32 i + 8 q + 4 lh + 0..3, column 64 fg + 32 j + l32) of
   // block (i, j), group q: ((row / 16) HID + column) 16 + row % 16
-  const uint32_t ks_lane = ((4 * rg * HID + 64 * fg + l32) << 4) + 4 * lh;
+  const uint32_t ks_lane = ((64 * fg + l32) << 4) + 4 * lh;
   auto ks_acc = [&](int i, int j, int q) -> uint32_t {
     return ks_lane + i * 32 * HID + (q >> 1) * 16 * HID + j * 32 * 16 + (q & 1) * 8;
   };
   for (uint32_t c = tid; c < HID; c += NT) wos[c] = a.w[OFF_WO + c];
+  Ring b;
+  deep_fill(b, frags(a.wb + offb_w(1), fg, lane));
   // the rows, four threads each with four inputs; every row has data (batches
   // are multiples of the tile)
   {
@@ -289,9 +343,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 #pragma unroll 1
   for (int l = 0; l < NL; ++l) {
     if (l == 0)
-      tile_product<NIN, false>(Ts, a.wb + offb_w(0), rg, fg, lane, acc);
+      tile_product<NIN, false>(Ts, a.wb + offb_w(0), fg, lane, acc);
     else
-      tile_product<HID, false>(Ts, a.wb + offb_w(l), rg, fg, lane, acc);
+      deep_product(Ts, frags(a.wb + offb_w(l), fg, lane),
+                   frags(l < NL - 1 ? a.wb + offb_w(l + 1) : a.wbt + offbt(NL - 1), fg, lane), lane, b, acc);
     __syncthreads();  // every wave has read the layer's input
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -310,7 +365,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         const uint32_t f = 64 * fg + 32 * j + l32;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const uint32_t R = 64 * rg + 32 * i + 8 * q + 4 * lh;
+          const uint32_t R = 32 * i + 8 * q + 4 * lh;
           if (zl) {
             u16x4 zv;
 #pragma unroll
@@ -373,7 +428,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const uint32_t R = 64 * rg + 32 * i + 8 * q + 4 * lh;
+        const uint32_t R = 32 * i + 8 * q + 4 * lh;
         u16x4 dv;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -387,26 +442,28 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   // backward through the hidden layers
 #pragma unroll 1
   for (int l = NL - 1; l >= 1; --l) {
-    tile_product<HID, false>(Ts, a.wbt + offbt(l), rg, fg, lane, acc);
-    __syncthreads();  // every wave has read dZ_l
+    u16x4 zp[2][2][4];  // Z_{l-1}, loaded before the product
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      u16x4 zp[2][4];  // Z_{l-1} of this row block, loaded before any is used
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          zp[j][q] = *reinterpret_cast<const u16x4 *>(a.Z[l - 1] + r0 * HID + ks_acc(i, j, q));
+          zp[i][j][q] = *reinterpret_cast<const u16x4 *>(a.Z[l - 1] + r0 * HID + ks_acc(i, j, q));
+    deep_product(Ts, frags(a.wbt + offbt(l), fg, lane), frags(a.wbt + offbt(l > 1 ? l - 1 : 1), fg, lane), lane, b, acc);
+    __syncthreads();  // every wave has read dZ_l
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const uint32_t k = 64 * fg + 32 * j + l32;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const uint32_t R = 64 * rg + 32 * i + 8 * q + 4 * lh;
+          const uint32_t R = 32 * i + 8 * q + 4 * lh;
           u16x4 dv;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
-            dv[c] = f2bf(acc[i][j][4 * q + c] * dsilu(bf2f(zp[j][q][c])));
+            dv[c] = f2bf(acc[i][j][4 * q + c] * dsilu(bf2f(zp[i][j][q][c])));
             Ts[(R + c) * HP + k] = dv[c];
           }
           *reinterpret_cast<u16x4 *>(a.dZ[l - 1] + r0 * HID + ks_acc(i, j, q)) = dv;
@@ -481,9 +538,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   for (int l = 0; l < NL; ++l) {
     const uint16_t *wl = a.wb + offb_w(l);
     if (l == 0)
-      tile_product<NIN, true>(Ts, wl, 0, fg, lane, acc);
+      tile_product<NIN, true>(Ts, wl, fg, lane, acc);
     else
-      tile_product<HID, true>(Ts, wl, 0, fg, lane, acc);
+      tile_product<HID, true>(Ts, wl, fg, lane, acc);
     const float *bl = a.w + off_b(l) + 64 * fg + 4 * lh;
     __syncthreads();  // every wave has read the layer's input
 #pragma unroll
@@ -875,6 +932,7 @@ void infer(fim_nn *n, const float *x, const float *mp, const uint32_t *sample, u
            float *out) {
   const InferArgs a{x, n->coords, mp, sample, m, n->wb, n->w, out, nreal, t_scale(n), delta};
   k_mlp_infer<<<(nreal + TR - 1) / TR, 256, CHAIN_LDS, n->stream>>>(a);
+
   HIPCHECK(hipGetLastError());
 }
 
@@ -901,6 +959,7 @@ uint32_t train_pass(fim_nn *n, const float *x, uint64_t seed, uint32_t B) {
   a.tp = n->tp;
   a.inv_b = 1.0f / (float)B;
   k_mlp_chain<<<B / TR, NT, CHAIN_LDS, n->stream>>>(a);
+
   // weight gradients: S spans of whole 32-row steps, one partial sum each
   const uint32_t S = std::min<uint32_t>(n->nsplit, B / 32);
   WGradArgs wa;
@@ -1040,10 +1099,8 @@ int fim_nn_create(const fim_mesh *mesh, const fim_nn_opts *o, fim_nn **out) {
       n->out = nn_alloc<float>(n, n->cap);
       n->parts = nn_alloc<float>(n, (size_t)n->nsplit * PST);
       n->tp = nn_alloc<float>(n, (size_t)(n->cap / TR) * NOUT);
-      HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_chain, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)CHAIN_LDS));
-      HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_infer, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)CHAIN_LDS));
+      for (const void *k : {(const void *)k_mlp_chain, (const void *)k_mlp_infer})
+        HIPCHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CHAIN_LDS));
       HIPCHECK(hipFuncSetAttribute((const void *)k_mlp_wgrad, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    WG_LDS * 2));
       n->coords = nn_alloc<float>(n, 3 * (size_t)n->nn);
