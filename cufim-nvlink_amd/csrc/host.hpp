@@ -2,14 +2,34 @@
 // device pack).  Internal to libcufim.so; the public surface is include/cufim.h.
 #pragma once
 
+#include <algorithm>
+#include <cstddef>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "cufim.h"
 
 namespace fim {
+
+// f(begin, end) over [0, n) on up to eight host threads, at least `least` each
+// (starting and joining four took 20 to 50 us).  f may not throw.
+template <class F>
+void parallel_ranges(size_t n, size_t least, F &&f) {
+  const size_t nt = std::max<size_t>(1, std::min<size_t>({8, (size_t)std::thread::hardware_concurrency(), n / least}));
+  std::vector<std::thread> ts;
+  ts.reserve(nt);
+  size_t t = 1;
+  try {
+    for (; t < nt; ++t) ts.emplace_back([&f, n, nt, t] { f(n * t / nt, n * (t + 1) / nt); });
+  } catch (const std::exception &) {  // no more threads: the rest on this one
+  }
+  f(0, n / nt);
+  if (t < nt) f(n * t / nt, n);
+  for (auto &w : ts) w.join();
+}
 
 // error carried to the C ABI as (code, message)
 struct Error : std::runtime_error {

@@ -4,7 +4,6 @@
 #include <cmath>
 #include <map>
 #include <numeric>
-#include <thread>
 
 #include "host.hpp"
 #include "local_solve.hpp"
@@ -205,15 +204,9 @@ int64_t converge_lds_bytes(int32_t nn_max, int32_t ne_max) {
 static void element_bounds(Pack &k) {
   k.bnd8.resize(12 * (size_t)k.ne_global);
   k.bnd_scale.resize((size_t)k.ne_global);
-  auto run = [&](int64_t b, int64_t e) {
-    for (int64_t i = b; i < e; ++i) cand_bounds(&k.geo64[6 * i], &k.bnd8[12 * i], &k.bnd_scale[i]);
-  };
-  const int64_t nt = std::max<int64_t>(1, std::min<int64_t>({8, (int64_t)std::thread::hardware_concurrency(),
-                                                             k.ne_global / 4096}));
-  std::vector<std::thread> ts;
-  for (int64_t t = 1; t < nt; ++t) ts.emplace_back(run, k.ne_global * t / nt, k.ne_global * (t + 1) / nt);
-  run(0, k.ne_global / nt);
-  for (auto &t : ts) t.join();
+  parallel_ranges((size_t)k.ne_global, 4096, [&](size_t b, size_t e) {
+    for (size_t i = b; i < e; ++i) cand_bounds(&k.geo64[6 * i], &k.bnd8[12 * i], &k.bnd_scale[i]);
+  });
 }
 
 Pack build_pack(const Mesh &m, const Partition &p, int32_t source) {

@@ -38,7 +38,6 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
-#include <thread>
 #include <string>
 #include <vector>
 
@@ -2289,17 +2288,6 @@ T *dalloc(size_t n, std::vector<void *> &owned) {
   HIPCHECK(hipMalloc(&p, n * sizeof(T)));
   owned.push_back(p);
   return static_cast<T *>(p);
-}
-
-// f(begin, end) over [0, n) on up to eight host threads, at least `least` each
-// (starting a thread costs about 50 us)
-template <class F>
-void parallel_ranges(size_t n, size_t least, F &&f) {
-  const size_t nt = std::max<size_t>(1, std::min<size_t>({8, (size_t)std::thread::hardware_concurrency(), n / least}));
-  std::vector<std::thread> ts;
-  for (size_t t = 1; t < nt; ++t) ts.emplace_back([&, t] { f(n * t / nt, n * (t + 1) / nt); });
-  f(0, n / nt);
-  for (auto &t : ts) t.join();
 }
 
 template <class T>
