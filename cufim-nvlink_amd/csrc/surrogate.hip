@@ -875,6 +875,11 @@ struct fim_nn {
   // activations (rows = cap, a multiple of the chain kernel's tile), k-step layout
   uint32_t cap = 0;
   uint16_t *X0 = nullptr, *Z[NL - 1] = {}, *dZ[NL] = {};
+  // pinned staging of what a call takes and gives (stage_n bytes: a map or the
+  // gradient; more goes the pageable way), and its device address
+  unsigned char *stage = nullptr, *stage_d = nullptr;
+  size_t stage_n = 0;
+  float *xin = nullptr;  // given rows, or the parameters of a chunk of solves
   float *tgt = nullptr, *out = nullptr, *parts = nullptr, *tp = nullptr;
   uint32_t nsplit = 1;  // row spans of the weight gradients (partial sums)
   // dataset
@@ -895,6 +900,7 @@ T *nn_alloc(fim_nn *n, size_t count) {
 void nn_destroy(fim_nn *n) {
   if (!n) return;
   for (void *p : n->owned) (void)hipFree(p);
+  if (n->stage) (void)hipHostFree(n->stage);
   if (n->stream) (void)hipStreamDestroy(n->stream);
   delete n;
 }
@@ -923,6 +929,20 @@ void ensure_rows(fim_nn *n, uint32_t rows) {
 
 // rows rounded up to whole tiles of the chain kernel
 uint32_t tile_rows(uint32_t rows) { return (rows + TR - 1) / TR * TR; }
+
+// `bytes` from src to dst in stream order; through the staging buffer at
+// `at` where it holds them (src may then be gone when the call returns, and
+// the bytes up to the returned end may not be written before the stream is
+// past the copy)
+size_t upload(fim_nn *n, void *dst, const void *src, size_t bytes, size_t at) {
+  if (at + bytes <= n->stage_n) {
+    std::memcpy(n->stage + at, src, bytes);
+    src = n->stage + at;
+    at += bytes;
+  }
+  HIPCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, n->stream));
+  return at;
+}
 
 float t_scale(const fim_nn *n) { return (float)(n->o.t_scale > 0 ? n->o.t_scale : 1e5); }
 
@@ -1097,6 +1117,10 @@ int fim_nn_create(const fim_mesh *mesh, const fim_nn_opts *o, fim_nn **out) {
       for (int l = 0; l < NL; ++l) n->dZ[l] = nn_alloc<uint16_t>(n, (size_t)n->cap * HID);
       n->tgt = nn_alloc<float>(n, n->cap);
       n->out = nn_alloc<float>(n, n->cap);
+      n->xin = nn_alloc<float>(n, (size_t)n->cap * NIN);
+      n->stage_n = std::max<size_t>(n->cap, NPAR + 1) * sizeof(float);
+      HIPCHECK(hipHostMalloc((void **)&n->stage, n->stage_n, hipHostMallocDefault));
+      HIPCHECK(hipHostGetDevicePointer((void **)&n->stage_d, n->stage, 0));
       n->parts = nn_alloc<float>(n, (size_t)n->nsplit * PST);
       n->tp = nn_alloc<float>(n, (size_t)(n->cap / TR) * NOUT);
       for (const void *k : {(const void *)k_mlp_chain, (const void *)k_mlp_infer})
@@ -1217,24 +1241,15 @@ int fim_nn_gradient(fim_nn *n, const float *x, const float *t, int32_t b, double
     HIPCHECK(hipSetDevice(n->dev));
     std::vector<float> ts(b);
     for (int32_t i = 0; i < b; ++i) ts[i] = t[i] / t_scale(n);
-    float *xd = nullptr;
-    HIPCHECK(hipMalloc(&xd, (size_t)b * NIN * sizeof(float)));
-    try {
-      HIPCHECK(hipMemcpyAsync(xd, x, (size_t)b * NIN * sizeof(float), hipMemcpyHostToDevice, n->stream));
-      HIPCHECK(hipMemcpyAsync(n->tgt, ts.data(), (size_t)b * sizeof(float), hipMemcpyHostToDevice, n->stream));
-      const uint32_t S = train_pass(n, xd, 0, (uint32_t)b);
-      k_reduce_parts<<<NPAR / 256 + 1, 256, 0, n->stream>>>(n->parts, S, n->g);
-      HIPCHECK(hipGetLastError());
-      float l = 0.0f;
-      HIPCHECK(hipMemcpyAsync(grad, n->g, NPAR * sizeof(float), hipMemcpyDeviceToHost, n->stream));
-      HIPCHECK(hipMemcpyAsync(&l, n->g + NPAR, sizeof(float), hipMemcpyDeviceToHost, n->stream));
-      HIPCHECK(hipStreamSynchronize(n->stream));
-      *loss = (double)l / b;
-    } catch (...) {
-      (void)hipFree(xd);
-      throw;
-    }
-    HIPCHECK(hipFree(xd));
+    const size_t at = upload(n, n->xin, x, (size_t)b * NIN * sizeof(float), 0);
+    (void)upload(n, n->tgt, ts.data(), (size_t)b * sizeof(float), at);
+    const uint32_t S = train_pass(n, n->xin, 0, (uint32_t)b);
+    k_reduce_parts<<<NPAR / 256 + 1, 256, 0, n->stream>>>(n->parts, S, reinterpret_cast<float *>(n->stage_d));
+    HIPCHECK(hipGetLastError());
+    HIPCHECK(hipStreamSynchronize(n->stream));
+    const float *g = reinterpret_cast<const float *>(n->stage);
+    std::memcpy(grad, g, NPAR * sizeof(float));
+    *loss = (double)g[NPAR] / b;
   });
 }
 
@@ -1263,18 +1278,10 @@ int fim_nn_predict(fim_nn *n, const float *x, int64_t count, float *t) {
     if (count > (int64_t)n->cap) throw Error(FIM_ELIMIT, "batch larger than the surrogate's row capacity");
     ensure_rows(n, tile_rows((uint32_t)count));
     HIPCHECK(hipSetDevice(n->dev));
-    float *xd = nullptr;
-    HIPCHECK(hipMalloc(&xd, (size_t)count * NIN * sizeof(float)));
-    try {
-      HIPCHECK(hipMemcpyAsync(xd, x, (size_t)count * NIN * sizeof(float), hipMemcpyHostToDevice, n->stream));
-      infer(n, xd, nullptr, nullptr, 0u, (uint32_t)count, 0.0f, n->out);
-      HIPCHECK(hipMemcpyAsync(t, n->out, (size_t)count * sizeof(float), hipMemcpyDeviceToHost, n->stream));
-      HIPCHECK(hipStreamSynchronize(n->stream));
-    } catch (...) {
-      (void)hipFree(xd);
-      throw;
-    }
-    HIPCHECK(hipFree(xd));
+    (void)upload(n, n->xin, x, (size_t)count * NIN * sizeof(float), 0);
+    infer(n, n->xin, nullptr, nullptr, 0u, (uint32_t)count, 0.0f, reinterpret_cast<float *>(n->stage_d));
+    HIPCHECK(hipStreamSynchronize(n->stream));
+    std::memcpy(t, n->stage, (size_t)count * sizeof(float));
   });
 }
 
@@ -1300,33 +1307,19 @@ int fim_nn_predict_max(fim_nn *n, int32_t count, const int64_t *sites, const flo
     HIPCHECK(hipSetDevice(n->dev));
     // solves per forward pass: as many whole samples as the rows hold
     const uint32_t per = std::max<uint32_t>(1u, n->cap / (uint32_t)m);
-    uint32_t *sd = nullptr;
-    float *md = nullptr, *od = nullptr;
-    try {
-      HIPCHECK(hipMalloc(&sd, sv.size() * sizeof(uint32_t)));
-      HIPCHECK(hipMalloc(&md, mp.size() * sizeof(float)));
-      HIPCHECK(hipMalloc(&od, (size_t)count * sizeof(float)));
-      HIPCHECK(hipMemcpyAsync(sd, sv.data(), sv.size() * sizeof(uint32_t), hipMemcpyHostToDevice, n->stream));
-      HIPCHECK(hipMemcpyAsync(md, mp.data(), mp.size() * sizeof(float), hipMemcpyHostToDevice, n->stream));
-      for (uint32_t j0 = 0; j0 < (uint32_t)count; j0 += per) {
-        const uint32_t nj = std::min<uint32_t>(per, (uint32_t)count - j0);
-        const uint32_t nreal = nj * (uint32_t)m;
-        infer(n, nullptr, md + (size_t)j0 * MAPP, sd, (uint32_t)m, nreal, 0.0f, n->out);
-        k_solve_max<<<std::min<uint32_t>((nj + 3) / 4, 4096), 256, 0, n->stream>>>(n->out, (uint32_t)m, nj,
-                                                                                  od + j0);
-        HIPCHECK(hipGetLastError());
-      }
-      HIPCHECK(hipMemcpyAsync(out, od, (size_t)count * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+    uint32_t *sd = reinterpret_cast<uint32_t *>(n->tgt);  // a training batch's targets: >= m words
+    size_t at = upload(n, sd, sv.data(), sv.size() * sizeof(uint32_t), 0);
+    for (uint32_t j0 = 0; j0 < (uint32_t)count; j0 += per) {
+      const uint32_t nj = std::min<uint32_t>(per, (uint32_t)count - j0);
+      (void)upload(n, n->xin, mp.data() + (size_t)j0 * MAPP, (size_t)nj * MAPP * sizeof(float), at);
+      infer(n, nullptr, n->xin, sd, (uint32_t)m, nj * (uint32_t)m, 0.0f, n->out);
+      k_solve_max<<<std::min<uint32_t>((nj + 3) / 4, 4096), 256, 0, n->stream>>>(
+          n->out, (uint32_t)m, nj, reinterpret_cast<float *>(n->stage_d));
+      HIPCHECK(hipGetLastError());
       HIPCHECK(hipStreamSynchronize(n->stream));
-    } catch (...) {
-      (void)hipFree(sd);
-      (void)hipFree(md);
-      (void)hipFree(od);
-      throw;
+      std::memcpy(out + j0, n->stage, nj * sizeof(float));
+      at = 0;
     }
-    HIPCHECK(hipFree(sd));
-    HIPCHECK(hipFree(md));
-    HIPCHECK(hipFree(od));
   });
 }
 
@@ -1335,9 +1328,9 @@ int fim_nn_predict_map(fim_nn *n, const int64_t *sites, int32_t n_sites, const f
     if (!n || !sites || !scales || !t) throw Error(FIM_EINVAL, "null argument");
     HIPCHECK(hipSetDevice(n->dev));
     const std::vector<float> mp = map_params(n, sites, n_sites, scales);
-    predict_map_device(n, mp, 0.0f, n->out);
-    HIPCHECK(hipMemcpyAsync(t, n->out, (size_t)n->nn * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+    predict_map_device(n, mp, 0.0f, reinterpret_cast<float *>(n->stage_d));
     HIPCHECK(hipStreamSynchronize(n->stream));
+    std::memcpy(t, n->stage, (size_t)n->nn * sizeof(float));
   });
 }
 

@@ -125,6 +125,26 @@ def test_partial_gradients_cover_every_row_once(small_slab, b):
     nn.close()
 
 
+@pytest.mark.parametrize("rows", [19584, 19648, 20864])
+def test_calls_around_the_staging_capacity(small_slab, rows):
+    """1.33 MB of staging hold rows and targets up to 19,621 rows and the rows
+    alone up to 20,848: the same predictions as in two parts, and the
+    gradient as the mean over them (as above)."""
+    _, m = small_slab
+    nn = F.Surrogate(m, seed=1)
+    nn.set_params(M.init_params(7))
+    rng = np.random.default_rng(4)
+    x = rng.uniform(-1, 1, (rows, M.NIN)).astype(np.float32)
+    t = rng.uniform(0.0, 2.0 * TS, rows).astype(np.float32)
+    h = rows // 128 * 64
+    assert np.array_equal(nn.predict(x), np.concatenate([nn.predict(x[:h]), nn.predict(x[h:])]))
+    g = nn.gradient(x, t)[1]
+    ref = (h * nn.gradient(x[:h], t[:h])[1].astype(np.float64) + (rows - h) * nn.gradient(x[h:], t[h:])[1]) / rows
+    for name, sl in _blocks():
+        assert np.linalg.norm(g[sl] - ref[sl]) <= 1e-2 * np.linalg.norm(ref[sl]), name
+    nn.close()
+
+
 def test_adam_steps_match_oracle(small_slab):
     """k_adam against the oracle's Adam: three steps with known gradients
     through the C ABI; FP32 masters and both moments agree with the FP64

@@ -536,3 +536,26 @@ def test_solver_group_maps_instances_to_contexts():
     for bad in (-1, 12):
         with pytest.raises(F.FimError):
             g.download(inst=bad)
+
+
+@pytest.mark.parametrize("sets", [
+    [], [[5]], [[1, 2, 3], (4,), np.array([7, 8])], [np.array([3.0]), [2.0, 1]], [[[1, 2]], [3]], [7, [1]],
+    [np.array([[4], [5]]), (6, 6, 6)], [range(2), [9]]])
+def test_all_site_sets_at_once_equal_one_by_one(sets):
+    want = np.array([F._sites3(x)[0] for x in sets], dtype=np.int64).reshape(len(sets), 3)
+    got = F._sites3_all(sets)
+    assert got.dtype == np.int64 and np.array_equal(got, want)
+    f = [np.arange(4.0) + i if i % 2 else [1.0, 2, 3, i] for i in range(len(sets))]
+    want = np.array([np.asarray(x, np.float32) for x in f], np.float32).reshape(len(sets), 4)
+    got = F._factors_all(f)
+    assert got.dtype == np.float32 and got.flags.c_contiguous and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("sets", [[[]], [[1, 2, 3, 4]], [[1], np.zeros(0, np.int64)], [{1, 2}], [["a"]]])
+def test_site_sets_that_are_refused_one_by_one_are_refused_at_once(sets):
+    with pytest.raises((AssertionError, TypeError, ValueError)):
+        [F._sites3(x) for x in sets]
+    with pytest.raises((AssertionError, TypeError, ValueError)):
+        F._sites3_all(sets)
+    with pytest.raises(ValueError):
+        F._factors_all([[1.0, 2, 3], [1.0, 2, 3, 4, 5]])
