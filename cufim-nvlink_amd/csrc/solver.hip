@@ -1539,6 +1539,61 @@ __global__ void k_fill(T *p, size_t n, T v) {
     p[i] = v;
 }
 
+// Several arrays filled in one launch (a context's reset was ten, at about 4 us
+// each on a small mesh): 16 bytes of each array's pattern at a time, and
+// the bytes left at its end.
+struct FillArgs {
+  struct {
+    void *p;       // 16-byte aligned
+    size_t bytes;
+    uint4 v;       // the pattern (of 1, 4 or 8 bytes, repeated)
+  } seg[10];
+  int n = 0;
+  template <class T>
+  void add(T *p, size_t count, T v) {
+    static_assert(sizeof(T) <= 8, "pattern");
+    unsigned char b[16];
+    for (size_t i = 0; i < 16; i += sizeof(T)) std::memcpy(b + i, &v, sizeof(T));
+    seg[n].p = p;
+    seg[n].bytes = count * sizeof(T);
+    std::memcpy(&seg[n++].v, b, 16);
+  }
+};
+
+__global__ __launch_bounds__(256) void k_fill_all(FillArgs a) {
+  const size_t first = blockIdx.x * (size_t)256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+  for (int k = 0; k < a.n; ++k) {
+    const size_t n16 = a.seg[k].bytes / 16;
+    const uint4 v = a.seg[k].v;
+    uint4 *p = static_cast<uint4 *>(a.seg[k].p);
+    for (size_t i = first; i < n16; i += step) p[i] = v;
+    if (first < a.seg[k].bytes % 16) {
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+      reinterpret_cast<unsigned char *>(p + n16)[first] = (unsigned char)(w[first / 4] >> 8 * (first % 4));
+    }
+  }
+}
+
+// Before a run: speed factors and windows from pinned memory, counters cleared
+// (two copies, a wait and a clear before)
+__global__ __launch_bounds__(256) void k_run_begin(const float *src, uint32_t nr, float *rscale, uint32_t nw,
+                                                   float *winst, unsigned long long *stats) {
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < nr + nw; i += gridDim.x * 256) {
+    if (i < nr)
+      rscale[i] = src[i];
+    else
+      winst[i - nr] = src[i];
+  }
+  if (stats && blockIdx.x == 0 && threadIdx.x < 8) stats[threadIdx.x] = 0ull;
+}
+
+// After a chunk of iterations: queued units and counters to pinned memory
+// (word 0; words 2..17)
+__global__ void k_chunk_end(const uint32_t *left, const uint32_t *stats, uint32_t *pin) {
+  if (threadIdx.x == 0) pin[0] = *left;
+  if (threadIdx.x < 16) pin[2 + threadIdx.x] = stats[threadIdx.x];
+}
+
 // min over copies of each global vertex
 __global__ void k_conv_gather(const float *phi, const uint32_t *g2c_dsp, const uint32_t *g2c,
                               uint32_t nn, size_t ib, float *out) {
@@ -2346,6 +2401,7 @@ struct fim_ctx {
   // launch that reads them: setting up a batch costs no device round trip
   // per instance
   std::vector<float> h_rscale, h_winst;
+  float *h_par = nullptr, *d_par = nullptr;  // the two on their way: pinned, and its device address
   bool params_dirty = false;
   uint32_t *d_flag = nullptr;   // n_inst: scratch for instance queries / lists
   uint32_t *d_inbox = nullptr;  // 2 x n_inst x interface entries
@@ -2374,7 +2430,7 @@ struct fim_ctx {
   // shared
   unsigned long long *d_stats = nullptr;
   uint32_t *h_pin = nullptr, *d_pin = nullptr;  // pinned host words and their device address
-  // seed staging: pinned host and device buffers of (instance, copy) pairs
+  // (instance, copy) pairs to seed: pinned, and the device address
   uint2 *h_seed = nullptr, *d_seed = nullptr;
   size_t seed_cap = 0;
   float *d_tmpf = nullptr;
@@ -2536,8 +2592,8 @@ void destroy_ctx(fim_ctx *c) {
   for (void *p : c->owned) (void)hipFree(p);
   if (c->h_pin) (void)hipHostFree(c->h_pin);
   if (c->h_map) (void)hipHostFree(c->h_map);
+  if (c->h_par) (void)hipHostFree(c->h_par);
   if (c->h_seed) (void)hipHostFree(c->h_seed);
-  if (c->d_seed) (void)hipFree(c->d_seed);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -2609,13 +2665,18 @@ uint32_t *noalloc_scratch(int dev) {
 
 // uploads the per-instance factors and windows set since the last upload
 // (the device must be current)
-void flush_params(fim_ctx *c) {
-  if (!c->params_dirty) return;
-  HIPCHECK(hipMemcpyAsync(c->d_rscale, c->h_rscale.data(), c->h_rscale.size() * sizeof(float),
-                          hipMemcpyHostToDevice, c->stream));
-  HIPCHECK(hipMemcpyAsync(c->d_winst, c->h_winst.data(), c->h_winst.size() * sizeof(float),
-                          hipMemcpyHostToDevice, c->stream));
-  HIPCHECK(hipStreamSynchronize(c->stream));
+void flush_params(fim_ctx *c, bool clear_stats = false) {
+  if (!c->params_dirty && !clear_stats) return;
+  const uint32_t nr = c->params_dirty ? (uint32_t)c->h_rscale.size() : 0u;
+  const uint32_t nw = c->params_dirty ? (uint32_t)c->h_winst.size() : 0u;
+  if (c->params_dirty) {
+    HIPCHECK(hipStreamSynchronize(c->stream));  // a kernel may still read the last ones (idle but after an error)
+    std::memcpy(c->h_par, c->h_rscale.data(), nr * sizeof(float));
+    std::memcpy(c->h_par + nr, c->h_winst.data(), nw * sizeof(float));
+  }
+  k_run_begin<<<blocks_for(nr + nw, 256), 256, 0, c->stream>>>(c->d_par, nr, c->d_rscale, nw, c->d_winst,
+                                                              clear_stats ? c->d_stats : nullptr);
+  HIPCHECK(hipGetLastError());
   c->params_dirty = false;
 }
 
@@ -2665,7 +2726,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
       HIPCHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
       HIPCHECK(hipEventCreate(&c->ev0));
       HIPCHECK(hipEventCreate(&c->ev1));
-      HIPCHECK(hipEventCreateWithFlags(&c->evc, hipEventDisableTiming));
+      HIPCHECK(hipEventCreate(&c->evc));
       if (o->mode != FIM_MODE_CONVERGE && o->mode != FIM_MODE_COMPAT)
         throw Error(FIM_EINVAL, "unknown mode");
       c->block = o->block ? o->block : (o->mode == FIM_MODE_CONVERGE ? 512 : 256);
@@ -2701,7 +2762,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
       c->d_g2c_dsp = dupload(p.g2c_dsp, ow);
       c->d_g2c = dupload(p.g2c, ow);
       c->d_stats = dalloc<unsigned long long>(8, ow);
-      HIPCHECK(hipHostMalloc((void **)&c->h_pin, 64, hipHostMallocDefault));
+      HIPCHECK(hipHostMalloc((void **)&c->h_pin, 128, hipHostMallocDefault));
       HIPCHECK(hipHostGetDevicePointer((void **)&c->d_pin, c->h_pin, 0));
       const size_t per = o->mode == FIM_MODE_CONVERGE ? sizeof(float) : sizeof(double) + sizeof(int32_t);
       HIPCHECK(hipHostMalloc((void **)&c->h_map, std::max<size_t>(c->nn * per, 64), hipHostMallocDefault));
@@ -2881,6 +2942,8 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->d_tmpf = dalloc<float>(c->nn, ow);
         k_fill<float><<<blocks_for(4 * (size_t)c->ninst, 256), 256, 0, c->stream>>>(c->d_rscale, 4 * (size_t)c->ninst, 1.0f);
         c->h_rscale.assign(4 * (size_t)c->ninst, 1.0f);
+        HIPCHECK(hipHostMalloc((void **)&c->h_par, 5 * (size_t)c->ninst * sizeof(float), hipHostMallocDefault));
+        HIPCHECK(hipHostGetDevicePointer((void **)&c->d_par, c->h_par, 0));
         // one resident wave of workgroups: registers, LDS and wave slots.
         // Workgroups of 256 put one wave on each SIMD, so the LDS carve
         // alone caps the waves per SIMD at 160 KB / carve; the band kernel
@@ -3037,24 +3100,25 @@ int fim_reset(fim_ctx *c) {
   return guarded([&] {
     if (!c) throw Error(FIM_EINVAL, "null context");
     HIPCHECK(hipSetDevice(c->dev));
+    FillArgs f;
     if (c->o.mode == FIM_MODE_CONVERGE) {
       const size_t ncs = (size_t)c->ninst * c->ncopy, nss = (size_t)c->ninst * c->nsub;
       settle(c);  // empties the inbox
-      k_fill<float><<<blocks_for(ncs, 256), 256, 0, c->stream>>>(c->d_phi, ncs, F_INF);
-      k_fill<uint8_t><<<blocks_for(ncs, 256), 256, 0, c->stream>>>(c->d_dirty, ncs, (uint8_t)0);
-      k_fill<uint32_t><<<blocks_for(2 * nss, 256), 256, 0, c->stream>>>(c->d_act, 2 * nss, 0u);
-      k_fill<float><<<blocks_for(nss, 256), 256, 0, c->stream>>>(c->d_wake, nss, F_INF);
-      k_fill<float><<<blocks_for(2 * nss, 256), 256, 0, c->stream>>>(c->d_wpush, 2 * nss, F_INF);
-      k_fill<uint32_t><<<1, 64, 0, c->stream>>>(c->d_cnt, 48, 0u);
-      k_fill<uint32_t><<<blocks_for(c->ninst, 256), 256, 0, c->stream>>>(c->d_start, c->ninst, 0u);
-      for (int k = 0; k < 3; ++k)
-        k_fill<uint32_t><<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>(c->wl[k].bcnt, c->nsub, 0u);
+      f.add(c->d_phi, ncs, F_INF);
+      f.add(c->d_dirty, ncs, (uint8_t)0);
+      f.add(c->d_act, 2 * nss, 0u);
+      f.add(c->d_wake, nss, F_INF);
+      f.add(c->d_wpush, 2 * nss, F_INF);
+      f.add(c->d_cnt, 48, 0u);
+      f.add(c->d_start, c->ninst, 0u);
+      for (int k = 0; k < 3; ++k) f.add(c->wl[k].bcnt, c->nsub, 0u);
     } else {
-      k_fill<double><<<blocks_for(c->ncopy, 256), 256, 0, c->stream>>>(c->d_phi64, c->ncopy, DBL_MAX);
-      k_fill<int8_t><<<blocks_for(c->ncopy, 256), 256, 0, c->stream>>>(c->d_st, c->ncopy, (int8_t)FIM_FAR);
-      k_fill<double><<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>(c->d_nexte, c->nsub, INFINITY);
-      k_fill<uint32_t><<<1, 64, 0, c->stream>>>(c->d_lcnt, 3, 0u);
+      f.add(c->d_phi64, c->ncopy, DBL_MAX);
+      f.add(c->d_st, c->ncopy, (int8_t)FIM_FAR);
+      f.add(c->d_nexte, c->nsub, (double)INFINITY);
+      f.add(c->d_lcnt, 3, 0u);
     }
+    k_fill_all<<<blocks_for(f.seg[0].bytes / 16 + 1, 256), 256, 0, c->stream>>>(f);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(c->stream));
   });
@@ -3071,17 +3135,15 @@ void seed_pairs(fim_ctx *c, const std::vector<uint2> &ic, double t0) {
   if (ic.size() > c->seed_cap) {
     HIPCHECK(hipStreamSynchronize(c->stream));
     if (c->h_seed) HIPCHECK(hipHostFree(c->h_seed));
-    if (c->d_seed) HIPCHECK(hipFree(c->d_seed));
     c->h_seed = nullptr;
     c->d_seed = nullptr;
     c->seed_cap = 0;
     const size_t cap = std::max<size_t>(ic.size(), 1024);
     HIPCHECK(hipHostMalloc((void **)&c->h_seed, cap * sizeof(uint2), hipHostMallocDefault));
-    HIPCHECK(hipMalloc(&c->d_seed, cap * sizeof(uint2)));
+    HIPCHECK(hipHostGetDevicePointer((void **)&c->d_seed, c->h_seed, 0));
     c->seed_cap = cap;
   }
   std::memcpy(c->h_seed, ic.data(), ic.size() * sizeof(uint2));
-  HIPCHECK(hipMemcpyAsync(c->d_seed, c->h_seed, ic.size() * sizeof(uint2), hipMemcpyHostToDevice, c->stream));
   const int g = blocks_for(ic.size(), 256);
   if (c->o.mode == FIM_MODE_CONVERGE) {
     k_conv_seed<<<g, 256, 0, c->stream>>>(c->d_seed, (uint32_t)ic.size(), (float)t0, c->d_c2s, c->d_phi,
@@ -3217,7 +3279,7 @@ struct RunState {
 
 void run_begin(fim_ctx *c, int32_t max_iters, bool reset_stats, RunState &r) {
   HIPCHECK(hipSetDevice(c->dev));
-  flush_params(c);
+  flush_params(c, reset_stats);
   // profile mode launches the same sequence of kernels without the graph
   // (events cannot be timed inside a graph) and times every compute launch
   if (c->o.profile && c->kev.empty()) {
@@ -3226,7 +3288,6 @@ void run_begin(fim_ctx *c, int32_t max_iters, bool reset_stats, RunState &r) {
   }
   if (!c->o.profile && !c->direct && !c->gexec) build_graph(c);
   if (reset_stats) {
-    HIPCHECK(hipMemsetAsync(c->d_stats, 0, 8 * sizeof(unsigned long long), c->stream));
     c->stats.compute_ms = 0.0;
     c->stats.compute_launches = 0;
   }
@@ -3248,7 +3309,8 @@ void run_chunk(fim_ctx *c, RunState &r) {
     HIPCHECK(hipGraphLaunch(c->gexec, c->stream));
   }
   r.done += c->graph_iters;
-  HIPCHECK(hipMemcpyAsync(c->h_pin, c->d_cnt, 4, hipMemcpyDeviceToHost, c->stream));
+  k_chunk_end<<<1, 64, 0, c->stream>>>(c->d_cnt, reinterpret_cast<const uint32_t *>(c->d_stats), c->d_pin);
+  HIPCHECK(hipGetLastError());
   HIPCHECK(hipEventRecord(c->evc, c->stream));
 }
 
@@ -3268,13 +3330,11 @@ bool run_collect(fim_ctx *c, RunState &r) {
 }
 
 void run_end(fim_ctx *c, RunState &r) {
-  HIPCHECK(hipSetDevice(c->dev));
-  HIPCHECK(hipEventRecord(c->ev1, c->stream));
-  unsigned long long st[8];
-  HIPCHECK(hipMemcpyAsync(st, c->d_stats, sizeof(st), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(hipStreamSynchronize(c->stream));
+  unsigned long long st[8];  // of the last chunk, whose event has completed
+  std::memcpy(st, c->h_pin + 2, sizeof(st));
   float ms = 0;
-  HIPCHECK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
+  HIPCHECK(hipSetDevice(c->dev));
+  HIPCHECK(hipEventElapsedTime(&ms, c->ev0, c->evc));
   c->stats.last_ms = ms;
   c->stats.activations = (int64_t)st[0];
   c->stats.local_iters = (int64_t)st[1];

@@ -705,3 +705,47 @@ def test_converge_edge_cases():
     again, _ = s.download(inst=0)
     assert np.array_equal(again, p0)
     s.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 9])
+@pytest.mark.parametrize("n_inst", [1, 3])
+def test_reset_leaves_nothing(n, n_inst):
+    """a reset after a run, at array lengths of every remainder by the 16-byte
+    fills: every vertex FAR, the counters of a run start at zero, the factors
+    set in between take effect, and the next run gives the maps of a context
+    that had none before"""
+    cfg = dict(cases.CUBE, nx=n, ny=n, nz=n + 1)
+    m = F.Mesh.gen_box(seed=3, **cfg)
+    p = F.Pack(m, F.PART_RCB, max_nn=64, seed=3)
+    far = np.finfo(np.float64).max
+
+    def run(s):
+        for i in range(n_inst):
+            s.set_scaling([1.0 + 0.25 * i] * 4, inst=i)
+            s.seed([i % m.nn], 0.0, inst=i)
+        s.run()
+        return [s.download(inst=i)[0] for i in range(n_inst)], s.stats()["activations"]
+
+    s = F.Solver(p, n_instances=n_inst, window=0.0)
+    want, acts = run(s)
+    for i in range(n_inst):
+        s.set_scaling([3.0] * 4, inst=i)
+        s.seed([m.nn - 1], 0.0, inst=i)
+    s.run()
+    s.reset()
+    for i in range(n_inst):
+        phi, st = s.download(inst=i)
+        assert (phi == far).all() and (st == 0).all()
+    got, again = run(s)
+    assert again == acts and all(np.array_equal(a, b) for a, b in zip(got, want))
+    s.close()
+    c = F.Solver(p, mode=F.MODE_COMPAT)
+    steps = []
+    for _ in range(2):
+        c.seed([0], 0.0)
+        steps.append([c.step(0.0, 2000.0, 2000.0, 1e6), *c.download()])
+        c.reset()
+        phi, st = c.download()
+        assert (phi == far).all() and (st == 0).all()
+    assert steps[0][0] == steps[1][0] and all(np.array_equal(a, b) for a, b in zip(steps[0][1:], steps[1][1:]))
+    c.close()
