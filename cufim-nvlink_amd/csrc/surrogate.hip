@@ -802,10 +802,13 @@ __device__ inline void put_bf16(uint32_t i, float w, uint16_t *wb, uint16_t *wbt
   }
 }
 
-// gradient and loss sum (element NPAR)
-__global__ __launch_bounds__(256) void k_reduce_parts(const float *P, uint32_t S, float *g) {
+// gradient and loss sum (element NPAR, which also goes to *loss)
+__global__ __launch_bounds__(256) void k_reduce_parts(const float *P, uint32_t S, float *g, float *loss) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i <= NPAR) g[i] = sum_parts(P, S, i);
+  if (i > NPAR) return;
+  const float v = sum_parts(P, S, i);
+  g[i] = v;
+  if (i == NPAR) *loss = v;
 }
 
 // Adam on the FP32 masters with the sum of S partial gradients; BF16 copies of
@@ -1244,7 +1247,8 @@ int fim_nn_gradient(fim_nn *n, const float *x, const float *t, int32_t b, double
     const size_t at = upload(n, n->xin, x, (size_t)b * NIN * sizeof(float), 0);
     (void)upload(n, n->tgt, ts.data(), (size_t)b * sizeof(float), at);
     const uint32_t S = train_pass(n, n->xin, 0, (uint32_t)b);
-    k_reduce_parts<<<NPAR / 256 + 1, 256, 0, n->stream>>>(n->parts, S, reinterpret_cast<float *>(n->stage_d));
+    k_reduce_parts<<<NPAR / 256 + 1, 256, 0, n->stream>>>(n->parts, S, reinterpret_cast<float *>(n->stage_d),
+                                                          n->g + NPAR);  // the last loss, as a step leaves it
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(n->stream));
     const float *g = reinterpret_cast<const float *>(n->stage);
