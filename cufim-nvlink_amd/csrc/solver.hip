@@ -908,9 +908,11 @@ __device__ inline void wave_append(bool pred, uint32_t l, uint16_t *list, uint32
 // are used instead of spilled; with WPE <= 4 a wave works on two rounds of
 // pairs side by side (ILP).
 //
-// What bounds it is latency: with 8 waves per SIMD the vector units issue 41-50 %
-// of the time and waves wait 65-70 % of theirs (L2 misses of records and
-// times, LDS round trips, barriers).  Cycles per item of the 2M slab (256 x 2
+// What bounds it: at 512 instances a launch, vector issue (73 % of one wave
+// instruction per SIMD and 4 cycles, 5.2e8 instructions in 1,172 us, 10.6 per
+// candidate), while waves wait 61 % of their cycles; with 128 instances, or a
+// single one, those waits (65-70 %: L2 misses of records and times, LDS round
+// trips, barriers), vector issue being 41-50 %.  Cycles per item of the 2M slab (256 x 2
 // instances, 2816 copies; a single solve, 1024 copies): staging 24k / 6.9k,
 // mark 13k / 7k, list and evaluate 79k / 27k, accept 17k / 5k, write-back 6k /
 // 3k, push 3k / 2.5k, next item 6k / 2.6k; 155k / 63k in all before the lists
