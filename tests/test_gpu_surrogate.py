@@ -265,6 +265,21 @@ def test_training_and_warm_start_reach_the_cold_fixed_point(small_slab):
     nn.close()
 
 
+@pytest.mark.parametrize("count", [19500, 19700])
+def test_predicted_maxima_of_many_solves(small_slab, count):
+    """as many solves as the staging holds at once (1.33 MB, 68 bytes each),
+    and more: the same rows, so the same bits as in a small call"""
+    cfg, m = small_slab
+    nn = F.Surrogate(m, seed=3)
+    nn.set_params(M.init_params(11))
+    solves = _draw(cfg, 50, 5)
+    sample = np.array([1, 7, m.nn - 1], dtype=np.int64)
+    want = nn.predict_max(solves, sample)
+    got = nn.predict_max((solves * (count // 50 + 1))[:count], sample)
+    assert np.array_equal(got, np.resize(want, count))
+    nn.close()
+
+
 @pytest.mark.parametrize("max_batch", [0, 64])
 def test_predicted_maximum_equals_the_map_maximum(small_slab, max_batch):
     """fim_nn_predict_max over a vertex sample equals the largest value of
