@@ -109,6 +109,10 @@ constexpr uint32_t kIterWord = 10;
 // needs no clearing; kPushed outranks kQueued.
 constexpr uint32_t kQueued = 1, kPushed = 2;
 __device__ inline uint32_t act_tag(uint32_t iter) { return 4u * (iter + 1u); }
+// Iterations have numbers below this: the last one queues items for the
+// iteration after it, and those flags still fit 32 bits.  A context that runs
+// on without a reset is renumbered before (k_conv_renumber).
+constexpr uint32_t kIterEnd = (1u << 30) - 2u;
 
 // Where items are queued: a list and its iteration's queue flags.
 struct Queue {
@@ -1497,6 +1501,25 @@ __global__ __launch_bounds__(256) void k_inst_active(Queue q, uint32_t *out) {
   if (threadIdx.x == 0) out[blockIdx.x] = any;
 }
 
+// Gives the next iteration the number `to` (to + 1 if its parity differs: inbox,
+// wake times and flags exist by parity), between runs.  What is queued
+// for it stays queued, for the same reason; flags of earlier iterations are
+// cleared; the instances' windows go on from where they are.
+__device__ inline uint32_t renumbered(uint32_t now, uint32_t to) { return to + ((now ^ to) & 1u); }
+__global__ __launch_bounds__(256) void k_conv_renumber(const uint32_t *iter, uint32_t to, uint32_t *act, size_t nss,
+                                                       uint32_t *start, uint32_t ninst) {
+  const uint32_t now = *iter, next = renumbered(now, to), tag = act_tag(now);
+  uint32_t *cur = act + (now & 1u) * nss, *other = act + (~now & 1u) * nss;
+  const size_t first = blockIdx.x * (size_t)256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+  for (size_t i = first; i < nss; i += step) {
+    const uint32_t f = cur[i];
+    cur[i] = f >= tag ? act_tag(next) + (f & 3u) : 0u;
+    other[i] = 0u;
+  }
+  for (size_t i = first; i < ninst; i += step) start[i] += next - now;
+}
+__global__ void k_iter_set(uint32_t *iter, uint32_t to) { *iter = renumbered(*iter, to); }
+
 // recycles finished instances: times to +inf, flags and wake times cleared,
 // and the instance's window restarts at the current iteration
 __global__ void k_inst_reset(const uint32_t *insts, uint32_t n, float *phi, uint8_t *dirty, float *wake,
@@ -2410,6 +2433,7 @@ struct fim_ctx {
   uint32_t *d_ifc = nullptr;    // per interface entry: its copy
   bool inbox_left = false;      // the last run stopped with pushes in the inbox
   bool direct_plan = false;     // a bucket is one work unit
+  uint32_t next_iter = 0;       // the next iteration's number, or one more
   uint2 *d_ifm = nullptr;
   uint32_t wps = 1;
   WorkList wl[3] = {};
@@ -2567,6 +2591,17 @@ void settle(fim_ctx *c) {
   k_conv_drain<<<dim3(std::min(blocks_for(c->n_if, 256), 256), std::min<uint32_t>(c->ninst, 1024u)), 256, 0,
                  c->stream>>>(a);
   HIPCHECK(hipGetLastError());
+}
+
+// continues the numbering of the iterations at `to`, or to + 1
+void renumber(fim_ctx *c, uint32_t to) {
+  const size_t nss = (size_t)c->ninst * c->nsub;
+  uint32_t *iter = c->wl[0].cnt + kIterWord;
+  k_conv_renumber<<<std::min(blocks_for(std::max<size_t>(nss, c->ninst), 256), 2048), 256, 0, c->stream>>>(
+      iter, to, c->d_act, nss, c->d_start, c->ninst);
+  k_iter_set<<<1, 1, 0, c->stream>>>(iter, to);
+  HIPCHECK(hipGetLastError());
+  c->next_iter = to + 1u;
 }
 
 void check_inst(const fim_ctx *c, int32_t inst) {
@@ -3113,6 +3148,7 @@ int fim_reset(fim_ctx *c) {
       f.add(c->d_wpush, 2 * nss, F_INF);
       f.add(c->d_cnt, 48, 0u);
       f.add(c->d_start, c->ninst, 0u);
+      c->next_iter = 0;
       for (int k = 0; k < 3; ++k) f.add(c->wl[k].bcnt, c->nsub, 0u);
     } else {
       f.add(c->d_phi64, c->ncopy, DBL_MAX);
@@ -3305,6 +3341,8 @@ void run_begin(fim_ctx *c, int32_t max_iters, bool reset_stats, RunState &r) {
 // chunk's completion event
 void run_chunk(fim_ctx *c, RunState &r) {
   HIPCHECK(hipSetDevice(c->dev));
+  if (c->next_iter + (uint32_t)c->graph_iters > kIterEnd) renumber(c, 0u);
+  c->next_iter += (uint32_t)c->graph_iters;
   if (c->o.profile || c->direct) {
     for (int i = 0; i < c->graph_iters; ++i) enqueue_iteration(c, i, c->o.profile != 0);
   } else {
@@ -3439,6 +3477,15 @@ int fim_run_multi(fim_ctx *const *cs, int32_t n, int32_t max_iters, int32_t *ite
       capped = capped || rs[i].left != 0;
     }
     if (capped) throw Error(FIM_ENOCONV, "iteration cap reached before convergence");
+  });
+}
+
+int fim_ctx_renumber(fim_ctx *c, uint32_t n) {
+  return guarded([&] {
+    if (!c || c->o.mode != FIM_MODE_CONVERGE || n >= kIterEnd) throw Error(FIM_EINVAL, "bad renumbering");
+    HIPCHECK(hipSetDevice(c->dev));
+    renumber(c, n);
+    HIPCHECK(hipStreamSynchronize(c->stream));
   });
 }
 

@@ -749,3 +749,47 @@ def test_reset_leaves_nothing(n, n_inst):
         assert (phi == far).all() and (st == 0).all()
     assert steps[0][0] == steps[1][0] and all(np.array_equal(a, b) for a, b in zip(steps[0][1:], steps[1][1:]))
     c.close()
+
+
+ITER_END = 2 ** 30 - 2  # iteration numbers stay below (csrc/solver.hip, kIterEnd)
+
+
+@pytest.mark.parametrize("n_inst,unit", [(1, 0), (5, 2)])
+@pytest.mark.parametrize("before", [4, 5, 10, 31])
+def test_iteration_numbers_start_over(n_inst, unit, before):
+    """a context whose iteration numbers run out `before` iterations later (it
+    has never been reset): runs with work queued and pushes on their way, a
+    recycled instance and later runs give bitwise the maps and activations of
+    a context that counts from 0"""
+    cfg = cases.scaled(cases.SLAB, 8)
+    m, _ = cases.box(cfg, seed=9)
+    p = F.Pack(m, F.PART_RCB, max_nn=200, seed=9)
+    srcs = [cases.pacing_sites(cfg, 1 + k % 3, seed=500 + k) for k in range(n_inst)]
+
+    def solves(number):
+        s = F.Solver(p, n_instances=n_inst, window=500.0, unit=unit, graph_iters=3)
+        if number is not None:
+            assert F.lib().fim_ctx_renumber(s.h, number) == 0
+        out, counts = [], []
+        s.seed_batch(srcs, 0.0)
+        for k in range(1000):
+            if s.advance(3, reset_stats=k == 0) == 0:
+                break
+        out += [s.download(inst=i)[0] for i in range(n_inst)]
+        counts.append(s.stats()["activations"])
+        assert not np.any(s.active())
+        for beat in range(2):
+            s.recycle([0])
+            s.seed(srcs[0][:1], 0.0)
+            s.run()
+            out.append(s.download()[0])
+            counts.append(s.stats()["activations"])
+        s.close()
+        return out, counts
+
+    want, n = solves(None)
+    got, k = solves(ITER_END - before)
+    for a, b in zip(want, got):
+        assert np.all(b < 1e30)
+        assert np.array_equal(a, b)
+    assert n == k
