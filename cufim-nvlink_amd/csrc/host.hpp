@@ -164,7 +164,8 @@ void ctx_init_field(fim_ctx *c, int32_t inst, bool all_active);
 }  // namespace fim
 
 // for tests of long runs, not part of cufim.h: the context's next iteration
-// gets the number n, or n + 1
+// gets the number n, or n + 1; in compat mode its next window, higher than
+// the last one's
 extern "C" int fim_ctx_renumber(fim_ctx *c, uint32_t n);
 
 struct fim_mesh {

@@ -2443,15 +2443,15 @@ struct fim_ctx {
   double *d_phi64 = nullptr;
   int8_t *d_st = nullptr;
   double *d_nexte = nullptr;  // per submesh: earliest window time a copy changes
-  // submesh lists of this and the last window (by parity), their counts
-  // (three in rotation), the stamps of the last window that listed a submesh,
-  // the pass's end counter and its records of changed shared vertices
+  // submesh lists of this and the last window (two in turn), their counts
+  // (three in turn), the stamps of the last window that listed a submesh (0:
+  // none), the pass's end counter and its records of changed shared vertices
   uint32_t *d_list = nullptr, *d_lcnt = nullptr, *d_mark = nullptr;
   CompatSub *d_csub = nullptr;
   uint4 *d_blob = nullptr;
   uint32_t *d_cshared = nullptr, *d_vrec = nullptr, *d_vcnt = nullptr;
   unsigned long long *d_done = nullptr;
-  uint32_t stamp = 0;
+  uint32_t stamp = 0, turn = 0;  // of the last window
   bool compat_small = false, compat_geo = false;  // k_compat_small, with geometry in LDS
   // shared
   unsigned long long *d_stats = nullptr;
@@ -3277,17 +3277,21 @@ int fim_step(fim_ctx *c, double phi_start, double cur_time, double dt, double fr
     if (c->o.mode != FIM_MODE_COMPAT) throw Error(FIM_ESTATE, "fim_step needs compat mode");
     HIPCHECK(hipSetDevice(c->dev));
     HIPCHECK(hipEventRecord(c->ev0, c->stream));
-    const uint32_t stamp = ++c->stamp;
-    uint32_t *list = c->d_list + (stamp & 1u) * (size_t)c->nsub, *last = c->d_list + ((stamp & 1u) ^ 1u) * (size_t)c->nsub;
-    const CompatSyncArgs sy{c->d_sub, last, c->d_lcnt + (stamp + 2) % 3, c->d_vrec, c->d_vcnt, c->d_g2c_dsp, c->d_g2c,
+    if (++c->stamp == 0u) {  // after 2^32 - 1 windows the stamps start over
+      k_fill<uint32_t><<<blocks_for(c->nsub, 256), 256, 0, c->stream>>>(c->d_mark, c->nsub, 0u);
+      c->stamp = 1u;
+    }
+    const uint32_t turn = c->turn = (c->turn + 1u) % 6u;
+    uint32_t *list = c->d_list + (turn & 1u) * (size_t)c->nsub, *last = c->d_list + ((turn & 1u) ^ 1u) * (size_t)c->nsub;
+    const CompatSyncArgs sy{c->d_sub, last, c->d_lcnt + (turn + 2) % 3, c->d_vrec, c->d_vcnt, c->d_g2c_dsp, c->d_g2c,
                             c->d_c2s, c->d_phi64, c->d_st, c->d_nexte, c->nsub, cur_time, list,
-                            c->d_lcnt + stamp % 3, c->d_lcnt + (stamp + 1) % 3, c->d_mark, stamp};
+                            c->d_lcnt + turn % 3, c->d_lcnt + (turn + 1) % 3, c->d_mark, c->stamp};
     // a wave for every submesh the last window can have listed, up to 8 waves per SIMD
     k_compat_sync<<<std::min<int>(blocks_for((size_t)c->nsub * 64, 256), 2048), 256, 0, c->stream>>>(sy);
     HIPCHECK(hipGetLastError());
     CompatArgs a = c->xa;
     a.list = list;
-    a.nlist = c->d_lcnt + stamp % 3;
+    a.nlist = c->d_lcnt + turn % 3;
     a.fw = front_width;
     a.cur = cur_time;
     a.phi_start = phi_start;
@@ -3482,9 +3486,10 @@ int fim_run_multi(fim_ctx *const *cs, int32_t n, int32_t max_iters, int32_t *ite
 
 int fim_ctx_renumber(fim_ctx *c, uint32_t n) {
   return guarded([&] {
-    if (!c || c->o.mode != FIM_MODE_CONVERGE || n >= kIterEnd) throw Error(FIM_EINVAL, "bad renumbering");
+    if (!c || (c->o.mode == FIM_MODE_CONVERGE && n >= kIterEnd)) throw Error(FIM_EINVAL, "bad renumbering");
     HIPCHECK(hipSetDevice(c->dev));
-    renumber(c, n);
+    if (c->o.mode == FIM_MODE_CONVERGE) renumber(c, n);
+    else c->stamp = n - 1u;
     HIPCHECK(hipStreamSynchronize(c->stream));
   });
 }

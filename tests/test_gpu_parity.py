@@ -8,6 +8,8 @@ Tolerances
     against the FP64 fixed point of the oracle, the per-config bound the
     solver is specified to.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -793,3 +795,32 @@ def test_iteration_numbers_start_over(n_inst, unit, before):
         assert np.all(b < 1e30)
         assert np.array_equal(a, b)
     assert n == k
+
+
+@pytest.mark.parametrize("max_nn", [128, 700])
+@pytest.mark.parametrize("before", [1, 2, 3, 7, 12])
+def test_window_numbers_start_over(max_nn, before):
+    """a context that has worked through 2^32 windows but `before`, in the
+    middle of a map (submeshes listed, shared vertices to be merged): bitwise
+    the times and states, and the pending copies after every window, of a
+    context that counts from 0"""
+    cfg = dict(cases.SLAB, nx=17, ny=13, nz=5, lx=17e3, ly=13e3, lz=5e3)
+    m, _ = cases.box(cfg, seed=5)
+    p = F.Pack(m, F.PART_RCB, max_nn=max_nn, seed=3)
+    fw, dt = m.front_width(), 2e3
+
+    def windows(number):
+        s = F.Solver(p, mode=F.MODE_COMPAT, local=F.LOCAL_REF, apd=20e3)
+        s.seed([0, 700], 0.0)
+        left = [s.step(0.0, dt, dt, fw)]
+        if number is not None:
+            assert F.lib().fim_ctx_renumber(s.h, C.c_uint32(number)) == 0
+        left += [s.step(k * dt, (k + 1) * dt, dt, fw) for k in range(1, 20)]
+        phi, st = s.download()
+        s.close()
+        return phi, st, left
+
+    want, got = windows(None), windows(2 ** 32 - before)
+    assert max(want[2][8:]) > 0
+    assert want[2] == got[2]
+    assert np.array_equal(want[0], got[0]) and np.array_equal(want[1], got[1])
