@@ -3101,8 +3101,6 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->d_vrec = dalloc<uint32_t>(p.if_l.size(), ow);
         c->d_vcnt = dalloc<uint32_t>(c->nsub, ow);
         c->d_done = dalloc<unsigned long long>(1, ow);
-        HIPCHECK(hipMemset(c->d_mark, 0, sizeof(uint32_t) * c->nsub));
-        HIPCHECK(hipMemset(c->d_done, 0, sizeof(unsigned long long)));
         HIPCHECK(hipFuncSetAttribute(compat_kernel_ptr(c), hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)c->lds_compat));
         int ncu = 256, per_cu = 0;
@@ -3155,6 +3153,9 @@ int fim_reset(fim_ctx *c) {
       f.add(c->d_st, c->ncopy, (int8_t)FIM_FAR);
       f.add(c->d_nexte, c->nsub, (double)INFINITY);
       f.add(c->d_lcnt, 3, 0u);
+      f.add(c->d_mark, c->nsub, 0u);
+      f.add(c->d_done, 1, 0ull);
+      c->stamp = 0u;
     }
     k_fill_all<<<blocks_for(f.seg[0].bytes / 16 + 1, 256), 256, 0, c->stream>>>(f);
     HIPCHECK(hipGetLastError());
