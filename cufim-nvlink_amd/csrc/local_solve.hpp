@@ -152,9 +152,10 @@ FIM_HD inline T cand_exact(const T g[6], const T ph[4], T inf) {
 // sum l_i x_i| (l_i >= 0, sum 1) is at least min_i (p_i + n . u_i).  n points
 // here from the centroid of the opposite face to the target.  b[3 T + j] is
 // the product for node T + 1 + j (mod 4) as a byte, (byte - 128) * scale, rounded
-// down after a margin of 1e-4 |u_i| that lies far above the rounding of the
-// products and of the FP32 candidates.  A face whose centroid (almost) meets
-// the target gives no direction: -|u_i|.
+// down after a margin of 1e-4 |u_i| for the rounding of lengths (of the
+// products, and of the FP32 candidates' terms in them); what grows with the
+// times is allowed for where the times are added (cand_bounds32).  A face
+// whose centroid (almost) meets the target gives no direction: -|u_i|.
 inline void cand_bounds(const double geo[6], uint8_t b[12], float *scale) {
   double hi = 0.0, v[12], top = 0.0;
   for (int k = 0; k < 6; ++k) hi = std::fmax(hi, geo[k]);
@@ -178,6 +179,29 @@ inline void cand_bounds(const double geo[6], uint8_t b[12], float *scale) {
   for (int a = 0; a < 12; ++a) {
     const double x = *scale > 0.0f ? std::floor(v[a] / *scale) + 128.0 : 0.0;
     b[a] = (uint8_t)std::fmin(255.0, std::fmax(0.0, x));
+  }
+}
+
+// The bounds of an element's four targets at node times ph, from the bytes of
+// cand_bounds (word k / 4, byte k % 4 is b[k]) and the scale sc.  Two FP32
+// additions here and up to three in a candidate round by half an ulp of the
+// time each, so each time counts as 2^-21 of itself less (four to eight ulp):
+// beyond 800 edge lengths an ulp of the time is more than the bytes' margin,
+// and a candidate an ulp lower than its target would be lost.
+FIM_HD inline void cand_bounds32(const uint32_t w[3], float sc, const float ph[4], float v[4]) {
+  const float zero = -128.0f * sc;
+  float p[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) p[k] = std::fmaf(ph[k], 1.0f - 0x1p-21f, zero);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    float x[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int k = 3 * t + j;
+      x[j] = std::fmaf((float)((w[k >> 2] >> (8 * (k & 3))) & 0xffu), sc, p[(t + 1 + j) & 3]);
+    }
+    v[t] = std::fmin(x[0], std::fmin(x[1], x[2]));
   }
 }
 

@@ -808,22 +808,12 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
 // a table, take 100 instructions and 30 more registers (28 % slower).
 __device__ inline uint32_t live_targets(const uint4 b, float hs, const float ph[4], const int f[4]) {
   const uint32_t w[3] = {b.x, b.y, b.z};
-  const float sc = __uint_as_float(b.w) * hs;
+  float v[4];
+  cand_bounds32(w, __uint_as_float(b.w) * hs, ph, v);
   const int nf = f[0] + f[1] + f[2] + f[3];
-  float p[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) p[k] = fmaf(-128.0f, sc, ph[k]);
   uint32_t tm = 0;
 #pragma unroll
-  for (int T = 0; T < 4; ++T) {
-    float v[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int k = 3 * T + j;
-      v[j] = fmaf((float)((w[k >> 2] >> (8 * (k & 3))) & 0xffu), sc, p[(T + 1 + j) & 3]);
-    }
-    tm |= (nf - f[T] > 0 && ph[T] > fminf(v[0], fminf(v[1], v[2]))) ? 1u << T : 0u;
-  }
+  for (int T = 0; T < 4; ++T) tm |= (nf - f[T] > 0 && ph[T] > v[T]) ? 1u << T : 0u;
   return tm;
 }
 // (element, target) pair ring of one wave in the band kernel: pairs left from

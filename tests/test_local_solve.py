@@ -210,3 +210,77 @@ def test_candidate_bounds_lie_below_every_candidate(shim):
             assert bound <= c, (k, t, bound, c, g, ph)
             tight += bound > min(ph[o]) + 0.3 * (c - min(ph[o]))
     assert tight > 4000  # they do bound: most lie well above the earliest node
+
+
+SHIM_LATE = r"""
+#include "local_solve.hpp"
+// smallest difference FP32 candidate - FP32 bound, and the number of
+// (element, target) pairs whose candidate lies below its bound
+extern "C" int ls_late(int n, const double *g, const float *ph, float *least) {
+  int bad = 0;
+  *least = 3e38f;
+  for (int i = 0; i < n; ++i) {
+    unsigned char b[12];
+    float scale, g32[6], sq[6], rc[6], v[4];
+    fim::cand_bounds(g + 6 * i, b, &scale);
+    uint32_t w[3] = {0, 0, 0};
+    for (int k = 0; k < 12; ++k) w[k / 4] |= (uint32_t)b[k] << 8 * (k % 4);
+    for (int k = 0; k < 6; ++k) {
+      g32[k] = (float)g[6 * i + k];
+      sq[k] = fim::csqrt(g32[k]);
+      rc[k] = 1.0f / g32[k];
+    }
+    const float *p = ph + 4 * i, inf = 3.0e38f;
+    fim::cand_bounds32(w, scale, p, v);
+    const float c[8] = {fim::cand_exact<0, float>(g32, p, inf), fim::cand_exact<1, float>(g32, p, inf),
+                        fim::cand_exact<2, float>(g32, p, inf), fim::cand_exact<3, float>(g32, p, inf),
+                        fim::cand_exact_sh<0, float>(g32, sq, rc, p, inf), fim::cand_exact_sh<1, float>(g32, sq, rc, p, inf),
+                        fim::cand_exact_sh<2, float>(g32, sq, rc, p, inf), fim::cand_exact_sh<3, float>(g32, sq, rc, p, inf)};
+    for (int k = 0; k < 8; ++k) {
+      if (!(v[k & 3] <= c[k])) ++bad;
+      if (c[k] - v[k & 3] < *least) *least = c[k] - v[k & 3];
+    }
+  }
+  return bad;
+}
+"""
+
+
+@pytest.mark.parametrize("edges", [0, 30, 1e3, 1e4, 1e6])
+def test_bounds_in_single_precision_lie_below_every_candidate_at_late_times(tmp_path, edges):
+    """the kernel's form of the bounds against the FP32 candidates, on
+    well-shaped elements under anisotropic metrics whose times lie `edges` edge
+    lengths after the start.  A candidate's additions round by at most 2.5 ulp
+    of its time together with the bound's, which has a margin of at least 4:
+    nothing is allowed for rounding."""
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    src = tmp_path / "late.cpp"
+    src.write_text(SHIM_LATE)
+    so = tmp_path / "late.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", f"-I{CSRC}",
+                    str(src), "-o", str(so)], check=True)
+    lib = C.CDLL(str(so))
+    lib.ls_late.argtypes = [C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_float), C.POINTER(C.c_float)]
+    rng = np.random.default_rng(int(edges) + 3)
+    n = 200000
+    base = np.array([[0.0, 0.0, 0.0], [1.0, 0.0, 0.0], [0.5, np.sqrt(3) / 2, 0.0],
+                     [0.5, np.sqrt(3) / 6, np.sqrt(2.0 / 3.0)]])
+    x = base + rng.uniform(-0.25, 0.25, (n, 4, 3))
+    f = rng.normal(size=(n, 3))
+    f /= np.linalg.norm(f, axis=1, keepdims=True)
+    slow = rng.uniform(1.0, 3.0, n)  # slowness along the fibre 1, across it up to 3
+    pairs = ((0, 1), (0, 2), (1, 2), (0, 3), (1, 3), (2, 3))
+    g = np.empty((n, 6))
+    for k, (a, b) in enumerate(pairs):
+        d = x[:, a] - x[:, b]
+        along = np.sum(d * f, axis=1)
+        g[:, k] = slow ** 2 * (np.sum(d * d, axis=1) - along ** 2) + along ** 2
+    g *= 600.0 ** 2
+    # times within a front's reach of each other, so that faces, triangles and
+    # edges all occur
+    ph = (600.0 * (edges + rng.uniform(0.0, 1.0, (n, 4)) * rng.choice([0.0, 0.1, 0.5, 1.5], (n, 1)))).astype(np.float32)
+    g = np.ascontiguousarray(g)
+    least = C.c_float()
+    bad = lib.ls_late(n, _ptr(g, C.c_double), _ptr(ph, C.c_float), C.byref(least))
+    assert bad == 0, (bad, least.value)
