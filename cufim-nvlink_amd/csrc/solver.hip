@@ -1343,7 +1343,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     // are pruning data of this kernel, not algorithmic bytes)
     uint32_t cnt = 0;
     for (uint32_t k = tid; k < new32; k += BS) cnt += __popc(eseen[k]);
-    cnt = wave_sum_small<9>(cnt);  // at most 8 words of 32 per thread
+    // up to 65,535 elements, so 2,048 / BS words of 32 per thread (8 with 256)
+    cnt = wave_sum_small<BS >= 256 ? 9 : BS == 128 ? 10 : 11>(cnt);
     if (lane == 0 && cnt) atomicAdd(&misc[3], cnt);
     if (lane == 0 && evals) atomicAdd(&misc[0], evals);
     // write back decreased copies and list the lowered interface copies

@@ -824,3 +824,19 @@ def test_window_numbers_start_over(max_nn, before):
     assert max(want[2][8:]) > 0
     assert want[2] == got[2]
     assert np.array_equal(want[0], got[0]) and np.array_equal(want[1], got[1])
+
+
+@pytest.mark.parametrize("block", [64, 128, 256, 512])
+def test_algorithmic_bytes_of_a_large_submesh(block):
+    """one submesh of 63,888 elements, all of them evaluated: 32 B each and
+    10 B a copy, whatever the workgroup's size (with 64 threads a lane adds up
+    to 1,024 of the evaluated elements' bits, with 128 up to 512)"""
+    m = F.Mesh.gen_box(seed=4, **dict(cases.CUBE, nx=22, ny=22, nz=22))
+    p = F.Pack(m, F.PART_RCB, max_nn=16000, max_ne=65535, seed=4)
+    assert p.info["nsub"] == 1 and p.info["ne_global"] == 63888
+    s = F.Solver(p, block=block)
+    s.seed([0], 0.0)
+    s.run()
+    st = s.stats()
+    s.close()
+    assert st["alg_bytes"] == st["activations"] * (32 * 63888 + 10 * p.info["nn_global"])
