@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <thread>
@@ -114,10 +115,6 @@ struct Pack {
   std::vector<float> hgt32;        // 4 per element: metric height of each node
                                    // above its opposite face, rounded down
   std::vector<double> geo64;       // 6 per element
-  std::vector<uint8_t> bnd8;       // 12 per element: for each node as target, lower bounds
-                                   // n . (x_target - x_i) of the other three nodes for a unit
-                                   // direction n, (byte - 128) * scale
-  std::vector<float> bnd_scale;    // 1 per element
   std::vector<uint8_t> ereg;       // 1 per element
   std::vector<uint32_t> c2g;       // per copy
   std::vector<uint32_t> c2s;       // per copy
@@ -138,6 +135,15 @@ struct Pack {
 };
 
 Pack build_pack(const Mesh &m, const Partition &p, int32_t source);
+
+// Candidate bounds of the elements (cand_bounds), for the band kernel's records
+struct ElementBounds {
+  std::vector<uint8_t> b;      // 12 per element: for each node as target, lower bounds
+                               // n . (x_target - x_i) of the other three nodes for a unit
+                               // direction n, (byte - 128) * scale
+  std::vector<float> scale;    // 1 per element
+};
+ElementBounds element_bounds(const Pack &k);
 
 // element-list entries the converge-mode band kernel keeps per pass (more
 // marked elements take further passes)
@@ -173,4 +179,8 @@ struct fim_mesh {
 };
 struct fim_pack {
   fim::Pack p;
+  // worked out for the first context that runs the band kernel (0.1 s for 2M
+  // elements), kept for those after it
+  mutable fim::ElementBounds bounds;
+  mutable std::once_flag bounds_once;
 };

@@ -201,12 +201,14 @@ int64_t converge_lds_bytes(int32_t nn_max, int32_t ne_max) {
          al(std::max<int64_t>(2 * nn64, ne_max < (1 << 14) ? 2560 : 0)) + 80 + 2 * al(4 * (nn64 / 32));
 }
 
-static void element_bounds(Pack &k) {
-  k.bnd8.resize(12 * (size_t)k.ne_global);
-  k.bnd_scale.resize((size_t)k.ne_global);
+ElementBounds element_bounds(const Pack &k) {
+  ElementBounds r;
+  r.b.resize(12 * (size_t)k.ne_global);
+  r.scale.resize((size_t)k.ne_global);
   parallel_ranges((size_t)k.ne_global, 4096, [&](size_t b, size_t e) {
-    for (size_t i = b; i < e; ++i) cand_bounds(&k.geo64[6 * i], &k.bnd8[12 * i], &k.bnd_scale[i]);
+    for (size_t i = b; i < e; ++i) cand_bounds(&k.geo64[6 * i], &r.b[12 * i], &r.scale[i]);
   });
+  return r;
 }
 
 Pack build_pack(const Mesh &m, const Partition &p, int32_t source) {
@@ -293,7 +295,6 @@ Pack build_pack(const Mesh &m, const Partition &p, int32_t source) {
     }
     for (int64_t l = 0; l < nn_s; ++l) g2l[p.l2g[p.s_vdsp[s] + l]] = -1;
   }
-  element_bounds(k);
   // global vertex -> copies, ascending submesh
   k.g2c_dsp.assign(m.nn + 1, 0);
   for (int64_t c = 0; c < k.ncopy; ++c) k.g2c_dsp[k.c2g[c] + 1]++;

@@ -793,7 +793,7 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
 //       and 1), nodes 2,3 (u16 each), geometry e12 e13 (f32)
 //   [1] geometry e23 e14 e24 e34 (f32)
 //   [2] candidate bounds: for the targets T = 0..3, n . (x_T - x_i) of the
-//       nodes i = T+1, T+2, T+3 (Pack::bnd8), their scale (f32)
+//       nodes i = T+1, T+2, T+3 (ElementBounds), their scale (f32)
 // Local copy ids are below 2^15, so the two region bits are free.
 
 // The targets with a source among the other nodes whose candidates can still
@@ -2864,6 +2864,8 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->d_n2e_le = dupload(p.n2e_le, ow);
         if (!o->staged) {
           if (c->nn_max > 32768) throw Error(FIM_ELIMIT, "submeshes above 32768 copies");
+          std::call_once(pk->bounds_once, [&] { pk->bounds = element_bounds(p); });
+          const ElementBounds &eb = pk->bounds;
           std::vector<uint4> rec(3 * (size_t)p.ne_global);
           parallel_ranges((size_t)p.ne_global, 65536, [&](size_t b, size_t end) {
             for (size_t e = b; e < end; ++e) {
@@ -2875,8 +2877,8 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
                                       (uint32_t)n[2] | ((uint32_t)n[3] << 16), fb(g[0]), fb(g[1]));
               rec[3 * e + 1] = make_uint4(fb(g[2]), fb(g[3]), fb(g[4]), fb(g[5]));
               uint32_t w[3];
-              std::memcpy(w, &p.bnd8[12 * e], 12);
-              rec[3 * e + 2] = make_uint4(w[0], w[1], w[2], fb(p.bnd_scale[e]));
+              std::memcpy(w, &eb.b[12 * e], 12);
+              rec[3 * e + 2] = make_uint4(w[0], w[1], w[2], fb(eb.scale[e]));
             }
           });
           c->d_erec = dupload(rec, ow);

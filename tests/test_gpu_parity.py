@@ -840,3 +840,28 @@ def test_algorithmic_bytes_of_a_large_submesh(block):
     st = s.stats()
     s.close()
     assert st["alg_bytes"] == st["activations"] * (32 * 63888 + 10 * p.info["nn_global"])
+
+
+def test_contexts_made_at_once_share_a_pack():
+    """the element bounds that contexts of a pack share are worked out by
+    the first of them: four threads making contexts of a fresh pack at once
+    get the maps of one made alone"""
+    import threading
+    cfg = cases.scaled(cases.SLAB, 8)
+    m, _ = cases.box(cfg, seed=9)
+    src = cases.pacing_sites(cfg, 2, seed=9)
+    want = _converge(m, F.Pack(m, F.PART_RCB, max_nn=300, seed=9), src)[0]
+    p = F.Pack(m, F.PART_RCB, max_nn=300, seed=9)
+    got, gate = [None] * 4, threading.Barrier(4)
+
+    def work(i):
+        gate.wait()
+        got[i] = _converge(m, p, src)[0]
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for g in got:
+        assert g is not None and np.array_equal(g, want)
