@@ -220,8 +220,6 @@ struct ConvArgs {
   uint32_t *old_cnt;     // counters of the list of the last iteration
   const uint32_t *start; // n_inst: iteration an instance was (re)seeded at; its
                          // window is window * (iter - start + 1)
-  const uint32_t *n2e_dsp;  // per copy: incident local elements (staged kernel)
-  const uint16_t *n2e_le;
   const uint4 *erec;        // band kernel: 48 B per element (below)
   const uint4 *adj;         // band kernel: per copy, four words of 8 incident local element ids
   const uint32_t *adj_ptr;  // copies of more than 32 elements: offset << 6 | words in adj_more
@@ -478,13 +476,10 @@ __device__ inline void push_lowered_scan(const Queue &nq, const SubInfo &si, uin
   }
 }
 
-// One workgroup per work item (instance, submesh).  STAGED copies the
-// submesh's elements (nodes + geometry) into LDS and finds the active
-// elements by scanning them every sweep; otherwise element data stays in
-// global memory (L2 / MALL resident) and the active elements are marked
-// from the flagged vertices through the vertex -> element adjacency, so an
-// activation costs in proportion to the band of the submesh it touches.
-template <int BS, bool STAGED>
+// The staged converge kernel (fim_opts.staged): one workgroup per work item
+// (instance, submesh) copies the submesh's elements (nodes + geometry) into
+// LDS and finds the active elements by scanning them every sweep.
+template <int BS>
 __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   float *phi_l = reinterpret_cast<float *>(lds);
@@ -492,12 +487,9 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
   uint32_t *flg = reinterpret_cast<uint32_t *>(lds + a.o_flg);
   uint32_t *tch = reinterpret_cast<uint32_t *>(lds + a.o_tch);
   uint32_t *dfr = reinterpret_cast<uint32_t *>(lds + a.o_dfr);
-  uint2 *el = reinterpret_cast<uint2 *>(lds + a.o_e2n);      // STAGED
-  float *gl = reinterpret_cast<float *>(lds + a.o_geo);       // STAGED
-  uint32_t *emark = reinterpret_cast<uint32_t *>(lds + a.o_e2n);  // !STAGED
-  uint32_t *eseen = reinterpret_cast<uint32_t *>(lds + a.o_geo);  // !STAGED
+  uint2 *el = reinterpret_cast<uint2 *>(lds + a.o_e2n);
+  float *gl = reinterpret_cast<float *>(lds + a.o_geo);
   uint16_t *elist = reinterpret_cast<uint16_t *>(lds + a.o_list);
-  uint16_t *vlist = reinterpret_cast<uint16_t *>(lds + a.o_vlist);  // !STAGED
   uint32_t *misc = reinterpret_cast<uint32_t *>(lds + a.o_misc);
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
@@ -515,7 +507,6 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
     const size_t cb = (size_t)inst * a.ncopy + si.coff;
     const uint32_t nn = si.nn, ne = si.ne;
     const uint32_t nv64 = (nn + 63u) & ~63u;
-    const uint32_t new32 = (ne + 31u) >> 5;
     // nothing in this submesh can act before the window reaches its wake
     // time: keep it queued without staging anything
     if (item.wake > W) {
@@ -554,97 +545,44 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
       }
     }
     const float *rs = a.rscale + 4 * (size_t)inst;
-    if (STAGED) {
-      // stage elements (geometry scaled by the instance's regional factor)
-      for (uint32_t e = tid; e < ne; e += BS) {
-        const size_t ge = (size_t)si.eoff + e;
-        el[e] = a.e2n[ge];
-        const float sc = rs[a.ereg[ge] & 3];
-        const float2 *g2 = reinterpret_cast<const float2 *>(a.geo + 6 * ge);
-        const float2 x0 = g2[0], x1 = g2[1], x2 = g2[2];
-        float *o = gl + 6 * e;
-        o[0] = x0.x * sc;
-        o[1] = x0.y * sc;
-        o[2] = x1.x * sc;
-        o[3] = x1.y * sc;
-        o[4] = x2.x * sc;
-        o[5] = x2.y * sc;
-      }
-    } else {
-      for (uint32_t k = tid; k < new32; k += BS) {
-        emark[k] = 0u;
-        eseen[k] = 0u;
-      }
+    // stage elements (geometry scaled by the instance's regional factor)
+    for (uint32_t e = tid; e < ne; e += BS) {
+      const size_t ge = (size_t)si.eoff + e;
+      el[e] = a.e2n[ge];
+      const float sc = rs[a.ereg[ge] & 3];
+      const float2 *g2 = reinterpret_cast<const float2 *>(a.geo + 6 * ge);
+      const float2 x0 = g2[0], x1 = g2[1], x2 = g2[2];
+      float *o = gl + 6 * e;
+      o[0] = x0.x * sc;
+      o[1] = x0.y * sc;
+      o[2] = x1.x * sc;
+      o[3] = x1.y * sc;
+      o[4] = x2.x * sc;
+      o[5] = x2.y * sc;
     }
     __syncthreads();
 
     int it = 0;
     bool capped = false;
     for (;;) {
-      if (tid == 0) {
-        misc[0] = 0u;
-        misc[2] = 0u;
+      if (tid == 0) misc[0] = 0u;
+      __syncthreads();
+      // active elements: any node flagged (wave ballot + per-wave base)
+      for (uint32_t e0 = 0; e0 < ne; e0 += BS) {
+        const uint32_t e = e0 + tid;
+        bool on = false;
+        if (e < ne) {
+          const uint2 q = el[e];
+          on = flag_at(flg, q.x & 0xffffu) || flag_at(flg, q.x >> 16) ||
+               flag_at(flg, q.y & 0xffffu) || flag_at(flg, q.y >> 16);
+        }
+        const uint64_t m = __ballot(on);
+        uint32_t base = 0;
+        if (lane == 0 && m) base = atomicAdd(&misc[0], (uint32_t)__popcll(m));
+        base = __shfl(base, 0);
+        if (on) elist[base + __popcll(m & lanes_below())] = (uint16_t)e;
       }
       __syncthreads();
-      if (STAGED) {
-        // active elements: any node flagged (wave ballot + per-wave base)
-        for (uint32_t e0 = 0; e0 < ne; e0 += BS) {
-          const uint32_t e = e0 + tid;
-          bool on = false;
-          if (e < ne) {
-            const uint2 q = el[e];
-            on = flag_at(flg, q.x & 0xffffu) || flag_at(flg, q.x >> 16) ||
-                 flag_at(flg, q.y & 0xffffu) || flag_at(flg, q.y >> 16);
-          }
-          const uint64_t m = __ballot(on);
-          uint32_t base = 0;
-          if (lane == 0 && m) base = atomicAdd(&misc[0], (uint32_t)__popcll(m));
-          base = __shfl(base, 0);
-          if (on) elist[base + __popcll(m & lanes_below())] = (uint16_t)e;
-        }
-        __syncthreads();
-      } else {
-        // flagged vertices -> compact list
-        for (uint32_t l0 = 0; l0 < nv64; l0 += BS) {
-          const uint32_t l = l0 + tid;
-          const bool on = l < nn && flag_at(flg, l);
-          const uint64_t m = __ballot(on);
-          uint32_t base = 0;
-          if (lane == 0 && m) base = atomicAdd(&misc[2], (uint32_t)__popcll(m));
-          base = __shfl(base, 0);
-          if (on) vlist[base + __popcll(m & lanes_below())] = (uint16_t)l;
-        }
-        __syncthreads();
-        const uint32_t nsrc = misc[2];
-        // mark the elements incident to them
-        for (uint32_t i = tid; i < nsrc; i += BS) {
-          const uint32_t c = si.coff + vlist[i];
-          const uint32_t kb = a.n2e_dsp[c], ke = a.n2e_dsp[c + 1];
-          for (uint32_t k = kb; k < ke; ++k) {
-            const uint32_t le = a.n2e_le[k];
-            atomicOr(&emark[le >> 5], 1u << (le & 31));
-          }
-        }
-        __syncthreads();
-        // marked elements -> compact list (and clear the marks)
-        for (uint32_t k0 = 0; k0 < new32; k0 += BS) {
-          const uint32_t k = k0 + tid;
-          uint32_t bits = 0;
-          if (k < new32) {
-            bits = emark[k];
-            emark[k] = 0u;
-            eseen[k] |= bits;
-          }
-          const uint32_t cnt = __popc(bits);
-          uint32_t base = cnt ? atomicAdd(&misc[0], cnt) : 0u;
-          while (bits) {
-            const uint32_t b = __ffs(bits) - 1;
-            bits &= bits - 1;
-            elist[base++] = (uint16_t)(k * 32 + b);
-          }
-        }
-        __syncthreads();
-      }
       const uint32_t nact = misc[0];
       if (nact == 0) break;
       if ((a.max_local > 0 && it >= a.max_local) || it >= kHardLocalCap) {
@@ -656,25 +594,10 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
       // candidates of the active elements
       for (uint32_t i = tid; i < nact; i += BS) {
         const uint32_t e = elist[i];
-        uint2 q;
+        const uint2 q = el[e];
         float g[6];
-        if (STAGED) {
-          q = el[e];
 #pragma unroll
-          for (int k = 0; k < 6; ++k) g[k] = gl[6 * e + k];
-        } else {
-          const size_t ge = (size_t)si.eoff + e;
-          q = a.e2n[ge];
-          const float sc = rs[a.ereg[ge] & 3];
-          const float2 *g2 = reinterpret_cast<const float2 *>(a.geo + 6 * ge);
-          const float2 x0 = g2[0], x1 = g2[1], x2 = g2[2];
-          g[0] = x0.x * sc;
-          g[1] = x0.y * sc;
-          g[2] = x1.x * sc;
-          g[3] = x1.y * sc;
-          g[4] = x2.x * sc;
-          g[5] = x2.y * sc;
-        }
+        for (int k = 0; k < 6; ++k) g[k] = gl[6 * e + k];
         const uint32_t nd[4] = {q.x & 0xffffu, q.x >> 16, q.y & 0xffffu, q.y >> 16};
         float ph[4];
         int f[4];
@@ -747,19 +670,8 @@ __global__ __launch_bounds__(BS) void k_conv_compute(ConvArgs a) {
     acts += it > 0;
     // algorithmic bytes of the activation: copies read and written (phi 4+4,
     // flag 1+1), interface entries (index 4, read 4, write 4) and the
-    // element data used (nodes 8 + geometry 24) -- all elements when staged,
-    // the distinct elements evaluated otherwise
-    uint32_t used = ne;
-    if (!STAGED) {
-      if (tid == 0) misc[3] = 0u;
-      __syncthreads();
-      uint32_t c = 0;
-      for (uint32_t k = tid; k < new32; k += BS) c += __popc(eseen[k]);
-      if (c) atomicAdd(&misc[3], c);
-      __syncthreads();
-      used = misc[3];
-    }
-    if (it > 0) abytes += 32ull * used + 10ull * nn + 12ull * si.ni;
+    // element data (nodes 8 + geometry 24)
+    if (it > 0) abytes += 32ull * ne + 10ull * nn + 12ull * si.ni;
     // write back decreased copies and push the lowered interface copies.
     // Deferred vertices (and sources left by the sweep cap) stay dirty and
     // the submesh is queued for the next iteration.
@@ -2474,14 +2386,14 @@ namespace {
 
 const void *conv_kernel_ptr(bool staged, int block, int wpe, bool pairs) {
   switch (block) {
-    case 64: return staged ? (const void *)k_conv_compute<64, true> : (const void *)k_conv_band<64, 8, false>;
-    case 128: return staged ? (const void *)k_conv_compute<128, true> : (const void *)k_conv_band<128, 8, false>;
+    case 64: return staged ? (const void *)k_conv_compute<64> : (const void *)k_conv_band<64, 8, false>;
+    case 128: return staged ? (const void *)k_conv_compute<128> : (const void *)k_conv_band<128, 8, false>;
     case 512:
-      if (staged) return (const void *)k_conv_compute<512, true>;
+      if (staged) return (const void *)k_conv_compute<512>;
       if (!pairs) return (const void *)k_conv_band<512, 8, false>;
       return wpe <= 4 ? (const void *)k_conv_band<512, 4, true> : (const void *)k_conv_band<512, 8, true>;
     default:
-      if (staged) return (const void *)k_conv_compute<256, true>;
+      if (staged) return (const void *)k_conv_compute<256>;
       if (pairs) {
         if (wpe <= 4) return (const void *)k_conv_band<256, 4, true>;
         if (wpe == 5) return (const void *)k_conv_band<256, 5, true>;
@@ -2860,8 +2772,6 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
             hg[e] = make_float4(p.hgt32[4 * e], p.hgt32[4 * e + 1], p.hgt32[4 * e + 2], p.hgt32[4 * e + 3]);
           c->d_hgt = dupload(hg, ow);
         }
-        c->d_n2e_dsp = dupload(p.n2e_dsp, ow);
-        c->d_n2e_le = dupload(p.n2e_le, ow);
         if (!o->staged) {
           if (c->nn_max > 32768) throw Error(FIM_ELIMIT, "submeshes above 32768 copies");
           std::call_once(pk->bounds_once, [&] { pk->bounds = element_bounds(p); });
@@ -2995,7 +2905,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->ca = ConvArgs{c->d_sub, c->d_e2n, c->d_geo32, c->d_hgt, c->d_ereg, c->d_rscale, c->d_phi,
                          c->d_dirty, c->d_act, c->d_wake, c->d_wpush, c->d_if_l, c->d_ifm, c->d_inbox, c->d_if_fo,
                          c->d_if_os, WorkList{}, WorkList{}, c->d_stats, nullptr, c->d_start,
-                         c->d_n2e_dsp, c->d_n2e_le, c->d_erec, c->d_adj, c->d_adj_ptr, c->d_adj_more,
+                         c->d_erec, c->d_adj, c->d_adj_ptr, c->d_adj_more,
                          c->nsub, c->ncopy, c->ninst, c->direct_plan ? 1u : 0u,
                          (float)(o->eps_rel > 0 ? o->eps_rel : 1e-6),
                          c->d_winst, o->local_iters, c->unit, c->maxch, (uint32_t)p.if_l.size(),
