@@ -199,7 +199,7 @@ struct ConvArgs {
   const SubInfo *sub;
   const uint2 *e2n;      // 4 x u16 local ids per element
   const float *geo;      // 6 per element
-  const float4 *hgt;     // per element: height of each node above its opposite face
+  const float4 *hgt;     // staged kernel, per element: height of each node above its opposite face
   const uint8_t *ereg;   // region per element
   const float *rscale;   // n_inst x 4 geometry multipliers (1/s^2)
   float *phi;            // n_inst x ncopy
@@ -2766,7 +2766,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
           throw Error(FIM_ELIMIT, "largest submesh needs " + std::to_string(c->lds_conv) +
                                       " B of LDS (limit 163840); use a smaller partition budget");
         c->d_geo32 = dupload(p.geo32, ow);
-        {
+        if (o->staged) {  // the band kernel's records have bounds of their own
           std::vector<float4> hg(p.ne_global);
           for (int64_t e = 0; e < p.ne_global; ++e)
             hg[e] = make_float4(p.hgt32[4 * e], p.hgt32[4 * e + 1], p.hgt32[4 * e + 2], p.hgt32[4 * e + 3]);

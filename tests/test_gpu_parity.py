@@ -865,3 +865,26 @@ def test_contexts_made_at_once_share_a_pack():
         t.join()
     for g in got:
         assert g is not None and np.array_equal(g, want)
+
+
+def test_device_memory_of_a_context_is_what_its_kernels_read():
+    """an unstaged context keeps 81 B an element (node ids 8, region 1,
+    geometry 24, record 48), 89 B a copy (ids 12, time 4, flag 1, adjacency 68,
+    vertex offsets at most 4), 60 B and twice 4 an interface copy: no heights,
+    which only the staged kernel reads.  8 MB for rounding and the rest, half
+    of what the heights of this mesh's 1.57 M elements take."""
+    def free():  # of the HIP runtime that the library is linked with
+        f, total = C.c_size_t(), C.c_size_t()
+        assert F.lib().hipMemGetInfo(C.byref(f), C.byref(total)) == 0
+        return f.value
+
+    m = F.Mesh.gen_box(seed=1, **dict(cases.CUBE, nx=64, ny=64, nz=64))
+    p = F.Pack(m, F.PART_RCB, max_nn=2816, seed=1)
+    F.Solver(p).close()  # what the first context of a process brings
+    before = free()
+    s = F.Solver(p)
+    used = before - free()
+    s.close()
+    i = p.info
+    need = 81 * i["ne_global"] + 89 * i["ncopy"] + 68 * i["n_iface_copies"]
+    assert used <= need + (8 << 20), (used, need)
