@@ -145,12 +145,29 @@ struct ElementBounds {
 };
 ElementBounds element_bounds(const Pack &k);
 
-// element-list entries the converge-mode band kernel keeps per pass (more
-// marked elements take further passes)
-constexpr int32_t kElistCap = 2032;
+// element-list entries the converge-mode band kernel keeps per pass at least
+// (more marked elements take further passes)
+constexpr uint32_t kElistCap = 2032;
+// (element, target) pair ring of one wave in the band kernel: pairs left from
+// earlier rounds of 64 ilp plus 4 targets of 64 elements
+constexpr uint32_t pair_ring(int ilp) { return 64u * (uint32_t)ilp + 256u; }
+// the band kernel evaluates pairs with workgroups of 256 and 512, where local
+// element ids fit 14 bits
+inline bool band_with_pairs(int block, int32_t ne_max) {
+  return (block == 256 || block == 512) && ne_max < (1 << 14);
+}
+// A list of at most one unit per submesh leaves the CUs with a few waves each
+// when the mesh has few submeshes: the band kernel gets registers for two pair
+// rounds side by side then
+inline bool few_submeshes(int64_t nsub, int cus) { return nsub <= 4 * (int64_t)cus; }
 
-// dynamic LDS bytes the converge-mode kernel needs for the largest submesh
-int64_t converge_lds_bytes(int32_t nn_max, int32_t ne_max);
+// Dynamic LDS of the converge-mode kernels for the largest submesh: byte
+// offsets, the entries of the element list, all bytes.
+struct ConvergeCarve {
+  uint32_t o_phin, o_flg, o_tch, o_dfr, o_e2n, o_geo, o_list, o_vlist, o_misc, o_wrt, o_ifc, elcap, bytes;
+};
+// ilp: pair rounds side by side, 0 without pairs
+ConvergeCarve converge_carve(int32_t nn_max, int32_t ne_max, int block, bool staged, int ilp);
 
 // solver-context hooks for the surrogate (csrc/surrogate.hip); device
 // pointers, work queued on the context's stream

@@ -263,7 +263,8 @@ int fim_pack_info(const fim_pack *p, fim_pack_info_t *info) {
     info->nn_max = k.nn_max;
     info->ne_max = k.ne_max;
     info->device_bytes_mesh = 32 * k.ne_global + 4 * k.ncopy;
-    info->lds_bytes = converge_lds_bytes(k.nn_max, k.ne_max);
+    const int ilp = !band_with_pairs(512, k.ne_max) ? 0 : few_submeshes(k.nsub, 256) ? 2 : 1;
+    info->lds_bytes = converge_carve(k.nn_max, k.ne_max, 512, false, ilp).bytes;
   });
 }
 

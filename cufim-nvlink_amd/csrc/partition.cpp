@@ -186,19 +186,44 @@ Partition partition_rcb(const Mesh &m, int max_nn, int max_ne, uint64_t seed) {
   return p;
 }
 
-int64_t converge_lds_bytes(int32_t nn_max, int32_t ne_max) {
-  // same carve as the default converge-mode kernel: vertex times and
-  // candidate minima (2 x f32 per vertex, rounded to 64), four vertex
-  // bitmasks, two element bitmasks, element list (u16), source list (u16),
-  // 8 counters, 4 region factors, 4 launch counters, interface-copy bits and entry counts
-  auto al = [](int64_t x) { return (x + 15) & ~int64_t(15); };
-  const int64_t nn64 = (nn_max + 63) & ~int64_t(63);
-  const int64_t ne32 = (ne_max + 31) / 32;
-  // (the source list doubles as the (element, target) pair rings of the
-  // four waves of a workgroup of 256: at least 4 x 320 u16)
-  return 2 * al(4 * nn64) + 4 * al(4 * (nn64 / 32)) + 2 * al(4 * ne32) +
-         al(2LL * std::min<int64_t>(ne_max, kElistCap)) +
-         al(std::max<int64_t>(2 * nn64, ne_max < (1 << 14) ? 2560 : 0)) + 80 + 2 * al(4 * (nn64 / 32));
+ConvergeCarve converge_carve(int32_t nn_max, int32_t ne_max, int block, bool staged, int ilp) {
+  auto al = [](uint32_t x) { return (x + 15u) & ~15u; };
+  const uint32_t nn64 = ((uint32_t)nn_max + 63u) & ~63u, ne = (uint32_t)ne_max, ne32 = (ne + 31u) / 32u;
+  const uint32_t vbits = al(4 * (nn64 / 32)), nw = (uint32_t)block / 64u;
+  ConvergeCarve c{};
+  // times and candidate minima at 0 and o_phin, then three vertex bitmasks
+  c.o_phin = al(4 * nn64);
+  c.o_flg = 2 * c.o_phin;
+  c.o_tch = c.o_flg + vbits;
+  c.o_dfr = c.o_tch + vbits;
+  c.o_e2n = c.o_dfr + vbits;
+  // staged: element nodes and geometry; unstaged: element bitmasks
+  c.o_geo = c.o_e2n + (staged ? al(8 * ne) : al(4 * ne32));
+  c.o_list = c.o_geo + (staged ? al(24 * ne) : al(4 * ne32));
+  if (staged) {
+    c.elcap = ne;
+    c.o_vlist = c.o_misc = c.o_list + al(2 * ne);
+    c.o_wrt = c.o_ifc = c.bytes = c.o_misc + 48u;  // 8 words, 4 region factors
+    return c;
+  }
+  // the source list doubles as the waves' pair rings; 8 counters and flags, 4
+  // region factors, 4 launch counters; a vertex bitmask, interface-copy bits
+  // and entry counts
+  const uint32_t vlist = al(std::max(2 * nn64, ilp ? nw * 2u * pair_ring(ilp) : 0u)), misc = 80u;
+  // The band kernel lists at most elcap elements per pass, an equal share per
+  // wave: all elements of a wave's words where they fit, else at least
+  // kElistCap, more if the LDS left over by the workgroups the wave slots admit
+  // (8 waves per SIMD) holds more
+  const uint32_t budget = (160u * 1024u / std::max(1u, 32u / nw)) & ~15u;
+  const uint32_t base = c.o_list + vlist + misc + 3u * vbits;
+  const uint32_t room = budget > base ? ((budget - base) / 2u) & ~7u : 0u;
+  c.elcap = std::min(32u * nw * ((ne32 + nw - 1u) / nw), std::max(kElistCap, room));
+  c.o_vlist = c.o_list + al(2 * c.elcap);
+  c.o_misc = c.o_vlist + vlist;
+  c.o_wrt = c.o_misc + misc;
+  c.o_ifc = c.o_wrt + vbits;
+  c.bytes = c.o_ifc + 2u * vbits;
+  return c;
 }
 
 ElementBounds element_bounds(const Pack &k) {

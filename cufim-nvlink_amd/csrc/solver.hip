@@ -728,11 +728,6 @@ __device__ inline uint32_t live_targets(const uint4 b, float hs, const float ph[
   for (int T = 0; T < 4; ++T) tm |= (nf - f[T] > 0 && ph[T] > v[T]) ? 1u << T : 0u;
   return tm;
 }
-// (element, target) pair ring of one wave in the band kernel: pairs left from
-// earlier rounds of 64 ilp plus 4 targets of 64 elements
-constexpr uint32_t pair_ring(int ilp) { return 64u * (uint32_t)ilp + 256u; }
-// counters and flags of a workgroup, region factors, launch counters
-constexpr uint32_t kMiscBytes = 80;
 
 // marks the two local elements of one adjacency word in the LDS bitmask; the
 // atomics return nothing, the list is built from the bitmask
@@ -2711,19 +2706,6 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
       HIPCHECK(hipMemset(c->d_stats, 0, 8 * sizeof(unsigned long long)));
       if (o->mode == FIM_MODE_CONVERGE) {
         c->lds_conv = 0;
-        const uint32_t nn64 = ((uint32_t)c->nn_max + 63u) & ~63u;
-        const uint32_t ne32 = ((uint32_t)c->ne_max + 31u) / 32u;
-        const uint32_t o_phin = al16(4 * nn64);
-        const uint32_t o_flg = o_phin + al16(4 * nn64);
-        const uint32_t o_tch = o_flg + al16(4 * (nn64 / 32));
-        const uint32_t o_dfr = o_tch + al16(4 * (nn64 / 32));
-        const uint32_t o_e2n = o_dfr + al16(4 * (nn64 / 32));
-        // staged: element nodes + geometry; unstaged: element mark bitmasks
-        const uint32_t o_geo = o_e2n + (o->staged ? al16(8 * (uint32_t)c->ne_max) : al16(4 * ne32));
-        const uint32_t o_list = o_geo + (o->staged ? al16(24 * (uint32_t)c->ne_max) : al16(4 * ne32));
-        // workgroups of 256 and 512 evaluate (element, target) pairs when
-        // local element ids fit 14 bits; the pair rings live in the source list
-        c->band_pairs = !o->staged && (c->block == 256 || c->block == 512) && c->ne_max < (1 << 14);
         c->unit = o->unit > 0 ? (uint32_t)o->unit : 2u;
         c->maxch = (c->ninst + c->unit - 1) / c->unit;
         if ((uint64_t)c->nsub * c->maxch >= (1ull << 32)) throw Error(FIM_ELIMIT, "too many work units");
@@ -2734,34 +2716,12 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->direct_plan = c->maxch == 1;
         int ncu = 256;
         HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->dev));
-        // A list of at most one unit per submesh leaves the CUs with a few waves
-        // each when the mesh has few submeshes: the kernel gets registers for
-        // two pair rounds side by side then (ILP of k_conv_band)
-        const bool few = c->band_pairs && c->direct_plan && o->waves == 0 && c->nsub <= 4u * (uint32_t)ncu;
+        c->band_pairs = !o->staged && band_with_pairs(c->block, c->ne_max);
+        const bool few = c->band_pairs && c->direct_plan && o->waves == 0 && few_submeshes(c->nsub, ncu);
         if (few) c->band_wpe = 4;
-        const uint32_t vlist_bytes =
-            o->staged ? 0u
-                      : al16(std::max<uint32_t>(2 * nn64, c->band_pairs ? (uint32_t)(c->block / 64) * 2u * pair_ring(few ? 2 : 1) : 0u));
-        const uint32_t misc_bytes = o->staged ? 48u : kMiscBytes;  // staged: 8 words, 4 region factors
-        const uint32_t tail_bytes = vlist_bytes + misc_bytes + (o->staged ? 0u : 3u * al16(4 * (nn64 / 32)));
-        // The band kernel lists at most elcap elements per pass, an equal share
-        // per wave: all elements of a wave's words where they fit, else at least
-        // kElistCap, more if the LDS left over by the workgroups the wave slots
-        // admit (8 waves per SIMD) holds more
-        uint32_t elcap = (uint32_t)c->ne_max;
-        if (!o->staged) {
-          const uint32_t nw = (uint32_t)c->block / 64u, wg_slots = std::max<uint32_t>(1u, 32u / nw);
-          const uint32_t budget = (160u * 1024u / wg_slots) & ~15u;
-          const uint32_t base = o_list + tail_bytes;
-          const uint32_t room = budget > base ? ((budget - base) / 2u) & ~7u : 0u;
-          elcap = std::min<uint32_t>(32u * nw * ((ne32 + nw - 1u) / nw), std::max<uint32_t>((uint32_t)kElistCap, room));
-        }
-        const uint32_t o_vlist = o_list + al16(2 * elcap);
-        const uint32_t o_misc = o_vlist + vlist_bytes;
-        const uint32_t o_wrt = o_misc + misc_bytes;
-        // unstaged: interface-copy bits and entry counts (2 x nn64/32 words)
-        const uint32_t o_ifc = o_wrt + (o->staged ? 0u : al16(4 * (nn64 / 32)));
-        c->lds_conv = o_ifc + (o->staged ? 0u : 2u * al16(4 * (nn64 / 32)));
+        const ConvergeCarve lds = converge_carve(c->nn_max, c->ne_max, c->block, o->staged != 0,
+                                                 !c->band_pairs ? 0 : few ? 2 : 1);
+        c->lds_conv = lds.bytes;
         if (c->lds_conv > 160 * 1024)
           throw Error(FIM_ELIMIT, "largest submesh needs " + std::to_string(c->lds_conv) +
                                       " B of LDS (limit 163840); use a smaller partition budget");
@@ -2909,8 +2869,8 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
                          c->nsub, c->ncopy, c->ninst, c->direct_plan ? 1u : 0u,
                          (float)(o->eps_rel > 0 ? o->eps_rel : 1e-6),
                          c->d_winst, o->local_iters, c->unit, c->maxch, (uint32_t)p.if_l.size(),
-                         c->wps, elcap, o_phin, o_flg, o_tch, o_dfr, o_e2n, o_geo, o_list, o_vlist, o_misc,
-                         o_wrt, o_ifc};
+                         c->wps, lds.elcap, lds.o_phin, lds.o_flg, lds.o_tch, lds.o_dfr, lds.o_e2n, lds.o_geo,
+                         lds.o_list, lds.o_vlist, lds.o_misc, lds.o_wrt, lds.o_ifc};
         c->n_if = (uint32_t)p.if_l.size();
       } else {
         const uint32_t nn = (uint32_t)c->nn_max;

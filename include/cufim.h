@@ -160,7 +160,8 @@ typedef struct {
   int64_t nsub, ncopy, n_iface_copies;
   int32_t nn_max, ne_max;
   int64_t device_bytes_mesh;  /* compact FP32 mesh bytes (plain mode)      */
-  int64_t lds_bytes;          /* dynamic LDS per workgroup (plain mode)    */
+  int64_t lds_bytes;          /* dynamic LDS per workgroup of a converge
+                                 context with default options              */
 } fim_pack_info_t;
 
 int fim_pack_build(const fim_mesh *m, const fim_part_opts *o, fim_pack **out);

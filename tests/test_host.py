@@ -559,3 +559,28 @@ def test_site_sets_that_are_refused_one_by_one_are_refused_at_once(sets):
         F._sites3_all(sets)
     with pytest.raises(ValueError):
         F._factors_all([[1.0, 2, 3], [1.0, 2, 3, 4, 5]])
+
+
+@pytest.mark.parametrize("max_nn", [20, 64, 100, 512, 1500, 2816])
+def test_pack_info_reports_the_whole_lds_carve(max_nn):
+    """lds_bytes of a pack, added up here part by part for a context with
+    default options: eight waves, one instance, two pair rounds of a wave side
+    by side on up to 4 x 256 submeshes"""
+    m = F.Mesh.gen_box(seed=1, **dict(cases.SLAB, nx=24, ny=24, nz=8))
+    i = F.Pack(m, F.PART_RCB, max_nn=max_nn, seed=1).info
+    assert (i["nsub"] > 1024) == (max_nn == 20) and i["ne_max"] < 2 ** 14
+    nn64 = -(-i["nn_max"] // 64) * 64
+    words = -(-i["ne_max"] // 32)
+    ring = 64 * (1 if i["nsub"] > 1024 else 2) + 256
+    up = lambda x: -(-x // 16) * 16  # noqa: E731
+    parts = [4 * nn64] * 2                    # times, candidate minima
+    parts += [nn64 // 8] * 6                  # four vertex bitmasks, interface-copy bits and counts
+    parts += [4 * words] * 2                  # two element bitmasks
+    parts += [max(2 * nn64, 8 * 2 * ring)]    # sources, or the eight waves' pair rings
+    parts += [80]                             # counters and factors
+    fixed = sum(up(x) for x in parts)
+    # the element list: every wave's share of the words, or what the LDS of one of four
+    # workgroups leaves, at least 2,032
+    room = max(0, (40960 - fixed) // 2 // 8 * 8)
+    want = fixed + up(2 * min(32 * 8 * -(-words // 8), max(2032, room)))
+    assert i["lds_bytes"] == want
