@@ -1620,7 +1620,6 @@ struct CompatArgs {
   const uint16_t *n2n_lv;
   double *phi;
   int8_t *st;
-  unsigned long long *stats;  // sweeps, slot evaluations
   double *nexte;              // per submesh: earliest window time its copies change
   const uint32_t *list;       // submeshes of this window (k_compat_sync), *nlist of them
   const uint32_t *nlist;
@@ -1720,12 +1719,9 @@ __device__ inline double compat_slot(const CompatArgs &a, const SubInfo &si, con
 constexpr unsigned long long kDmaxBits = 0x7fefffffffffffffull;  // DBL_MAX
 
 // The candidates of every slot k0 <= k < k1 whose owner has state `want`,
-// merged into the owner's minimum (FP64 bits, LDS integer min); returns the
-// slots this thread evaluated.
-__device__ inline unsigned long long compat_slots(const CompatArgs &a, const SubInfo &si,
-                                                  const double *phi_l, const int8_t *st_l, uint32_t k0,
-                                                  uint32_t k1, int8_t want, unsigned long long *tmin) {
-  unsigned long long n = 0;
+// merged into the owner's minimum (FP64 bits, LDS integer min).
+__device__ inline void compat_slots(const CompatArgs &a, const SubInfo &si, const double *phi_l, const int8_t *st_l,
+                                    uint32_t k0, uint32_t k1, int8_t want, unsigned long long *tmin) {
   for (uint32_t k = k0 + threadIdx.x; k < k1; k += blockDim.x) {
     const int t = a.n2e_pos[k];
     const size_t ge = (size_t)si.eoff + a.n2e_le[k];
@@ -1735,9 +1731,7 @@ __device__ inline unsigned long long compat_slots(const CompatArgs &a, const Sub
     if (st_l[owner] != want) continue;
     const double v = compat_slot(a, si, phi_l, st_l, ge, nd, t);
     atomicMin(&tmin[owner], (unsigned long long)__double_as_longlong(v));
-    ++n;
   }
-  return n;
 }
 
 template <int BS>
@@ -1751,7 +1745,6 @@ __global__ __launch_bounds__(BS) void k_compat_compute(CompatArgs a) {
   int8_t *snap = reinterpret_cast<int8_t *>(lds + a.o_snap);
   uint32_t *misc = reinterpret_cast<uint32_t *>(lds + a.o_misc);
   const uint32_t tid = threadIdx.x;
-  unsigned long long sweeps = 0, slots = 0;
   unsigned long long *evslot = reinterpret_cast<unsigned long long *>(misc + 2);
   const uint32_t nlist = *a.nlist;
   uint32_t pend_wg = 0;  // thread 0
@@ -1790,13 +1783,12 @@ __global__ __launch_bounds__(BS) void k_compat_compute(CompatArgs a) {
     const uint32_t k0 = a.n2e_dsp[si.coff], k1 = a.n2e_dsp[si.coff + nn];
     unsigned long long *tmin = reinterpret_cast<unsigned long long *>(tphi);
     while (active > 0) {
-      ++sweeps;
       // a: candidates of narrow vertices, one thread per slot; times are
       // >= 0, so the minimum of the FP64 bit patterns as integers is the
       // minimum of the values and does not depend on the order
       for (uint32_t l = tid; l < nn; l += BS) tmin[l] = kDmaxBits;
       __syncthreads();
-      slots += compat_slots(a, si, phi_l, st_l, k0, k1, FIM_NARROW, tmin);
+      compat_slots(a, si, phi_l, st_l, k0, k1, FIM_NARROW, tmin);
       __syncthreads();
       // b: reduce, window test, convergence test
       for (uint32_t l = tid; l < nn; l += BS) {
@@ -1830,7 +1822,7 @@ __global__ __launch_bounds__(BS) void k_compat_compute(CompatArgs a) {
       // d: candidates of marked vertices, one thread per slot
       for (uint32_t l = tid; l < nn; l += BS) tmin[l] = kDmaxBits;
       __syncthreads();
-      slots += compat_slots(a, si, phi_l, st_l, k0, k1, FIM_NEIG, tmin);
+      compat_slots(a, si, phi_l, st_l, k0, k1, FIM_NEIG, tmin);
       __syncthreads();
       // e: accept improvements
       for (uint32_t l = tid; l < nn; l += BS) {
@@ -1894,9 +1886,6 @@ __global__ __launch_bounds__(BS) void k_compat_compute(CompatArgs a) {
     }
   }
   if (tid == 0) compat_finish(a, nlist, pend_wg);
-  if (tid == 0 && sweeps) atomicAdd(&a.stats[0], sweeps);
-  for (int off = 32; off > 0; off >>= 1) slots += __shfl_xor(slots, off);
-  if ((tid & 63) == 0 && slots) atomicAdd(&a.stats[1], slots);
 }
 
 // geometry index of e12 e13 e23 e14 e24 e34 after relabelling for target t
@@ -1955,7 +1944,6 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   const double lo = a.phi_start - a.fw;
   const uint32_t nlist = *a.nlist;
   uint32_t s = a.list[blockIdx.x];  // gridDim <= nsub entries; read with nlist
-  unsigned long long sweeps = 0, slots = 0;
   uint32_t pend_wg = 0;  // thread 0
   auto offer = [&](int8_t st, double p) { return (st >= FIM_NARROW && p > lo) ? p : DBL_MAX; };
   for (uint32_t i = blockIdx.x; i < nlist; i += gridDim.x) {
@@ -2049,13 +2037,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4, 8))) void
             v = cand_ref_a(e12, e13, e23, e14, e24, e34, p1, p2, p3);
           atomicMin(&tmin[node(t)], (unsigned long long)__double_as_longlong(v));
         }
-        slots += n;
       };
       for (uint32_t par = 0;; par ^= 1u) {
         __syncthreads();
         const uint32_t n = misc[par];
         if (n == 0) break;  // uniform
-        ++sweeps;
         // a: candidates of narrow copies
         evaluate(lp, n);
         __syncthreads();
@@ -2171,11 +2157,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4, 8))) void
       a.vcnt[s] = misc[6];
     }
   }
-  if (tid == 0) {
-    compat_finish(a, nlist, pend_wg);
-    if (sweeps) atomicAdd(&a.stats[0], sweeps);
-    if (slots) atomicAdd(&a.stats[1], slots);
-  }
+  if (tid == 0) compat_finish(a, nlist, pend_wg);
 }
 
 // Start of a window.  sync_step2 (min over the copies of each shared vertex)
@@ -2972,7 +2954,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->grid = (int)std::min<uint32_t>(c->nsub, (uint32_t)(ncu * std::max(per_cu, 1)));
         c->lds_conv = 0;
         c->xa = CompatArgs{c->d_sub, c->d_e2n, c->d_geo64, c->d_n2e_dsp, c->d_n2e_le, c->d_n2e_pos,
-                           c->d_n2n_dsp, c->d_n2n_lv, c->d_phi64, c->d_st, c->d_stats,
+                           c->d_n2n_dsp, c->d_n2n_lv, c->d_phi64, c->d_st,
                            c->d_nexte, nullptr, nullptr, c->d_cshared, c->d_vrec, c->d_vcnt,
                            c->d_done, c->d_pin, c->nsub,
                            o->local == FIM_LOCAL_EXACT ? 1 : 0, 0, 0, 0, 0, o->apd > 0 ? o->apd : 3e5,
