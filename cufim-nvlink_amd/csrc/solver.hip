@@ -2867,6 +2867,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         const uint32_t s_tmin = 2 * al16(8 * nn), s_st = s_tmin + al16(8 * nn);
         const uint32_t s_misc = s_st + al16(nn), s_blob = s_misc + al16(32 + 2 * 4 * ((uint32_t)c->block / 32));
         uint32_t chunks = 0, words = 0, gwords = 0;  // largest submesh
+        uint64_t total = 0, gtotal = 0;              // all
         std::vector<CompatSub> cs(p.nsub);
         for (int64_t q = 0; q < p.nsub; ++q) {
           const SubInfo &si = p.sub[q];
@@ -2877,25 +2878,27 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
           chunks = std::max(chunks, nch);
           words = std::max(words, w);
           gwords = std::max(gwords, w + 3 * si.ne);
+          total += w;
+          gtotal += w + 3 * si.ne;
         }
         // k_compat_small needs a thread per copy and its data in LDS; 40 KB
         // leave a CU the four workgroups that its registers admit.  Without
         // the geometry in LDS (submeshes of 256 copies, say) it comes from L2.
+        // A submesh's place in the blocks is a number of words in 32 bits.
         const uint32_t lists = 2 * al16(8 * chunks);
         constexpr uint32_t kSmallLds = 40 * 1024;
         c->compat_small = nn <= (uint32_t)c->block && (uint32_t)c->ne_max < (kNoSlot >> 2) && chunks < (1u << 16) &&
-                          s_blob + 16 * words + lists <= kSmallLds;
-        c->compat_geo = c->compat_small && s_blob + 16 * gwords + lists <= kSmallLds;
+                          s_blob + 16 * words + lists <= kSmallLds && total < (1ull << 32);
+        c->compat_geo = c->compat_small && s_blob + 16 * gwords + lists <= kSmallLds && gtotal < (1ull << 32);
         const uint32_t s_lp = s_blob + 16 * (c->compat_geo ? gwords : words), s_lq = s_lp + al16(8 * chunks);
         if (c->compat_small) {
           c->lds_compat = s_blob + 16 * (c->compat_geo ? gwords : words) + lists;
-          size_t total = 0;
+          total = 0;
           for (CompatSub &q : cs) {
             if (c->compat_geo) q.nw += 3 * q.ne;
             q.boff = (uint32_t)total;
             total += q.nw;
           }
-          if (total >= (1ull << 32)) throw Error(FIM_ELIMIT, "submesh blocks above 2^32 words");
           std::unique_ptr<void, void (*)(void *)> mem(std::malloc(16 * std::max<size_t>(total, 1)), std::free);
           if (!mem) throw std::bad_alloc();
           uint4 *blob = static_cast<uint4 *>(mem.get());
