@@ -36,7 +36,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -2160,6 +2159,60 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   if (tid == 0) compat_finish(a, nlist, pend_wg);
 }
 
+// Assembles the submeshes' blocks (CompatSub), one workgroup per submesh, from
+// the plain arrays.  On the host, and copied from there, the 144 MB of the 2M-tet
+// slab took 10 ms more of a context's creation (20 against 10; 8.5 with the
+// general kernel alone).
+struct CompatBlockArgs {
+  const CompatSub *csub;
+  const uint2 *e2n;
+  const uint32_t *n2e_dsp;
+  const uint16_t *n2e_le;
+  const uint8_t *n2e_pos;
+  const uint4 *geo;  // FP64 geometry, three words an element; null: not in the blocks
+  uint4 *blob;
+  uint32_t nsub;
+};
+__global__ __launch_bounds__(256) void k_compat_block(CompatBlockArgs a) {
+  __shared__ uint32_t off[512 + 1];  // chunks before each copy; at most 512 copies (k_compat_small)
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t s = blockIdx.x; s < a.nsub; s += gridDim.x) {
+    const CompatSub q = a.csub[s];
+    const uint32_t nd = (2 * (q.nn + 1) + 15) / 16, nel = (8 * q.ne + 15) / 16, nsl = (8 * q.nch + 15) / 16;
+    uint4 *block = a.blob + q.boff;
+    const uint32_t *dsp = a.n2e_dsp + q.coff;
+    if (tid < 3) block[(tid == 0 ? nd : tid == 1 ? nd + nel : nd + nel + nsl) - 1] = make_uint4(0u, 0u, 0u, 0u);  // ends
+    if (tid < 64) {
+      uint32_t before = 0;
+      for (uint32_t l0 = 0; l0 < q.nn; l0 += 64) {
+        const uint32_t l = l0 + tid, n = l < q.nn ? (dsp[l + 1] - dsp[l] + 3) / 4 : 0u;
+        uint32_t sum = n;
+        for (int d = 1; d < 64; d <<= 1) {
+          const uint32_t x = __shfl_up(sum, d);
+          if (tid >= (uint32_t)d) sum += x;
+        }
+        if (l < q.nn) off[l] = before + sum - n;
+        before += __shfl(sum, 63);
+      }
+      if (tid == 0) off[q.nn] = before;
+    }
+    __syncthreads();
+    uint16_t *o = reinterpret_cast<uint16_t *>(block);
+    for (uint32_t l = tid; l <= q.nn; l += 256) o[l] = (uint16_t)off[l];
+    uint2 *en = reinterpret_cast<uint2 *>(block + nd);
+    for (uint32_t e = tid; e < q.ne; e += 256) en[e] = a.e2n[(size_t)q.eoff + e];
+    uint16_t *sl = reinterpret_cast<uint16_t *>(block + nd + nel);
+    for (uint32_t l = tid; l < q.nn; l += 256) {
+      const uint32_t kb = dsp[l], n = dsp[l + 1] - kb;
+      for (uint32_t k = 0; k < (n + 3) / 4 * 4; ++k)
+        sl[4 * off[l] + k] = k < n ? (uint16_t)((uint32_t)a.n2e_le[kb + k] << 2 | a.n2e_pos[kb + k]) : kNoSlot;
+    }
+    if (a.geo)
+      for (uint32_t i = tid; i < 3 * q.ne; i += 256) block[nd + nel + nsl + i] = a.geo[3 * (size_t)q.eoff + i];
+    __syncthreads();  // off is free
+  }
+}
+
 // Start of a window.  sync_step2 (min over the copies of each shared vertex)
 // and the list of submeshes the window's pass has to run on: those whose
 // copies' own clocks are due (nexte; -inf when something is narrow or next)
@@ -2256,6 +2309,14 @@ T *dupload(const std::vector<T> &v, std::vector<void *> &owned) {
   if (!v.empty()) HIPCHECK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
   return p;
 }
+
+// device buffers of a scope
+struct Buffers {
+  std::vector<void *> v;
+  ~Buffers() {
+    for (void *p : v) (void)hipFree(p);
+  }
+};
 
 }  // namespace
 }  // namespace fim
@@ -2869,17 +2930,21 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         uint32_t chunks = 0, words = 0, gwords = 0;  // largest submesh
         uint64_t total = 0, gtotal = 0;              // all
         std::vector<CompatSub> cs(p.nsub);
-        for (int64_t q = 0; q < p.nsub; ++q) {
-          const SubInfo &si = p.sub[q];
-          uint32_t nch = 0;
-          for (uint32_t l = 0; l < si.nn; ++l) nch += (p.n2e_dsp[si.coff + l + 1] - p.n2e_dsp[si.coff + l] + 3) / 4;
-          const uint32_t w = (2 * (si.nn + 1) + 15) / 16 + (8 * si.ne + 15) / 16 + (8 * nch + 15) / 16;
-          cs[q] = CompatSub{si.coff, si.nn, si.eoff, si.ne, si.ioff, 0u, w, nch};
-          chunks = std::max(chunks, nch);
-          words = std::max(words, w);
-          gwords = std::max(gwords, w + 3 * si.ne);
-          total += w;
-          gtotal += w + 3 * si.ne;
+        parallel_ranges((size_t)p.nsub, 512, [&](size_t b, size_t e) {
+          for (size_t q = b; q < e; ++q) {
+            const SubInfo &si = p.sub[q];
+            uint32_t nch = 0;
+            for (uint32_t l = 0; l < si.nn; ++l) nch += (p.n2e_dsp[si.coff + l + 1] - p.n2e_dsp[si.coff + l] + 3) / 4;
+            const uint32_t w = (2 * (si.nn + 1) + 15) / 16 + (8 * si.ne + 15) / 16 + (8 * nch + 15) / 16;
+            cs[q] = CompatSub{si.coff, si.nn, si.eoff, si.ne, si.ioff, 0u, w, nch};
+          }
+        });
+        for (const CompatSub &q : cs) {
+          chunks = std::max(chunks, q.nch);
+          words = std::max(words, q.nw);
+          gwords = std::max(gwords, q.nw + 3 * q.ne);
+          total += q.nw;
+          gtotal += q.nw + 3 * q.ne;
         }
         // k_compat_small needs a thread per copy and its data in LDS; 40 KB
         // leave a CU the four workgroups that its registers admit.  Without
@@ -2899,32 +2964,16 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
             q.boff = (uint32_t)total;
             total += q.nw;
           }
-          std::unique_ptr<void, void (*)(void *)> mem(std::malloc(16 * std::max<size_t>(total, 1)), std::free);
-          if (!mem) throw std::bad_alloc();
-          uint4 *blob = static_cast<uint4 *>(mem.get());
-          parallel_ranges((size_t)p.nsub, 256, [&](size_t b, size_t e) {
-            for (size_t i = b; i < e; ++i) {
-              const CompatSub &q = cs[i];
-              const size_t nd = (2 * (q.nn + 1) + 15) / 16, nel = (8 * q.ne + 15) / 16, nsl = (8 * q.nch + 15) / 16;
-              uint16_t *d = reinterpret_cast<uint16_t *>(blob + q.boff), *en = d + 8 * nd, *sl = en + 8 * nel;
-              blob[q.boff + nd - 1] = blob[q.boff + nd + nel - 1] = blob[q.boff + nd + nel + nsl - 1] =
-                  make_uint4(0u, 0u, 0u, 0u);  // the sections' ends
-              std::memcpy(en, &p.e2n_l[4 * (size_t)q.eoff], 8 * (size_t)q.ne);
-              uint32_t ch = 0;
-              for (uint32_t l = 0; l < q.nn; ++l) {
-                const uint32_t kb = p.n2e_dsp[q.coff + l], n = p.n2e_dsp[q.coff + l + 1] - kb;
-                d[l] = (uint16_t)ch;
-                for (uint32_t k = 0; k < (n + 3) / 4 * 4; ++k)
-                  sl[4 * ch + k] = k < n ? (uint16_t)(p.n2e_le[kb + k] << 2 | p.n2e_pos[kb + k]) : kNoSlot;
-                ch += (n + 3) / 4;
-              }
-              d[q.nn] = (uint16_t)ch;
-              if (c->compat_geo) std::memcpy(sl + 8 * nsl, &p.geo64[6 * (size_t)q.eoff], 48 * (size_t)q.ne);
-            }
-          });
           c->d_csub = dupload(cs, ow);
           c->d_blob = dalloc<uint4>(total, ow);
-          HIPCHECK(hipMemcpy(c->d_blob, blob, 16 * total, hipMemcpyHostToDevice));
+          Buffers tmp;
+          const CompatBlockArgs ba{c->d_csub, c->d_e2n, dupload(p.n2e_dsp, tmp.v), dupload(p.n2e_le, tmp.v),
+                                   dupload(p.n2e_pos, tmp.v),
+                                   c->compat_geo ? reinterpret_cast<const uint4 *>(dupload(p.geo64, tmp.v)) : nullptr,
+                                   c->d_blob, c->nsub};
+          k_compat_block<<<(int)std::min<uint32_t>(c->nsub, 65536u), 256, 0, c->stream>>>(ba);
+          HIPCHECK(hipGetLastError());
+          HIPCHECK(hipStreamSynchronize(c->stream));
         }
         if (!c->compat_geo) c->d_geo64 = dupload(p.geo64, ow);
         if (!c->compat_small) {
@@ -2941,10 +2990,14 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->d_mark = dalloc<uint32_t>(c->nsub, ow);
         c->d_lcnt = dalloc<uint32_t>(3, ow);
         {
-          std::vector<uint32_t> cs(p.ncopy, kNoVertex);
-          for (uint32_t v : p.grp_v)
-            for (uint32_t k = p.g2c_dsp[v]; k < p.g2c_dsp[v + 1]; ++k) cs[p.g2c[k]] = v;
-          c->d_cshared = dupload(cs, ow);
+          std::vector<uint32_t> sh(p.ncopy);
+          parallel_ranges((size_t)p.ncopy, 65536, [&](size_t b, size_t e) {
+            for (size_t i = b; i < e; ++i) {
+              const uint32_t v = p.c2g[i];
+              sh[i] = p.g2c_dsp[v + 1] - p.g2c_dsp[v] > 1 ? v : kNoVertex;
+            }
+          });
+          c->d_cshared = dupload(sh, ow);
         }
         c->d_vrec = dalloc<uint32_t>(p.if_l.size(), ow);
         c->d_vcnt = dalloc<uint32_t>(c->nsub, ow);
