@@ -81,7 +81,7 @@ def kernel_source_digest():
     measured on."""
     import hashlib
     h = hashlib.sha256()
-    for f in ("solver.hip", "local_solve.hpp"):
+    for f in ("solver.hip", "local_solve.hpp", "host.hpp", "partition.cpp"):
         for line in open(os.path.join(ROOT, "cufim-nvlink_amd", "csrc", f)).read().splitlines():
             code = re.sub(r"//.*$", "", line).rstrip()
             if code:

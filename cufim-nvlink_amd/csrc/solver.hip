@@ -1245,8 +1245,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     }
     // algorithmic bytes: copies (phi 4+4, flag 1+1), interface entries
     // (4+4+4) and the distinct elements evaluated (32 B: 24 B of FP32
-    // geometry + 8 B of node ids; the 16 B of node heights in the record
-    // are pruning data of this kernel, not algorithmic bytes)
+    // geometry + 8 B of node ids; the record's 16 B of candidate bounds and
+    // their scale are pruning data of this kernel, not algorithmic bytes)
     uint32_t cnt = 0;
     for (uint32_t k = tid; k < new32; k += BS) cnt += __popc(eseen[k]);
     // up to 65,535 elements, so 2,048 / BS words of 32 per thread (8 with 256)
@@ -1912,7 +1912,7 @@ __device__ inline uint32_t compat_relabel(int t) {
 //     so a slot reads three words and no states;
 //   - the downwind neighbours of just-frozen copies are found through the
 //     elements (copies are neighbours when they share one);
-//   - a sweep in which nothing froze has two barriers, any other six;
+//   - a sweep in which nothing froze has three barriers, any other five or six;
 //   - the submesh's data comes straight into LDS, in flight together with the
 //     copies' times, so a submesh waits for memory three times in all.
 // Full slab, 10,152 submeshes of at most 128 copies, 150 windows of 2 ms: a
