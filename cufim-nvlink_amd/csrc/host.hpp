@@ -161,6 +161,11 @@ inline bool band_with_pairs(int block, int32_t ne_max) {
 // rounds side by side then
 inline bool few_submeshes(int64_t nsub, int cus) { return nsub <= 4 * (int64_t)cus; }
 
+// Elements per wave of a workgroup up to which a submesh's sweeps are listed by
+// few waves (GATHER of k_conv_band): always, and while the launch's units fill
+// at least half of its workgroups
+constexpr uint32_t kGatherAlways = 256, kGatherFull = 640;
+
 // Dynamic LDS of the converge-mode kernels for the largest submesh: byte
 // offsets, the entries of the element list, all bytes.
 struct ConvergeCarve {

@@ -821,7 +821,22 @@ __device__ inline void wave_append(bool pred, uint32_t l, uint16_t *list, uint32
 // as long as its longest item (107k cycles), a batch's launch is 1,450 items
 // deep.  Loading the next 64 listed elements ahead of the current ones gained
 // nothing.
-template <int BS, int WPE, bool PAIRS>
+//
+// GATHER: a sweep of few sources marks too few elements to give every wave a
+// full round, and eight nearly empty rounds cost as many instructions as eight
+// full ones.  Where the CUs are busy (the units fill half of the workgroups or
+// more), submeshes of up to kGatherFull elements a wave have such a sweep
+// listed by one wave for every 32 sources (about 20 elements each): 271 maps of
+// a 44k-tet mesh in submeshes of 769 copies, workgroups of 512, 16.6 ms against
+// 20.8 with all waves; 423 maps of a 180k-tet shell in two contexts 74 against
+// 93.  With the line at 1,280 elements a wave some batches gained another 10 %,
+// others lost 20 % (149 maps on 42 submeshes 42 against 34 ms): their sweeps are
+// a chain of rounds, and 512 maps of the 2M-tet slab take 228 instead of 205 ms
+// with few waves.  So do launches that leave the CUs half empty.  Up to
+// kGatherAlways elements a wave, a wave has hardly a word of the bitmask, and
+// few waves list at any load (a single solve on 3,534 submeshes of 256 copies:
+// 9.0 against 10.2 ms).
+template <int BS, int WPE, bool PAIRS, bool GATHER>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) void k_conv_band(ConvArgs) {
   extern __shared__ __align__(16) unsigned char lds[];
   const KArgs k0 = kargs();
@@ -842,13 +857,14 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
   // [8..11] the instance's region factors, [12..19] launch counters
   uint32_t *misc = reinterpret_cast<uint32_t *>(lds + k0->o_misc);
   const float *rsl = reinterpret_cast<const float *>(misc + 8);
-  constexpr uint32_t NW = BS / 64;
+  constexpr uint32_t NW = BS / 64, LNW = NW == 8 ? 3 : NW == 4 ? 2 : NW == 2 ? 1 : 0;
   constexpr int ILP = WPE <= 4 ? 2 : 1;
   uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   UnitCursor cursor;
   const uint32_t iter_now = start_iteration();
+  const bool full = GATHER && 2u * k0->cur.cnt[0] >= gridDim.x;
   // counters of the launch (thread 0): activations, sweeps, element
   // evaluations, algorithmic bytes
   unsigned long long *ctr = reinterpret_cast<unsigned long long *>(misc + 12);
@@ -868,7 +884,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
     const uint32_t nn = si.nn, ne = si.ne;
     const uint32_t nv64 = (nn + 63u) & ~63u;
     const uint32_t new32 = (ne + 31u) >> 5;  // element bitmask words
-    const uint32_t nww = wave < new32 ? (new32 - wave + NW - 1) / NW : 0u;  // words of this wave
+    const bool gather = GATHER && ne <= (full ? kGatherFull : kGatherAlways) * NW;
     if (item.wake > W) {
       defer_item<BS>(si, item, inst, s, iter_now, &misc[5]);
       continue;
@@ -976,15 +992,19 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
       for (uint32_t i = tid; i < nsrc; i += BS) mark_incident(adj, adj_ptr, adj_more, vlist[i], emark);
       __syncthreads();
       if (tid == 0) misc[2] = 0u;  // every thread has read the source count
-      // Each wave lists and evaluates the marked elements of its own words of
-      // the bitmask (every NW-th: neighbours go to different waves), without a
-      // barrier in between.  Lane i holds word i: offsets from a wave prefix sum
+      // Each wave, or each of a few, lists and evaluates the marked elements of
+      // its own words of the bitmask (every NW-th: neighbours go to different
+      // waves), without a barrier in between.  Lane i holds word i: offsets from a wave prefix sum
       // of the word counts (<= 32, six bits) with one ballot per bit, then two
       // words at a time, a lane per bit.  A pass lists at most wcap elements;
       // what is left of the words stays marked for the next pass (the sweep
       // still evaluates every marked element against the same times).
+      uint32_t lw = LNW;  // 2^lw waves
+      if (GATHER && gather && nsrc < 128u)
+        lw = __builtin_amdgcn_readfirstlane(min(LNW, nsrc < 32u ? 0u : nsrc < 64u ? 1u : 2u));
+      const uint32_t nw = 1u << lw, nww = wave < min(nw, new32) ? (new32 - wave + nw - 1) >> lw : 0u;
       for (uint32_t i0 = 0; i0 < nww;) {
-        const uint32_t kw = wave + NW * (i0 + lane);
+        const uint32_t kw = wave + ((i0 + lane) << lw);
         const uint32_t rest = i0 + lane < nww ? emark[kw] : 0u;
         const uint32_t n = __popc(rest);
         uint32_t pos = 0, tot = 0;
@@ -1023,7 +1043,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE, 8))) vo
           const uint32_t bit = lane & 31u, tw = hi ? (two ? t2 : 0u) : t1;
           if ((tw >> bit) & 1u)
             wlist[(hi ? p2 : p1) + __popc(tw & ((1u << bit) - 1u))] =
-                (uint16_t)((wave + NW * (word0 + (hi ? i2 : i1))) * 32 + bit);
+                (uint16_t)((wave + ((word0 + (hi ? i2 : i1)) << lw)) * 32 + bit);
         }
         __builtin_amdgcn_wave_barrier();
         const uint32_t nact = min(tot, wcap);
@@ -2416,44 +2436,54 @@ struct fim_ctx {
   int grid = 0, block = 256, graph_iters = 8;
   int band_wpe = 8;  // waves per SIMD the band kernel's registers are sized for
   bool band_pairs = false;  // band kernel evaluates (element, target) pairs
+  bool band_gather = false; // its GATHER variant
   bool direct = false;      // launch iterations directly instead of replaying the graph
   fim_stats_t stats{};
 };
 
 namespace {
 
-const void *conv_kernel_ptr(bool staged, int block, int wpe, bool pairs) {
+template <bool GATHER>
+const void *band_pairs_ptr(int block, int wpe) {
+  if (block == 512) return (const void *)k_conv_band<512, 8, true, GATHER>;
+  if (wpe == 5) return (const void *)k_conv_band<256, 5, true, GATHER>;
+  if (wpe == 6) return (const void *)k_conv_band<256, 6, true, GATHER>;
+  if (wpe == 7) return (const void *)k_conv_band<256, 7, true, GATHER>;
+  return (const void *)k_conv_band<256, 8, true, GATHER>;
+}
+
+const void *conv_kernel_ptr(const fim_ctx *c) {
+  const int block = c->block, wpe = c->band_wpe;
+  if (c->o.staged) switch (block) {
+      case 64: return (const void *)k_conv_compute<64>;
+      case 128: return (const void *)k_conv_compute<128>;
+      case 512: return (const void *)k_conv_compute<512>;
+      default: return (const void *)k_conv_compute<256>;
+    }
+  if (c->band_pairs) {
+    if (wpe <= 4)
+      return block == 512 ? (const void *)k_conv_band<512, 4, true, false> : (const void *)k_conv_band<256, 4, true, false>;
+    return c->band_gather ? band_pairs_ptr<true>(block, wpe) : band_pairs_ptr<false>(block, wpe);
+  }
   switch (block) {
-    case 64: return staged ? (const void *)k_conv_compute<64> : (const void *)k_conv_band<64, 8, false>;
-    case 128: return staged ? (const void *)k_conv_compute<128> : (const void *)k_conv_band<128, 8, false>;
-    case 512:
-      if (staged) return (const void *)k_conv_compute<512>;
-      if (!pairs) return (const void *)k_conv_band<512, 8, false>;
-      return wpe <= 4 ? (const void *)k_conv_band<512, 4, true> : (const void *)k_conv_band<512, 8, true>;
+    case 64: return (const void *)k_conv_band<64, 8, false, false>;
+    case 128: return (const void *)k_conv_band<128, 8, false, false>;
+    case 512: return (const void *)k_conv_band<512, 8, false, false>;
     default:
-      if (staged) return (const void *)k_conv_compute<256>;
-      if (pairs) {
-        if (wpe <= 4) return (const void *)k_conv_band<256, 4, true>;
-        if (wpe == 5) return (const void *)k_conv_band<256, 5, true>;
-        if (wpe == 6) return (const void *)k_conv_band<256, 6, true>;
-        if (wpe == 7) return (const void *)k_conv_band<256, 7, true>;
-        return (const void *)k_conv_band<256, 8, true>;
-      }
-      if (wpe <= 5) return (const void *)k_conv_band<256, 5, false>;
-      if (wpe == 6) return (const void *)k_conv_band<256, 6, false>;
-      if (wpe == 7) return (const void *)k_conv_band<256, 7, false>;
-      return (const void *)k_conv_band<256, 8, false>;
+      if (wpe <= 5) return (const void *)k_conv_band<256, 5, false, false>;
+      if (wpe == 6) return (const void *)k_conv_band<256, 6, false, false>;
+      if (wpe == 7) return (const void *)k_conv_band<256, 7, false, false>;
+      return (const void *)k_conv_band<256, 8, false, false>;
   }
 }
 
 void launch_conv_compute(fim_ctx *c, const ConvArgs &a) {
   void *args[] = {const_cast<ConvArgs *>(&a)};
-  HIPCHECK(hipLaunchKernel(conv_kernel_ptr(c->o.staged != 0, c->block, c->band_wpe, c->band_pairs), dim3(c->grid),
-                           dim3(c->block), args, c->lds_conv, c->stream));
+  HIPCHECK(hipLaunchKernel(conv_kernel_ptr(c), dim3(c->grid), dim3(c->block), args, c->lds_conv, c->stream));
 }
 
 void set_lds_attr(fim_ctx *c) {
-  const void *f = conv_kernel_ptr(c->o.staged != 0, c->block, c->band_wpe, c->band_pairs);
+  const void *f = conv_kernel_ptr(c);
   HIPCHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->lds_conv));
 }
 
@@ -2896,14 +2926,20 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
           c->band_wpe = lds_cap <= 5u ? 5 : (lds_cap >= 8u ? 8 : (int)lds_cap);
           if (o->waves > 0) c->band_wpe = std::min(c->band_wpe, std::max(o->waves, 5));
         }
-        set_lds_attr(c);
-        int per_cu = 0;
-        HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, conv_kernel_ptr(o->staged != 0, c->block, c->band_wpe, c->band_pairs), c->block,
-            c->lds_conv));
-        per_cu = std::max(per_cu, 1);
-        c->grid = o->grid > 0 ? o->grid : ncu * per_cu;
-        c->grid = std::max(c->grid, (int)kXcd);  // every XCD eighth needs a workgroup
+        auto size_grid = [&] {
+          set_lds_attr(c);
+          int per_cu = 0;
+          HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, conv_kernel_ptr(c), c->block, c->lds_conv));
+          c->grid = o->grid > 0 ? o->grid : ncu * std::max(per_cu, 1);
+          c->grid = std::max(c->grid, (int)kXcd);  // every XCD eighth needs a workgroup
+        };
+        size_grid();
+        // GATHER, where the submeshes on average, and a launch of all units, would
+        // use it (its tests cost the others 1 %)
+        const uint64_t per_wave = (uint64_t)c->ne / c->nsub / ((uint32_t)c->block / 64u);
+        const bool fills = 2u * (uint64_t)c->nsub * c->maxch >= (uint64_t)c->grid;
+        c->band_gather = c->band_pairs && !few && per_wave <= (fills ? kGatherFull : kGatherAlways);
+        if (c->band_gather) size_grid();
         c->lds_compat = 0;
         c->ca = ConvArgs{c->d_sub, c->d_e2n, c->d_geo32, c->d_hgt, c->d_ereg, c->d_rscale, c->d_phi,
                          c->d_dirty, c->d_act, c->d_wake, c->d_wpush, c->d_if_l, c->d_ifm, c->d_inbox, c->d_if_fo,

@@ -888,3 +888,28 @@ def test_device_memory_of_a_context_is_what_its_kernels_read():
     i = p.info
     need = 81 * i["ne_global"] + 89 * i["ncopy"] + 68 * i["n_iface_copies"]
     assert used <= need + (8 << 20), (used, need)
+
+
+@pytest.mark.parametrize("block,max_nn", [(256, 150), (256, 450), (512, 40), (512, 320), (512, 900), (512, 1300)])
+def test_lists_of_few_waves_change_nothing(block, max_nn):
+    """sweeps listed by few waves (a grid that the units fill, small submeshes)
+    and by all waves (a grid that they do not): bitwise the same maps, on
+    submeshes below, between and above the two sizes per wave, at one and at
+    several instances a unit, and within the oracle's tolerance"""
+    cfg = cases.scaled(cases.SLAB, 4)
+    m, om = cases.box(cfg, seed=6)
+    p = F.Pack(m, F.PART_RCB, max_nn=max_nn, seed=6)
+    n_inst = 7
+    srcs = [cases.pacing_sites(cfg, 1 + k % 3, seed=40 + k) for k in range(n_inst)]
+    maps = []
+    for grid, unit in ((16, 1), (16, 3), (65536, 1), (0, 2)):
+        s = F.Solver(p, n_instances=n_inst, block=block, grid=grid, unit=unit, window=2000.0, local_iters=3)
+        s.seed_batch(srcs, 0.0)
+        s.run()
+        maps.append([s.download(inst=i)[0] for i in range(n_inst)])
+        s.close()
+    for got in maps[1:]:
+        for a, b in zip(maps[0], got):
+            assert np.array_equal(a, b)
+    ref, _ = O.fim_solve(om, srcs[0], variant=O.LOCAL_EXACT)
+    _check_fp32(maps[0][0], ref)
