@@ -97,12 +97,17 @@ struct WorkList {
   uint32_t *bcnt;   // nsub: queued instances per submesh
   uint32_t *bins;   // nsub x ninst instance ids
   uint32_t *plan;   // work units
-  uint32_t *cnt;    // [0] units, [1] queued pairs, [2..9] per-XCD unit counters,
-                    // [10] number of the iteration that works through the list
+  uint32_t *cnt;    // [0] units, [1] queued pairs, [2] number of the iteration that
+                    // works through the list, from kGrab per-XCD unit counters
 };
 
 constexpr uint32_t kXcd = 8;
-constexpr uint32_t kIterWord = 10;
+constexpr uint32_t kIterWord = 2;
+// A unit counter has a 128 B line to itself: with all eight and the unit count
+// in one line, the XCDs' accesses to it limited launches of many small units (357
+// maps on 128 submeshes, one instance a unit: 66.2 ms, with lines of their own
+// and the own counter asked first 34.6; 395 maps on 127: 77.0 -> 32.5).
+constexpr uint32_t kCntLine = 32, kGrab = kCntLine, kCntWords = kGrab + kXcd * kCntLine;
 
 // Queue flags of the items of iteration k: act = 4 (k + 1) + why, so a flag
 // needs no clearing; kPushed outranks kQueued.
@@ -191,7 +196,7 @@ __global__ __launch_bounds__(1024) void k_conv_plan(PlanArgs a) {
     a.cnt[0] = base_sh;
     a.cnt[1] = items_sh;
   }
-  if (tid < kXcd) a.cnt[2 + tid] = 0u;
+  if (tid < kXcd) a.cnt[kGrab + kCntLine * tid] = 0u;
 }
 
 struct ConvArgs {
@@ -266,32 +271,38 @@ struct UnitCursor {
   uint32_t s = 0, base = 0, n_in = 0, i = 0;
   bool first = true;
 
-  // a further unit from the eighths' counters (own eighth first), U if none is
-  // left.  The first wave looks at all eight at once: one round trip for the
-  // workgroup that finds nothing (one after the other took 6 us, at the end of
-  // every launch); when no eighth has more units than workgroups, none.
+  // a further unit from the eighths' counters, U if none is left.  The own
+  // eighth's counter is asked alone: most units come from it, and eight reads
+  // for each unit cost launches of many small units 4 %.  When it has none left,
+  // the first wave looks at all eight at once (one after the other took 6 us, at
+  // the end of every launch); when no eighth has more units than workgroups, no
+  // counter is asked.
   __device__ static uint32_t fetch(const uint32_t *cnt, uint32_t U, uint32_t *slot) {
     const uint32_t G = gridDim.x;
     if ((U + kXcd - 1) / kXcd <= G / kXcd) return U;
     if (threadIdx.x < 64) {
-      uint32_t *grab = const_cast<uint32_t *>(cnt) + 2;
       const uint32_t y = (blockIdx.x + threadIdx.x) % kXcd;
+      uint32_t *grab = const_cast<uint32_t *>(cnt) + kGrab + kCntLine * y;
       const UnitRange R = xcd_range(U, y, G);
       const uint32_t dyn = R.b + R.nb;
       uint32_t got = U;
-      for (;;) {
+      if (threadIdx.x == 0 && dyn < R.e) {
+        const uint32_t v = dyn + atomicAdd(grab, 1u);
+        if (v < R.e) got = v;
+      }
+      got = __builtin_amdgcn_readfirstlane(got);
+      while (got == U) {
         // a plain read of the counter skips exhausted eighths without an atomic
         const bool open = threadIdx.x < kXcd && dyn < R.e &&
-                          dyn + __hip_atomic_load(&grab[y], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < R.e;
+                          dyn + __hip_atomic_load(grab, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < R.e;
         const uint64_t m = __ballot(open);
         if (m == 0) break;
         const int w = __ffsll((unsigned long long)m) - 1;
         if ((int)threadIdx.x == w) {
-          const uint32_t v = dyn + atomicAdd(&grab[y], 1u);
+          const uint32_t v = dyn + atomicAdd(grab, 1u);
           if (v < R.e) got = v;
         }
         got = __shfl(got, w);
-        if (got < U) break;
       }
       if (threadIdx.x == 0) *slot = got;
     }
@@ -347,6 +358,7 @@ __device__ inline uint32_t start_iteration() {
       if (k->cur.cnt[0] > 0) atomicAdd(&k->stats[3], 1ull);
     }
     if (k->direct && threadIdx.x < kIterWord) k->old_cnt[threadIdx.x] = 0u;
+    if (k->direct && threadIdx.x < kXcd) k->old_cnt[kGrab + kCntLine * threadIdx.x] = 0u;
   }
   return iter;
 }
@@ -2904,12 +2916,12 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->d_act = dalloc<uint32_t>(2 * nss, ow);
         c->d_wake = dalloc<float>(nss, ow);
         c->d_wpush = dalloc<float>(2 * nss, ow);
-        c->d_cnt = dalloc<uint32_t>(48, ow);  // 16 words per list
+        c->d_cnt = dalloc<uint32_t>(3 * kCntWords, ow);
         for (int k = 0; k < 3; ++k) {
           c->wl[k].bcnt = dalloc<uint32_t>(c->nsub, ow);
           c->wl[k].bins = dalloc<uint32_t>(nss, ow);
           c->wl[k].plan = dalloc<uint32_t>((size_t)c->nsub * c->maxch, ow);
-          c->wl[k].cnt = c->d_cnt + 16 * k;
+          c->wl[k].cnt = c->d_cnt + kCntWords * k;
         }
         c->d_rscale = dalloc<float>(4 * (size_t)c->ninst, ow);
         c->d_tmpf = dalloc<float>(c->nn, ow);
@@ -3081,7 +3093,7 @@ int fim_reset(fim_ctx *c) {
       f.add(c->d_act, 2 * nss, 0u);
       f.add(c->d_wake, nss, F_INF);
       f.add(c->d_wpush, 2 * nss, F_INF);
-      f.add(c->d_cnt, 48, 0u);
+      f.add(c->d_cnt, 3 * kCntWords, 0u);
       f.add(c->d_start, c->ninst, 0u);
       c->next_iter = 0;
       for (int k = 0; k < 3; ++k) f.add(c->wl[k].bcnt, c->nsub, 0u);
