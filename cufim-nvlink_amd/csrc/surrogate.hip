@@ -882,7 +882,9 @@ struct fim_nn {
   // gradient; more goes the pageable way), and its device address
   unsigned char *stage = nullptr, *stage_d = nullptr;
   size_t stage_n = 0;
-  float *xin = nullptr;  // given rows, or the parameters of a chunk of solves
+  // given rows, or the parameters of a chunk of solves: in the place of the
+  // partial gradients, which are written once the chain kernel has read the rows
+  float *xin = nullptr;
   float *tgt = nullptr, *out = nullptr, *parts = nullptr, *tp = nullptr;
   uint32_t nsplit = 1;  // row spans of the weight gradients (partial sums)
   // dataset
@@ -1120,11 +1122,11 @@ int fim_nn_create(const fim_mesh *mesh, const fim_nn_opts *o, fim_nn **out) {
       for (int l = 0; l < NL; ++l) n->dZ[l] = nn_alloc<uint16_t>(n, (size_t)n->cap * HID);
       n->tgt = nn_alloc<float>(n, n->cap);
       n->out = nn_alloc<float>(n, n->cap);
-      n->xin = nn_alloc<float>(n, (size_t)n->cap * NIN);
       n->stage_n = std::max<size_t>(n->cap, NPAR + 1) * sizeof(float);
       HIPCHECK(hipHostMalloc((void **)&n->stage, n->stage_n, hipHostMallocDefault));
       HIPCHECK(hipHostGetDevicePointer((void **)&n->stage_d, n->stage, 0));
-      n->parts = nn_alloc<float>(n, (size_t)n->nsplit * PST);
+      n->parts = nn_alloc<float>(n, std::max((size_t)n->nsplit * PST, (size_t)n->cap * NIN));
+      n->xin = n->parts;
       n->tp = nn_alloc<float>(n, (size_t)(n->cap / TR) * NOUT);
       for (const void *k : {(const void *)k_mlp_chain, (const void *)k_mlp_infer})
         HIPCHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CHAIN_LDS));

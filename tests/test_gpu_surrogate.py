@@ -5,6 +5,8 @@ Tolerances: the oracle rounds to BF16 where the GPU does, so forward values
 agree to FP32-accumulation level (relative 1e-2 of the output spread) and
 gradients per parameter block to 2e-2 relative L2 with cosine > 0.999.
 Warm-started maps must equal cold maps within 1e-4 x max(T)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -143,6 +145,35 @@ def test_calls_around_the_staging_capacity(small_slab, rows):
     for name, sl in _blocks():
         assert np.linalg.norm(g[sl] - ref[sl]) <= 1e-2 * np.linalg.norm(ref[sl]), name
     nn.close()
+
+
+@pytest.mark.parametrize("max_batch", [1 << 18, 1 << 20])
+def test_device_memory_of_a_network(max_batch):
+    """given rows (64 B a row) have the place of the partial gradients (40 x
+    1.33 MB), whichever is larger, and a gradient comes out the same in either
+    case.  5,664 B a row of activations, 8 of targets and results, 16.25 of
+    tile sums; seven arrays of parameters; 8 MB for rounding and the rest, half of
+    what the rows of the smaller batch take."""
+    def free():  # of the HIP runtime that the library is linked with
+        f, total = C.c_size_t(), C.c_size_t()
+        assert F.lib().hipMemGetInfo(C.byref(f), C.byref(total)) == 0
+        return f.value
+
+    m = F.Mesh.gen_box(seed=3, **cases.CUBE)
+    rng = np.random.default_rng(4)
+    x = rng.uniform(-1, 1, (4160, M.NIN)).astype(np.float32)
+    t = rng.uniform(0.0, 2.0 * TS, 4160).astype(np.float32)
+    small = F.Surrogate(m, seed=1, max_maps=1, max_batch=4160)
+    want = small.gradient(x, t)
+    small.close()
+    before = free()
+    nn = F.Surrogate(m, seed=1, max_maps=1, max_batch=max_batch)
+    used = before - free()
+    got = nn.gradient(x, t)
+    nn.close()
+    assert got[0] == want[0] and np.array_equal(got[1], want[1])
+    need = int(5688.25 * max_batch) + max(40 * 1334528, 64 * max_batch) + 7 * 4 * M.NPARAMS
+    assert used <= need + (8 << 20), (used, need)
 
 
 def test_adam_steps_match_oracle(small_slab):
