@@ -2245,6 +2245,15 @@ __global__ __launch_bounds__(256) void k_compat_block(CompatBlockArgs a) {
   }
 }
 
+// per copy: its vertex if it has other copies, else kNoVertex
+__global__ __launch_bounds__(256) void k_compat_shared(const uint32_t *c2g, const uint32_t *g2c_dsp, uint32_t *cshared,
+                                                       uint32_t ncopy) {
+  for (uint32_t c = blockIdx.x * 256 + threadIdx.x; c < ncopy; c += gridDim.x * 256) {
+    const uint32_t v = c2g[c];
+    cshared[c] = g2c_dsp[v + 1] - g2c_dsp[v] > 1u ? v : kNoVertex;
+  }
+}
+
 // Start of a window.  sync_step2 (min over the copies of each shared vertex)
 // and the list of submeshes the window's pass has to run on: those whose
 // copies' own clocks are due (nexte; -inf when something is narrow or next)
@@ -2767,6 +2776,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
       c->g2c_dsp = p.g2c_dsp;
       c->g2c = p.g2c;
       auto &ow = c->owned;
+      Buffers tmp;  // what only kernels of this call read: until the stream is past them
       c->d_sub = dupload(p.sub, ow);
       {
         std::vector<uint2> e2(p.ne_global);
@@ -3014,14 +3024,12 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
           }
           c->d_csub = dupload(cs, ow);
           c->d_blob = dalloc<uint4>(total, ow);
-          Buffers tmp;
           const CompatBlockArgs ba{c->d_csub, c->d_e2n, dupload(p.n2e_dsp, tmp.v), dupload(p.n2e_le, tmp.v),
                                    dupload(p.n2e_pos, tmp.v),
                                    c->compat_geo ? reinterpret_cast<const uint4 *>(dupload(p.geo64, tmp.v)) : nullptr,
                                    c->d_blob, c->nsub};
           k_compat_block<<<(int)std::min<uint32_t>(c->nsub, 65536u), 256, 0, c->stream>>>(ba);
           HIPCHECK(hipGetLastError());
-          HIPCHECK(hipStreamSynchronize(c->stream));
         }
         if (!c->compat_geo) c->d_geo64 = dupload(p.geo64, ow);
         if (!c->compat_small) {
@@ -3037,16 +3045,9 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
         c->d_list = dalloc<uint32_t>(2 * (size_t)c->nsub, ow);
         c->d_mark = dalloc<uint32_t>(c->nsub, ow);
         c->d_lcnt = dalloc<uint32_t>(3, ow);
-        {
-          std::vector<uint32_t> sh(p.ncopy);
-          parallel_ranges((size_t)p.ncopy, 65536, [&](size_t b, size_t e) {
-            for (size_t i = b; i < e; ++i) {
-              const uint32_t v = p.c2g[i];
-              sh[i] = p.g2c_dsp[v + 1] - p.g2c_dsp[v] > 1 ? v : kNoVertex;
-            }
-          });
-          c->d_cshared = dupload(sh, ow);
-        }
+        c->d_cshared = dalloc<uint32_t>(c->ncopy, ow);
+        k_compat_shared<<<blocks_for(c->ncopy, 256), 256, 0, c->stream>>>(c->d_c2g, c->d_g2c_dsp, c->d_cshared, c->ncopy);
+        HIPCHECK(hipGetLastError());
         c->d_vrec = dalloc<uint32_t>(p.if_l.size(), ow);
         c->d_vcnt = dalloc<uint32_t>(c->nsub, ow);
         c->d_done = dalloc<unsigned long long>(1, ow);
