@@ -820,9 +820,9 @@ __device__ inline void wave_append(bool pred, uint32_t l, uint16_t *list, uint32
 // are used instead of spilled; with WPE <= 4 a wave works on two rounds of
 // pairs side by side (ILP).
 //
-// What bounds it: at 512 instances a launch, vector issue (73 % of one wave
-// instruction per SIMD and 4 cycles, 5.2e8 instructions in 1,172 us, 10.6 per
-// candidate), while waves wait 61 % of their cycles; with 128 instances, or a
+// What bounds it: at 512 instances a launch, vector issue (75 % of one wave
+// instruction per SIMD and 4 cycles, 5.2e8 instructions in 1,120 us, 10.5 per
+// candidate), while waves wait 60 % of their cycles; with 128 instances, or a
 // single one, those waits (65-70 %: L2 misses of records and times, LDS round
 // trips, barriers), vector issue being 41-50 %.  Cycles per item of the 2M slab (256 x 2
 // instances, 2816 copies; a single solve, 1024 copies): staging 24k / 6.9k,
@@ -2193,8 +2193,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 
 // Assembles the submeshes' blocks (CompatSub), one workgroup per submesh, from
 // the plain arrays.  On the host, and copied from there, the 144 MB of the 2M-tet
-// slab took 10 ms more of a context's creation (20 against 10; 8.5 with the
-// general kernel alone).
+// slab took 10 ms more of a context's creation (20 against 9 to 10; 8.2 with the
+// general kernel alone; this kernel takes 0.1).
 struct CompatBlockArgs {
   const CompatSub *csub;
   const uint2 *e2n;

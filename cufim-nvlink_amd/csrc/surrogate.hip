@@ -196,8 +196,9 @@ __device__ inline void tile_product(const uint16_t *Ts, const uint16_t *__restri
 // across layers and barriers: b holds the first DEEP steps of this layer's
 // weights on entry and of `next`'s on return.  170 registers, so two waves a
 // SIMD; with the Z of the backward loaded before the product as well, the
-// training kernel takes 167 against 175 us for 65,536 rows and 47 against
-// 61 us for 4,160 (four waves a SIMD, two steps); eight steps 169 and 47.
+// training kernel took 167 against 175 us for 65,536 rows and 47 against
+// 61 us for 4,160 (four waves a SIMD, two steps), eight steps 169 and 47, all on
+// one device; others take 156 to 169 us for the same code.
 // Inference, whose epilogue is shorter, is faster with four waves (267
 // against 310 us for 362,894 rows).
 constexpr int DEEP = 4;
@@ -280,8 +281,8 @@ struct ChainArgs {
 //     dZ_l in LDS; every dZ_l goes to HBM in the k-step layout.
 // Rounding to BF16 where the separate-kernel formulation stores values:
 // Z, H and dZ; SiLU'(Z) of the stored Z.
-// At 65,536 rows 372 MB out and 218 MB in, in 157 us (3.8 TB/s): memory and the
-// two barriers a layer bound it (86.4 GFLOP, 0.55 PFLOP/s).
+// At 65,536 rows 372 MB out and 220 MB in, in 156 to 169 us by device (3.5 to 3.8
+// TB/s): memory and the two barriers a layer bound it (86.4 GFLOP, 0.51 to 0.55 PFLOP/s).
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mlp_chain(ChainArgs a) {
   extern __shared__ __align__(16) unsigned char chain_lds[];
   uint16_t *Ts = reinterpret_cast<uint16_t *>(chain_lds);
@@ -586,7 +587,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 // waves of 32 x 16 (K = 16: the inputs; the other half of the 32-wide product
 // repeats them and is dropped).  Layer 0's workgroups also add up their span's
 // share of the output-layer gradient and the loss.  At 65,536 rows it reads
-// 373 MB and writes 53 in 97 us (4.4 TB/s, of 4.7 TB/s that a large copy reaches).
+// 373 MB and writes 53 in 96 to 99 us (4.3 to 4.4 TB/s, of 4.7 TB/s that a large copy reaches).
 // ---------------------------------------------------------------------------
 struct WGradArgs {
   const uint16_t *dZ[NL];   // k-step layout, HID columns
