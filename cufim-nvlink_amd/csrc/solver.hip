@@ -23,7 +23,7 @@
 //    units; otherwise an iteration is one launch.  Each
 //    instance's time window counts from its own start iteration, so a
 //    converged instance can be recycled and seeded again mid-run.
-//    Iterations are captured in a hipGraph; the host reads one counter per
+//    Iterations are recorded in a hipGraph; the host reads one counter per
 //    graph launch.
 //
 //  compat (FP64, reference local update): one workgroup per submesh runs the
@@ -2448,9 +2448,11 @@ struct fim_ctx {
   uint32_t *d_tmpu = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
+  hipGraphNode_t node = nullptr;  // the last one, while the graph is built
+  bool building = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t evc = nullptr;  // end of an iteration chunk's read-back
-  std::vector<hipEvent_t> kev;  // profile: events around each captured compute launch
+  std::vector<hipEvent_t> kev;  // profile: events around each compute launch
   ConvArgs ca{};
   CompatArgs xa{};
   uint32_t lds_conv = 0, lds_compat = 0;
@@ -2498,9 +2500,27 @@ const void *conv_kernel_ptr(const fim_ctx *c) {
   }
 }
 
+// a kernel of an iteration: into the context's stream or, while its graph is
+// built, as the graph's next node
+void launch(fim_ctx *c, const void *f, dim3 grid, dim3 block, void **args, uint32_t lds) {
+  if (!c->building) {
+    HIPCHECK(hipLaunchKernel(f, grid, block, args, lds, c->stream));
+    return;
+  }
+  hipKernelNodeParams n{};
+  n.func = const_cast<void *>(f);
+  n.gridDim = grid;
+  n.blockDim = block;
+  n.kernelParams = args;  // copied by the call
+  n.sharedMemBytes = lds;
+  hipGraphNode_t node;
+  HIPCHECK(hipGraphAddKernelNode(&node, c->graph, c->node ? &c->node : nullptr, c->node ? 1 : 0, &n));
+  c->node = node;
+}
+
 void launch_conv_compute(fim_ctx *c, const ConvArgs &a) {
   void *args[] = {const_cast<ConvArgs *>(&a)};
-  HIPCHECK(hipLaunchKernel(conv_kernel_ptr(c), dim3(c->grid), dim3(c->block), args, c->lds_conv, c->stream));
+  launch(c, conv_kernel_ptr(c), dim3(c->grid), dim3(c->block), args, c->lds_conv);
 }
 
 void set_lds_attr(fim_ctx *c) {
@@ -2535,8 +2555,8 @@ int blocks_for(size_t n, int bs) { return (int)std::max<size_t>(1, std::min<size
 void launch_plan(fim_ctx *c, int l, int z) {
   PlanArgs pa{c->wl[l].bcnt, c->wl[l].plan, c->wl[l].cnt, z >= 0 ? c->wl[z].bcnt : nullptr,
               c->nsub, c->unit, c->maxch};
-  k_conv_plan<<<1, 1024, 0, c->stream>>>(pa);
-  HIPCHECK(hipGetLastError());
+  void *args[] = {&pa};
+  launch(c, (const void *)k_conv_plan, dim3(1), dim3(1024), args, 0);
 }
 
 // one global iteration k: work lists rotate over three buffers; iteration k
@@ -2555,17 +2575,24 @@ void enqueue_iteration(fim_ctx *c, int k, bool timed) {
   if (!c->direct_plan) launch_plan(c, q, p);
 }
 
+// The iterations as a chain of kernel nodes.  (Captured from the stream, they
+// failed, and so did the other's call, where another thread used the null
+// stream meanwhile, for instance to create a context.)
 void build_graph(fim_ctx *c) {
-  HIPCHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+  HIPCHECK(hipGraphCreate(&c->graph, 0));
+  c->building = true;
+  c->node = nullptr;
   try {
     for (int i = 0; i < c->graph_iters; ++i) enqueue_iteration(c, i, false);
+    c->building = false;
+    HIPCHECK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
   } catch (...) {
-    hipGraph_t g;
-    (void)hipStreamEndCapture(c->stream, &g);
+    c->building = false;
+    (void)hipGraphDestroy(c->graph);
+    c->graph = nullptr;
+    c->gexec = nullptr;
     throw;
   }
-  HIPCHECK(hipStreamEndCapture(c->stream, &c->graph));
-  HIPCHECK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
 }
 
 // the list that the next run starts on, for kernels between runs
@@ -2746,7 +2773,7 @@ int fim_create(const fim_pack *pk, const fim_opts *o, fim_ctx **out) {
       HIPCHECK(hipSetDevice(c->dev));
       (void)noalloc_scratch(c->dev);  // once per device: fim_support_noalloc's scratch
       // CUFIM_DIRECT_LAUNCH=1 launches the iterations' kernels directly instead
-      // of replaying a captured graph (the same kernel sequence): for tools
+      // of replaying the graph of them (the same kernel sequence): for tools
       // that cannot trace graph launches
       {
         const char *dl = std::getenv("CUFIM_DIRECT_LAUNCH");

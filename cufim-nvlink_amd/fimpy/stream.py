@@ -14,7 +14,7 @@ def stream_solve(solver, sets, scales=None, on_map=None, check_iters=6, max_iter
     on_map(solve_index, inst) is called for every converged map before its
     instance is reused.  Returns the number of global iterations run, as the
     device counts them (iterations that processed work; fim_advance runs
-    whole captured graphs, so one call may run more than check_iters);
+    whole graphs, so one call may run more than check_iters);
     max_iters caps that count."""
     n = solver.n_instances
     slot = [-1] * n

@@ -190,7 +190,7 @@ typedef struct {
                          /* converge mode, 256 in compat mode)               */
   int32_t local_iters;   /* max local iterations per activation (0 = until
                             locally converged)                              */
-  int32_t graph_iters;   /* global iterations per captured graph, rounded up
+  int32_t graph_iters;   /* global iterations per graph, rounded up
                             to a multiple of 3 (0 = 6)                      */
   int32_t grid;          /* workgroups of the persistent kernels (0 = auto)  */
   double eps_rel;        /* convergence threshold (0 = 1e-6, reference)      */
@@ -273,7 +273,7 @@ int fim_step(fim_ctx *c, double phi_start, double cur_time, double dt,
 int fim_run(fim_ctx *c, int32_t max_iters, int32_t *iters);
 /* Continuous batching (no counterpart in the reference, which solves one map
  * per process).  fim_advance runs at least `iters` global iterations (whole
- * captured graphs) or until nothing is queued, without FIM_ENOCONV; *left
+ * graphs) or until nothing is queued, without FIM_ENOCONV; *left
  * (may be NULL) receives the queued work units left.  Device counters
  * accumulate until a call with reset_stats != 0.  fim_active writes, per
  * instance, 1 if it still has queued work and 0 if its map is converged.

@@ -867,6 +867,36 @@ def test_contexts_made_at_once_share_a_pack():
         assert g is not None and np.array_equal(g, want)
 
 
+def test_contexts_come_and_go_while_others_run():
+    """distinct contexts are independent: threads that create a context, build
+    its graph in the first run and destroy it, again and again, beside each
+    other get the maps of one context alone"""
+    import threading
+    cfg = cases.scaled(cases.SLAB, 8)
+    m, _ = cases.box(cfg, seed=9)
+    src = cases.pacing_sites(cfg, 2, seed=9)
+    p = F.Pack(m, F.PART_RCB, max_nn=300, seed=9)
+    want = _converge(m, p, src)[0]
+    bad, gate = [], threading.Barrier(6)
+
+    def work(i):
+        gate.wait()
+        try:
+            for k in range(12):
+                n = 1 + (i + k) % 4  # with and without a plan kernel
+                if not np.array_equal(_converge(m, p, src, n_instances=n)[0], want):
+                    bad.append((i, k, n))
+        except F.FimError as e:
+            bad.append((i, str(e)))
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, bad
+
+
 def test_device_memory_of_a_context_is_what_its_kernels_read():
     """an unstaged context keeps 81 B an element (node ids 8, region 1,
     geometry 24, record 48), 89 B a copy (ids 12, time 4, flag 1, adjacency 68,
